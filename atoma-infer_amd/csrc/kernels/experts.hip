@@ -12,18 +12,18 @@
 //                 gets inside its expert's range is not fixed; no result depends on it, since every row of a product
 //                 is computed by itself;
 //   expert_gemm   C[row(slot)] = (scale[slot] * A[src(slot)]) . W[expert]^T for all slots, tile by tile: true float32
-//                 multiply-adds over float32 or bfloat16 operands, K in ascending order, so a row's result does not
-//                 depend on the batch around it.  src is the slot's token (first product: the token's input, times its
+//                 multiply-adds (gemm_f32_tile.h) over float32 or bfloat16 operands, every row's sums in the same
+//                 order, so a row's result does not depend on the batch around it.  src is the slot's token (first product: the token's input, times its
 //                 score) or the slot itself (second product); the second product writes choice c of token t to row
 //                 c * T + t, so that the choices of a token lie in planes which the next norm adds in order.
 //                 act = 2 squares what is positive of a result and drops the rest (experts without a gate: relu^2);
 //                 out_scale[slot] multiplies a result (experts whose weight applies to their output).
-#include "common.h"
 #include "gate_act.h"
+#include "gemm_f32_tile.h"
 
 using namespace atoma;
 
-constexpr int kTileM = 64, kTileN = 64, kStepK = 16;
+constexpr int kTileM = 64, kTileN = 64;
 
 // Up to 64 experts: lane e holds expert e and counts the experts that go before it (a larger score, or the same and a
 // lower index), which is its place; the scores of the others come through scalar registers, one after the other, and no
@@ -233,67 +233,49 @@ route_group_kernel(const int32_t* __restrict__ ids, int n_slots, int experts, in
   for (int s = threadIdx.x; s < n_slots; s += 1024) perm[atomicAdd(&cursor[ids[s]], 1)] = s;
 }
 
-template <typename TA, typename TW, typename TC>
+template <bool VEC, typename TA, typename TW, typename TC>
 __global__ void __launch_bounds__(256)
 expert_gemm_kernel(const TA* __restrict__ a, int lda, int a_div, const float* __restrict__ scale,
                    const TW* __restrict__ w, TC* __restrict__ c, int ldc, int N, int K,
                    const int32_t* __restrict__ perm, const int32_t* __restrict__ offsets,
                    const int32_t* __restrict__ tiles, int top, int plane_rows, int act,
                    const float* __restrict__ out_scale) {
-  __shared__ float as[kStepK][kTileM + 4];
-  __shared__ float ws[kStepK][kTileN + 4];
-  __shared__ int32_t slot_of[kTileM];
+  __shared__ __attribute__((aligned(16))) float lds[2 * (kTileM + kTileN) * kF32Row];
   const int e = tiles[2 * blockIdx.y];
   if (e < 0) return;
   const int row0 = tiles[2 * blockIdx.y + 1], row_end = offsets[e + 1];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
   const int n0 = blockIdx.x * kTileN;
-  if (tid < kTileM) slot_of[tid] = row0 + tid < row_end ? perm[row0 + tid] : -1;
-  __syncthreads();
   const TW* we = w + (size_t)e * N * K;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kStepK) {
+  auto slot_of = [&](int r) { return row0 + r < row_end ? perm[row0 + r] : -1; };
+  f32x4_t acc[kTileN / 32][kTileM / 32];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int el = tid + i * 256;
-      const int r = el >> 4, kk = el & 15, k = k0 + kk;
-      const int slot = slot_of[r];
-      float av = 0.f;
-      if (slot >= 0 && k < K) {
-        av = to_f32(a[(size_t)(slot / a_div) * lda + k]);
-        if (scale) av *= scale[slot];
-      }
-      as[kk][r] = av;
-      ws[kk][r] = (n0 + r < N && k < K) ? to_f32(we[(size_t)(n0 + r) * K + k]) : 0.f;
-    }
-    __syncthreads();
+  for (int i = 0; i < kTileN / 32; ++i)
 #pragma unroll
-    for (int kk = 0; kk < kStepK; ++kk) {
-      float av[4], wv[4];
+    for (int j = 0; j < kTileM / 32; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32_tile<kTileM, kTileN, VEC, TA, TW>(
+      lds, K,
+      [&](int r) {
+        const int slot = slot_of(r);
+        return slot >= 0 ? a + (size_t)(slot / a_div) * lda : nullptr;
+      },
+      [&](int r) { return n0 + r < N ? we + (size_t)(n0 + r) * K : nullptr; },
+      [&](int r) { return scale != nullptr ? scale[slot_of(r)] : 1.f; }, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = as[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wv[j] = ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int slot = slot_of[ty * 4 + i];
+  for (int j = 0; j < kTileM / 32; ++j) {
+    const int slot = slot_of((wave >> 1) * (kTileM / 2) + j * 16 + (lane & 15));
     if (slot < 0) continue;
     const size_t row = plane_rows > 0 ? (size_t)(slot % top) * plane_rows + slot / top : (size_t)slot;
     const float os = out_scale != nullptr ? out_scale[slot] : 1.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      float v = acc[i][j];
-      if (act == 2) v = v > 0.f ? v * v : 0.f;
-      if (n < N) c[row * ldc + n] = from_f32<TC>(v * os);
-    }
+    for (int i = 0; i < kTileN / 32; ++i)
+#pragma unroll
+      for (int l = 0; l < 4; ++l) {
+        const int n = n0 + (wave & 1) * (kTileN / 2) + i * 16 + (lane >> 4) * 4 + l;
+        float v = acc[i][j][l];
+        if (act == 2) v = v > 0.f ? v * v : 0.f;
+        if (n < N) c[row * ldc + n] = from_f32<TC>(v * os);
+      }
   }
 }
 
@@ -579,15 +561,23 @@ extern "C" int atoma_expert_gemm(const void* a, int a_dtype, int lda, int a_div,
   if (K <= 0 || lda < K || ldc < N || a_div <= 0 || top <= 0 || max_tiles > 65535 || (act != 0 && act != 2))
     return ATOMA_ERR_SHAPE;
   dim3 grid((N + kTileN - 1) / kTileN, max_tiles), block(256);
-#define ATOMA_EG(TA, TW, TC)                                                                                       \
-  hipLaunchKernelGGL((expert_gemm_kernel<TA, TW, TC>), grid, block, 0, stream, (const TA*)a, lda, a_div, scale,     \
+#define ATOMA_EG_(V, TA, TW, TC)                                                                                   \
+  hipLaunchKernelGGL((expert_gemm_kernel<V, TA, TW, TC>), grid, block, 0, stream, (const TA*)a, lda, a_div, scale, \
                      (const TW*)w, (TC*)c, ldc, N, K, perm, offsets, tiles, top, plane_rows, act, out_scale)
+  // (pieces of four values: at most 16 bytes)
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0;
+#define ATOMA_EG(TA, TW, TC)                \
+  do {                                      \
+    if (vec) ATOMA_EG_(true, TA, TW, TC);   \
+    else ATOMA_EG_(false, TA, TW, TC);      \
+  } while (0)
   if (a_dtype == kF32 && w_dtype == kF32 && c_dtype == kF32) ATOMA_EG(float, float, float);
   else if (a_dtype == kF32 && w_dtype == kBF16 && c_dtype == kF32) ATOMA_EG(float, bf16_t, float);
   else if (a_dtype == kBF16 && w_dtype == kBF16 && c_dtype == kF32) ATOMA_EG(bf16_t, bf16_t, float);
   else if (a_dtype == kBF16 && w_dtype == kBF16 && c_dtype == kBF16) ATOMA_EG(bf16_t, bf16_t, bf16_t);
   else return ATOMA_ERR_DTYPE;
 #undef ATOMA_EG
+#undef ATOMA_EG_
   ATOMA_LAUNCH_CHECK();
   return 0;
 }

@@ -2,7 +2,7 @@
 
 Which kernel runs is decided by the operands, never by the model:
 
-* any float32 operand -> the true float32 kernel (plain FMAs, no matrix-core mode);
+* any float32 operand -> the true float32 kernels (float32 multiply-adds, no reduced-precision mode);
 * bfloat16 x bfloat16 -> the hand-written MFMA kernels where their shape conditions hold (skinny products that
   stream the weight once, and float32-output products for logits), the library product (hipBLASLt through
   ``torch.matmul``, as the reference uses cuBLAS through candle for its linears: models/src/llama.rs:269-271,

@@ -103,6 +103,20 @@ def test_gemm_generic(m, n, k, adt, wdt, cdt):
     assert (c2.double().cpu() - want2).abs().max() <= tol * want2.abs().max()
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 4096, 64), (17, 4112, 544), (33, 31, 96), (64, 100, 2048), (65, 130, 256), (200, 70, 4128),
+                                   (300, 5000, 36), (1000, 1030, 100), (2049, 2047, 68), (4100, 2000, 33)])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_gemm_generic_kernels(m, n, k, wdt):
+    """The streaming kernel (blocks of 16, 32, 64 rows, K split into uneven shares) and the tiles of 64 and of 128, with
+    rows, columns and values of K left over.  A float32 sum of k products in any order is within k 2^-24 of the sum of
+    their absolute values."""
+    from atoma_infer_amd.kernels import ops
+    a, w = rnd(m, k, seed=1), rnd(n, k, dtype=wdt, seed=2)
+    c = ops.gemm_generic(a, w, torch.float32)
+    want = a.double() @ w.double().T
+    assert bool(((c.double() - want).abs() <= k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 48, 64])
 @pytest.mark.parametrize("n,k", [(16, 32), (100, 64), (3072, 2048), (2048, 8192), (1000, 96), (40000, 128),
                                  (70000, 64)])
