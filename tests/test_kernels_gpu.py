@@ -318,6 +318,39 @@ def test_paged_attention(nh, nkv, hd, page, window, entries, kind):
         row += c
 
 
+@pytest.mark.parametrize("page", [4, 5, 16, 24, 32])
+@pytest.mark.parametrize("hd,nh,nkv", [(40, 6, 2), (64, 8, 2), (136, 3, 1), (16, 17, 1)])
+def test_generic_attention_masks(hd, nh, nkv, page):
+    """Sixteen rows a workgroup from neighbouring tokens, across the ends of requests: against the plain formula, and what a
+    row does not see (a later token, another request) may be anything, NaN and infinities too.  (Blocks with such values are
+    added in another order: weights that sum to 1 over at most 50 values, so within 50 * 2^-24 of the largest value.)"""
+    from atoma_infer_amd.kernels import ops
+    starts, counts, window = [0, 21, 130], [37, 41, 3], 50
+    lens = [s + c for s, c in zip(starts, counts)]
+    t = sum(counts)
+    q = torch.randn(t, nh * hd, generator=torch.Generator().manual_seed(3))
+    outs = []
+    for spoil in (False, True):
+        def edit(ks, vs):
+            if spoil:
+                vs[0][10], ks[0][11], vs[0][12] = float("nan"), float("inf"), float("-inf")
+                vs[1][61] = float("nan")
+        ks, vs, kc, vc, bt = paged_setup(lens, nkv, hd, page, torch.float32, seed=hd, edit=edit)
+        ctx, out = FakeCtx(starts, counts), torch.empty(t, nh * hd, device=DEV)
+        ops.paged_attention_generic(q.to(DEV), kc, vc, out, bt, ctx.token_seq, ctx.positions, hd ** -0.5, window, page, nh, nkv, hd)
+        outs.append(out.cpu())
+        if not spoil:
+            row = 0
+            for e, (s, c) in enumerate(zip(starts, counts)):
+                want = plain_attention(q[row:row + c].view(c, nh, hd), ks[e], vs[e], s, hd ** -0.5, window, nh // nkv)
+                assert (out[row:row + c].double().cpu() - want.reshape(c, -1)).abs().max() < 2e-5 * want.abs().max()
+                row += c
+    clean = list(range(10)) + list(range(37, 37 + 40)) + list(range(78, 81))
+    largest = max(float(v[torch.isfinite(v)].abs().max()) for v in vs)
+    assert (outs[0][clean] - outs[1][clean]).abs().max() <= 50 * 2.0 ** -24 * largest
+    assert bool(outs[1][10].isnan().all()) and bool(outs[1][77].isnan().all())
+
+
 TWO_PIECE_CASES = [c for c in ATTN_CASES if c[2] <= 64] + [
     # groups of 1, 3, 8, 33 and 40 heads (tiles of 256, 255, 256, 264, 240 rows; the last pieces are short or half
     # empty), one token, a window, portions beside decoded tokens
