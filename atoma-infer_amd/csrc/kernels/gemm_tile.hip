@@ -1,0 +1,412 @@
+// bfloat16 x bfloat16 products on the matrix cores for many rows of activations (prompts, large batches):
+// X[M, K] * W[N, K]^T with float32 accumulation, in tiles of BM rows of X against BN rows of W a workgroup.
+//
+// Bound by the matrix cores, and behind them by LDS: a wave's tile of TM x TN blocks of 16 x 16 reads 1 KB of LDS a block
+// row and block column for TM * TN MFMAs.  So tiles are as large as the launch allows (256 x 256 by eight waves), and:
+//
+//   * both operands go from memory to LDS directly (buffer_load ... lds, 16 bytes a lane), S buffers of 64 values of K in
+//     turn, so that no register holds them on the way and S - 1 steps are in flight while one is multiplied;
+//   * a row of a buffer is 128 bytes and its eight 16-byte pieces lie in the order piece ^ (row % 8): a wave's LDS reads
+//     (16 rows, four pieces) then fall on different banks.  The loads do the permuting: lane l of a load fetches piece
+//     (l % 8) ^ (l / 8) of its row, since what it stores is always in lane order;
+//   * a step's fragments of 32 values of K are read while the MFMAs of the 32 before run, across the end of the step
+//     too: one barrier a step stands between the reads of its last fragments and those of the next step's first, with
+//     MFMAs on either side of it;
+//   * the first operand of the MFMA is W, so a lane's four results are neighbouring columns of one row of X: two pairs
+//     of a rotation, or (with W's rows in blocks of 16 gate rows and their 16 up rows) gate and up of the same output;
+//   * workgroups are numbered so that each of the eight XCDs, which take them in turn, gets a run of tiles that lie
+//     in a patch of four rows of tiles: its L2 then serves most of what they share (the gate-up product of Llama 1B
+//     with 2,048 rows 125 -> 119 us against rows of eight, its down product 72 -> 67).
+//
+// What leaves: float32 (whole, or a plane a K slice), bfloat16, the float32 residual rows with the sums added, silu(gate) *
+// up in bfloat16, or q rotated in bfloat16 and k, v in the paged cache.
+//
+// Needs K % 64 == 0, N % 16 == 0 and 16-byte aligned rows; the host wrapper checks and otherwise refuses.
+#include "common.h"
+#include "rope_store.h"
+
+using namespace atoma;
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+enum Epilogue : int { kOutF32 = 0, kOutBF16 = 1, kOutResid = 2, kOutSilu = 3, kOutRope = 4 };
+
+struct TileOut {
+  void* c;               // float32 [slices][M][ldc], bfloat16 [M][ldc], or the float32 residual rows [M][ldc]
+  int ldc;
+  size_t plane;          // elements between the planes of two K slices
+  RopeArgs rope;
+};
+
+// BM x BN: a workgroup's tile; WM x WN: its waves; S: LDS buffers.
+template <int BM_, int BN_, int WM_, int WN_, int S_>
+struct Tile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_, NW = WM * WN;
+  static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;                  // blocks of 16 of a wave
+  static constexpr int QX = BM / 8, XI = (QX + NW - 1) / NW;                  // loads of eight rows: a step's, a wave's
+  static constexpr int QW = BN / 8, WI = (QW + NW - 1) / NW;
+  static constexpr int XBUF = BM * 128, BUF = (BM + BN) * 128, LDS = S * BUF;  // bytes; X's rows, then W's
+  // what a wave may still have on its way when the next step has to be there: the S - 2 steps behind it
+  static constexpr int NEWER = (S - 2) * (XI + WI);
+  static_assert(S >= 2 && LDS <= 160 * 1024 && NEWER + XI + WI < 64, "");
+};
+
+// silu(g) * u on its way to bfloat16: the hardware's exponential and reciprocal (each within 1 ulp of float32), where expf and
+// a division cost a tile's epilogue 10 us (64 results a lane)
+__device__ __forceinline__ float silu_times(float g, float u) {
+  return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896f)) * u;
+}
+
+constexpr int kPatch = 4;      // rows of tiles in a patch
+
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+template <typename C>
+struct Frag { bf16x8 w[C::TN], x[C::TM]; };
+
+// Q loads of eight rows, I of them this wave's (one that has less than others repeats the last: the same bytes to the same
+// place)
+template <int Q, int I, int NW>
+__device__ __forceinline__ void issue(char* __restrict__ dst, rsrc_t src, int k, const uint32_t (&vo)[I], int wave) {
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)(dst + min(i * NW + wave, Q - 1) * 1024), 16, vo[i], k, 0, 0);
+}
+
+template <typename C>
+__device__ __forceinline__ void read(const char* __restrict__ rd, int half, uint32_t xr, uint32_t wr, int lane, Frag<C>& f) {
+  const uint32_t col = (uint32_t)((half * 4 + (lane >> 4)) ^ (lane & 7)) * 16;
+#pragma unroll
+  for (int i = 0; i < C::TN; ++i) f.w[i] = *reinterpret_cast<const bf16x8*>(rd + wr + i * 2048 + col);
+#pragma unroll
+  for (int j = 0; j < C::TM; ++j) f.x[j] = *reinterpret_cast<const bf16x8*>(rd + xr + j * 2048 + col);
+}
+
+template <typename C>
+__device__ __forceinline__ void multiply(const Frag<C>& f, f32x4 (&acc)[C::TN][C::TM]) {
+#pragma unroll
+  for (int j = 0; j < C::TM; ++j)
+#pragma unroll
+    for (int i = 0; i < C::TN; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[i], f.x[j], acc[i][j], 0, 0, 0);
+}
+
+// a read of LDS behind every few MFMAs
+template <typename C>
+__device__ __forceinline__ void interleave() {
+  constexpr int reads = C::TM + C::TN, per = C::TM * C::TN / reads > 0 ? C::TM * C::TN / reads : 1;
+#pragma unroll
+  for (int i = 0; i < reads; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, per, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x8, C::TM * C::TN, 0);
+}
+
+// Step s behind its barrier: f1 holds the last fragments of step s, rd is the buffer of step s + 1, wr that of step s, which
+// nobody reads any more and which the loads of step s + S (at byte k of the rows) go to.  (That the two pointers promise
+// not to overlap is what keeps the compiler from waiting for those loads before the reads.)
+template <typename C>
+__device__ __forceinline__ void step(const char* __restrict__ rd, char* __restrict__ wr, bool more, rsrc_t xb, rsrc_t wb, int k,
+                                     const uint32_t (&xo)[C::XI], const uint32_t (&wo)[C::WI], int wave, uint32_t xr, uint32_t wrow,
+                                     int lane, Frag<C>& f0, Frag<C>& f1, f32x4 (&acc)[C::TN][C::TM]) {
+  if (more) {
+    issue<C::QX, C::XI, C::NW>(wr, xb, k, xo, wave);
+    issue<C::QW, C::WI, C::NW>(wr + C::XBUF, wb, k, wo, wave);
+  }
+  read<C>(rd, 0, xr, wrow, lane, f0);
+  multiply<C>(f1, acc);
+  interleave<C>();
+  __builtin_amdgcn_sched_barrier(0);
+  read<C>(rd, 1, xr, wrow, lane, f1);
+  multiply<C>(f0, acc);
+  interleave<C>();
+}
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  const bf16x2 v = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+// The rotary epilogue of a wave's tile of ROWS x COLS sums, which lie in LDS row by row: rows from m0, columns from n0.
+// (Written out for the sums in registers, with four-byte stores and a trip to memory for every row's position and slot, it
+// took 13 us of 43 for Llama 1B with 2,048 rows; 9 of 37 now.)
+//   q and k: a lane takes sixteen columns of a row, eight rotation pairs: columns 2 i, 2 i + 1 become columns i of the
+//     head's lower and of its upper half; eight and eight of them leave as 16 bytes each, to the query's row or to the runs
+//     of the key tile, which holds a token's columns in eights;
+//   values: a lane takes a column of four rows; where those are neighbours in the value tile they leave together.
+// (hd is a multiple of 16, so sixteen columns from a multiple of 16 on lie in one head.)
+// Lane r holds row r's position, page and place in the page (page < 0: no cache write), asked for before the product: a trip
+// to memory every time round the loops is what they cannot afford.
+template <int ROWS, int COLS>
+__device__ __forceinline__ void rope_tile(const float* __restrict__ sums, int m0, int M, int n0, int N, int pos_of, int page_of,
+                                          int off_of, const RopeArgs& ra, uint16_t* __restrict__ q_out, int ldq, int lane) {
+  static_assert(ROWS <= 64, "a lane a row");
+  const int hd = ra.hd, half = hd >> 1, rotated = (ra.nh + ra.nkv) * hd;
+  constexpr int BLOCKS = COLS / 16;
+  const int live = min(BLOCKS, (N - n0) / 16), turned = min(live, max(0, rotated - n0) / 16);       // (N >= n0 here)
+#pragma unroll 1
+  for (int first = 0; first < ROWS * turned; first += 64) {
+    const int item = first + lane, r = item / turned, b = item - r * turned, m = m0 + r;
+    const int pos = __shfl(pos_of, r, 64), page = __shfl(page_of, r, 64), off = __shfl(off_of, r, 64);
+    if (r >= ROWS || m >= M) continue;
+    const int n = n0 + b * 16, head = n / hd, i0 = (n - head * hd) >> 1;
+    const f32x4* const cp = reinterpret_cast<const f32x4*>(ra.cos_t + (size_t)pos * half + i0);
+    const f32x4* const sp = reinterpret_cast<const f32x4*>(ra.sin_t + (size_t)pos * half + i0);
+    const f32x4 c[2] = {cp[0], cp[1]}, sn[2] = {sp[0], sp[1]};
+    const f32x4* const x = reinterpret_cast<const f32x4*>(sums + r * COLS + b * 16);
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const f32x4 v = x[p];
+      const float c0 = c[p >> 1][(p & 1) * 2], c1 = c[p >> 1][(p & 1) * 2 + 1], s0 = sn[p >> 1][(p & 1) * 2], s1 = sn[p >> 1][(p & 1) * 2 + 1];
+      lo[p] = pack_bf16(v[0] * c0 - v[1] * s0, v[2] * c1 - v[3] * s1);
+      hi[p] = pack_bf16(v[1] * c0 + v[0] * s0, v[3] * c1 + v[2] * s1);
+    }
+    if (head >= ra.nh && page < 0) continue;
+    uint16_t *to, *to_hi;
+    if (head < ra.nh) {
+      to = q_out + (size_t)m * ldq + (size_t)head * hd + i0;
+      to_hi = to + half;
+    } else {
+      uint16_t* const tile = ra.kcache + ((size_t)page * ra.nkv + (head - ra.nh)) * ra.page_size * hd;
+      to = tile + key_offset(off, i0, ra.page_size);
+      to_hi = tile + key_offset(off, i0 + half, ra.page_size);
+    }
+    *reinterpret_cast<uint4*>(to) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    *reinterpret_cast<uint4*>(to_hi) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  }
+  if (turned >= live) return;
+  const int columns = (live - turned) * 16;
+#pragma unroll 1
+  for (int first = 0; first < ROWS / 4 * columns; first += 64) {
+    const int item = first + lane, r = item / columns * 4, cc = item - item / columns * columns;
+    int page[4], off[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) page[t] = __shfl(page_of, r + t, 64), off[t] = __shfl(off_of, r + t, 64);
+    if (r >= ROWS || m0 + r >= M) continue;
+    const int n = n0 + turned * 16 + cc, head = (n - rotated) / hd, d = n - rotated - head * hd;
+    uint16_t v[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) v[t] = (uint16_t)pack_bf16(sums[(r + t) * COLS + turned * 16 + cc], 0.f);
+    auto place = [&](int t) {
+      return ra.vcache + ((size_t)page[t] * ra.nkv + head) * ra.page_size * hd + value_offset(d, off[t], hd, ra.page_size);
+    };
+    if ((ra.page_size & 3) == 0 && page[0] >= 0 && (off[0] & 3) == 0 && page[1] == page[0] && page[2] == page[0] &&
+        page[3] == page[0] && off[1] == off[0] + 1 && off[2] == off[0] + 2 && off[3] == off[0] + 3) {
+      *reinterpret_cast<uint2*>(place(0)) = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
+    } else {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (page[t] >= 0) *place(t) = v[t];
+    }
+  }
+}
+
+// at most n loads of this wave still on their way; reads: and none of its LDS reads
+template <int N, bool READS>
+__device__ __forceinline__ void wait() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((READS ? 0 : 15) << 8) | ((N >> 4) << 14));
+}
+__device__ __forceinline__ void meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+#endif
+
+template <typename C, int EPI>
+__global__ void __launch_bounds__(64 * C::NW, C::NW >= 8 ? 2 : 1)
+gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int ldx, int ldw, int k_len,
+                 TileOut out) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  // the tile: this XCD's run of the order, patches of kPatch rows of tiles, column by column
+  const int mt = (M + C::BM - 1) / C::BM, nt = (N + C::BN - 1) / C::BN;
+  const int share = (mt * nt) >> 3, rest = (mt * nt) & 7, xcd = blockIdx.x & 7;
+  const int id = xcd * share + min(xcd, rest) + (blockIdx.x >> 3);
+  const int patch = id / (kPatch * nt), pm = min(kPatch, mt - patch * kPatch), in = id - patch * kPatch * nt;
+  const int m0 = (patch * kPatch + in % pm) * C::BM, n0 = (in / pm) * C::BN;
+  const int k0 = blockIdx.y * k_len;
+
+  const int rows_x = min(C::BM, M - m0), rows_w = min(C::BN, N - n0);
+  // (rows past the end: the last one, never stored)
+  const int lr = lane >> 3;
+  const uint32_t piece = ((lane & 7) ^ lr) * 16;
+  uint32_t xo[C::XI], wo[C::WI];
+#pragma unroll
+  for (int i = 0; i < C::XI; ++i) xo[i] = (uint32_t)min(min(i * C::NW + wave, C::QX - 1) * 8 + lr, rows_x - 1) * ldx * 2 + piece;
+#pragma unroll
+  for (int i = 0; i < C::WI; ++i) wo[i] = (uint32_t)min(min(i * C::NW + wave, C::QW - 1) * 8 + lr, rows_w - 1) * ldw * 2 + piece;
+  const rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (size_t)m0 * ldx + k0), 0, ((rows_x - 1) * ldx + k_len) * 2, 0x00027000);
+  const rsrc_t wb = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * ldw + k0), 0, ((rows_w - 1) * ldw + k_len) * 2, 0x00027000);
+
+  f32x4 acc[C::TN][C::TM];
+#pragma unroll
+  for (int i = 0; i < C::TN; ++i)
+#pragma unroll
+    for (int j = 0; j < C::TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const uint32_t xr = (wm * (C::BM / C::WM) + r16) * 128, wr = C::XBUF + (wn * (C::BN / C::WN) + r16) * 128;
+
+  int pos_of = 0, page_of = -1, off_of = 0;
+  if constexpr (EPI == kOutRope) {
+    const int row = m0 + wm * (C::BM / C::WM) + lane;
+    if (lane < C::BM / C::WM && row < M) {
+      const int slot = out.rope.slot_mapping[row];
+      pos_of = out.rope.positions[row];
+      if (slot >= 0) page_of = slot / out.rope.page_size, off_of = slot - page_of * out.rope.page_size;
+    }
+  }
+
+  const int steps = k_len / 64;
+#pragma unroll
+  for (int s = 0; s < C::S; ++s)
+    if (s < steps) {
+      issue<C::QX, C::XI, C::NW>(lds + s * C::BUF, xb, s * 128, xo, wave);
+      issue<C::QW, C::WI, C::NW>(lds + s * C::BUF + C::XBUF, wb, s * 128, wo, wave);
+    }
+  if (C::S <= steps) wait<C::NEWER + C::XI + C::WI, false>();
+  else wait<0, false>();
+  meet();
+  Frag<C> f0, f1;
+  read<C>(lds, 0, xr, wr, lane, f0);
+  read<C>(lds, 1, xr, wr, lane, f1);
+  multiply<C>(f0, acc);
+  int cur = 0, nxt = C::BUF;
+  for (int s = 0; s + 1 < steps; ++s) {
+    // step s + 1 has landed, for this wave here and for all behind the barrier, and so are all reads of step s done
+    if (s + C::S <= steps) wait<C::NEWER, true>();
+    else wait<0, true>();
+    meet();
+    step<C>(lds + nxt, lds + cur, s + C::S < steps, xb, wb, (s + C::S) * 128, xo, wo, wave, xr, wr, lane, f0, f1, acc);
+    cur = nxt;
+    nxt = nxt + C::BUF == C::LDS ? 0 : nxt + C::BUF;
+  }
+  multiply<C>(f1, acc);
+
+  if constexpr (EPI == kOutRope) {
+    constexpr int ROWS = C::TM * 16, COLS = C::TN * 16;
+    static_assert(ROWS * COLS * 4 * C::NW <= 160 * 1024, "");
+    wait<0, true>();
+    meet();                  // everybody's reads of the last step are done
+    float* const sums = reinterpret_cast<float*>(lds) + wave * (ROWS * COLS);
+#pragma unroll
+    for (int j = 0; j < C::TM; ++j)
+#pragma unroll
+      for (int i = 0; i < C::TN; ++i) *reinterpret_cast<f32x4*>(sums + (j * 16 + r16) * COLS + i * 16 + kg * 4) = acc[i][j];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    const int nw = n0 + wn * COLS;
+    if (nw < N) rope_tile<ROWS, COLS>(sums, m0 + wm * ROWS, M, nw, N, pos_of, page_of, off_of, out.rope,
+                                          (uint16_t*)out.c, out.ldc, lane);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < C::TM; ++j) {
+    const int m = m0 + wm * (C::BM / C::WM) + j * 16 + r16;
+    const int nw = n0 + wn * (C::BN / C::WN);
+    if (m >= M) continue;
+    if constexpr (EPI == kOutSilu) {
+      uint16_t* const row = (uint16_t*)out.c + (size_t)m * out.ldc;
+#pragma unroll
+      for (int i = 0; i + 1 < C::TN; i += 2) {         // blocks of 16 gate rows, then the 16 up rows of the same outputs
+        if (nw + i * 16 >= N) continue;
+        const int n = (nw + i * 16) / 2 + kg * 4;
+        uint2 v;
+        __bf16* const o = reinterpret_cast<__bf16*>(&v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (__bf16)silu_times(acc[i][j][e], acc[i + 1][j][e]);
+        *reinterpret_cast<uint2*>(row + n) = v;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < C::TN; ++i) {
+        const int n = nw + i * 16 + kg * 4;
+        if (nw + i * 16 >= N) continue;                // (N is a multiple of 16: a block is there or is not)
+        const f32x4 v = acc[i][j];
+        if constexpr (EPI == kOutF32) {
+          *reinterpret_cast<f32x4*>((float*)out.c + blockIdx.y * out.plane + (size_t)m * out.ldc + n) = v;
+        } else if constexpr (EPI == kOutResid) {
+          f32x4* const p = reinterpret_cast<f32x4*>((float*)out.c + (size_t)m * out.ldc + n);
+          *p = *p + v;
+        } else {
+          uint2 u;
+          __bf16* const o = reinterpret_cast<__bf16*>(&u);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (__bf16)v[e];
+          *reinterpret_cast<uint2*>((uint16_t*)out.c + (size_t)m * out.ldc + n) = u;
+        }
+      }
+    }
+  }
+#endif
+}
+
+template <typename C, int EPI>
+static int launch(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
+                  hipStream_t stream) {
+  // (every device that the kernel is launched on has its own setting)
+  constexpr int lds = EPI == kOutRope && C::BM * C::BN * 4 > C::LDS ? C::BM * C::BN * 4 : C::LDS;      // (the rotary epilogue's sums)
+  const hipError_t e = hipFuncSetAttribute((const void*)gemm_tile_kernel<C, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return (int)e;
+  const int64_t tiles = (int64_t)((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
+  if (tiles > 0x7fffffff) return ATOMA_ERR_SHAPE;
+  hipLaunchKernelGGL((gemm_tile_kernel<C, EPI>), dim3((int)tiles, slices), dim3(64 * C::NW), lds, stream,
+                     (const uint16_t*)x, (const uint16_t*)w, M, N, ldx, ldw, K / slices, out);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+template <int EPI>
+static int pick(int tile, const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
+                hipStream_t stream) {
+  constexpr bool GATED = EPI == kOutSilu;
+  (void)GATED;
+#define ATOMA_TILE(...) return launch<Tile<__VA_ARGS__>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream)
+  switch (tile) {
+    case 0: if constexpr (EPI != kOutRope) ATOMA_TILE(256, 256, 2, 4, 2); break;      // (its sums do not fit LDS)
+    case 1: ATOMA_TILE(256, 128, 4, 2, 3);
+    case 2: ATOMA_TILE(128, 128, 2, 4, 4);
+    case 3: ATOMA_TILE(128, 64, 2, 2, 4);
+    case 4: if constexpr (!GATED) ATOMA_TILE(256, 160, 4, 2, 3); break;     // (a wave's blocks are not in pairs)
+    case 5: if constexpr (!GATED) ATOMA_TILE(256, 96, 4, 2, 3); break;
+  }
+#undef ATOMA_TILE
+  return ATOMA_ERR_SHAPE;
+}
+
+// x [M, K] and w [N, K] bfloat16.  kind: what leaves (see Epilogue); tile: which of the tiles above; slices: parts of K, a
+// float32 plane each (kind 0 only).  rope: positions, cos_t, sin_t, kcache, vcache, slot_mapping and sizes (kind 4 only).
+extern "C" int atoma_gemm_tile(const void* x, const void* w, void* c, int kind, int tile, int M, int N, int K, int ldx,
+                               int ldw, int ldc, int slices, const int32_t* positions, const float* cos_t, const float* sin_t,
+                               void* kcache, void* vcache, const int32_t* slot_mapping, int page_size, int nh, int nkv, int hd, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || slices <= 0 || K % (64 * slices) || N % 16 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || ldx > (1 << 21) ||
+      ldw > (1 << 21) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || (slices > 1 && kind != kOutF32) || slices > 65535 || ldc % 4 ||
+      ((uintptr_t)c & (kind == kOutF32 || kind == kOutResid ? 15 : 7)))
+    return ATOMA_ERR_SHAPE;
+  TileOut out{c, ldc, (size_t)M * ldc, 
+              RopeArgs{positions, cos_t, sin_t, (uint16_t*)kcache, (uint16_t*)vcache, slot_mapping, page_size, nh, nkv, hd}};
+  if (kind == kOutRope) {
+    if (N != (nh + 2 * nkv) * hd || hd % 16 || ldc < nh * hd || nh <= 0 || nkv <= 0 || page_size <= 0 || !positions || !cos_t ||
+        !sin_t || !kcache || !vcache || !slot_mapping || ldc % 8 ||
+        (((uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)c | (uintptr_t)cos_t | (uintptr_t)sin_t) & 15))
+      return ATOMA_ERR_SHAPE;
+    return pick<kOutRope>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
+  }
+  if (kind == kOutSilu) {
+    if (N % 32 || ldc < N / 2) return ATOMA_ERR_SHAPE;
+    return pick<kOutSilu>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
+  }
+  if (ldc < N) return ATOMA_ERR_SHAPE;
+  if (kind == kOutF32) return pick<kOutF32>(tile, x, w, M, N, K, ldx, ldw, slices, out, stream);
+  if (kind == kOutBF16) return pick<kOutBF16>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
+  if (kind == kOutResid) return pick<kOutResid>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
+  return ATOMA_ERR_SHAPE;
+}

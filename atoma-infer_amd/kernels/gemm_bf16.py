@@ -6,13 +6,16 @@
   output is wanted (logits), running it over blocks of 64 rows of x;
 * the library product (hipBLASLt through ``torch.mm``) for products with many rows of x (more than 64; more
   than 32 on large weights; more than 16 for float32 output), as the reference uses a library for its linears;
+  what parts ask for with an epilogue (``try_tile_*``, ``try_add_resid``, ``linear_planes``) goes to the tile kernel
+  instead wherever that is the quicker one;
 * nothing (None) when the shape fits neither: the caller then runs the float32 FMA kernel.
 """
 from __future__ import annotations
 
 import ctypes
 import dataclasses
-from typing import Optional
+import functools
+from typing import Optional, Tuple
 
 import torch
 
@@ -251,6 +254,125 @@ def _library_wins(m: int, n: int, k: int, out_dtype: torch.dtype) -> bool:
     return m > LIBRARY_MIN_M_WIDE and n * k >= (1 << 24)
 
 
+# -- tiles for many rows (csrc/kernels/gemm_tile.hip) ------------------------------------------------------------------
+TILE_F32, TILE_BF16, TILE_RESID, TILE_SILU, TILE_ROPE = range(5)
+# the kernel's tiles: (rows of x, rows of w, microseconds a workgroup spends beside its steps, microseconds a step of 64
+# values of K), measured on MI355X with a workgroup on each of the 256 CUs
+TILES = ((256, 256, 10.0, 1.37), (256, 128, 9.0, 0.88), (128, 128, 7.4, 0.503), (128, 64, 5.8, 0.34),
+         (256, 160, 9.0, 1.0), (256, 96, 7.0, 0.727))
+TILES_SILU = (0, 1, 2, 3)         # those with a wave's blocks of 16 rows of w in pairs
+TILES_ROPE = (1, 2, 3, 4, 5)      # those whose sums fit LDS
+TILE_CUS = 256
+TILE_MAX_SLICES = 8
+_tile_lib = None
+
+
+def tile_lib():
+    global _tile_lib
+    if _tile_lib is None:
+        _tile_lib = load_hip_module("gemm_tile")
+    return _tile_lib
+
+
+@functools.lru_cache(maxsize=4096)
+def tile_plan(m: int, n: int, k: int, kind: int, planes: bool = False) -> Tuple[int, int, float]:
+    """(tile, K slices, estimated microseconds) for x [m, k] @ w [n, k]^T: the tile whose rounds over the CUs are
+    shortest.  A round lasts as long as a workgroup does, so few large tiles lose to small ones where they leave CUs idle,
+    and with ``planes`` K may be cut into slices for the same reason; their planes then cost a write and a read."""
+    best = None
+    for tile, (bm, bn, fixed, per_step) in enumerate(TILES):
+        if (kind == TILE_SILU and tile not in TILES_SILU) or (kind == TILE_ROPE and tile not in TILES_ROPE):
+            continue
+        groups = -(-m // bm) * -(-n // bn)
+        slices = 1
+        while slices <= (TILE_MAX_SLICES if planes else 1) and k % (64 * slices) == 0:
+            steps = k // (64 * slices)
+            us = -(-groups * slices // TILE_CUS) * (fixed + steps * per_step)
+            us *= 0.8 + 0.2 * min(1.0, groups * slices / TILE_CUS)      # (a round that leaves CUs idle is quicker)
+            if slices > 1:
+                us += slices * m * n * 8 / 4e6
+            if (best is None or us < best[2]) and (slices == 1 or steps >= 4):
+                best = (tile, slices, us)
+            slices *= 2
+    return best
+
+
+def _library_us(m: int, n: int, k: int) -> float:
+    """Roughly what the library's product takes (microseconds): fitted to 65 to 4,096 rows at the layer shapes of the Llamas,
+    within a tenth of most."""
+    return 2.0 * m * n * k / 1.4e9 + 0.0028 * k + 4.0
+
+
+@functools.lru_cache(maxsize=4096)
+def _tile_wins(m: int, n: int, k: int, kind: int) -> bool:
+    """Whether the tile kernel takes a product that the library could take too, from the estimates of both.  Whole rounds
+    over the CUs are what decides it: with the sums added to the residual rows and the norm behind them, N 2,048 and K
+    8,192, 1,024 / 1,300 / 2,048 / 3,000 rows take 49 / 70 / 80 / 116 us against the library's 58 / 67 / 85 / 107.
+    A product that leaves gated or rotated saves the kernel that would do it, which the library's estimate counts:
+    gate-up of Llama 1B with SiLU-multiply, 80 / 300 / 1,024 / 2,048 rows, 16 / 32 / 58 / 108 us against 22 / 35 / 70 /
+    132 (at the 8B width 600 rows 181 against 158); q, k, v of Llama 1B with rotation and cache write, 200 / 2,048 rows,
+    20 / 37 us against 23 / 46, of Llama 3B 2,048 rows 69 against 82, of Llama 8B 120 against 106.  The rotary
+    epilogue costs a workgroup 7 us."""
+    rotary = kind == TILE_ROPE
+    tile, slices, us = tile_plan(m, n, k, kind, kind in (TILE_F32, TILE_RESID))
+    if rotary:
+        us += 7.0 * -(-(-(-m // TILES[tile][0]) * -(-n // TILES[tile][1])) // TILE_CUS)
+        return us <= 1.05 * (_library_us(m, n, k) + 9.0 + m * n * 1.2e-6)
+    if kind == TILE_SILU:
+        return us <= 1.22 * (_library_us(m, n, k) + 3.0 + m * n * 6.6e-7)
+    return us <= 1.1 * _library_us(m, n, k)
+
+
+def _tile_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.dim() == 2 and w.dim() == 2
+            and x.shape[0] > SKINNY_MAX_M and x.shape[1] == w.shape[1] and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0
+            and max(x.stride(0), w.stride(0)) <= 1 << 21 and _aligned(x) and _aligned(w))
+
+
+def tile_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: int, tile: int, slices: int = 1, rope=None) -> None:
+    """``out`` from x [M, K] @ w [N, K]^T by the tile kernel: float32 planes [slices, M, N] (or [M, N]), bfloat16 [M, N],
+    the float32 rows the product is added to, silu(gate) * up [M, N / 2], or rotated q [M, nh hd] (``rope``: positions,
+    cos, sin, kcache, vcache, slot_mapping, page_size, nh, nkv, hd)."""
+    m, k = x.shape
+    tensors, sizes = (rope[:6], rope[6:]) if rope is not None else ((None,) * 6, (0,) * 4)
+    _check(tile_lib().atoma_gemm_tile(_p(x), _p(w), _p(out), kind, tile, m, w.shape[0], k, x.stride(0), w.stride(0),
+                                      out.stride(-2), slices, *(_p(t) for t in tensors), *(int(v) for v in sizes),
+                                      _stream()), "gemm_tile")
+
+
+def try_tile_swiglu(x, w: torch.Tensor, act="silu") -> Optional[torch.Tensor]:
+    """``try_linear_swiglu`` for more rows than it takes, SiLU only: silu(gate) * up of x @ w^T, w [2 I, K] in blocks of 16
+    rows, by the tile kernel; None where that does not take the shape."""
+    if act != "silu" or isinstance(x, Begun) or w.shape[0] % 32 or not _tile_ok(x, w):
+        return None
+    (m, k), n = x.shape, w.shape[0]
+    if not _tile_wins(m, n, k, TILE_SILU):
+        return None
+    out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+    tile_product(x, w, out, TILE_SILU, tile_plan(m, n, k, TILE_SILU)[0])
+    return out
+
+
+def try_tile_rope(x, w: torch.Tensor, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
+                  vcache: torch.Tensor, slot_mapping: torch.Tensor, page_size: int, nh: int, nkv: int, hd: int,
+                  ) -> Optional[torch.Tensor]:
+    """``try_linear_rope`` for more rows than it takes: q rotated as the result, k and v in the cache, by the tile kernel;
+    None where that does not take the shape, or the library's product and the rotary kernel are quicker."""
+    if (isinstance(x, Begun) or not _tile_ok(x, w) or w.shape[0] != (nh + 2 * nkv) * hd or hd % 16
+            or any(t.data_ptr() % 16 for t in (cos, sin, kcache, vcache))
+            or kcache.dtype is not torch.bfloat16 or vcache.dtype is not torch.bfloat16
+            or cos.dtype is not torch.float32 or cos.shape[1] != hd // 2 or not cos.is_contiguous()
+            or not sin.is_contiguous() or not kcache.is_contiguous() or not vcache.is_contiguous()):
+        return None
+    (m, k), n = x.shape, w.shape[0]
+    if not _tile_wins(m, n, k, TILE_ROPE):
+        return None
+    out = torch.empty((m, nh * hd), dtype=torch.bfloat16, device=x.device)
+    tile_product(x, w, out, TILE_ROPE, tile_plan(m, n, k, TILE_ROPE)[0],
+                 rope=(positions, cos, sin, kcache, vcache, slot_mapping, page_size, nh, nkv, hd))
+    return out
+
+
 def _probe_mm_out_dtype() -> bool:
     """Whether this torch has ``mm(..., out_dtype=float32)`` for bfloat16 operands (float32 accumulation either way)."""
     doc = getattr(torch.mm, "__doc__", "") or ""
@@ -317,13 +439,22 @@ def _probe_addmm_out_dtype() -> bool:
 _ADDMM_OUT_DTYPE = _probe_addmm_out_dtype()
 
 
-def try_addmm_resid(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor) -> bool:
-    """``resid += x @ w^T`` by the library (hipBLASLt with beta = 1: the float32 sums of the product are added to the
-    float32 rows in place, so the product's own result is never written or read again), for products of more rows
-    than the streaming kernels take; False, nothing done, where that is not the choice."""
+def try_add_resid(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor) -> bool:
+    """``resid += x @ w^T`` for products of more rows than the streaming kernels take: the float32 sums of the product are
+    added to the float32 rows in place, so the product's own result is never written or read again.  By the tile kernel,
+    or by the library (hipBLASLt with beta = 1) for sizes that it does not take.  False, nothing done, where that is not
+    the choice: few rows, or rows for which float32 planes of K slices are (``linear_planes``)."""
     m = x.shape[0]
-    if not (_ADDMM_OUT_DTYPE and m > SKINNY_MAX_M and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16
+    if not (m > SKINNY_MAX_M and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16
             and resid.dtype is torch.float32 and resid.is_contiguous() and tuple(resid.shape) == (m, w.shape[0])):
+        return False
+    if _tile_ok(x, w) and _tile_wins(m, w.shape[0], x.shape[1], TILE_RESID):
+        tile, slices, _ = tile_plan(m, w.shape[0], x.shape[1], TILE_RESID, True)
+        if slices > 1:
+            return False
+        tile_product(x, w, resid, TILE_RESID, tile)
+        return True
+    if not _ADDMM_OUT_DTYPE:
         return False
     torch.addmm(resid, x, w.t(), out_dtype=torch.float32, out=resid)
     return True
@@ -341,10 +472,18 @@ def tile_weight_planes(w: torch.Tensor) -> Optional[TiledWeight]:
 
 
 def linear_planes(x: torch.Tensor, w: torch.Tensor, tiled: Optional[TiledWeight] = None) -> Optional[torch.Tensor]:
-    """For M <= 64: float32 planes [slices, M, N] whose sum is x @ w^T (K split over the grid), else None.
-    ``tiled``: the copy of ``w`` that ``tile_weight_planes`` made, read in its place by 17 rows and more."""
+    """Float32 planes [slices, M, N] whose sum is x @ w^T (K split over the grid): for M <= 64, and for more rows where the
+    tile kernel is quicker than the library; else None.
+    ``tiled``: the copy of ``w`` that ``tile_weight_planes`` made, read in its place by 17 to 64 rows."""
     m, k = x.shape
     n = w.shape[0]
+    if _tile_ok(x, w):
+        if not _tile_wins(m, n, k, TILE_F32):
+            return None
+        tile, slices, _ = tile_plan(m, n, k, TILE_F32, True)
+        out = torch.empty((slices, m, n), dtype=torch.float32, device=x.device)
+        tile_product(x, w, out, TILE_F32, tile, slices)
+        return out
     if m > SKINNY_MAX_M or not skinny_ok(x, w):
         return None
     rt, wk, slices = _plan(m, n, k, True)

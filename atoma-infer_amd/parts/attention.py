@@ -180,6 +180,9 @@ class PagedAttention(Mixer):
             qkv = gemm_bf16.try_linear_rope(x, w, ctx.positions, tables[0], tables[1], k_cache, v_cache,
                                             cache.slot_mapping, cache.page_size, nh, nkv, hd,
                                             tiled=self.w_qkv_tiled)
+            if qkv is None:
+                qkv = gemm_bf16.try_tile_rope(x, w, ctx.positions, tables[0], tables[1], k_cache, v_cache,
+                                              cache.slot_mapping, cache.page_size, nh, nkv, hd)
         if qkv is None:
             x = as_tensor(x)
         if qkv is not None:

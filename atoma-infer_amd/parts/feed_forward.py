@@ -5,7 +5,7 @@ values (``kernels.ops.gate_activation``).
 gate and up are fused into one [2 I, width] matrix at load time, so one product feeds the SiLU-multiply kernel.
 When I is a multiple of 16 the rows are interleaved in blocks of 16 (16 gate rows, then the 16 up rows of the
 same outputs): a lane of the weight-streaming MFMA product then holds a gate value and its up value, and the
-activation runs in that product's epilogue for few rows of x.
+activation runs in that product's epilogue (so does the tile kernel's, for many rows).
 """
 from __future__ import annotations
 
@@ -71,6 +71,8 @@ class SwiGLU(FeedForward):
         if self.block and x.dtype is torch.bfloat16 and self.w_gate_up.dtype is torch.bfloat16:
             from ..kernels import gemm_bf16
             h = gemm_bf16.try_linear_swiglu(x, self.w_gate_up, self.w_gate_up_tiled, self.activation)
+            if h is None:
+                h = gemm_bf16.try_tile_swiglu(x, self.w_gate_up, self.activation)
         if h is None:
             h = ops.swiglu(linear(x, self.w_gate_up), block=self.block, act=self.activation)
         return linear_delta(h, self.w_down, sink, self.w_down_tiled)

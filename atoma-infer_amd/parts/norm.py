@@ -82,7 +82,7 @@ class RMSNorm(Norm):
                               next_norm.act_dtype)
 
     # the norm begun by its neighbours (bfloat16 steps of at most 16 rows): see kernels/gemm_bf16.py; with many rows
-    # the library adds its product to the residual rows itself, and the norm reads them once
+    # the product is added to the residual rows by its own kernel, and the norm reads them once
     def add_product(self, resid, x, w, tiled=None):
         if self.act_dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16:
             return None
@@ -92,7 +92,7 @@ class RMSNorm(Norm):
         if y is not None:
             y.norm = self
             return y
-        if gemm_bf16.try_addmm_resid(as_tensor(x), w, resid):
+        if gemm_bf16.try_add_resid(as_tensor(x), w, resid):
             return Normed(self.add_norm(resid, None), self)
         return None
 

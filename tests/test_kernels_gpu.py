@@ -666,6 +666,86 @@ def test_gemm_with_rotary_epilogue(m, nh, nkv, hd, k, planes, monkeypatch):
                                      hd) is None   # too many rows
 
 
+@pytest.mark.parametrize("tile", range(6))
+@pytest.mark.parametrize("m,n,k", [(65, 16, 64), (130, 272, 128), (257, 544, 192), (600, 48, 1024), (300, 1056, 576)])
+def test_gemm_tile(tile, m, n, k):
+    """Every tile at edges of its rows, columns and buffers (1, 2, 3, 9 and 16 steps), every result it can leave.  A float32
+    sum of k products in any order is within k 2^-24 of the sum of their absolute values; bfloat16 rounds to 2^-9."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    wide = rnd(m, k + 8, dtype=torch.bfloat16, seed=1)
+    x, w = wide[:, 8:], rnd(n, k, dtype=torch.bfloat16, seed=2)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    bound = k * 2.0 ** -24 * size
+    for slices in (1, 2, 8):
+        if k % (64 * slices) == 0:
+            c = torch.full((slices, m, n), 7.0, device=DEV)
+            gb.tile_product(x, w, c, gb.TILE_F32, tile, slices)
+            assert bool(((c.double().sum(0) - want).abs() <= bound).all())
+    c = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    gb.tile_product(x, w, c, gb.TILE_BF16, tile)
+    assert bool(((c.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all())
+    r0 = rnd(m, n, seed=3)
+    r = r0.clone()
+    gb.tile_product(x, w, r, gb.TILE_RESID, tile)
+    assert bool(((r.double() - r0.double() - want).abs() <= bound + 2.0 ** -23 * (r0.double().abs() + want.abs())).all())
+    if n % 32 == 0 and tile in gb.TILES_SILU:
+        c = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+        gb.tile_product(x, w, c, gb.TILE_SILU, tile)
+        z = want.view(m, n // 32, 2, 16)
+        ref = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(m, n // 2)
+        assert bool(((c.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
+
+
+def test_gemm_tile_planned():
+    """The tile kernel where parts call it: planes of K slices, sums into the residual rows, and what it does not take."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    x, w = rnd(100, 8192, dtype=torch.bfloat16, seed=1), rnd(256, 8192, dtype=torch.bfloat16, seed=2)
+    want = x.double() @ w.double().T
+    planes = gb.linear_planes(x, w)
+    assert planes.dim() == 3 and planes.shape[0] > 1 and not gb.try_add_resid(x, w, torch.zeros(100, 256, device=DEV))
+    assert (planes.double().sum(0) - want).abs().max() <= 1e-5 * want.abs().max()
+    x, w = rnd(2048, 256, dtype=torch.bfloat16, seed=3), rnd(2048, 256, dtype=torch.bfloat16, seed=4)
+    r = torch.ones(2048, 2048, device=DEV)
+    assert gb.try_add_resid(x, w, r)
+    want = x.double() @ w.double().T + 1.0
+    assert (r.double() - want).abs().max() <= 1e-5 * want.abs().max()
+    assert gb.try_tile_swiglu(rnd(64, 256, dtype=torch.bfloat16), w) is None          # (few rows)
+    assert gb.try_tile_swiglu(rnd(70, 96, dtype=torch.bfloat16), rnd(64, 96, dtype=torch.bfloat16)) is None   # (K % 64)
+    assert gb.try_tile_swiglu(rnd(70, 264, dtype=torch.bfloat16)[:, 4:260], w) is None                       # (not aligned)
+
+
+@pytest.mark.parametrize("m", [65, 90, 300])
+@pytest.mark.parametrize("nh,nkv,hd,k,page", [(8, 2, 64, 128, 16), (6, 2, 48, 64, 16), (4, 1, 128, 192, 32), (2, 2, 16, 64, 5)])
+def test_gemm_tile_rope(m, nh, nkv, hd, k, page):
+    """q, k, v with rotary encoding and the cache write by the tile kernel, against the product and the rotary kernel apart in
+    float32: the difference is the rounding to bfloat16."""
+    from atoma_infer_amd.kernels import gemm_bf16, ops
+    from atoma_infer_amd.cache.layout import pack_keys, pack_values
+    pages, n = -(-(m + 8) // page) + 2, (nh + 2 * nkv) * hd
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    g = torch.Generator().manual_seed(5)
+    pos = torch.randint(0, 90, (m,), generator=g).int().to(DEV)
+    slots = torch.randperm(pages * page, generator=g)[:m].int()
+    slots[m // 2:] = torch.arange(m - m // 2).int() + 3 * (m % 2)          # (neighbours, aligned to four or not)
+    slots[: m // 2] = torch.arange(pages * page)[m - m // 2 + 3:][torch.randperm(pages * page - (m - m // 2 + 3), generator=g)[: m // 2]].int()
+    slots[2] = -1
+    slots = slots.to(DEV)
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    gg = torch.Generator().manual_seed(9)
+    kc = pack_keys(torch.randn(pages, nkv, page, hd, generator=gg).bfloat16()).to(DEV)
+    vc = pack_values(torch.randn(pages, nkv, hd, page, generator=gg).bfloat16()).to(DEV)
+    kf, vf, q2 = kc.float(), vc.float(), torch.empty(m, nh * hd, device=DEV)
+    ops.rope_cache_write(ops.gemm_generic(x, w, torch.float32), pos, cos, sin, hd, kf, vf, slots, page, nh, nkv, hd, q2)
+    for tile in gemm_bf16.TILES_ROPE:
+        k1, v1, q1 = kc.clone(), vc.clone(), torch.empty(m, nh * hd, dtype=torch.bfloat16, device=DEV)
+        gemm_bf16.tile_product(x, w, q1, gemm_bf16.TILE_ROPE, tile, rope=(pos, cos, sin, k1, v1, slots, page, nh, nkv, hd))
+        for got, want in ((q1, q2), (k1, kf), (v1, vf)):
+            assert bool(((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max()).all())
+    assert gemm_bf16.try_tile_rope(x, w, pos, cos, sin, kc, vc, slots, page, nh, nkv, hd) is not None
+    assert gemm_bf16.try_tile_rope(x[:64], w, pos, cos, sin, kc, vc, slots, page, nh, nkv, hd) is None       # (few rows)
+
+
 def _rms(x, g, eps):
     x = x.double()
     return x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps) * g.double()
