@@ -438,6 +438,103 @@ expert_gemm_mfma_kernel(const uint16_t* __restrict__ a, const uint16_t* __restri
   }
 }
 
+// Few places an expert (decode steps): the product only streams the chosen experts' weights, and what bounds it is the bytes
+// in flight.  A workgroup takes 32 rows of an expert's weight against a tile of up to 16 places; its four waves split K,
+// fetch both operands straight from memory, two batches of four steps in turn, and meet in LDS.  With the scores given
+// (scale) the inputs are the tokens' rows themselves, scaled and rounded as gather_scale does it, so that no kernel has
+// to lay them out before.  8 experts of 1,024 columns at width 2,048, 8 places each, with the grouping: 25 us, where the
+// tiles of 64 places (128 columns of K a step, one step ahead: 34 + 18 us alone) and gather_scale took 50.
+constexpr int kStreamPlaces = 16, kStreamWaves = 4;
+
+template <int ACT, bool GATHER, bool SCALED>
+__global__ void __launch_bounds__(64 * kStreamWaves)
+expert_stream_kernel(const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const int32_t* __restrict__ tiles,
+                     const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm, int K, int N, int lda, int top,
+                     const float* __restrict__ scale, void* __restrict__ c, int ldc, int plane_rows,
+                     const float* __restrict__ out_scale, GateAct gate) {
+  constexpr int U = 4;
+  __shared__ f32x4 red[kStreamWaves - 1][2][64];
+  const int e = tiles[2 * blockIdx.y];
+  if (e < 0) return;
+  const int row0 = tiles[2 * blockIdx.y + 1], rows = min(kStreamPlaces, offsets[e + 1] - row0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * 32, k_len = K / kStreamWaves, k_begin = wave * k_len;
+  const int place = row0 + min(r16, rows - 1), slot = perm[place];      // (rows past the tile: its last, never stored)
+  const uint16_t* const ap = a + (size_t)(GATHER ? slot / top : place) * lda + k_begin + kg * 8;
+  const float sc = SCALED ? scale[slot] : 1.f;
+  const uint16_t* const wp = w + ((size_t)e * N + n0 + r16) * K + k_begin + kg * 8;
+  const size_t block = (size_t)16 * K;
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  bf16x8 wf[2][U][2], af[2][U];
+  auto load = [&](int buf, int k0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) wf[buf][u][s] = *reinterpret_cast<const bf16x8*>(wp + s * block + k0 + u * 32);
+      af[buf][u] = *reinterpret_cast<const bf16x8*>(ap + k0 + u * 32);
+    }
+  };
+  auto one = [&](bf16x8 x, const bf16x8 (&y)[2]) {
+    if constexpr (SCALED) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = (__bf16)((float)x[i] * sc);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y[s], x, acc[s], 0, 0, 0);
+  };
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) one(af[buf][u], wf[buf][u]);
+  };
+  const int batches = k_len / (32 * U);
+  if (batches > 0) load(0, 0);
+  int b = 0;
+  for (; b + 2 <= batches; b += 2) {
+    load(1, (b + 1) * 32 * U);
+    multiply(0);
+    if (b + 2 < batches) load(0, (b + 2) * 32 * U);
+    multiply(1);
+  }
+  if (b < batches) multiply(0);
+  for (int k = batches * 32 * U; k < k_len; k += 32) {
+    bf16x8 y[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) y[s] = *reinterpret_cast<const bf16x8*>(wp + s * block + k);
+    one(*reinterpret_cast<const bf16x8*>(ap + k), y);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) red[wave - 1][s][lane] = acc[s];
+  }
+  __syncthreads();
+  if (wave > 0 || r16 >= rows) return;
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int i = 0; i < kStreamWaves - 1; ++i) acc[s] += red[i][s][lane];
+  if constexpr (ACT == 1) {          // 16 gate rows, then the 16 up rows of the same outputs
+    uint16_t* const dst = (uint16_t*)c + (size_t)place * ldc + n0 / 2 + kg * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[i] = f32_to_bf16_bits(gated(acc[0][i], acc[1][i], gate));
+  } else if constexpr (ACT == 2) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = acc[s][i];
+        ((uint16_t*)c)[(size_t)place * ldc + n0 + s * 16 + kg * 4 + i] = f32_to_bf16_bits(v > 0.f ? v * v : 0.f);
+      }
+  } else {
+    const size_t row = plane_rows > 0 ? (size_t)(slot % top) * plane_rows + slot / top : (size_t)place;
+    const float os = out_scale != nullptr ? out_scale[slot] : 1.0f;
+    float* const dst = (float*)c + row * ldc + n0 + kg * 4;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[s * 16 + i] = acc[s][i] * os;
+  }
+}
+
 // out[t, i] = relu(u[t, i])^2 * sigmoid(u[t, off_gate]) for an expert that every token uses: its first product's
 // result u [T, ld] holds the ff columns of the expert and, at off_gate, the token's gate (off_gate < 0: no gate).
 template <typename TI, typename TO>
@@ -509,6 +606,37 @@ extern "C" int atoma_expert_gemm_mfma(const void* a, const void* w, void* c, int
   return 0;
 }
 
+// The product for few places an expert.  gather: a is [tokens, K] (row stride lda) and a place's input is its token's row,
+// times scale[slot] where given; else a is [places, K].  tiles as route_group makes them for 16 places.
+extern "C" int atoma_expert_stream(const void* a, int lda, int gather, const float* scale, const void* w, void* c, int ldc,
+                                   int N, int K, const int32_t* perm, const int32_t* offsets, const int32_t* tiles,
+                                   int max_tiles, int top, int plane_rows, int act, const float* out_scale, int gate_kind,
+                                   float limit, float slope, hipStream_t stream) {
+  if (max_tiles <= 0 || N <= 0) return 0;
+  if (K <= 0 || K % (32 * kStreamWaves) || N % 32 || lda < K || lda % 8 || top <= 0 || max_tiles > 65535 || ((uintptr_t)a & 15) ||
+      ((uintptr_t)w & 15) || act < 0 || act > 2 || !gate_act_ok(gate_kind, limit) || ldc < (act == 1 ? N / 2 : N) ||
+      (act != 0 && (plane_rows > 0 || out_scale != nullptr)) || (scale != nullptr && !gather))
+    return ATOMA_ERR_SHAPE;
+  const GateAct gate{gate_kind, limit, slope};
+  const dim3 grid(N / 32, max_tiles), block(64 * kStreamWaves);
+#define ATOMA_ES(ACT, G, S)                                                                                            \
+  hipLaunchKernelGGL((expert_stream_kernel<ACT, G, S>), grid, block, 0, stream, (const uint16_t*)a, (const uint16_t*)w, tiles, \
+                     offsets, perm, K, N, lda, top, scale, c, ldc, plane_rows, out_scale, gate)
+#define ATOMA_ES_(ACT)                          \
+  do {                                          \
+    if (scale != nullptr) ATOMA_ES(ACT, true, true); \
+    else if (gather) ATOMA_ES(ACT, true, false); \
+    else ATOMA_ES(ACT, false, false);           \
+  } while (0)
+  if (act == 1) ATOMA_ES_(1);
+  else if (act == 2) ATOMA_ES_(2);
+  else ATOMA_ES_(0);
+#undef ATOMA_ES_
+#undef ATOMA_ES
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
 extern "C" int atoma_route_topk(const float* logits, int ld, int experts, int top, int32_t* ids, float* weights,
                                 int n_tokens, int score, const float* correction, float scale, const float* bias,
                                 int groups, int groups_keep, hipStream_t stream) {
@@ -544,7 +672,7 @@ extern "C" int atoma_route_max_tiles(int n_slots, int experts, int tile_m) {
 extern "C" int atoma_route_group(const int32_t* ids, int n_slots, int experts, int32_t* perm, int32_t* offsets,
                                  int32_t* tiles, int max_tiles, int tile_m, hipStream_t stream) {
   if (n_slots <= 0) return 0;
-  if (experts <= 0 || experts > 1024 || (tile_m != 64 && tile_m != 128) ||
+  if (experts <= 0 || experts > 1024 || (tile_m != 16 && tile_m != 64 && tile_m != 128) ||
       max_tiles < atoma_route_max_tiles(n_slots, experts, tile_m))
     return ATOMA_ERR_SHAPE;
   hipLaunchKernelGGL(route_group_kernel, dim3(1), dim3(1024), 0, stream, ids, n_slots, experts, perm, offsets, tiles,

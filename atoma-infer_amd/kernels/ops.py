@@ -756,7 +756,7 @@ def route_topk(logits: torch.Tensor, top: int, score: str = "sigmoid", correctio
 
 def route_group(ids: torch.Tensor, experts: int, tile_m: int = 64):
     """Slots (token, choice) ordered by expert: (perm int32 [slots], offsets int32 [experts + 1], tiles int32
-    [max_tiles, 2] of (expert or -1, first place in perm)); a tile holds up to ``tile_m`` (64 or 128) places."""
+    [max_tiles, 2] of (expert or -1, first place in perm)); a tile holds up to ``tile_m`` (16, 64 or 128) places."""
     _dev(ids)
     _i32(ids, "ids")
     n = ids.numel()
@@ -838,6 +838,40 @@ def expert_gemm_mfma(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, perm, 
         _p(a), _p(w), _p(out), cols, n, k, _p(perm), _p(offsets), _p(tiles), tiles.shape[0], int(top),
         n_slots // top if planes else 0, 1 if swiglu else 2 if relu2 else 0, int(tile_m), _p(out_scale),
         *_gate_args(act), _stream()), "expert_gemm_mfma")
+
+
+EXPERT_STREAM_PLACES = 16
+
+
+def expert_stream_ok(x: torch.Tensor, n: int, k: int) -> bool:
+    """Whether ``expert_stream`` takes inputs x [., k] for weights of n rows."""
+    return (n % 32 == 0 and k % 128 == 0 and x.dim() == 2 and x.stride(1) == 1 and x.data_ptr() % 16 == 0
+            and (x.shape[0] == 1 or x.stride(0) % 8 == 0))
+
+
+def expert_stream(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, perm, offsets, tiles, top: int, *, gather: bool,
+                  scale: Optional[torch.Tensor] = None, swiglu: bool = False, planes: bool = False, relu2: bool = False,
+                  out_scale: Optional[torch.Tensor] = None, act="silu") -> None:
+    """``expert_gemm_mfma`` for few places an expert, with ``tiles`` of 16 places.  ``gather``: a is [T, K], a place's input
+    its token's row (times ``scale`` [slots], rounded to bfloat16, where given); else a is [places, K]."""
+    _dev(a, w, out, perm, offsets, tiles, scale, out_scale)
+    _need(not (swiglu and relu2) and (gather or scale is None), "expert_stream: one activation, scores with tokens only")
+    for t in (scale, out_scale):
+        if t is not None:
+            _f32(t, "scale", perm.numel())
+    n_slots = perm.numel()
+    e, n, k = w.shape
+    _need(a.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and w.is_contiguous() and a.shape[1] == k
+          and a.shape[0] * (top if gather else 1) == n_slots and expert_stream_ok(a, n, k), "expert_stream: operands do not fit")
+    cols = n // 2 if swiglu else n
+    _need(out.is_contiguous() and out.numel() == n_slots * cols and out.shape[-1] == cols
+          and out.dtype is (torch.bfloat16 if swiglu or relu2 else torch.float32)
+          and not ((swiglu or relu2) and (planes or out_scale is not None)), "expert_stream: bad out")
+    _need(offsets.numel() == e + 1 and tiles.dim() == 2 and tiles.shape[1] == 2, "expert_stream: bad grouping")
+    _check(_module("experts").atoma_expert_stream(
+        _p(a), a.stride(0) if a.shape[0] > 1 else k, int(gather), _p(scale), _p(w), _p(out), cols, n, k, _p(perm), _p(offsets),
+        _p(tiles), tiles.shape[0], int(top), n_slots // top if planes else 0, 1 if swiglu else 2 if relu2 else 0,
+        _p(out_scale), *_gate_args(act), _stream()), "expert_stream")
 
 
 def relu2_gate(u: torch.Tensor, ff: int, off_gate: int, out_dtype: torch.dtype) -> torch.Tensor:

@@ -41,6 +41,13 @@ from .feed_forward import SwiGLU
 from .linear import linear, linear_delta
 
 
+# places an expert, on average, up to which the streaming kernel takes the products (beyond, an expert's weight is read
+# again for every tile of 16 places).  Grouping, inputs and both products with 8 experts of 1,024 columns at width 2,048, 1 /
+# 8 / 32 / 48 / 64 places an expert: 23 / 25 / 42 / 59 / 74 us against 50 / 50 / 59 / 66 / 72 by tiles of 64; 4 of 32 experts of
+# 2,048 columns for 1 / 8 / 64 / 100 tokens: 24 / 98 / 147 / 168 against 63 / 147 / 201 / 215
+STREAM_PLACES = 24
+
+
 class RoutedExperts(FeedForward):
     def __init__(self, width: int, intermediate: int, experts: int, top: int, score: str = "sigmoid",
                  scale: float = 1.0, correction: bool = False, expert: str = "swiglu", shared: int = 0,
@@ -149,6 +156,17 @@ class RoutedExperts(FeedForward):
         slots = t * self.top
         flat = weights.view(-1)
         w_in, w_out = (flat, None) if self.weighs_input else (None, flat)
+        rows = self.w_gate_up.shape[1]
+        if (self.mfma and x.dtype is torch.bfloat16 and slots <= STREAM_PLACES * self.experts
+                and ops.expert_stream_ok(x, rows, self.width) and self.width % 32 == 0 and self.inter % 128 == 0):
+            # few places an expert: its weight is streamed, and the tokens' rows are read where they lie
+            perm, offsets, tiles = ops.route_group(ids.view(-1), self.experts, ops.EXPERT_STREAM_PLACES)
+            h = torch.empty((slots, self.inter), dtype=torch.bfloat16, device=x.device)
+            ops.expert_stream(x, self.w_gate_up, h, perm, offsets, tiles, self.top, gather=True, scale=w_in,
+                              swiglu=self.gated, relu2=not self.gated, act=self.activation)
+            out = torch.empty((self.top, t, self.width), dtype=torch.float32, device=x.device)
+            ops.expert_stream(h, self.w_down, out, perm, offsets, tiles, self.top, gather=False, planes=True, out_scale=w_out)
+            return out
         if self.mfma and x.dtype is torch.bfloat16:
             # tiles of 128 places where an expert has about a hundred or more (prompts): a weight fragment then
             # serves twice as many rows

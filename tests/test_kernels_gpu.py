@@ -351,6 +351,38 @@ def test_generic_attention_masks(hd, nh, nkv, page):
     assert bool(outs[1][10].isnan().all()) and bool(outs[1][77].isnan().all())
 
 
+@pytest.mark.parametrize("counts", [(1, 0, 3), (16, 17, 0, 33, 1), (5, 5, 5, 5)])
+@pytest.mark.parametrize("n,k", [(32, 128), (96, 640), (64, 1152)])
+def test_expert_stream(counts, n, k):
+    """Tiles of 16 places, full, short and none, uneven batches of K, every result: the same tokens chosen ``top`` times over,
+    against float64.  Sums are within k 2^-24 of the sum of absolute values, bfloat16 results within 2^-8 beyond that."""
+    from atoma_infer_amd.kernels import ops
+    experts, top = len(counts), 1
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)]).int()
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))].to(DEV)
+    t = ids.numel()
+    wide = rnd(t, k + 8, dtype=torch.bfloat16, seed=2)
+    x, w, score = wide[:, 8:], rnd(experts, n, k, dtype=torch.bfloat16, seed=3), rnd(t, seed=4).abs()
+    perm, offsets, tiles = ops.route_group(ids, experts, ops.EXPERT_STREAM_PLACES)
+    for scale in (None, score):
+        xin = x if scale is None else (x.float() * scale[:, None]).bfloat16()
+        want = torch.einsum("tk,tnk->tn", xin.double(), w.double()[ids.long()])
+        bound = k * 2.0 ** -24 * torch.einsum("tk,tnk->tn", xin.double().abs(), w.double().abs()[ids.long()])
+        out = torch.empty(top, t, n, device=DEV)
+        ops.expert_stream(x, w, out, perm, offsets, tiles, top, gather=True, scale=scale, planes=True, out_scale=score)
+        assert bool(((out[0].double() - want * score[:, None].double()).abs() <= (2 * bound + 1e-7 * want.abs()) * score[:, None]).all())
+        p = perm.long()
+        relu = torch.empty(t, n, dtype=torch.bfloat16, device=DEV)
+        ops.expert_stream(x, w, relu, perm, offsets, tiles, top, gather=True, scale=scale, relu2=True)
+        ref = want[p].clamp(min=0) ** 2
+        assert bool(((relu.double() - ref).abs() <= 2.0 ** -7 * ref + 1e-5 * ref.abs().max()).all())
+        gate = torch.empty(t, n // 2, dtype=torch.bfloat16, device=DEV)
+        ops.expert_stream(xin[p].contiguous(), w, gate, perm, offsets, tiles, top, gather=False, swiglu=True)
+        z = want[p].view(t, n // 32, 2, 16)
+        ref = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(t, n // 2)
+        assert bool(((gate.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-5 * ref.abs().max()).all())
+
+
 TWO_PIECE_CASES = [c for c in ATTN_CASES if c[2] <= 64] + [
     # groups of 1, 3, 8, 33 and 40 heads (tiles of 256, 255, 256, 264, 240 rows; the last pieces are short or half
     # empty), one token, a window, portions beside decoded tokens
