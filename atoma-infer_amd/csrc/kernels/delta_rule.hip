@@ -7,10 +7,10 @@
 //                      inputs before an entry's first token come from the request's state), q and k to unit length per
 //                      head (q also times dim^-1/2), beta = sigmoid(b), g = exp(-exp(A_log) softplus(a + dt_bias));
 //   delta_conv_state   per request: the last taps - 1 inputs of the convolution, for the request's next step;
-//   delta_scan         per (request, head, 16 columns of S): the recurrence over the entry's tokens in order, S read from
+//   delta_scan         per (request, head, 8 columns of S): the recurrence over the entry's tokens in order, S read from
 //                      the request's state slot before and written back after.  A column of S lives in the registers
-//                      of 16 neighbouring lanes (dim / 16 rows each, rounded up), so a token costs a lane a few dozen
-//                      multiply-adds and one four-step exchange among those lanes; the tokens' inputs pass LDS in
+//                      of 32 neighbouring lanes (dim / 32 rows each, rounded up), so a token costs a lane a dozen or
+//                      two multiply-adds and one five-step exchange among those lanes; the tokens' inputs pass LDS in
 //                      blocks, fetched a block ahead;
 //   delta_out          per token and head: o / sqrt(mean(o^2) + eps) * w * sigmoid(gate), in the activation dtype.
 // The order of every sum depends on the sizes alone, so a token's result does not depend on how the request was cut
@@ -113,34 +113,39 @@ delta_conv_state_kernel(const float* __restrict__ proj, DeltaShape sh, const int
   }
 }
 
-// Sum over the 16 lanes of a DPP row; every lane gets the same sum (the pairs of each step add the same two numbers).
-__device__ __forceinline__ float row16_sum(float x) {
+// Sum over the 32 lanes of half a wave; every lane gets the same sum (the pairs of each step add the same two numbers).
+__device__ __forceinline__ float half_sum(float x) {
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xf, 0xf, false));    // lanes i ^ 1
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xf, 0xf, false));    // lanes i ^ 2
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xf, 0xf, false));   // the other quad of 8
   x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x140, 0xf, 0xf, false));   // the other half of 16
-  return x;
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);                                       // the other 16
 }
 
-// R: rows of S a lane holds.  16 lanes (a DPP row) share a column of S, so dim <= 16 R; a wave holds 4 columns, a
-// workgroup of four waves 16.  The tokens' q, k, decay (for the head), v (for the 16 columns), beta and k . q pass
-// LDS in blocks of TB tokens: the next block is fetched from memory while this one is worked on, so the walk over the
-// tokens waits for LDS only.
+// R: rows of S a lane holds.  32 lanes share a column of S, so dim <= 32 R; a wave holds 2 columns, a workgroup of four
+// waves 8.  The tokens' q, k, decay (for the head), v (for the 8 columns), beta and k . q pass LDS in blocks of TB tokens:
+// the next block is fetched from memory while this one is worked on, and the next token's rows are read from LDS while
+// this one's are worked on.
+// Bound by a wave's instructions for a token, one after the other (a prompt has a workgroup for 8 columns of a head and
+// nothing else to fill the CUs with), so a column has 32 lanes of few rows: two layers of Somesun at the 1b sizes, eight
+// prompts of 11,000 tokens together and 64 decoded tokens each, 5.46 -> 4.74 ms (16 lanes of twice the rows before).
 template <int R>
 __global__ void __launch_bounds__(256)
 delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vn,
                   const float* __restrict__ beta, const float* __restrict__ decay, const float* __restrict__ kq,
                   DeltaShape sh, const int32_t* __restrict__ q_start, const int32_t* __restrict__ state_slots,
                   float* __restrict__ state, size_t state_stride, size_t s_offset, float* __restrict__ o) {
-  constexpr int DP = 16 * R;                   // dim rounded up; rows beyond dim hold zeros
-  constexpr int TB = R <= 8 ? 16 : 8;          // tokens a block
+  constexpr int DP = 32 * R;                   // dim rounded up; rows beyond dim hold zeros
+  constexpr int TB = R <= 4 ? 16 : 8;          // tokens a block
+  constexpr int COLS = 8;
   constexpr int PER = TB * DP / 256;           // elements of q (k, decay) a thread fetches a block
-  __shared__ float sq[2][TB][DP], sk[2][TB][DP], sg[2][TB][DP];
-  __shared__ float sv[2][TB][16], sb[2][TB], skq[2][TB];
+  __shared__ __attribute__((aligned(16))) float sq[2][TB][DP], sk[2][TB][DP], sg[2][TB][DP];
+  __shared__ float sv[2][TB][COLS], sb[2][TB], skq[2][TB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int part = lane & 15;
-  const int col_local = wave * 4 + (lane >> 4);
-  const int col = blockIdx.x * 16 + col_local;
+  const int part = lane & 31;
+  const int col_local = wave * 2 + (lane >> 5);
+  const int col = blockIdx.x * COLS + col_local;
   const int h = blockIdx.y, e = blockIdx.z;
   const int kv = h / (sh.heads / sh.kv_heads);
   const int dim = sh.dim, vdim = sh.vdim;
@@ -155,69 +160,76 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn, co
 
   const int nqk = sh.kv_heads * dim, nd = sh.heads * dim, nv = sh.heads * vdim;
   float pq[PER], pk[PER], pg[PER], pv = 0.f, pb = 0.f, pkq = 0.f;
-  // block b's share of this thread: element idx = tid + j * 256 of [TB][DP]; v: thread tid of [TB][16]; beta, k . q: tid < TB
+  // block b's share of this thread: element idx = tid + j * 256 of [TB][DP]; v: thread tid of [TB][COLS]; beta, k . q: tid < TB
+  // (No load stands under a condition, which the compiler would wait for where the branches meet: what lies beyond the
+  // entry's tokens is fetched from the last one and never used, what lies beyond dim or vdim becomes zero on the way to LDS.)
   auto fetch = [&](int b) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int idx = tid + j * 256, tok = idx / DP, i = idx % DP;
-      const int n = b * TB + tok;
-      const bool ok = n < count && i < dim;
-      const size_t t = (size_t)(first + n);
-      pq[j] = ok ? qn[t * nqk + (size_t)kv * dim + i] : 0.f;
-      pk[j] = ok ? kn[t * nqk + (size_t)kv * dim + i] : 0.f;
-      pg[j] = ok ? decay[t * nd + (size_t)h * dim + i] : 0.f;
+      const int idx = tid + j * 256, tok = idx / DP, i = min(idx % DP, dim - 1);
+      const size_t t = (size_t)(first + min(b * TB + tok, count - 1));
+      pq[j] = qn[t * nqk + (size_t)kv * dim + i];
+      pk[j] = kn[t * nqk + (size_t)kv * dim + i];
+      pg[j] = decay[t * nd + (size_t)h * dim + i];
     }
-    if (tid < TB * 16) {
-      const int tok = tid >> 4, c = blockIdx.x * 16 + (tid & 15);
-      const int n = b * TB + tok;
-      pv = (n < count && c < vdim) ? vn[(size_t)(first + n) * nv + (size_t)h * vdim + c] : 0.f;
-    }
-    if (tid < TB) {
-      const bool ok = b * TB + tid < count;
-      pb = ok ? beta[(size_t)(first + b * TB + tid) * sh.heads + h] : 0.f;
-      pkq = ok ? kq[(size_t)(first + b * TB + tid) * sh.kv_heads + kv] : 0.f;
-    }
+    const size_t tv = (size_t)(first + min(b * TB + tid / COLS, count - 1)), tb = (size_t)(first + min(b * TB + tid, count - 1));
+    pv = vn[tv * nv + (size_t)h * vdim + min((int)blockIdx.x * COLS + tid % COLS, vdim - 1)];
+    pb = beta[tb * sh.heads + h];
+    pkq = kq[tb * sh.kv_heads + kv];
   };
   auto stash = [&](int buf) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int idx = tid + j * 256, tok = idx / DP, i = idx % DP;
-      sq[buf][tok][i] = pq[j];
-      sk[buf][tok][i] = pk[j];
-      sg[buf][tok][i] = pg[j];
+      sq[buf][tok][i] = i < dim ? pq[j] : 0.f;
+      sk[buf][tok][i] = i < dim ? pk[j] : 0.f;
+      sg[buf][tok][i] = i < dim ? pg[j] : 0.f;
     }
-    if (tid < TB * 16) sv[buf][tid >> 4][tid & 15] = pv;
+    if (tid < TB * COLS) sv[buf][tid / COLS][tid % COLS] = pv;
     if (tid < TB) sb[buf][tid] = pb, skq[buf][tid] = pkq;
+  };
+  struct Rows { float k[R], g[R], q[R], v, b, kq; };
+  auto load = [&](Rows& x, int buf, int tok) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) x.k[r] = sk[buf][tok][i0 + r], x.g[r] = sg[buf][tok][i0 + r], x.q[r] = sq[buf][tok][i0 + r];
+    x.v = sv[buf][tok][col_local], x.b = sb[buf][tok], x.kq = skq[buf][tok];
+  };
+  auto token = [&](const Rows& x, int n) {
+    float d1 = 0.f, d2 = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      s[r] *= x.g[r];
+      d1 = fmaf(s[r], x.k[r], d1);
+      d2 = fmaf(s[r], x.q[r], d2);
+    }
+    d1 = half_sum(d1);
+    d2 = half_sum(d2);
+    const float u = x.b * (x.v - d1);
+    // o = S_new^T q with S_new = diag(g) S + k u^T
+    if (part == 0 && col_ok) o[(size_t)(first + n) * nv + (size_t)h * vdim + col] = fmaf(u, x.kq, d2);
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = fmaf(x.k[r], u, s[r]);
   };
   const int blocks = (count + TB - 1) / TB;
   if (blocks > 0) {
     fetch(0);
     stash(0);
   }
+  // (the state has arrived, which the compiler would else make sure of in front of every block's tokens, by waiting for
+  // everything, the next block's fetch with it)
+  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
   __syncthreads();
   for (int b = 0; b < blocks; ++b) {
     const int buf = b & 1;
     if (b + 1 < blocks) fetch(b + 1);
     const int n_tok = min(TB, count - b * TB);
-#pragma unroll 2
-    for (int tok = 0; tok < n_tok; ++tok) {
-      float d1 = 0.f, d2 = 0.f;
-      float kr[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        kr[r] = sk[buf][tok][i0 + r];
-        s[r] *= sg[buf][tok][i0 + r];
-        d1 = fmaf(s[r], kr[r], d1);
-        d2 = fmaf(s[r], sq[buf][tok][i0 + r], d2);
-      }
-      d1 = row16_sum(d1);
-      d2 = row16_sum(d2);
-      const float u = sb[buf][tok] * (sv[buf][tok][col_local] - d1);
-      // o = S_new^T q with S_new = diag(g) S + k u^T
-      if (part == 0 && col_ok)
-        o[(size_t)(first + b * TB + tok) * nv + (size_t)h * vdim + col] = fmaf(u, skq[buf][tok], d2);
-#pragma unroll
-      for (int r = 0; r < R; ++r) s[r] = fmaf(kr[r], u, s[r]);
+    Rows x, y;
+    load(x, buf, 0);
+    for (int tok = 0; tok < n_tok; tok += 2) {
+      load(y, buf, min(tok + 1, TB - 1));
+      token(x, b * TB + tok);
+      load(x, buf, min(tok + 2, TB - 1));
+      if (tok + 1 < n_tok) token(y, b * TB + tok + 1);
     }
     if (b + 1 < blocks) stash(buf ^ 1);
     __syncthreads();
@@ -320,15 +332,14 @@ extern "C" int atoma_delta_scan(const float* qn, const float* kn, const float* v
   DeltaShape sh{heads, kv_heads, dim, vdim, taps, 1, 0, 0, 0, 0};
   if (!shape_ok(sh) || n_entries > 65535 || heads > 65535) return ATOMA_ERR_SHAPE;
   const size_t s_offset = (size_t)(taps - 1) * (2 * kv_heads * dim + heads * vdim);
-  dim3 grid((vdim + 15) / 16, heads, n_entries), block(256);
+  dim3 grid((vdim + 7) / 8, heads, n_entries), block(256);
 #define ATOMA_SCAN(R_)                                                                                            \
   hipLaunchKernelGGL((delta_scan_kernel<R_>), grid, block, 0, stream, qn, kn, vn, beta, decay, kq, sh, q_start,   \
                      state_slots, state, state_stride, s_offset, o)
-  if (dim <= 16) ATOMA_SCAN(1);
-  else if (dim <= 32) ATOMA_SCAN(2);
-  else if (dim <= 64) ATOMA_SCAN(4);
-  else if (dim <= 128) ATOMA_SCAN(8);
-  else ATOMA_SCAN(16);
+  if (dim <= 32) ATOMA_SCAN(1);
+  else if (dim <= 64) ATOMA_SCAN(2);
+  else if (dim <= 128) ATOMA_SCAN(4);
+  else ATOMA_SCAN(8);
 #undef ATOMA_SCAN
   ATOMA_LAUNCH_CHECK();
   return 0;
