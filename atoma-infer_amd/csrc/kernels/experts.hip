@@ -254,12 +254,9 @@ expert_gemm_kernel(const TA* __restrict__ a, int lda, int a_div, const float* __
     for (int j = 0; j < kTileM / 32; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   f32_tile<kTileM, kTileN, VEC, TA, TW>(
       lds, K,
-      [&](int r) {
-        const int slot = slot_of(r);
-        return slot >= 0 ? a + (size_t)(slot / a_div) * lda : nullptr;
-      },
-      [&](int r) { return n0 + r < N ? we + (size_t)(n0 + r) * K : nullptr; },
-      [&](int r) { return scale != nullptr ? scale[slot_of(r)] : 1.f; }, acc);
+      [&](int r) { return a + (size_t)(perm[min(row0 + r, row_end - 1)] / a_div) * lda; },
+      [&](int r) { return we + (size_t)min(n0 + r, N - 1) * K; },
+      [&](int r) { return scale != nullptr ? scale[perm[min(row0 + r, row_end - 1)]] : 1.f; }, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < kTileM / 32; ++j) {
@@ -693,7 +690,7 @@ extern "C" int atoma_expert_gemm(const void* a, int a_dtype, int lda, int a_div,
   hipLaunchKernelGGL((expert_gemm_kernel<V, TA, TW, TC>), grid, block, 0, stream, (const TA*)a, lda, a_div, scale, \
                      (const TW*)w, (TC*)c, ldc, N, K, perm, offsets, tiles, top, plane_rows, act, out_scale)
   // (pieces of four values: at most 16 bytes)
-  const bool vec = K % 4 == 0 && lda % 4 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0;
+  const bool vec = K % kF32Step == 0 && lda % 4 == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)w & 15) == 0;
 #define ATOMA_EG(TA, TW, TC)                \
   do {                                      \
     if (vec) ATOMA_EG_(true, TA, TW, TC);   \

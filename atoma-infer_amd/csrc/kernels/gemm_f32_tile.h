@@ -16,32 +16,32 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 constexpr int kF32Step = 32, kF32Row = kF32Step + 4;
 
-// four neighbouring values of K of one row, from k on; zeros from K on.  VEC: rows are aligned to four values and K is a
-// multiple of four.
+// four neighbouring values of K of one row as they come from memory, from k on; zeros from K on.  VEC: rows are aligned to
+// four values and K is a multiple of the step, so that no load stands under a condition (the compiler waits for such a
+// load where its branches meet, and the next step's fetch would not run under this one's products).
+template <typename T> struct F32Raw { f32x4_t v; };
+template <> struct F32Raw<bf16_t> { uint2 v; };
 template <bool VEC, typename T>
-__device__ __forceinline__ f32x4_t f32_load4(const T* __restrict__ row, int k, int K) {
-  f32x4_t v = f32x4_t{0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ F32Raw<T> f32_load4(const T* __restrict__ row, int k, int K) {
+  F32Raw<T> r;
   if constexpr (VEC) {
-    if (k < K) {
-      if constexpr (sizeof(T) == 4) {
-        v = *reinterpret_cast<const f32x4_t*>(row + k);
-      } else {
-        const uint2 u = *reinterpret_cast<const uint2*>(row + k);
-        v = f32x4_t{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                    __uint_as_float(u.y & 0xffff0000u)};
-      }
-    }
+    r.v = *reinterpret_cast<const decltype(r.v)*>(row + k);
   } else {
+    T* const e = reinterpret_cast<T*>(&r.v);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (k + i < K) v[i] = to_f32(row[k + i]);
+    for (int i = 0; i < 4; ++i) e[i] = k + i < K ? row[k + i] : from_f32<T>(0.f);
   }
-  return v;
+  return r;
+}
+__device__ __forceinline__ f32x4_t f32_wide(const F32Raw<float>& r) { return r.v; }
+__device__ __forceinline__ f32x4_t f32_wide(const F32Raw<bf16_t>& r) {
+  return f32x4_t{__uint_as_float(r.v.x << 16), __uint_as_float(r.v.x & 0xffff0000u), __uint_as_float(r.v.y << 16),
+                 __uint_as_float(r.v.y & 0xffff0000u)};
 }
 
 // acc[i][j] (i: blocks of 16 rows of W, j: blocks of 16 rows of A, of this wave's quarter): lane l holds rows
-// 4 (l / 16) .. + 3 of W's block against row l % 16 of A's.  row_a(r), row_w(r): the pointer to row r of the tile, or
-// null for a row that is all zeros; scale(r) multiplies row r of A.
+// 4 (l / 16) .. + 3 of W's block against row l % 16 of A's.  row_a(r), row_w(r): the pointer to row r of the tile
+// (of any row that can be read, for one past the end: its results are never stored); scale(r) multiplies row r of A.
 template <int TM, int TN, bool VEC, typename TA, typename TW, typename RowA, typename RowW, typename Scale>
 __device__ __forceinline__ void f32_tile(float* __restrict__ lds, int K, RowA row_a, RowW row_w, Scale scale,
                                          f32x4_t (&acc)[TN / 32][TM / 32]) {
@@ -54,17 +54,16 @@ __device__ __forceinline__ void f32_tile(float* __restrict__ lds, int K, RowA ro
   float sa[PA];
   const TW* pw[PW];
 #pragma unroll
-  for (int i = 0; i < PA; ++i) pa[i] = row_a(r0 + i * 32), sa[i] = pa[i] ? scale(r0 + i * 32) : 0.f;
+  for (int i = 0; i < PA; ++i) pa[i] = row_a(r0 + i * 32), sa[i] = scale(r0 + i * 32);
 #pragma unroll
   for (int i = 0; i < PW; ++i) pw[i] = row_w(r0 + i * 32);
-  f32x4_t va[PA], vw[PW];
+  F32Raw<TA> va[PA];
+  F32Raw<TW> vw[PW];
   auto fetch = [&](int k) {
 #pragma unroll
-    for (int i = 0; i < PA; ++i)
-      va[i] = pa[i] ? f32_load4<VEC>(pa[i], k + k4, K) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < PA; ++i) va[i] = f32_load4<VEC>(pa[i], k + k4, K);
 #pragma unroll
-    for (int i = 0; i < PW; ++i)
-      vw[i] = pw[i] ? f32_load4<VEC>(pw[i], k + k4, K) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < PW; ++i) vw[i] = f32_load4<VEC>(pw[i], k + k4, K);
   };
   fetch(0);
   int buf = 0;
@@ -72,9 +71,9 @@ __device__ __forceinline__ void f32_tile(float* __restrict__ lds, int K, RowA ro
     float* const as = lds + buf * BUF;
     float* const ws = as + TM * kF32Row;
 #pragma unroll
-    for (int i = 0; i < PA; ++i) *reinterpret_cast<f32x4_t*>(as + (r0 + i * 32) * kF32Row + k4) = va[i] * sa[i];
+    for (int i = 0; i < PA; ++i) *reinterpret_cast<f32x4_t*>(as + (r0 + i * 32) * kF32Row + k4) = f32_wide(va[i]) * sa[i];
 #pragma unroll
-    for (int i = 0; i < PW; ++i) *reinterpret_cast<f32x4_t*>(ws + (r0 + i * 32) * kF32Row + k4) = vw[i];
+    for (int i = 0; i < PW; ++i) *reinterpret_cast<f32x4_t*>(ws + (r0 + i * 32) * kF32Row + k4) = f32_wide(vw[i]);
     __syncthreads();      // (the other buffer was last read before the barrier of the step before)
     if (k + kF32Step < K) fetch(k + kF32Step);
     const float* const aw = as + ((wave >> 1) * (TM / 2) + r16) * kF32Row + kg * 4;

@@ -15,8 +15,9 @@
 //
 // Measured on MI355X, float32 rows against bfloat16 weights, beside the one kernel of vector multiply-adds before (a tile
 // of 64 x 64 a workgroup, 4 x 4 outputs a thread): the four layers of Llama 1B sizes and its head, 836 rows in one step
-// and 16 steps of 4 rows, 106.5 -> 12.5 ms in all; gate-up (16,384 x 2,048) with 836 rows 727 us (77 TFLOP/s; the
-// card's float32 product of 8,192^3 reaches 153), with 4 rows 22.7 us; the head (128,256 x 2,048) with 4 rows 133 us.
+// and 16 steps of 4 rows, 106.5 -> 9.8 ms in all; gate-up (16,384 x 2,048) with 836 rows 622 us (90 TFLOP/s, 727 with
+// loads under conditions; the card's float32 product of 8,192^3 reaches 153), with 4 rows 17.5 us (22.7 with one batch of
+// loads in flight); the head (128,256 x 2,048) with 4 rows 117 us (133).
 //
 // The order in which an output's K products are summed depends on the kernel and on (N, K), not on its row's place.
 #include "gemm_f32_tile.h"
@@ -35,8 +36,8 @@ f32_tile_kernel(const TA* __restrict__ a, const TW* __restrict__ w, TC* __restri
 #pragma unroll
     for (int j = 0; j < T / 32; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   f32_tile<T, T, VEC, TA, TW>(
-      lds, K, [&](int r) { return m0 + r < M ? a + (size_t)(m0 + r) * lda : nullptr; },
-      [&](int r) { return n0 + r < N ? w + (size_t)(n0 + r) * ldw : nullptr; }, [](int) { return 1.f; }, acc);
+      lds, K, [&](int r) { return a + (size_t)min(m0 + r, M - 1) * lda; },
+      [&](int r) { return w + (size_t)min(n0 + r, N - 1) * ldw; }, [](int) { return 1.f; }, acc);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < T / 32; ++j) {
@@ -52,17 +53,17 @@ f32_tile_kernel(const TA* __restrict__ a, const TW* __restrict__ w, TC* __restri
   }
 }
 
-// eight neighbouring values of a row as float32 (16-byte aligned)
-__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
-  const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 4);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = lo[i], v[4 + i] = hi[i];
+// eight neighbouring values of a row as they come from memory (16-byte aligned), and one of them as float32
+template <typename T> struct Eight { f32x4_t lo, hi; };
+template <> struct Eight<bf16_t> { uint4 v; };
+__device__ __forceinline__ void fetch8(const float* p, Eight<float>& x) {
+  x.lo = *reinterpret_cast<const f32x4_t*>(p), x.hi = *reinterpret_cast<const f32x4_t*>(p + 4);
 }
-__device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
-  const uint4 u = *reinterpret_cast<const uint4*>(p);
-  const uint32_t q[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[2 * i] = __uint_as_float(q[i] << 16), v[2 * i + 1] = __uint_as_float(q[i] & 0xffff0000u);
+__device__ __forceinline__ void fetch8(const bf16_t* p, Eight<bf16_t>& x) { x.v = *reinterpret_cast<const uint4*>(p); }
+__device__ __forceinline__ float value8(const Eight<float>& x, int e) { return e < 4 ? x.lo[e & 3] : x.hi[e & 3]; }
+__device__ __forceinline__ float value8(const Eight<bf16_t>& x, int e) {
+  const uint32_t q = e < 2 ? x.v.x : e < 4 ? x.v.y : e < 6 ? x.v.z : x.v.w;
+  return __uint_as_float(e & 1 ? q & 0xffff0000u : q << 16);
 }
 
 // MT blocks of 16 rows of A; WK waves that split K (K % 32 == 0; rows of A and W aligned to 16 bytes).  A step is 32
@@ -84,33 +85,47 @@ f32_stream_kernel(const TA* __restrict__ a, const TW* __restrict__ w, TC* __rest
   f32x4_t acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  int s = begin;
-  for (; s + U <= end; s += U) {
-    float wv[U][8], av[U][MT][8];
+  // two batches of U steps in turn: while the MFMAs of one run, the loads of the other are on their way
+  Eight<TW> wv[2][U];
+  Eight<TA> av[2][U][MT];
+  auto load = [&](int buf, int s) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      load8(wp + (s + u) * 32, wv[u]);
+      fetch8(wp + (s + u) * 32, wv[buf][u]);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) load8(ap[m] + (s + u) * 32, av[u][m]);
+      for (int m = 0; m < MT; ++m) fetch8(ap[m] + (s + u) * 32, av[buf][u][m]);
     }
+  };
+  auto multiply = [&](int buf) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int e = 0; e < 8; ++e)
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][e], av[u][m][e], acc[m], 0, 0, 0);
+          acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(value8(wv[buf][u], e), value8(av[buf][u][m], e), acc[m], 0, 0, 0);
+  };
+  const int batches = (end - begin) / U;
+  if (batches > 0) load(0, begin);
+  int b = 0;
+  for (; b + 2 <= batches; b += 2) {
+    load(1, begin + (b + 1) * U);
+    multiply(0);
+    if (b + 2 < batches) load(0, begin + (b + 2) * U);
+    multiply(1);
   }
-  for (; s < end; ++s) {
-    float wv[8], av[MT][8];
-    load8(wp + s * 32, wv);
+  if (b < batches) multiply(0);
+  for (int s = begin + batches * U; s < end; ++s) {
+    Eight<TW> wl;
+    Eight<TA> al[MT];
+    fetch8(wp + s * 32, wl);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) load8(ap[m] + s * 32, av[m]);
+    for (int m = 0; m < MT; ++m) fetch8(ap[m] + s * 32, al[m]);
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[e], av[m][e], acc[m], 0, 0, 0);
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(value8(wl, e), value8(al[m], e), acc[m], 0, 0, 0);
   }
   if (wave > 0) {
 #pragma unroll
@@ -160,7 +175,7 @@ static int launch(const TA* a, const TW* w, TC* c, int M, int N, int K, int lda,
     ATOMA_LAUNCH_CHECK();
     return 0;
   }
-  const bool vec = aligned && K % 4 == 0;
+  const bool vec = aligned && K % kF32Step == 0;
   const int T = large >= kCUs ? 128 : 64;
   if (ceil_div(M, T) > 65535) return ATOMA_ERR_SHAPE;
   const dim3 grid(ceil_div(N, T), ceil_div(M, T)), block(256);
