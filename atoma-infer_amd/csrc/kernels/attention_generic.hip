@@ -24,7 +24,8 @@
 //
 // Measured on MI355X (float32, 32 heads over 8 of 64 columns, four layers; before: a wave per token and head, the values
 // read one token and 64 columns at a time, columns 64 bytes apart): 836 tokens of four prompts and sixteen steps of four
-// decoded tokens with 40 to 530 keys, 11.8 -> 2.1 ms in all: 79 us a layer for the prompts, 28 for four decoded tokens.
+// decoded tokens with 40 to 530 keys, 11.8 -> 1.25 ms in all: 63 us a layer for the prompts, 16 for four decoded tokens
+// (79 and 28 with loads under conditions, a block's values asked for behind its scores).
 // Bound by the chain of page number, keys and values of a wave's few blocks.
 #include "common.h"
 #include "cache_layout.h"
@@ -63,9 +64,11 @@ __device__ __forceinline__ f32x4 load4(const bf16_t* p) {
                __uint_as_float(u.y & 0xffff0000u)};
 }
 
-// HB: columns of keys and of values that the registers hold (32, 64, 128 or 256); NW: waves that share the keys.
-template <int HB, int NW, typename TQ, typename TC>
-__global__ void __launch_bounds__(64 * NW)
+// HB: columns of keys and of values that the registers hold (32, 64, 128 or 256); NW: waves that share the keys.  EXACT: keys
+// and values have HB columns and a block of sixteen keys lies in one page, in the MFMA's order: then no load stands under a
+// condition, all of a block's are on their way together, and the next block's page numbers with them.
+template <int HB, int NW, bool EXACT, typename TQ, typename TC>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, HB > 128 ? 1 : 8)))
 paged_attention_generic_kernel(const TQ* __restrict__ q, const TC* __restrict__ kcache, const TC* __restrict__ vcache,
                                TQ* __restrict__ out, GenericAttnArgs a) {
   constexpr int KG = HB / 32, VT = HB / 16;
@@ -86,7 +89,7 @@ paged_attention_generic_kernel(const TQ* __restrict__ q, const TC* __restrict__ 
   const float slope = a.slopes ? a.slopes[h] : 0.f;
   const int runs = a.hd / 8;
   const size_t k_tile = (size_t)a.page_size * a.hd, v_tile = (size_t)a.page_size * a.vd;
-  const bool whole_runs = (a.page_size & 15) == 0;      // a block of sixteen keys lies in one page, in the MFMA's order
+  const bool whole_runs = EXACT || (a.page_size & 15) == 0;
 
   float qv[KG][8];
 #pragma unroll
@@ -118,20 +121,43 @@ paged_attention_generic_kernel(const TQ* __restrict__ q, const TC* __restrict__ 
 #pragma unroll
     for (int v = 0; v < VT; ++v) acc[v] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // keys that nobody here may see are never read: their pages may be another request's by now
+    auto exists = [&](int j) { return j <= p_max && (j < kept || j >= first_min); };
+    auto base_of = [&](int b) { return 16 * (b < kept_blocks ? b : from + b - kept_blocks); };
+    auto key_of = [&](int base) { return exists(base + r16) ? base + r16 : p_max; };
+    // page numbers: of the lane's key, and of the block's values
+    int k_page = 0, v_page_no = 0;
+    auto pages_of = [&](int b) {
+      const int base = base_of(b < visits ? b : visits - 1);
+      k_page = table[key_of(base) / a.page_size];
+      if (whole_runs) v_page_no = table[base / a.page_size];
+    };
+    pages_of(wave);
     for (int b = wave; b < visits; b += NW) {
-      const int base = 16 * (b < kept_blocks ? b : from + b - kept_blocks);
-      // keys that nobody here may see are never read: their pages may be another request's by now
-      auto exists = [&](int j) { return j <= p_max && (j < kept || j >= first_min); };
-      const int j_key = exists(base + r16) ? base + r16 : p_max;
-      const TC* kt = kcache + ((size_t)table[j_key / a.page_size] * a.nkv + kvh) * k_tile + (size_t)(j_key % a.page_size) * 8;
+      const int base = base_of(b), j_key = key_of(base);
+      const TC* kt = kcache + ((size_t)k_page * a.nkv + kvh) * k_tile + (size_t)(j_key % a.page_size) * 8;
+      const size_t v_page = ((size_t)v_page_no * a.nkv + kvh) * v_tile;
+      const int v_off = whole_runs ? base % a.page_size : 0;
+      f32x4 vv[VT];
+      float kv[KG][8];
+      if constexpr (EXACT) {
+#pragma unroll
+        for (int g = 0; g < KG; ++g) load8(kt + (size_t)(kg + 4 * g) * a.page_size * 8, kv[g]);
+#pragma unroll
+        for (int v = 0; v < VT; ++v) vv[v] = load4(vcache + v_page + value_offset(v * 16 + r16, v_off + 4 * kg, HB, 16));
+      }
+      pages_of(b + NW);
       f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < KG; ++g) {
-        const int run = kg + 4 * g;
-        float kv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (run < runs) load8(kt + (size_t)run * a.page_size * 8, kv);
+        if constexpr (!EXACT) {
+          const int run = kg + 4 * g;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[g][e], sc, 0, 0, 0);
+          for (int e = 0; e < 8; ++e) kv[g][e] = 0.f;
+          if (run < runs) load8(kt + (size_t)run * a.page_size * 8, kv[g]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[g][e], qv[g][e], sc, 0, 0, 0);
       }
       // the lane's four keys of row r16
       bool vis[4], all_seen = true, all_there = true;
@@ -154,18 +180,15 @@ paged_attention_generic_kernel(const TQ* __restrict__ q, const TC* __restrict__ 
       l = l * corr + (pj[0] + pj[1] + pj[2] + pj[3]);
       m = m_new;
       // the lane's column of every sixteen, tokens 4 kg .. + 3
-      f32x4 vv[VT];
-      const size_t v_page = whole_runs ? ((size_t)table[base / a.page_size] * a.nkv + kvh) * v_tile : 0;
-      const int v_off = whole_runs ? base % a.page_size : 0;
       const bool all_rows = __all(all_seen);
       bool finite = true;
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
         const int d = v * 16 + r16;
-        vv[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (d < a.vd) {
+        if constexpr (!EXACT) vv[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (EXACT || d < a.vd) {
           if (whole_runs) {
-            vv[v] = load4(vcache + v_page + value_offset(d, v_off + 4 * kg, a.vd, a.page_size));
+            if constexpr (!EXACT) vv[v] = load4(vcache + v_page + value_offset(d, v_off + 4 * kg, a.vd, a.page_size));
             if (!all_there) {
 #pragma unroll
               for (int i = 0; i < 4; ++i) vv[v][i] = exists(base + 4 * kg + i) ? vv[v][i] : 0.f;
@@ -261,10 +284,23 @@ static void launch_generic(const TQ* q, const TC* kcache, const TC* vcache, TQ* 
   // (decode steps have another request in every token: a token a workgroup, and eight waves for its keys)
   a.tokens = one_each ? 1 : group >= kRows ? 1 : kRows / group;
   const dim3 grid((a.n_tokens + a.tokens - 1) / a.tokens, a.nkv * pieces);
-  if ((size_t)grid.x * grid.y < 512)
-    hipLaunchKernelGGL((paged_attention_generic_kernel<HB, 8, TQ, TC>), grid, dim3(512), 0, stream, q, kcache, vcache, out, a);
-  else
-    hipLaunchKernelGGL((paged_attention_generic_kernel<HB, 4, TQ, TC>), grid, dim3(256), 0, stream, q, kcache, vcache, out, a);
+  const bool exact = a.hd == HB && a.vd == HB && a.page_size % 16 == 0;
+  const bool many = (size_t)grid.x * grid.y >= 512;
+#define ATOMA_GEN(NW, E)                                                                                                  \
+  hipLaunchKernelGGL((paged_attention_generic_kernel<HB, NW, E, TQ, TC>), grid, dim3(64 * NW), 0, stream, q, kcache, vcache, \
+                     out, a)
+  // (wide heads hold more registers than eight waves a workgroup have)
+  if constexpr (HB <= 64) {
+    if (!many && exact) ATOMA_GEN(8, true);
+    else if (!many) ATOMA_GEN(8, false);
+    else if (exact) ATOMA_GEN(4, true);
+    else ATOMA_GEN(4, false);
+  } else {
+    (void)many;
+    if (exact) ATOMA_GEN(4, true);
+    else ATOMA_GEN(4, false);
+  }
+#undef ATOMA_GEN
 }
 
 extern "C" int atoma_paged_attention_generic(const void* q, int q_stride, const void* kcache, const void* vcache,
