@@ -669,7 +669,7 @@ extern "C" int atoma_route_max_tiles(int n_slots, int experts, int tile_m) {
 extern "C" int atoma_route_group(const int32_t* ids, int n_slots, int experts, int32_t* perm, int32_t* offsets,
                                  int32_t* tiles, int max_tiles, int tile_m, hipStream_t stream) {
   if (n_slots <= 0) return 0;
-  if (experts <= 0 || experts > 1024 || (tile_m != 16 && tile_m != 64 && tile_m != 128) ||
+  if (experts <= 0 || experts > 1024 || (tile_m != 16 && tile_m != 64 && tile_m != 128 && tile_m != 256) ||
       max_tiles < atoma_route_max_tiles(n_slots, experts, tile_m))
     return ATOMA_ERR_SHAPE;
   hipLaunchKernelGGL(route_group_kernel, dim3(1), dim3(1024), 0, stream, ids, n_slots, experts, perm, offsets, tiles,

@@ -40,6 +40,17 @@ struct TileOut {
   RopeArgs rope;
 };
 
+// Rows of X in groups, each against a weight of its own (experts): a row of tiles is one entry of a list (group, first row),
+// a group's rows end where the next one's begin, and the float32 result of row `place` goes, times scale, to the row of its
+// slot: choice slot % top of token slot / top, in plane slot % top of plane_rows rows.
+struct Groups {
+  const int32_t* tiles;      // [max_tiles][2]; group -1: nothing
+  const int32_t* offsets;    // [groups + 1]
+  const int32_t* perm;       // [places]: the place's slot
+  const float* scale;        // [slots] or null
+  int top, plane_rows;
+};
+
 // BM x BN: a workgroup's tile; WM x WN: its waves; S: LDS buffers.
 template <int BM_, int BN_, int WM_, int WN_, int S_>
 struct Tile {
@@ -224,21 +235,29 @@ __device__ __forceinline__ void meet() {
 }
 #endif
 
-template <typename C, int EPI>
+// (rows: M of X, or the entries of the groups' list times BM)
+template <typename C, int EPI, bool GROUPED>
 __global__ void __launch_bounds__(64 * C::NW, C::NW >= 8 ? 2 : 1)
-gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int M, int N, int ldx, int ldw, int k_len,
-                 TileOut out) {
+gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int rows, int N, int ldx, int ldw, int k_len,
+                 TileOut out, Groups groups) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
   // the tile: this XCD's run of the order, patches of kPatch rows of tiles, column by column
-  const int mt = (M + C::BM - 1) / C::BM, nt = (N + C::BN - 1) / C::BN;
+  const int mt = (rows + C::BM - 1) / C::BM, nt = (N + C::BN - 1) / C::BN;
   const int share = (mt * nt) >> 3, rest = (mt * nt) & 7, xcd = blockIdx.x & 7;
   const int id = xcd * share + min(xcd, rest) + (blockIdx.x >> 3);
   const int patch = id / (kPatch * nt), pm = min(kPatch, mt - patch * kPatch), in = id - patch * kPatch * nt;
-  const int m0 = (patch * kPatch + in % pm) * C::BM, n0 = (in / pm) * C::BN;
+  const int mi = patch * kPatch + in % pm, n0 = (in / pm) * C::BN;
   const int k0 = blockIdx.y * k_len;
+  int m0 = mi * C::BM, M = rows;
+  if constexpr (GROUPED) {
+    const int g = groups.tiles[2 * mi];
+    if (g < 0) return;
+    m0 = groups.tiles[2 * mi + 1], M = groups.offsets[g + 1];
+    w += (size_t)g * N * ldw;
+  }
 
   const int rows_x = min(C::BM, M - m0), rows_w = min(C::BN, N - n0);
   // (rows past the end: the last one, never stored)
@@ -318,6 +337,13 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const int m = m0 + wm * (C::BM / C::WM) + j * 16 + r16;
     const int nw = n0 + wn * (C::BN / C::WN);
     if (m >= M) continue;
+    size_t to_row = 0;
+    float to_scale = 1.f;
+    if constexpr (EPI == kOutF32 && GROUPED) {
+      const int slot = groups.perm[m];
+      to_row = (size_t)(slot % groups.top) * groups.plane_rows + slot / groups.top;
+      if (groups.scale) to_scale = groups.scale[slot];
+    }
     if constexpr (EPI == kOutSilu) {
       uint16_t* const row = (uint16_t*)out.c + (size_t)m * out.ldc;
 #pragma unroll
@@ -336,7 +362,9 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
         const int n = nw + i * 16 + kg * 4;
         if (nw + i * 16 >= N) continue;                // (N is a multiple of 16: a block is there or is not)
         const f32x4 v = acc[i][j];
-        if constexpr (EPI == kOutF32) {
+        if constexpr (EPI == kOutF32 && GROUPED) {
+          *reinterpret_cast<f32x4*>((float*)out.c + to_row * out.ldc + n) = v * to_scale;
+        } else if constexpr (EPI == kOutF32) {
           *reinterpret_cast<f32x4*>((float*)out.c + blockIdx.y * out.plane + (size_t)m * out.ldc + n) = v;
         } else if constexpr (EPI == kOutResid) {
           f32x4* const p = reinterpret_cast<f32x4*>((float*)out.c + (size_t)m * out.ldc + n);
@@ -354,17 +382,17 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 #endif
 }
 
-template <typename C, int EPI>
+template <typename C, int EPI, bool GROUPED = false>
 static int launch(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
-                  hipStream_t stream) {
+                  hipStream_t stream, const Groups& groups = Groups{}) {
   // (every device that the kernel is launched on has its own setting)
   constexpr int lds = EPI == kOutRope && C::BM * C::BN * 4 > C::LDS ? C::BM * C::BN * 4 : C::LDS;      // (the rotary epilogue's sums)
-  const hipError_t e = hipFuncSetAttribute((const void*)gemm_tile_kernel<C, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  const hipError_t e = hipFuncSetAttribute((const void*)gemm_tile_kernel<C, EPI, GROUPED>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return (int)e;
   const int64_t tiles = (int64_t)((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
   if (tiles > 0x7fffffff) return ATOMA_ERR_SHAPE;
-  hipLaunchKernelGGL((gemm_tile_kernel<C, EPI>), dim3((int)tiles, slices), dim3(64 * C::NW), lds, stream,
-                     (const uint16_t*)x, (const uint16_t*)w, M, N, ldx, ldw, K / slices, out);
+  hipLaunchKernelGGL((gemm_tile_kernel<C, EPI, GROUPED>), dim3((int)tiles, slices), dim3(64 * C::NW), lds, stream,
+                     (const uint16_t*)x, (const uint16_t*)w, M, N, ldx, ldw, K / slices, out, groups);
   ATOMA_LAUNCH_CHECK();
   return 0;
 }
@@ -414,5 +442,33 @@ extern "C" int atoma_gemm_tile(const void* x, const void* w, void* c, int kind, 
   if (kind == kOutF32) return pick<kOutF32>(tile, x, w, M, N, K, ldx, ldw, slices, out, stream);
   if (kind == kOutBF16) return pick<kOutBF16>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
   if (kind == kOutResid) return pick<kOutResid>(tile, x, w, M, N, K, ldx, ldw, 1, out, stream);
+  return ATOMA_ERR_SHAPE;
+}
+
+// The same for rows in groups (see Groups): x [places, K], w [groups, N, K], tiles [max_tiles][2] for tiles of the rows that
+// `tile` has.  kind 0: float32 planes by slot, [top][plane_rows][N]; kind 3: silu(gate) * up, bfloat16 [places, N / 2].
+extern "C" int atoma_gemm_tile_groups(const void* x, const void* w, void* c, int kind, int tile, int N, int K, const int32_t* tiles,
+                                      int max_tiles, const int32_t* offsets, const int32_t* perm, const float* scale, int top,
+                                      int plane_rows, hipStream_t stream) {
+  if (max_tiles <= 0 || N <= 0) return 0;
+  if (K <= 0 || K % 64 || N % 32 || K > (1 << 21) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)c & 15) ||
+      max_tiles > (1 << 20) || top <= 0 || plane_rows <= 0 || (kind == kOutSilu && scale != nullptr))
+    return ATOMA_ERR_SHAPE;
+  const TileOut out{c, kind == kOutSilu ? N / 2 : N, 0, RopeArgs{}};
+  const Groups groups{tiles, offsets, perm, scale, top, plane_rows};
+#define ATOMA_TILE(BM, ...)                                                                                                \
+  do {                                                                                                                     \
+    if (kind == kOutSilu)                                                                                                  \
+      return launch<Tile<BM, __VA_ARGS__>, kOutSilu, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);     \
+    if (kind == kOutF32)                                                                                                   \
+      return launch<Tile<BM, __VA_ARGS__>, kOutF32, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);      \
+  } while (0)
+  switch (tile) {
+    case 0: ATOMA_TILE(256, 256, 2, 4, 2); break;
+    case 1: ATOMA_TILE(256, 128, 4, 2, 3); break;
+    case 2: ATOMA_TILE(128, 128, 2, 4, 4); break;
+    case 3: ATOMA_TILE(128, 64, 2, 2, 4); break;
+  }
+#undef ATOMA_TILE
   return ATOMA_ERR_SHAPE;
 }

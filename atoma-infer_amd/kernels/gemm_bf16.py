@@ -350,6 +350,37 @@ def tile_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: int,
                                       _stream()), "gemm_tile")
 
 
+@functools.lru_cache(maxsize=4096)
+def tile_groups_plan(slots: int, groups: int, n_up: int, n_down: int, width: int, inter: int) -> Tuple[int, int, int]:
+    """(rows of a tile, tile of the first product, tile of the second) for ``slots`` rows in ``groups`` groups of about the same
+    size: x [., width] @ [n_up, width]^T, then [., inter] @ [n_down, inter]^T."""
+    best = None
+    for bm in (128, 256):
+        rows = -(-slots // (groups * bm)) * groups if slots >= groups else slots
+        choice, total = [], 0.0
+        for n, k in ((n_up, width), (n_down, inter)):
+            us, tile = min((-(-rows * -(-n // TILES[t][1]) // TILE_CUS) * (TILES[t][2] + k // 64 * TILES[t][3]), t)
+                           for t in TILES_SILU if TILES[t][0] == bm)
+            choice.append(tile)
+            total += us
+        if best is None or total < best[0]:
+            best = (total, bm, *choice)
+    return best[1:]
+
+
+def tile_groups(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: int, tile: int, tiles: torch.Tensor,
+                offsets: torch.Tensor, perm: torch.Tensor, top: int, scale: Optional[torch.Tensor] = None) -> None:
+    """The tile kernel over rows in groups: x [places, K] in the order of ``perm``, w [groups, N, K], ``tiles`` and ``offsets`` as
+    ``ops.route_group`` makes them for the tile's rows.  TILE_SILU: out bfloat16 [places, N / 2]; TILE_F32: out float32
+    [top, T, N] by slot, times ``scale`` [slots]."""
+    _, n, k = w.shape
+    if not (x.is_contiguous() and w.is_contiguous() and out.is_contiguous() and x.shape == (perm.numel(), k)
+            and k % 64 == 0 and n % 32 == 0 and offsets.numel() == w.shape[0] + 1):
+        raise ValueError("tile_groups: operands do not fit")
+    _check(tile_lib().atoma_gemm_tile_groups(_p(x), _p(w), _p(out), kind, tile, n, k, _p(tiles), tiles.shape[0], _p(offsets),
+                                             _p(perm), _p(scale), int(top), perm.numel() // top, _stream()), "gemm_tile_groups")
+
+
 def try_tile_swiglu(x, w: torch.Tensor, act="silu") -> Optional[torch.Tensor]:
     """``try_linear_swiglu`` for more rows than it takes, SiLU only: silu(gate) * up of x @ w^T, w [2 I, K] in blocks of 16
     rows, by the tile kernel; None where that does not take the shape."""

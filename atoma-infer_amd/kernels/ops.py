@@ -756,7 +756,7 @@ def route_topk(logits: torch.Tensor, top: int, score: str = "sigmoid", correctio
 
 def route_group(ids: torch.Tensor, experts: int, tile_m: int = 64):
     """Slots (token, choice) ordered by expert: (perm int32 [slots], offsets int32 [experts + 1], tiles int32
-    [max_tiles, 2] of (expert or -1, first place in perm)); a tile holds up to ``tile_m`` (16, 64 or 128) places."""
+    [max_tiles, 2] of (expert or -1, first place in perm)); a tile holds up to ``tile_m`` (16, 64, 128 or 256) places."""
     _dev(ids)
     _i32(ids, "ids")
     n = ids.numel()

@@ -43,9 +43,11 @@ from .linear import linear, linear_delta
 
 # places an expert, on average, up to which the streaming kernel takes the products (beyond, an expert's weight is read
 # again for every tile of 16 places).  Grouping, inputs and both products with 8 experts of 1,024 columns at width 2,048, 1 /
-# 8 / 32 / 48 / 64 places an expert: 23 / 25 / 42 / 59 / 74 us against 50 / 50 / 59 / 66 / 72 by tiles of 64; 4 of 32 experts of
-# 2,048 columns for 1 / 8 / 64 / 100 tokens: 24 / 98 / 147 / 168 against 63 / 147 / 201 / 215
-STREAM_PLACES = 24
+# 8 / 16 places an expert: 23 / 25 / 26 us against 50 / 50 / 52 by tiles of 64; 4 of 32 experts of 2,048 columns for 1 / 8 / 64 /
+# 100 tokens: 24 / 98 / 147 / 164 against 63 / 147 / 201 / 215.  Beyond, SiLU's go to the tile kernel of the dense products: the
+# 32 experts with 200 / 400 / 1,024 / 2,048 tokens 217 / 230 / 330 / 401 us against 262 streamed and 216 / 249 / 360 / 561 by
+# tiles of 64 and 128, which other activations keep; the 8 with 64 / 200 / 2,048 tokens 49 / 63 / 292 against 72 / 113 / 456
+STREAM_PLACES = 20
 
 
 class RoutedExperts(FeedForward):
@@ -166,6 +168,18 @@ class RoutedExperts(FeedForward):
                               swiglu=self.gated, relu2=not self.gated, act=self.activation)
             out = torch.empty((self.top, t, self.width), dtype=torch.float32, device=x.device)
             ops.expert_stream(h, self.w_down, out, perm, offsets, tiles, self.top, gather=False, planes=True, out_scale=w_out)
+            return out
+        if (self.mfma and x.dtype is torch.bfloat16 and self.gated and self.activation == "silu"
+                and self.width % 64 == 0 and self.inter % 64 == 0):
+            # many places an expert: the tile kernel of the dense products, a row of tiles an expert's run of places
+            from ..kernels import gemm_bf16 as gb
+            tile_m, up, down = gb.tile_groups_plan(slots, self.experts, rows, self.width, self.width, self.inter)
+            perm, offsets, tiles = ops.route_group(ids.view(-1), self.experts, tile_m)
+            xs = ops.gather_scale(x, w_in, perm, self.top)
+            h = torch.empty((slots, self.inter), dtype=torch.bfloat16, device=x.device)
+            gb.tile_groups(xs, self.w_gate_up, h, gb.TILE_SILU, up, tiles, offsets, perm, self.top)
+            out = torch.empty((self.top, t, self.width), dtype=torch.float32, device=x.device)
+            gb.tile_groups(h, self.w_down, out, gb.TILE_F32, down, tiles, offsets, perm, self.top, w_out)
             return out
         if self.mfma and x.dtype is torch.bfloat16:
             # tiles of 128 places where an expert has about a hundred or more (prompts): a weight fragment then

@@ -383,6 +383,35 @@ def test_expert_stream(counts, n, k):
         assert bool(((gate.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-5 * ref.abs().max()).all())
 
 
+@pytest.mark.parametrize("tile", range(4))
+@pytest.mark.parametrize("counts,n,k", [((3, 0, 300), 64, 64), ((128, 257, 1), 288, 192), ((90, 90, 90, 90), 544, 640)])
+def test_gemm_tile_groups(tile, counts, n, k):
+    """The tile kernel over experts' runs of places: whole, short and empty tiles, both results, against float64 (bounds as in
+    ``test_expert_stream``)."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb, ops
+    top = 2
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)]).int()
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))]
+    ids = ids[: len(ids) // top * top].to(DEV)
+    t = ids.numel()
+    x, w, score = rnd(t, k, dtype=torch.bfloat16, seed=2), rnd(len(counts), n, k, dtype=torch.bfloat16, seed=3), rnd(t, seed=4).abs()
+    perm, offsets, tiles = ops.route_group(ids, len(counts), gb.TILES[tile][0])
+    expert = ids.long()[perm.long()]            # (of a place)
+    want = torch.stack([x[i].double() @ w[expert[i]].double().T for i in range(t)])
+    size = torch.stack([x[i].double().abs() @ w[expert[i]].double().abs().T for i in range(t)])
+    for scale in (None, score):
+        out = torch.full((top, t // top, n), 7.0, device=DEV)
+        gb.tile_groups(x, w, out, gb.TILE_F32, tile, tiles, offsets, perm, top, scale)
+        got = out.transpose(0, 1).reshape(t, n)[perm.long()].double()
+        f = (torch.ones_like(score) if scale is None else scale)[perm.long()][:, None].double()
+        assert bool(((got - want * f).abs() <= (k * 2.0 ** -24 * size + 2.0 ** -23 * want.abs()) * f).all())
+    gate = torch.empty(t, n // 2, dtype=torch.bfloat16, device=DEV)
+    gb.tile_groups(x, w, gate, gb.TILE_SILU, tile, tiles, offsets, perm, top)
+    z = want.view(t, n // 32, 2, 16)
+    ref = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(t, n // 2)
+    assert bool(((gate.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
+
+
 TWO_PIECE_CASES = [c for c in ATTN_CASES if c[2] <= 64] + [
     # groups of 1, 3, 8, 33 and 40 heads (tiles of 256, 255, 256, 264, 240 rows; the last pieces are short or half
     # empty), one token, a window, portions beside decoded tokens
