@@ -484,7 +484,7 @@ LOWRANK_UP_MAX_TOKENS = 32      # beyond, the general product reads a tile of th
 
 def lowrank_up(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x float32 [T, K] (row stride free) times w [N, K] transposed, float32 out, for few tokens and a small K: the
-    second half of a low-rank map (float32 multiply-adds in ascending order of k, as the general product's)."""
+    second half of a low-rank map (float32 multiply-adds in ascending order of k)."""
     _dev(x, w)
     t, k = x.shape
     n = w.shape[0]

@@ -136,14 +136,14 @@ class PagedAttention(Mixer):
         from ..kernels import attention_bf16
         if cache_dtype is torch.bfloat16 and self.hd % 16:
             import warnings
-            warnings.warn(f"bfloat16 attention with heads of {self.hd} columns runs the general kernel (one wave per "
-                          f"token and head), many times slower than the matrix-core kernel, which takes head sizes "
+            warnings.warn(f"bfloat16 attention with heads of {self.hd} columns runs the general kernel (float32 "
+                          f"matrix instructions), many times slower than the bfloat16 kernel, which takes head sizes "
                           f"that are multiples of 16", stacklevel=2)
             return None
         if cache_dtype is torch.bfloat16 and not attention_bf16.page_ok(page_size):
             import warnings
-            warnings.warn(f"bfloat16 attention with pages of {page_size} tokens runs the general kernel (one wave per "
-                          f"token and head), many times slower than the matrix-core kernel, which needs pages of a "
+            warnings.warn(f"bfloat16 attention with pages of {page_size} tokens runs the general kernel (float32 "
+                          f"matrix instructions), many times slower than the bfloat16 kernel, which needs pages of a "
                           f"multiple of 16 tokens ([cache] block_size = 16, 32, 64, ...)", stacklevel=2)
         if cache_dtype is not torch.bfloat16 or not attention_bf16.page_ok(page_size):
             return None
