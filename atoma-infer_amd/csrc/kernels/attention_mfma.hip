@@ -64,9 +64,18 @@ constexpr int RUNS = PAGE / 16;        // runs of 16 tokens a page; a run of val
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kSlack = 8.0f;   // see the softmax in the kernel
 
+// Whether prompt tiles may share their keys through LDS (see the shared walk in the kernel): heads whose keys and values divide
+// into whole kilobytes a wave.  From kSharedMinKeys keys on: with 32 / 24 heads of 128 over 8 KV heads, four prompts of 500 tokens
+// take 26.7 us either way / 23.3 against 24.0, two of 1,000 33.9 against 37.2 with every wave's own loads.
+constexpr bool kShared = !BIASED && VD == HD && HD % 64 == 0 && HD <= 128;
+constexpr int kSharedMinKeys = 512, kSharedSlots = 4;
+constexpr size_t kSharedBytes = kShared ? (size_t)HD * 128 * 2 * kSharedSlots : 0;      // of LDS: a slot is 64 keys or values
+
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((address_space(3))) char* lds_bytes;
+typedef const __attribute__((address_space(3))) bf16x8* lds_frag;
 
 struct Task {
   int32_t entry;    // row of the block tables; < 0: nothing to do
@@ -200,11 +209,12 @@ __device__ __forceinline__ void merge_parts(const float* __restrict__ part_o, co
 // instructions (about a hundred a block and piece, a third of their time the sixteen exponentials), so portions
 // behind long prefixes gain (2,048 tokens behind 30,720: 741 -> 682 us at head size 64, behind 63,488: 1,495 ->
 // 1,355, behind 14,336: 376 -> 363); short prompts lose, because twice as few waves, each with a chain twice as
-// long, fill the GPU worse.  The host asks for two pieces from 16,384 keys on.
-// (the registers that the bias takes would cost heads of up to 64 columns the fourth wave of a SIMD, and with it the
+// long, fill the GPU worse.  The host asks for two pieces from 16,384 keys on where the tile's waves do not share their keys
+// through LDS (kShared), which is quicker there.
+// (the registers that the bias or the shared walk take would cost heads of 64 columns the fourth wave of a SIMD, and with it the
 // second workgroup of a CU; asked to, the compiler finds them)
 template <int TASKS, int KSPLIT, int RT = 1>
-__global__ void __launch_bounds__(64 * TASKS * KSPLIT, (BIASED && HD == 64 && VD == 64 && KSPLIT > 1 && RT == 1) ? 4 : 1)
+__global__ void __launch_bounds__(64 * TASKS * KSPLIT, (HD == 64 && VD == 64 && KSPLIT > 1 && RT == 1) ? 4 : 1)
 attention_mfma_kernel(const Task* __restrict__ tasks, int n_tasks, int nkv, const uint16_t* __restrict__ q,
                       int q_stride, int nh, const int32_t* __restrict__ block_tables, int max_blocks, int window,
                       const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
@@ -367,6 +377,68 @@ attention_mfma_kernel(const Task* __restrict__ tasks, int n_tasks, int nkv, cons
     }
   };
 
+  auto rescale = [&](int t, float bmax) {
+    // The reference point m of a row's exponentials follows its maximum only in jumps: as long as no row of the
+    // wave has grown by more than kSlack (in powers of two) beyond its m, m stays, the weights may exceed one (by
+    // at most 2^kSlack, nothing to float32 sums or to bfloat16 weights, whose precision is relative) and the
+    // accumulators need no rescaling, which is most of a block's vector work.  out = o / l does not depend on m.
+    const float m_new = fmaxf(m[t], bmax);
+    const bool grew = __ballot(m_new > m[t] + kSlack) != 0;    // (-inf + kSlack = -inf: a row's first key always counts)
+    if (grew) {
+      const float corr = __builtin_amdgcn_exp2f(m[t] - ((m_new == -INFINITY) ? 0.f : m_new));
+      l[t] *= corr;
+#pragma unroll
+      for (int dt = 0; dt < DTILES; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[t][dt][i] *= corr;
+      m[t] = m_new;
+    }
+  };
+  // Online softmax; accumulator element i is key kb + (i/4)*8 + hg*4 + i%4.  The running maximum is kept in
+  // units of the scaled score (score * scale * log2 e), so one fused multiply-add feeds exp2.  Only blocks
+  // that touch a row's own position, the window's edge or the end of the key range need the mask.
+  auto soften = [&](int t, f32x16& s, int rk, int kb, int k_end, float* sv) {
+    const bool edge = rk + 31 > p_lo || rk < lo_hi || kb + 32 > k_end;
+    float bmax = -INFINITY;
+    if constexpr (BIASED) {
+#pragma unroll
+      for (int i = 1; i < 16; ++i) s[i] = fmaf(per_key[t], (float)((i >> 2) * 8 + (i & 3)), s[i]);
+    }
+    // the bias of this lane's first key, in the units of the exponentials
+    const float at = BIASED ? per_key[t] * sc2 * (float)(rk + hg * 4 - p_row[t]) : 0.f;
+    if (edge) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int off = (i >> 2) * 8 + hg * 4 + (i & 3), key = rk + off;
+        const bool ok = key <= p_row[t] && (key >= lo_row[t] || (BIASED && key < keep)) && kb + off < k_end;
+        sv[i] = ok ? s[i] : -INFINITY;
+        bmax = fmaxf(bmax, sv[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        sv[i] = s[i];
+        bmax = fmaxf(bmax, sv[i]);
+      }
+    }
+    if constexpr (BIASED) {
+      bmax = fmaf(bmax, sc2, at);      // (the halves' first keys differ)
+      bmax = fmaxf(bmax, from_other_half(bmax, hg != 0));
+    } else {
+      bmax = fmaxf(bmax, from_other_half(bmax, hg != 0)) * sc2;
+    }
+    rescale(t, bmax);
+    const float m_use = (m[t] == -INFINITY) ? 0.f : m[t];
+    const float less = BIASED ? at - m_use : -m_use;
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      sv[i] = __builtin_amdgcn_exp2f(fmaf(sv[i], sc2, less));
+      psum += sv[i];
+    }
+    l[t] += psum;      // this lane's half of the row's sum; the halves meet after the last block
+  };
+
   // Keys run one block ahead of the values.  A block's values are asked for when its turn begins and arrive while
   // S^T and the softmax run; the next block's keys are asked for as soon as S^T has used the registers of this
   // block's, and arrive while the softmax and the P.V products run.  So no fragment needs registers of its own to wait
@@ -413,67 +485,11 @@ attention_mfma_kernel(const Task* __restrict__ tasks, int n_tasks, int nkv, cons
       asm volatile("" ::: "memory");
     }
 
-    // Online softmax; accumulator element i is key kb + (i/4)*8 + hg*4 + i%4.  The running maximum is kept in
-    // units of the scaled score (score * scale * log2 e), so one fused multiply-add feeds exp2.  Only blocks
-    // that touch a row's own position, the window's edge or the end of the key range need the mask.
-    const bool edge = rk + 31 > p_lo || rk < lo_hi || kb + 32 > k_end;
 #pragma unroll
     for (int t = 0; t < RT; ++t) {
       if (!piece_on[t]) continue;
       float sv[16];
-      float bmax = -INFINITY;
-      if constexpr (BIASED) {
-#pragma unroll
-        for (int i = 1; i < 16; ++i) s[t][i] = fmaf(per_key[t], (float)((i >> 2) * 8 + (i & 3)), s[t][i]);
-      }
-      // the bias of this lane's first key, in the units of the exponentials
-      const float at = BIASED ? per_key[t] * sc2 * (float)(rk + hg * 4 - p_row[t]) : 0.f;
-      if (edge) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int off = (i >> 2) * 8 + hg * 4 + (i & 3), key = rk + off;
-          const bool ok = key <= p_row[t] && (key >= lo_row[t] || (BIASED && key < keep)) && kb + off < k_end;
-          sv[i] = ok ? s[t][i] : -INFINITY;
-          bmax = fmaxf(bmax, sv[i]);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          sv[i] = s[t][i];
-          bmax = fmaxf(bmax, sv[i]);
-        }
-      }
-      if constexpr (BIASED) {
-        bmax = fmaf(bmax, sc2, at);      // (the halves' first keys differ)
-        bmax = fmaxf(bmax, from_other_half(bmax, hg != 0));
-      } else {
-        bmax = fmaxf(bmax, from_other_half(bmax, hg != 0)) * sc2;
-      }
-      // The reference point m of a row's exponentials follows its maximum only in jumps: as long as no row of the
-      // wave has grown by more than kSlack (in powers of two) beyond its m, m stays, the weights may exceed one (by
-      // at most 2^kSlack, nothing to float32 sums or to bfloat16 weights, whose precision is relative) and the
-      // accumulators need no rescaling, which is most of a block's vector work.  out = o / l does not depend on m.
-      const float m_new = fmaxf(m[t], bmax);
-      const bool grew = __ballot(m_new > m[t] + kSlack) != 0;    // (-inf + kSlack = -inf: a row's first key always counts)
-      if (grew) {
-        const float corr = __builtin_amdgcn_exp2f(m[t] - ((m_new == -INFINITY) ? 0.f : m_new));
-        l[t] *= corr;
-#pragma unroll
-        for (int dt = 0; dt < DTILES; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[t][dt][i] *= corr;
-        m[t] = m_new;
-      }
-      const float m_use = (m[t] == -INFINITY) ? 0.f : m[t];
-      const float less = BIASED ? at - m_use : -m_use;
-      float psum = 0.f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        sv[i] = __builtin_amdgcn_exp2f(fmaf(sv[i], sc2, less));
-        psum += sv[i];
-      }
-      l[t] += psum;      // this lane's half of the row's sum; the halves meet after the last block
-
+      soften(t, s[t], rk, kb, k_end, sv);
       // O^T += V^T P^T
       const bf16x8 pf0 = pack8(sv), pf1 = pack8(sv + 8);
 #pragma unroll
@@ -483,9 +499,185 @@ attention_mfma_kernel(const Task* __restrict__ tasks, int n_tasks, int nkv, cons
       }
     }
   };
-  int kb = k_first;
-  for (; kb + STRIDE < k_end; kb += STRIDE) turn(kb, std::true_type{});
-  if (kb < k_end) turn(kb, std::false_type{});
+  // The shared walk: the four tasks of a prompt tile see the same keys, so their eight waves take them through LDS together,
+  // 64 keys a turn, the two waves of a task 32 each (as in the walk above, and in the same order: the results' bits are the same).
+  // Every wave loading its own fragments asks for 16 KB of keys and values (heads of 128) per 16 MFMAs, four times what the L1
+  // can hold in flight for eight waves: what bounded it were those loads (27 % of the matrix cores' rate at 2,048 tokens behind
+  // 14,336).  Here a turn brings 32 KB for all eight waves, memory to LDS directly (buffer_load ... lds; a page's tile is already in
+  // the order of the fragments, so a load copies a kilobyte and every read of LDS is a straight one, free of bank conflicts).
+  //   * Turn t multiplies the keys of turn t + 1 while it weighs the scores of turn t: matrix instructions, exponentials and sums
+  //     of one wave in one stretch without branches, dealt by sched_group_barrier.  (Two groups of waves half a turn apart, one
+  //     at the matrix cores and one at the exponentials, with two barriers a turn: 543 us where this takes 509.)
+  //   * Four slots of keys and of values: those of turn t + 4 (values: t + 3) are asked for when turn t begins, three turns ahead.
+  //   * Page numbers come by scalar loads a turn ahead, and are waited for before the turn ends: a scalar load in flight would
+  //     make the compiler wait for all LDS reads at once.
+  // 32 heads of 128, us: 2,048 tokens 65 -> 52, behind 2,048 146 -> 112, behind 14,336 698 -> 509 (1.0 PFLOP/s, the clock then
+  // falls to 1.7 GHz).  32 heads of 64, whose exponentials weigh as much as their MFMAs: 2,048 tokens 32.8 -> 32.4, behind 2,048 72 -> 65,
+  // behind 16,384 380 -> 321 (two pieces a wave: about 370).
+  bool shared = false;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (kShared && TASKS == 4 && KSPLIT == 2 && RT == 1) {
+    // (the host lists a tile's tasks in fours; chunks of decoded tokens, whose tasks see different keys, walk on their own)
+    const int first = (blockIdx.x / nkv) * TASKS;
+    const bool whole = first + TASKS <= n_tasks;
+    const Task lead = tasks[whole ? first : 0];
+    shared = whole && lead.entry >= 0 && lead.dest < 0 && lead.k_end - lead.k_begin >= kSharedMinKeys;
+#pragma unroll
+    for (int i = 1; i < TASKS; ++i) {
+      const Task other = tasks[whole ? first + i : 0];
+      shared = shared && (other.entry < 0 || (other.dest < 0 && other.entry == lead.entry && other.k_begin == lead.k_begin &&
+                                              other.k_end == lead.k_end));
+    }
+    if (shared) {
+      extern __shared__ __attribute__((aligned(1024))) char ring[];
+      typedef __amdgpu_buffer_rsrc_t rsrc_t;
+      typedef const __attribute__((address_space(4))) int32_t* table_ptr;
+      // a run of 16 keys of one head, a turn's four runs; loads of a kilobyte: of a run, and of a wave (keys and values each)
+      constexpr int RUN = HD * 32, TILE = 4 * RUN, LOADS = HD >= 32 ? HD / 32 : 1, PW = HD >= 64 ? HD / 64 : 1;
+      const int kb0 = __builtin_amdgcn_readfirstlane(lead.k_begin), ke = __builtin_amdgcn_readfirstlane(lead.k_end);
+      const int turns = (ke - kb0 + 63) / 64;
+      const table_ptr pages = (table_ptr)(uintptr_t)(block_tables + (size_t)__builtin_amdgcn_readfirstlane(lead.entry) * max_blocks);
+      const lds_bytes keys = (lds_bytes)ring, vals = keys + kSharedSlots * TILE;
+      // The first key of the run that this wave's load j of turn t's keys takes; beyond the range, the last key's run (what it
+      // brings is masked)
+      auto key_in = [&](int t, int j) { return (uint32_t)min(ke - 1, kb0 + t * 64 + (j * 8 + wave) / LOADS * 16); };
+      uint32_t pk[PW], pv[PW];         // pages of the next keys to be asked for, and of the values, which are a turn behind
+      auto ask_pages = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < PW; ++j) pv[j] = pk[j], pk[j] = (uint32_t)pages[key_in(t, j) / (uint32_t)PAGE];
+      };
+      const uint32_t k_bytes = (uint32_t)k_page_stride * 2, v_bytes = (uint32_t)v_page_stride * 2;
+      const uint32_t k_off = ((uint32_t)(lane >> 4) * PAGE + (lane & 15)) * 16, v_off = lane * 16;
+      // the keys of turn t to kd, the values of turn t - 1 to vd
+      auto issue = [&](lds_bytes __restrict__ kd, lds_bytes __restrict__ vd, int t) {
+#pragma unroll
+        for (int j = 0; j < PW; ++j) {
+          const int run = (j * 8 + wave) / LOADS, piece = (j * 8 + wave) % LOADS, to = run * RUN + piece * 1024;
+          const uint32_t rk = RUNS == 1 ? 0 : key_in(t, j) / 16 % RUNS, rv = RUNS == 1 ? 0 : key_in(t - 1, j) / 16 % RUNS;
+          const rsrc_t ks = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)k_tiles + (uint64_t)pk[j] * k_bytes), 0, PAGE * HD * 2, 0x00027000);
+          const rsrc_t vs = __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)v_tiles + (uint64_t)pv[j] * v_bytes), 0, PAGE * VD * 2, 0x00027000);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(ks, (__attribute__((address_space(3))) void*)(kd + to), 16, k_off,
+                                                   rk * 256 + piece * (4 * PAGE * 16), 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(vs, (__attribute__((address_space(3))) void*)(vd + to), 16, v_off,
+                                                   rv * (32 * VD) + piece * 1024, 0, 0);
+        }
+      };
+      auto meet = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+      };
+      // at most n loads on their way, no LDS read
+      constexpr auto waits = [](int n) { return (n & 15) | (7 << 4) | ((n >> 4) << 14); };
+      constexpr int NEWER = 2 * PW * (kSharedSlots - 2);
+      const uint32_t k_at = (2 * part + (c >> 4)) * RUN + hg * 256 + (c & 15) * 16, v_at = 2 * part * RUN + lane * 16;
+      bf16x8 pf[2], kfs[KSTEPS], vfs[2][DTILES];
+      auto read_keys = [&](const lds_bytes __restrict__ rk) {
+#pragma unroll
+        for (int st = 0; st < KSTEPS; ++st) kfs[st] = *(lds_frag)(rk + k_at + st * 512);
+      };
+      auto scores = [&](f32x16& d) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) d[i] = 0.f;
+#pragma unroll
+        for (int st = 0; st < KSTEPS; ++st) d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfs[st], qf[0][st], d, 0, 0, 0);
+      };
+      auto weighted = [&]() {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int dt = 0; dt < DTILES; ++dt) o[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfs[j][dt], pf[j], o[0][dt], 0, 0, 0);
+      };
+      // Turn t: rk holds the keys of turn t + 1, rv the values of turn t; tk and tv, the slots of turn t's keys and of turn t - 1's
+      // values, which nobody reads any more, take those of turns t + kSharedSlots and one before it.  s: this turn's scores, next:
+      // the next one's.  (That the pointers promise not to overlap keeps the compiler from waiting for the loads before the reads.)
+      auto share = [&](const lds_bytes __restrict__ rk, const lds_bytes __restrict__ rv, lds_bytes __restrict__ tk, lds_bytes __restrict__ tv,
+                       int t, f32x16& s, f32x16& next, auto behind) __attribute__((always_inline)) {
+        meet();
+        const bool more = t + kSharedSlots - 1 < turns;
+        if (more) issue(tk, tv, t + kSharedSlots);
+        read_keys(rk);
+        if constexpr (decltype(behind)::value) weighted();          // the turn before's weights with its values
+        const int kb = kb0 + t * 64 + 32 * part;
+        float bmax = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) bmax = fmaxf(bmax, s[i]);
+        if (kb + 31 > p_lo || kb < lo_hi || kb + 32 > ke) {
+          bmax = -INFINITY;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = kb + (i >> 2) * 8 + hg * 4 + (i & 3);
+            s[i] = key <= p_row[0] && key >= lo_row[0] && key < ke ? s[i] : -INFINITY;
+            bmax = fmaxf(bmax, s[i]);
+          }
+        }
+        bmax = fmaxf(bmax, from_other_half(bmax, hg != 0)) * sc2;
+        rescale(0, bmax);
+        const float less = (m[0] == -INFINITY) ? 0.f : -m[0];
+        ask_pages(t + kSharedSlots + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        scores(next);
+        float sv[16], psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          sv[i] = __builtin_amdgcn_exp2f(fmaf(s[i], sc2, less));
+          psum += sv[i];
+        }
+        l[0] += psum;
+        pf[0] = pack8(sv), pf[1] = pack8(sv + 8);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int dt = 0; dt < DTILES; ++dt) vfs[j][dt] = *(lds_frag)(rv + v_at + j * RUN + dt * 1024);
+#pragma unroll
+        for (int i = 0; i < KSTEPS; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                // a matrix instruction,
+          __builtin_amdgcn_sched_group_barrier(0x400, 16 / KSTEPS, 0);    // its share of the exponentials,
+          __builtin_amdgcn_sched_group_barrier(0x2, 40 / KSTEPS, 0);      // of the other vector instructions
+          __builtin_amdgcn_sched_group_barrier(0x100, 2 * DTILES / KSTEPS > 0 ? 2 * DTILES / KSTEPS : 1, 0);   // and of the LDS reads
+        }
+        // (nothing of this stretch may sink below it)
+        asm volatile("" : "+v"(pf[0]), "+v"(pf[1]), "+v"(l[0]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < PW; ++j) asm volatile("" ::"s"(pk[j]));
+        if (more) __builtin_amdgcn_s_waitcnt(waits(NEWER));
+        else __builtin_amdgcn_s_waitcnt(waits(0));
+      };
+      auto at = [&](int t) { return t % kSharedSlots * TILE; };
+#pragma unroll
+      for (int j = 0; j < PW; ++j) pk[j] = (uint32_t)pages[key_in(0, j) / (uint32_t)PAGE];
+#pragma unroll
+      for (int t = 0; t < kSharedSlots; ++t) {        // (the values before turn 0: turn 0's, into a slot that is written anew)
+        ask_pages(t);
+        issue(keys + t * TILE, vals + at(t + kSharedSlots - 1), t);
+      }
+      ask_pages(kSharedSlots);
+      __builtin_amdgcn_s_waitcnt(waits(NEWER));
+      meet();
+      f32x16 s0, s1;
+      read_keys(keys);
+      scores(s0);
+      share(keys + at(1), vals, keys, vals + at(kSharedSlots - 1), 0, s0, s1, std::false_type{});
+      int t = 1;
+      for (; t + 1 < turns; t += 2) {
+        share(keys + at(t + 1), vals + at(t), keys + at(t), vals + at(t + kSharedSlots - 1), t, s1, s0, std::true_type{});
+        share(keys + at(t + 2), vals + at(t + 1), keys + at(t + 1), vals + at(t + kSharedSlots), t + 1, s0, s1, std::true_type{});
+      }
+      if (t < turns) share(keys + at(t + 1), vals + at(t), keys + at(t), vals + at(t + kSharedSlots - 1), t, s1, s0, std::true_type{});
+      weighted();
+      __builtin_amdgcn_s_waitcnt(waits(0));
+      meet();         // (the merge below writes where the slots were)
+    }
+  }
+#endif
+  if (!shared) {
+    int kb = k_first;
+    for (; kb + STRIDE < k_end; kb += STRIDE) turn(kb, std::true_type{});
+    if (kb < k_end) turn(kb, std::false_type{});
+  }
 
   if constexpr (KSPLIT > 1) {
     // Merge the shares of a task: the waves with part > 0 lay down (m, l, o), lane by lane; the wave with part 0
@@ -780,7 +972,7 @@ extern "C" int atoma_attention_mfma(const void* q, int q_stride, const void* kca
   if (ksplit == 1 && !kSplit2Fits && (size_t)n_tasks * nkv <= 1024) ATOMA_ATTN(1, 1, 0);
   else if (ksplit == 1) ATOMA_ATTN(4, 1, 0);
   else if (ksplit == 2 && row_tiles == 2) ATOMA_ATTN(4, 2, 2 * kMerge2Bytes, (kTwoPieces ? 2 : 1));
-  else if (ksplit == 2 && kSplit2Fits) ATOMA_ATTN(4, (kSplit2Fits ? 2 : 1), kMerge2Bytes);
+  else if (ksplit == 2 && kSplit2Fits) ATOMA_ATTN(4, (kSplit2Fits ? 2 : 1), (kSharedBytes > kMerge2Bytes ? kSharedBytes : kMerge2Bytes));
   else if (ksplit == 4 && kSplit4Fits) ATOMA_ATTN(2, (kSplit4Fits ? 4 : 1), kMerge4Bytes);
   else if (ksplit == 8 && kSplit8Fits) ATOMA_ATTN(1, (kSplit8Fits ? 8 : 1), kMerge8Bytes);
   else return ATOMA_ERR_SHAPE;

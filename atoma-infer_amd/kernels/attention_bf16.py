@@ -92,6 +92,13 @@ def max_row_tiles_for(hd: int, vd: Optional[int] = None) -> int:
     return 2 if max(hd, vd or hd) <= 64 else 1
 
 
+def shares_keys(hd: int, vd: Optional[int] = None, biased: bool = False) -> bool:
+    """Whether the waves of a prompt tile take long key ranges through LDS together (``kShared`` in the kernel module): a wave
+    of one piece of rows then keeps more of the GPU busy than one of two (2,048 tokens behind 16,384, 32 heads of 64: 321 us
+    against about 370), so such layers ask for one."""
+    return not biased and (vd is None or vd == hd) and hd in (64, 128)
+
+
 # (request, KV head) pairs from which on a decoded token's keys are not cut into chunks: measured on MI355X (256 CUs),
 # half as many pairs as CUs win at contexts from 2,000 to 32,000 tokens; with 64 pairs chunks win from 2,000 keys on
 WHOLE_MIN_PAIRS = 128

@@ -569,6 +569,50 @@ def test_gemm_tile_groups(tile, counts, n, k):
     assert bool(((gate.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
 
 
+# prompt tiles of 512 keys and more: their waves take the keys through LDS together, 64 a turn.  (nh, nkv, hd, page, window, entries)
+SHARED_CASES = [
+    # 8, 9 and 12 turns; the last one full, of one key, of 33 keys (a whole wave's share is masked) and of 63
+    (4, 1, 64, 16, 0, [(480, 32), (481, 32), (700, 33), (735, 32)]),
+    (4, 1, 128, 16, 0, [(480, 32), (481, 32), (700, 33), (735, 32)]),
+    # a tile of 511 keys (its waves walk alone) beside one of 543; heads that leave pieces of the tile empty
+    (6, 2, 128, 16, 0, [(0, 520), (600, 17)]),
+    (3, 3, 64, 16, 0, [(500, 140)]),
+    # windows and chunks, whose walks begin inside a page and not at 0
+    (8, 2, 64, 16, 600, [(1000, 70), (0, 640)]),
+    (4, 2, 128, 16, 777, [(900, 60)]),
+    # pages of several runs of 16 keys; a turn's runs lie in up to four pages
+    (8, 2, 64, 48, 0, [(590, 40)]),
+    (4, 2, 128, 32, 0, [(611, 50)]),
+    (8, 2, 64, 64, 523, [(701, 45), (0, 600)]),
+    (2, 2, 128, 64, 0, [(1029, 131)]),
+]
+
+
+@pytest.mark.parametrize("nh,nkv,hd,page,window,entries", SHARED_CASES)
+def test_attention_tiles_that_share_their_keys(nh, nkv, hd, page, window, entries, monkeypatch):
+    """Against 64 bits; weights and results are rounded to bfloat16 once each (2^-9), and the weights of a row add up to 1."""
+    from atoma_infer_amd.kernels import attention_bf16
+    attention_bf16.lib(hd, page=page)
+    monkeypatch.setattr(attention_bf16, "max_waves_for", lambda *a: 2)       # two waves a task, as in steps that fill the GPU
+    starts, counts = [s for s, _ in entries], [c for _, c in entries]
+    ks, vs, kc, vc, bt = paged_setup([s + c for s, c in entries], nkv, hd, page, torch.bfloat16, seed=hd + nh + page)
+    t = sum(counts)
+    g = torch.Generator().manual_seed(1)
+    qkv = (torch.randn(t, (nh + 2 * nkv) * hd, generator=g) * 1.5).bfloat16().to(DEV)
+    out = torch.full((t, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ctx, cache = FakeCtx(starts, counts), FakeCache(bt, page)
+    assert attention_bf16.try_attention(qkv, kc, vc, out, ctx, cache, hd ** -0.5, window, nh, nkv, hd)
+    plan = [v for k, v in ctx.scratch.items() if k[0] == "attention_tasks_adhoc"][0]
+    assert plan[1][3] == 2 and attention_bf16.shares_keys(hd)
+    row = 0
+    for e, (s0, c) in enumerate(entries):
+        q = qkv[row:row + c, : nh * hd].cpu().view(c, nh, hd)
+        want = plain_attention(q, ks[e], vs[e], s0, hd ** -0.5, window, nh // nkv).reshape(c, nh * hd)
+        got = out[row:row + c].double().cpu()
+        assert bool(((got - want).abs() <= 2.0 ** -9 * want.abs() + 2.0 ** -9 * vs[e].abs().max()).all()), f"entry {e} ({s0}, {c})"
+        row += c
+
+
 TWO_PIECE_CASES = [c for c in ATTN_CASES if c[2] <= 64] + [
     # groups of 1, 3, 8, 33 and 40 heads (tiles of 256, 255, 256, 264, 240 rows; the last pieces are short or half
     # empty), one token, a window, portions beside decoded tokens
