@@ -155,77 +155,48 @@ static int sample_splits(int n_rows, int vocab) {
   return s < 1 ? 1 : s > kMaxSplits ? kMaxSplits : s;
 }
 
-__global__ void __launch_bounds__(kSampThreads)
-sample_kernel(const float* __restrict__ logits, int ld, int vocab, const float* __restrict__ temperature,
-              const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
-              float* __restrict__ weights, int32_t* __restrict__ out_token, float* __restrict__ out_logit) {
-  __shared__ ArgMax am[kSampWaves];
-  __shared__ uint32_t hist_k[kBins];       // top-k search: how many weights fall into each bin
-  __shared__ uint32_t hist_pn[kBins];      // top-p search: how many, and their mass
-  __shared__ u64 hist_pm[kBins];
-  __shared__ u64 wave_u64[kSampWaves];
-  __shared__ uint32_t wave_u32[kSampWaves];
-  __shared__ u64 slice_mass[kSampWaves * kSlices];
-  __shared__ uint32_t slice_rank[kSampWaves * kSlices];
-  __shared__ int sel_s;
-  __shared__ u64 rest_u64;
-  __shared__ uint32_t rest_u32;
+// What a block that draws a row by itself needs of LDS
+struct RowShared {
+  ArgMax am[kSampWaves];
+  uint32_t hist_k[kBins];       // top-k search: how many weights fall into each bin
+  uint32_t hist_pn[kBins];      // top-p search: how many, and their mass
+  u64 hist_pm[kBins];
+  u64 wave_u64[kSampWaves];
+  uint32_t wave_u32[kSampWaves];
+  u64 slice_mass[kSampWaves * kSlices];
+  uint32_t slice_rank[kSampWaves * kSlices];
+  int sel_s;
+  u64 rest_u64;
+  uint32_t rest_u32;
+};
 
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const float* lr = logits + (size_t)row * ld;
-  float* w = weights + (size_t)row * vocab;
-  const float temp = temperature[row];
-
-  // A greedy row is shared by the gridDim.y blocks of its row: one block reads a large vocabulary no faster than one
-  // CU can load (a row of 128k logits: 10 us).  Each takes a stretch of the row and leaves its best; the block that
-  // finishes last picks among them (stores and loads that go through to memory, a device-wide counter that it leaves
-  // at zero: no fence that would flush a cache).  Rows that draw keep one block: its walks share what they find.
-  const int parts = gridDim.y, part = blockIdx.y;
-  if (parts > 1) {
-    if (temp > 0.f) {
-      if (part > 0) return;
-    } else {
-      const int len = ((vocab + parts * 4 - 1) / (parts * 4)) * 4;
-      const int lo = part * len, hi = lo + len < vocab ? lo + len : vocab;
-      ArgMax a = {-INFINITY, 0x7fffffff};
-      if (lo < hi) sweep(lr + lo, hi - lo, [&](float v, int i) { a = better(a, ArgMax{v, i + lo}); });
-      a = block_argmax(a, am);
-      if (tid == 0) {
-        __hip_atomic_store(&split_val[row * kMaxSplits + part], a.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&split_idx[row * kMaxSplits + part], a.i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);
-        const int before = __hip_atomic_fetch_add(&split_count[row], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before + 1 == parts) {
-          __hip_atomic_store(&split_count[row], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          ArgMax r = {-INFINITY, 0x7fffffff};
-          for (int p = 0; p < parts; ++p) {
-            ArgMax b;
-            b.v = __hip_atomic_load(&split_val[row * kMaxSplits + p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            b.i = __hip_atomic_load(&split_idx[row * kMaxSplits + p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            r = better(r, b);
-          }
-          if ((unsigned)r.i >= (unsigned)vocab) r.i = 0;   // a row of NaN has no largest value: still name a token
-          out_token[row] = r.i;
-          out_logit[row] = lr[r.i];
-        }
-      }
-      return;
-    }
-  }
+// The whole of a row by one block: its largest logit, or the draw (k <= 0: no top-k cut; p >= 1: no top-p cut; u: the number in
+// [0, 1) that draws)
+__device__ __forceinline__ void sample_row(RowShared& sh, const float* __restrict__ lr, float* __restrict__ w, int vocab, float temp, int k, float p,
+                           float u, int32_t* __restrict__ out_token, float* __restrict__ out_logit) {
+  ArgMax* const am = sh.am;
+  uint32_t* const hist_k = sh.hist_k;
+  uint32_t* const hist_pn = sh.hist_pn;
+  u64* const hist_pm = sh.hist_pm;
+  u64* const wave_u64 = sh.wave_u64;
+  uint32_t* const wave_u32 = sh.wave_u32;
+  u64* const slice_mass = sh.slice_mass;
+  uint32_t* const slice_rank = sh.slice_rank;
+  int& sel_s = sh.sel_s;
+  u64& rest_u64 = sh.rest_u64;
+  uint32_t& rest_u32 = sh.rest_u32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
   ArgMax a = {-INFINITY, 0x7fffffff};
   sweep(lr, vocab, [&](float v, int i) { a = better(a, ArgMax{v, i}); });
   a = block_argmax(a, am);
   if ((unsigned)a.i >= (unsigned)vocab) a.i = 0;       // a row of NaN has no largest value: still name a token
   if (tid == 0) {          // the answer of a greedy row, and of a row whose weights are no numbers
-    out_token[row] = a.i;
-    out_logit[row] = lr[a.i];
+    *out_token = a.i;
+    *out_logit = lr[a.i];
   }
   if (!(temp > 0.f)) return;
 
-  const int k = top_k[row];
-  const float p = top_p[row];
   const bool cut_k = k > 0 && k < vocab, cut_p = p < 1.0f, cut = cut_k || cut_p;
 
   // Each wave owns a contiguous stretch of the vocabulary, cut into kSlices slices of whole pieces of 256 values
@@ -475,7 +446,7 @@ sample_kernel(const float* __restrict__ logits, int ld, int vocab, const float* 
     kept += wave_u64[i];
   }
   if (kept == 0) return;                           // weights that are no numbers: the default answer stands
-  u64 target = (u64)((double)uniform[row] * (double)kept);
+  u64 target = (u64)((double)u * (double)kept);
   if (target >= kept) target = kept - 1;           // (kept >= 2^40: the largest weight is always kept)
   if (tid < kAllSlices && before <= target && target < before + mine) {
     sel_s = tid;
@@ -527,9 +498,59 @@ sample_kernel(const float* __restrict__ logits, int ld, int vocab, const float* 
   }
   if (lane == 0) {
     const int c = pick >= 0 ? pick : a.i;
-    out_token[row] = c;
-    out_logit[row] = lr[c];
+    *out_token = c;
+    *out_logit = lr[c];
   }
+}
+
+__global__ void __launch_bounds__(kSampThreads)
+sample_kernel(const float* __restrict__ logits, int ld, int vocab, const float* __restrict__ temperature,
+              const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
+              float* __restrict__ weights, int32_t* __restrict__ out_token, float* __restrict__ out_logit) {
+  __shared__ RowShared sh;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const float* lr = logits + (size_t)row * ld;
+  const float temp = temperature[row];
+
+  // A greedy row is shared by the gridDim.y blocks of its row: one block reads a large vocabulary no faster than one
+  // CU can load (a row of 128k logits: 10 us).  Each takes a stretch of the row and leaves its best; the block that
+  // finishes last picks among them (stores and loads that go through to memory, a device-wide counter that it leaves
+  // at zero: no fence that would flush a cache).  Rows that draw keep one block: its walks share what they find.
+  const int parts = gridDim.y, part = blockIdx.y;
+  if (parts > 1) {
+    if (temp > 0.f) {
+      if (part > 0) return;
+    } else {
+      const int len = ((vocab + parts * 4 - 1) / (parts * 4)) * 4;
+      const int lo = part * len, hi = lo + len < vocab ? lo + len : vocab;
+      ArgMax a = {-INFINITY, 0x7fffffff};
+      if (lo < hi) sweep(lr + lo, hi - lo, [&](float v, int i) { a = better(a, ArgMax{v, i + lo}); });
+      a = block_argmax(a, sh.am);
+      if (tid == 0) {
+        __hip_atomic_store(&split_val[row * kMaxSplits + part], a.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&split_idx[row * kMaxSplits + part], a.i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        const int before = __hip_atomic_fetch_add(&split_count[row], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before + 1 == parts) {
+          __hip_atomic_store(&split_count[row], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          ArgMax r = {-INFINITY, 0x7fffffff};
+          for (int p = 0; p < parts; ++p) {
+            ArgMax b;
+            b.v = __hip_atomic_load(&split_val[row * kMaxSplits + p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            b.i = __hip_atomic_load(&split_idx[row * kMaxSplits + p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            r = better(r, b);
+          }
+          if ((unsigned)r.i >= (unsigned)vocab) r.i = 0;   // a row of NaN has no largest value: still name a token
+          out_token[row] = r.i;
+          out_logit[row] = lr[r.i];
+        }
+      }
+      return;
+    }
+  }
+
+  sample_row(sh, lr, weights + (size_t)row * vocab, vocab, temp, top_k[row], top_p[row], uniform[row], out_token + row, out_logit + row);
 }
 
 extern "C" int atoma_sample(const float* logits, int ld, int n_rows, int vocab, const float* temperature,
@@ -671,7 +692,7 @@ split_max_kernel(const float* __restrict__ logits, int ld, int vocab, SplitRow* 
 }
 
 // the row's largest logit from its parts' (the same in every thread)
-__device__ __forceinline__ ArgMax split_row_max(const SplitRow& r, int parts, int vocab) {
+template <typename Row> __device__ __forceinline__ ArgMax row_max(const Row& r, int parts, int vocab) {
   ArgMax a = {-INFINITY, 0x7fffffff};
   for (int p = 0; p < parts; ++p) a = better(a, ArgMax{r.part_max_v[p], r.part_max_i[p]});
   if ((unsigned)a.i >= (unsigned)vocab) a.i = 0;       // a row of NaN has no largest value: still name a token
@@ -716,7 +737,7 @@ split_weights_kernel(const float* __restrict__ logits, int ld, int vocab, const 
   const float temp = temperature[row];
   const int k = top_k[row];
   const float p = top_p[row];
-  const ArgMax a = split_row_max(r, parts, vocab);
+  const ArgMax a = row_max(r, parts, vocab);
   if (part == 0 && tid == 0) {       // the answer of a greedy row, and of a row whose weights are no numbers
     out_token[row] = a.i;
     out_logit[row] = lr[a.i];
@@ -1106,6 +1127,247 @@ split_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts
   }
 }
 
+// ---- rows that all keep few weights (a top-k cut of at most kFewMaxK): three launches ---------------------------
+// The search above walks the row once a level, since it knows nothing of where the k-th weight lies.  With a small k a part can
+// contribute its own k largest values at most, so the first walk, which looks for the largest logit anyway, also lists them, and
+// the search runs over the lists of a row in the LDS of one block.  The weights rise with the logits, so a part needs neither the
+// row's largest logit nor the temperature for its list.  What is left are the two walks that nothing can replace: the largest logit
+// (with the lists), then the mass of all weights where a top-p cut asks for a share of it.
+//   A part's list: the values not below a floor that at least k + kFewSpare threads' largest values reach, found by two levels of
+// histogram over those 1,024 values (not the part's 16,384).  The spare ones put the floor's weight below the k-th weight even if one
+// part holds all k; where it is not clearly below (values tied by the hundred, or a list that is too long, or values that are no
+// numbers) the block that draws takes the row by itself as sample_kernel does: the tokens are the same in every case.
+// 64 rows of 128,256 logits, top-k 50 and top-p 0.9: the three launches take 15 + 7.5 + 9.5 us, 30 with what lies between them, where
+// the search's six take 77.  The lists stop at a k of 128, which two weights a lane of the last launch hold.
+constexpr int kFewMaxK = 128, kFewSpare = 16;
+constexpr int kFewCap = 384;                      // of a part's list
+constexpr int kFewNear = 1024;                    // weights in the k-th one's bin or above
+constexpr uint32_t kFewRefused = 0xffffffffu;
+struct FewRow {
+  u64 part_mass[kMaxParts];          // of a part: the mass of its weights (rows with a top-p cut)
+  float part_max_v[kMaxParts];       // its largest logit and that one's index
+  int32_t part_max_i[kMaxParts];
+  float part_floor[kMaxParts];       // every value that is not below this is in the list
+  uint32_t part_count[kMaxParts];    // length of the list; kFewRefused: there is none
+  uint2 list[kMaxParts][kFewCap];    // (bits of the logit, index in the row), in no order
+};
+static_assert(sizeof(FewRow) % 16 == 0, "rows of scratch stay aligned");
+
+// unsigned numbers in the order of the floats
+__device__ __forceinline__ uint32_t rising(float v) {
+  const uint32_t b = __float_as_uint(v);
+  return b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ float from_rising(uint32_t u) {
+  return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
+}
+
+// launch 1: a part's largest logit and its list
+__global__ void __launch_bounds__(kSampThreads)
+few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __restrict__ rows, const int32_t* __restrict__ top_k,
+                const float* __restrict__ temperature) {
+  __shared__ ArgMax am[kSampWaves];
+  __shared__ uint32_t hist[2][kBins];
+  __shared__ uint32_t wave_u32[kSampWaves];
+  __shared__ int sel_s;
+  __shared__ uint32_t rest_s, count;
+  const int row = blockIdx.x, parts = gridDim.y, part = blockIdx.y, tid = threadIdx.x;
+  FewRow& r = rows[row];
+  int lo, hi;
+  part_range(vocab, parts, part, lo, hi);
+  PartValues pv;
+  load_part(logits + (size_t)row * ld, lo, hi, pv);
+  const int k = top_k[row];
+  const float temp = temperature[row];
+  hist[0][tid] = 0;
+  hist[1][tid] = 0;
+  if (tid == 0) count = 0;
+  ArgMax a = {-INFINITY, 0x7fffffff};
+  bool odd = false;
+  for_part(pv, lo, hi, [&](float v, int i) {
+    a = better(a, ArgMax{v, i});
+    odd |= !(v < INFINITY);
+  });
+  const uint32_t top = rising(a.v);
+  a = block_argmax(a, am);
+  if (tid == 0) {
+    r.part_max_v[part] = a.v;
+    r.part_max_i[part] = a.i;
+  }
+  if (!(temp > 0.f)) return;                       // (a greedy row needs no more)
+  if (__syncthreads_or(odd) || k <= 0 || k > kFewMaxK) {
+    if (tid == 0) r.part_count[part] = kFewRefused;
+    return;
+  }
+  int sel0, sel1;
+  uint32_t want = (uint32_t)(k + kFewSpare);
+  atomicAdd(&hist[0][top >> 22], 1u);
+  __syncthreads();
+  select_bin<uint32_t>(hist[0], want, sel0, want, wave_u32, &sel_s, &rest_s);
+  if ((int)(top >> 22) == sel0) atomicAdd(&hist[1][(top >> 12) & (kBins - 1)], 1u);
+  __syncthreads();
+  select_bin<uint32_t>(hist[1], want, sel1, want, wave_u32, &sel_s, &rest_s);
+  const uint32_t least = rising(-INFINITY) + 1;    // (weights of zero are never drawn)
+  uint32_t edge = ((uint32_t)sel0 << 22) | ((uint32_t)sel1 << 12);
+  const bool all = edge < least;
+  if (all) edge = least;
+  if (top >= edge) {
+    for_part(pv, lo, hi, [&](float v, int i) {
+      if (rising(v) < edge) return;
+      const uint32_t at = atomicAdd(&count, 1u);
+      if (at < kFewCap) r.list[part][at] = make_uint2(__float_as_uint(v), (uint32_t)i);
+    });
+  }
+  __syncthreads();
+  if (tid == 0) {
+    r.part_floor[part] = all ? -INFINITY : from_rising(edge);
+    r.part_count[part] = count <= kFewCap ? count : kFewRefused;
+  }
+}
+
+// launch 2 (left out where no row has a top-p cut): the mass of a part's weights
+__global__ void __launch_bounds__(kSampThreads)
+few_mass_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __restrict__ rows, const float* __restrict__ top_p,
+                const float* __restrict__ temperature) {
+  __shared__ u64 wave_u64[kSampWaves];
+  const int row = blockIdx.x, parts = gridDim.y, part = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  FewRow& r = rows[row];
+  int lo, hi;
+  part_range(vocab, parts, part, lo, hi);
+  PartValues pv;
+  load_part(logits + (size_t)row * ld, lo, hi, pv);
+  const float temp = temperature[row], p = top_p[row];
+  if (!(temp > 0.f) || !(p < 1.0f)) return;
+  const ArgMax a = row_max(r, parts, vocab);
+  const float inv_t = 1.4426950408889634f / temp;
+  uint32_t hi_sum = 0, lo_sum = 0;
+  for_part(pv, lo, hi, [&](float v, int) {
+    uint32_t fh, fl;
+    fixed_parts(__builtin_amdgcn_exp2f((v - a.v) * inv_t), fh, fl);
+    hi_sum += fh;
+    lo_sum += fl;
+  });
+  const u64 mass = wave_total(((u64)hi_sum << 20) + lo_sum);
+  if (lane == 0) wave_u64[wave] = mass;
+  __syncthreads();
+  if (tid == 0) {
+    u64 all = 0;
+    for (int i = 0; i < kSampWaves; ++i) all += wave_u64[i];
+    r.part_mass[part] = all;
+  }
+}
+
+// launch 3, a block a row: the k largest weights of the lists, the shortest run of them that reaches the mass top-p asks for, and the
+// draw among those, in the row's order.
+__global__ void __launch_bounds__(kSampThreads)
+few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, int masses, FewRow* __restrict__ rows,
+                float* __restrict__ weights, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+                const float* __restrict__ top_p, const float* __restrict__ uniform, int32_t* __restrict__ out_token, float* __restrict__ out_logit) {
+  __shared__ RowShared sh;
+  __shared__ u64 near[kFewNear];                   // (bits of the weight, all ones less the index): larger ones are kept first
+  __shared__ u64 kept_key[kFewMaxK];               // those kept, falling
+  __shared__ u64 kept_mass[kFewMaxK];
+  __shared__ uint32_t n_near;
+  constexpr int kPerLane = kFewCap / kWave;
+  static_assert(kSampWaves == kMaxParts && kFewMaxK == 2 * kWave, "a wave a list, two kept weights a lane");
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const FewRow& r = rows[row];
+  // a wave takes a part's list, its length and its floor in one trip to memory
+  const int mine = wave < parts ? wave : 0;
+  uint2 got[kPerLane];
+#pragma unroll
+  for (int j = 0; j < kPerLane; ++j) got[j] = r.list[mine][j * kWave + lane];
+  const uint32_t listed = r.part_count[mine];
+  const float floor_v = r.part_floor[mine];
+  const float temp = temperature[row], p = masses ? top_p[row] : 1.0f, u = uniform[row];
+  const int k = top_k[row];
+  const float* lr = logits + (size_t)row * ld;
+  const ArgMax a = row_max(r, parts, vocab);
+  if (!(temp > 0.f)) {
+    if (tid == 0) out_token[row] = a.i, out_logit[row] = lr[a.i];
+    return;
+  }
+  const float inv_t = 1.4426950408889634f / temp;
+  // whether the lists hold what the draw needs; if so, it is made
+  auto from_lists = [&]() -> bool {
+    sh.hist_k[tid] = 0;
+    if (tid == 0) n_near = 0;
+    // (the longest list there is fits: counts beyond it are refusals)
+    if (__syncthreads_or(wave < parts && listed > kFewCap) || !(a.v > -INFINITY) || !(inv_t < INFINITY) || k <= 0 || k > kFewMaxK)
+      return false;
+    const int n = wave < parts ? (int)listed : 0;
+    uint32_t bits[kPerLane];
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+      bits[j] = __float_as_uint(__builtin_amdgcn_exp2f((__uint_as_float(got[j].x) - a.v) * inv_t));
+      if (j * kWave + lane < n) atomicAdd(&sh.hist_k[(bits[j] >> 20) & (kBins - 1)], 1u);
+    }
+    __syncthreads();
+    int sel;
+    uint32_t rest;
+    select_bin<uint32_t>(sh.hist_k, (uint32_t)k, sel, rest, sh.wave_u32, &sh.sel_s, &sh.rest_u32);
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+      if (j * kWave + lane < n && (int)(bits[j] >> 20) >= sel) {          // (sel < 0: fewer than k weights above zero, all kept)
+        const uint32_t at = atomicAdd(&n_near, 1u);
+        if (at < kFewNear) near[at] = ((u64)bits[j] << 32) | (uint32_t)~got[j].y;
+      }
+    }
+    __syncthreads();
+    const int m = (int)n_near;
+    if (m > kFewNear) return false;
+    const int n_k = m < k ? m : k;
+    if (tid < m) {
+      const u64 key = near[tid];
+      int rank = 0;
+      for (int i = 0; i < m; ++i) rank += near[i] > key;
+      if (rank < n_k) {
+        kept_key[rank] = key;
+        kept_mass[rank] = fixed_of(__uint_as_float((uint32_t)(key >> 32)));
+      }
+    }
+    __syncthreads();
+    // Nothing that the lists leave out may weigh as much as the k-th weight: the weight of a part's floor must lie below it by more than
+    // exp2 can be off, or be too small to be drawn.
+    const float last = m < k ? 0.f : __uint_as_float((uint32_t)(kept_key[k - 1] >> 32));
+    const float edge = __builtin_amdgcn_exp2f((floor_v - a.v) * inv_t);
+    const bool below = edge < 0x1p-41f || edge * (1.0f + 0x1p-20f) < last;
+    if (__syncthreads_or(wave < parts && !below)) return false;
+    if (wave > 0) return true;
+    const int at0 = 2 * lane, at1 = 2 * lane + 1;
+    const u64 m0 = at0 < n_k ? kept_mass[at0] : 0, m1 = at1 < n_k ? kept_mass[at1] : 0;
+    const u64 incl1 = wave_prefix(m0 + m1), incl0 = incl1 - m1;
+    int n_kept = n_k;
+    if (p < 1.0f) {
+      u64 total = 0;
+      for (int q = 0; q < parts; ++q) total += r.part_mass[q];
+      const double need = ceil((double)p * (double)total);
+      u64 want = need < 1.0 ? 1ull : (u64)need;
+      if (want > total) want = total;
+      const int reach = 1 + __popcll(__ballot(at0 < n_k && incl0 < want)) + __popcll(__ballot(at1 < n_k && incl1 < want));
+      n_kept = reach < n_k ? reach : n_k;
+    }
+    const int last_at = n_kept - 1;
+    const u64 kept = __shfl(last_at & 1 ? incl1 : incl0, last_at >> 1, 64);
+    u64 target = (u64)((double)u * (double)kept);
+    if (target >= kept) target = kept - 1;           // (kept >= 2^40: the largest weight is always kept)
+    // the one at which the running sum in the row's order passes the target
+    const u64 key0 = kept_key[at0 < n_kept ? at0 : 0], key1 = kept_key[at1 < n_kept ? at1 : 0];
+    const uint32_t i0 = ~(uint32_t)key0, i1 = ~(uint32_t)key1;
+    u64 run0 = 0, run1 = 0;
+    for (int i = 0; i < n_kept; ++i) {
+      const uint32_t at = ~(uint32_t)kept_key[i];
+      const u64 mass = kept_mass[i];
+      run0 += at <= i0 ? mass : 0;
+      run1 += at <= i1 ? mass : 0;
+    }
+    if (at0 < n_kept && run0 > target && run0 - m0 <= target) out_token[row] = (int32_t)i0, out_logit[row] = lr[i0];
+    if (at1 < n_kept && run1 > target && run1 - m1 <= target) out_token[row] = (int32_t)i1, out_logit[row] = lr[i1];
+    return true;
+  };
+  if (!from_lists()) sample_row(sh, lr, weights + (size_t)row * vocab, vocab, temp, k, p, u, out_token + row, out_logit + row);
+}
+
 // parts a row: so many that the blocks of all rows fill the GPU, and that a part's weights fit the draw's registers
 static int split_parts(int n_rows, int vocab) {
   int parts = (256 + n_rows - 1) / n_rows;
@@ -1114,13 +1376,17 @@ static int split_parts(int n_rows, int vocab) {
   return parts > kMaxParts ? (least <= kMaxParts ? kMaxParts : 0) : parts;
 }
 
-extern "C" size_t atoma_sample_split_scratch_bytes(int n_rows) { return (size_t)(n_rows > 0 ? n_rows : 0) * sizeof(SplitRow); }
+extern "C" size_t atoma_sample_split_scratch_bytes(int n_rows) {
+  return (size_t)(n_rows > 0 ? n_rows : 0) * (sizeof(SplitRow) > sizeof(FewRow) ? sizeof(SplitRow) : sizeof(FewRow));
+}
 
 // atoma_sample for steps in which rows draw: the same tokens from six short launches (see above).  scratch: at
 // least atoma_sample_split_scratch_bytes(n_rows) bytes, 16-byte aligned, whatever they hold.  Vocabularies too
 // large for sixteen parts (above 262,144) are refused: atoma_sample takes them.  cuts == 0: the caller knows that
 // no row has a top-k or top-p cut; the three launches of the search are left out, and top_k and top_p are not read
-// (a row that has a cut all the same is drawn from all of its weights).
+// (a row that has a cut all the same is drawn from all of its weights).  cuts == 2: the caller knows that every row that
+// draws has a top-k cut of at most 128, and that none has a top-p cut (top_p is not read); cuts == 3: the same, but rows may have
+// a top-p cut.  Two or three short launches; a row with another top-k all the same is drawn by one block.
 extern "C" int atoma_sample_split(const float* logits, int ld, int n_rows, int vocab, const float* temperature,
                                   const int32_t* top_k, const float* top_p, const float* uniform, float* weights,
                                   void* scratch, int cuts, int32_t* out_token, float* out_logit, hipStream_t stream) {
@@ -1128,8 +1394,18 @@ extern "C" int atoma_sample_split(const float* logits, int ld, int n_rows, int v
   if (vocab <= 0 || ld < vocab || scratch == nullptr || ((uintptr_t)scratch & 15) != 0) return ATOMA_ERR_SHAPE;
   const int parts = split_parts(n_rows, vocab);
   if (parts <= 0) return ATOMA_ERR_SHAPE;
-  SplitRow* rows = static_cast<SplitRow*>(scratch);
   const dim3 grid(n_rows, parts), block(kSampThreads);
+  if (cuts >= 2) {
+    FewRow* few = static_cast<FewRow*>(scratch);
+    hipLaunchKernelGGL(few_list_kernel, grid, block, 0, stream, logits, ld, vocab, few, top_k, temperature);
+    if (cuts == 3) hipLaunchKernelGGL(few_mass_kernel, grid, block, 0, stream, logits, ld, vocab, few, top_p, temperature);
+    hipLaunchKernelGGL(few_draw_kernel, dim3(n_rows), block, 0, stream, logits, ld, vocab, parts, cuts == 3, few, weights,
+                       temperature, top_k,
+                       top_p, uniform, out_token, out_logit);
+    ATOMA_LAUNCH_CHECK();
+    return 0;
+  }
+  SplitRow* rows = static_cast<SplitRow*>(scratch);
   hipLaunchKernelGGL(split_max_kernel, grid, block, 0, stream, logits, ld, vocab, rows);
   hipLaunchKernelGGL(split_weights_kernel, grid, block, 0, stream, logits, ld, vocab, temperature, top_k, top_p, weights,
                      rows, out_token, out_logit, cuts);

@@ -1476,12 +1476,13 @@ def rglru_scan(gates: torch.Tensor, u: torch.Tensor, g: torch.Tensor, ba, bi, sp
     return out
 
 
+FEW_MAX_K = 128                # the largest top-k of rows that ``sample_packed(few=True)`` is for
 SPLIT_MAX_VOCAB = 262144       # the largest vocabulary whose rows ``sample_packed(split=True)`` cuts into parts
 
 
 def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor,
                   uniform: torch.Tensor, workspace: Optional[torch.Tensor] = None, split: bool = False,
-                  cuts: bool = True) -> torch.Tensor:
+                  cuts: bool = True, few: bool = False, top_p_cuts: bool = True) -> torch.Tensor:
     """Per row of float32 ``logits`` [S, V]: argmax where temperature <= 0, else a draw (see sampling.hip).
 
     Returns one float32 tensor [2, S]: row 0 holds the tokens (int32 bits), row 1 the logits of the chosen tokens,
@@ -1489,7 +1490,10 @@ def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
     launches instead of one long one (the same tokens; quicker when rows draw from a large vocabulary: one block
     walks a row with top-k and top-p in over 100 us); vocabularies beyond ``SPLIT_MAX_VOCAB`` keep the one launch.
     ``cuts=False`` (with ``split``): the caller knows that no row has a top-k or top-p cut, and the three launches
-    that search for them are left out (``top_k`` and ``top_p`` are then not read).
+    that search for them are left out (``top_k`` and ``top_p`` are then not read).  ``few=True`` (with ``split``): the caller
+    knows that every row that draws has a top-k cut of at most ``FEW_MAX_K``; three launches that list each part's largest logits
+    then take the place of the search (the same tokens; a row with another cut is drawn by one block), two where it also knows
+    that there is no top-p cut (``top_p_cuts=False``: ``top_p`` is then not read).
     """
     _dev(logits, temperature, top_k, top_p, uniform)
     _need(logits.dim() == 2 and logits.dtype is torch.float32 and logits.stride(1) == 1, "logits must be float32 [S, V]")
@@ -1509,7 +1513,8 @@ def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
         scratch = torch.empty((int(lib.atoma_sample_split_scratch_bytes(s)) + 3) // 4, dtype=torch.int32,
                               device=logits.device)
         _check(lib.atoma_sample_split(_p(logits), ld, s, v, _p(temperature), _p(top_k), _p(top_p), _p(uniform),
-                                      _p(workspace), _p(scratch), 1 if cuts else 0, _p(out[0]), _p(out[1]), _stream()),
+                                      _p(workspace), _p(scratch), (3 if top_p_cuts else 2) if few and cuts else 1 if cuts else 0,
+                                      _p(out[0]), _p(out[1]), _stream()),
                "sample (split)")
         return out
     _check(core().atoma_sample(_p(logits), ld, s, v, _p(temperature), _p(top_k),

@@ -112,8 +112,10 @@ class Sampler:
             ops.repeat_penalty(logits, pen[0], pen[1], m[3])
         # (rows that draw are shared by several blocks each: a block walks a row of a large vocabulary too slowly)
         cuts = any(not pl.greedy and (pl.top_k > 0 or pl.top_p < 1.0) for pl in plans)
+        few = all(pl.greedy or 0 < pl.top_k <= ops.FEW_MAX_K for pl in plans)
         out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2],
-                                split=not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB, cuts=cuts)
+                                split=not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB, cuts=cuts, few=few,
+                                top_p_cuts=any(pl.top_p < 1.0 for pl in plans if not pl.greedy))
         tok, lg = out[0].view(torch.int32), out[1]
         host, pool = self._host_buffer(s)
         host.copy_(out, non_blocking=True)

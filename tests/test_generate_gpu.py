@@ -301,6 +301,47 @@ def test_rows_shared_by_several_blocks_draw_the_same_tokens(rows, vocab):
     assert torch.equal(one[0].view(torch.int32), four[0].view(torch.int32))
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 128256), (9, 128256), (14, 200003), (70, 50001), (300, 40000), (3, 262144), (2, 700)])
+def test_rows_that_keep_few_weights_draw_the_same_tokens(rows, vocab):
+    """The launches that list each part's largest logits against the one launch of a block a row: the same tokens and logits bit for
+    bit, whatever the rows look like: all large logits in one part, thousands of ties, fewer finite logits than k, infinities and
+    NaN, hardly any spread, temperatures that leave one weight or all of them; k from 1 to the largest listed, and beyond it."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows * 3 + vocab)
+    logits = torch.randn(rows, vocab, generator=g) * 3.0
+    modes = [(0.8, 50, 0.9), (0.8, 50, 1.0), (0.0, 0, 1.0), (1.0, 1, 0.5), (1.5, ops.FEW_MAX_K, 0.99), (0.7, 3, 0.9), (0.02, 40, 0.95),
+             (50.0, 100, 0.3), (0.9, ops.FEW_MAX_K + 1, 0.9), (0.8, 0, 0.9), (1e-38, 40, 0.9)]
+    pick = [modes[i % len(modes)] for i in range(rows)]
+    if rows >= 9:
+        logits[0, :300] += 30.0                          # all that is kept lies in the first part
+        logits[1, vocab // 2:vocab // 2 + 20] += 40.0    # a few neighbours far above the others
+        logits[3] = -float("inf")                        # fewer finite logits than k ...
+        logits[3, [7, 30000, vocab - 1]] = torch.tensor([1.0, 1.0, 0.5])
+        pick[3] = (1.0, 50, 0.99)
+        logits[4, 100:5000] = 11.5                       # thousands of ties, some of them kept
+        logits[5] = logits[5].round()                    # whole numbers: the k-th weight is one of a thousand equal ones
+        logits[6, 11] = float("nan")
+        logits[7] = 2.0 + 1e-6 * logits[7]               # (a handful of different floats)
+    if rows >= 70:
+        logits[11] = 0.0
+        logits[12, 9] = float("inf")
+        logits[13] = -float("inf")
+        logits[14, ::2] = -0.0
+        logits[14, 1::2] = 0.0
+        logits[15] = -1e30 * (1.0 + logits[15].abs())
+    dev = lambda x, dt: torch.tensor(x, dtype=dt, device="cuda:0")
+    lg = logits.cuda()
+    t, k, p = (dev([m[i] for m in pick], dt) for i, dt in ((0, torch.float32), (1, torch.int32), (2, torch.float32)))
+    same = lambda a, b: (torch.equal(a[0].view(torch.int32), b[0].view(torch.int32)) and torch.equal(a[1].isnan(), b[1].isnan())
+                         and torch.equal(a[1].nan_to_num(), b[1].nan_to_num()))
+    for u in (0.0, 0.31, 0.5, 0.93, 0.999999):
+        uu = dev([(u + 0.37 * i) % 1.0 for i in range(rows)], torch.float32)
+        assert same(ops.sample_packed(lg, t, k, p, uu), ops.sample_packed(lg, t, k, p, uu, split=True, few=True)), u
+    # a caller that knows of no top-p cut
+    no_p = torch.ones_like(p)
+    assert same(ops.sample_packed(lg, t, k, no_p, uu), ops.sample_packed(lg, t, k, p, uu, split=True, few=True, top_p_cuts=False))
+
+
 def test_the_sampler_shares_the_rows_of_a_large_vocabulary():
     """Through the engine's sampler: a step whose rows draw from 128k logits goes to the launches that share every
     row among several blocks, with the search left out when no row has a cut; the tokens are those of a block a row
