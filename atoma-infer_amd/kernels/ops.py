@@ -1477,6 +1477,7 @@ def rglru_scan(gates: torch.Tensor, u: torch.Tensor, g: torch.Tensor, ba, bi, sp
 
 
 FEW_MAX_K = 128                # the largest top-k of rows that ``sample_packed(few=True)`` is for
+_split = None                  # the draw by parts and the size of its scratch memory, once loaded
 SPLIT_MAX_VOCAB = 262144       # the largest vocabulary whose rows ``sample_packed(split=True)`` cuts into parts
 
 
@@ -1508,13 +1509,20 @@ def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
     out = torch.empty((2, s), dtype=torch.float32, device=logits.device)
     ld = logits.stride(0) if s > 1 else v
     if split and v <= SPLIT_MAX_VOCAB:
-        lib = core()
-        lib.atoma_sample_split_scratch_bytes.restype = ctypes.c_size_t
-        scratch = torch.empty((int(lib.atoma_sample_split_scratch_bytes(s)) + 3) // 4, dtype=torch.int32,
-                              device=logits.device)
-        _check(lib.atoma_sample_split(_p(logits), ld, s, v, _p(temperature), _p(top_k), _p(top_p), _p(uniform),
-                                      _p(workspace), _p(scratch), (3 if top_p_cuts else 2) if few and cuts else 1 if cuts else 0,
-                                      _p(out[0]), _p(out[1]), _stream()),
+        global _split
+        if _split is None:
+            lib = core()
+            lib.atoma_sample_split_scratch_bytes.restype = ctypes.c_size_t
+            i, ptr = ctypes.c_int, ctypes.c_void_p
+            # (with the types of its arguments known, a call takes plain numbers: 8 us less a step)
+            lib.atoma_sample_split.argtypes = [ptr, i, i, i] + [ptr] * 6 + [i, ptr, ptr, ptr]
+            _split = lib.atoma_sample_split, lib.atoma_sample_split_scratch_bytes
+        draw, scratch_bytes = _split
+        scratch = torch.empty((scratch_bytes(s) + 3) // 4, dtype=torch.int32, device=logits.device)
+        at = out.data_ptr()
+        _check(draw(logits.data_ptr(), ld, s, v, temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), uniform.data_ptr(),
+                    workspace.data_ptr(), scratch.data_ptr(), (3 if top_p_cuts else 2) if few and cuts else 1 if cuts else 0,
+                    at, at + 4 * s, _stream()),
                "sample (split)")
         return out
     _check(core().atoma_sample(_p(logits), ld, s, v, _p(temperature), _p(top_k),

@@ -52,3 +52,14 @@ def test_uniform_is_a_pure_function_in_the_unit_interval():
     assert xs == [uniform(42, i) for i in range(2000)]
     assert abs(sum(xs) / len(xs) - 0.5) < 0.03 and len(set(xs)) > 1990
     assert uniform(42, 0) != uniform(43, 0)
+
+
+def test_a_steps_uniform_numbers_written_natively_are_the_functions():
+    import ctypes
+
+    from atoma_infer_amd.sampling.sampler import write_uniforms
+    seeds = [0, 1, 42, -1, 2 ** 63, 2 ** 64 - 1, 2 ** 64 + 5] * 40
+    counters = [i * i for i in range(len(seeds))]
+    got = (ctypes.c_float * len(seeds))()
+    write_uniforms(seeds, counters, ctypes.addressof(got))
+    assert list(got) == [uniform(s, c) for s, c in zip(seeds, counters)]
