@@ -82,6 +82,47 @@ template <int NWAVES> __device__ __forceinline__ float block_max(float v, float*
 // Element type codes of the C interface.
 enum DType : int { kF32 = 0, kBF16 = 1 };
 
+// A barrier for what passes LDS: unlike __syncthreads it does not wait for the wave's loads from and stores to memory.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// One token of a causal convolution over time whose earlier inputs lie in the rows of `rows` (keep of them, `channels` apart), the
+// last tap on `in`: added to y in the order of the taps.  x: the rows' values where there are at most four, which push_inputs then
+// moves down by one row.
+__device__ __forceinline__ float convolve_one(const float* rows, const float* __restrict__ taps, int keep, int channels, float in, float y,
+                                              float (&x)[4]) {
+  if (keep == 0) return fmaf(taps[0], in, y);
+  if (keep <= 4) {                        // (in one stretch: one trip to memory)
+    float w[4];
+    const float last = taps[keep];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int at = min(j, keep - 1);
+      x[j] = rows[at * channels];
+      w[j] = taps[at];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y = j < keep ? fmaf(w[j], x[j], y) : y;
+    return fmaf(last, in, y);
+  }
+  for (int j = 0; j < keep; ++j) y = fmaf(taps[j], rows[(size_t)j * channels], y);
+  return fmaf(taps[keep], in, y);
+}
+__device__ __forceinline__ void push_inputs(float* rows, int keep, int channels, float in, const float (&x)[4], bool held) {
+  if (keep <= 0) return;
+  if (held && keep <= 4) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+      if (r + 1 < keep) rows[(size_t)r * channels] = x[r + 1];
+  } else {      // (ascending, so that a row is read before it is overwritten)
+    for (int r = 0; r + 1 < keep; ++r) rows[(size_t)r * channels] = rows[(size_t)(r + 1) * channels];
+  }
+  rows[(size_t)(keep - 1) * channels] = in;
+}
+
 }  // namespace atoma
 
 // Error codes of the C interface beyond hipError_t values (which are positive): negative numbers.

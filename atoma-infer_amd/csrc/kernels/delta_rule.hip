@@ -2,7 +2,7 @@
 //
 // Per token and head (q, k of size dim, unit length; v of size vdim; beta a scalar; g a decay per key channel):
 //   S <- diag(g) S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q          (the read-out sees the token's write)
-// Everything here is float32.  Four kernels:
+// Everything here is float32.  Four kernels, and delta_step, which does the work of all four for a step of single tokens:
 //   delta_prepare      per token: short causal convolution over time and SiLU of the q, k, v projections (the taps - 1
 //                      inputs before an entry's first token come from the request's state), q and k to unit length per
 //                      head (q also times dim^-1/2), beta = sigmoid(b), g = exp(-exp(A_log) softplus(a + dt_bias));
@@ -27,6 +27,8 @@ struct DeltaShape {
   int ldp;                 // row stride of the projections
   int off_q, off_k, off_v, off_b;   // first columns of the q, k, v and b projections in a row
 };
+
+constexpr int kStepThreads = 1024;      // of a workgroup of a step of single tokens
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float softplusf_(float x) { return x > 20.f ? x : log1pf(expf(x)); }
@@ -272,6 +274,167 @@ delta_out_kernel(const float* __restrict__ o, const float* __restrict__ gate_pre
   }
 }
 
+// A step of single tokens (every entry has one): all of the above in one launch, a workgroup a (q/k head, entry) with the heads that
+// read that q/k head, so that what the convolution reads and replaces of the request's state belongs to one workgroup.  The state's
+// columns, `PASSES` a thread at a time, are asked for before anything else and arrive while convolution, unit lengths and decays are
+// made; the heads' outputs are normed from LDS.  Every sum is added in the order of the kernels above: the same bits.
+// Bound by its trips to memory (the slot, then the state) and by what a CU moves of the state, 256 KB for two heads of 128 x 128: with
+// eight requests of 8 heads over 4 q/k heads 32 workgroups, 12.6 us for the launch, where the four take 29.5 (prepare 11.7, the
+// convolution's state 5.1, scan 8.2, output 5.2).  (With the loads of the state, the taps and the gates each waited for by itself: 15.8.)
+template <int R, int G, int LANES, typename TO>
+__global__ void __launch_bounds__(kStepThreads)
+delta_step_kernel(const float* __restrict__ proj, DeltaShape sh, const int32_t* __restrict__ q_start,
+                  const int32_t* __restrict__ state_slots, float* __restrict__ state, size_t state_stride, size_t s_offset,
+                  const float* __restrict__ taps_w, const float* __restrict__ dt_pre, int ld_dt, const float* __restrict__ dt_bias,
+                  const float* __restrict__ a_log, const float* __restrict__ gate_pre, int ld_gate,
+                  const float* __restrict__ norm_w, float eps, TO* __restrict__ out, bool vec) {
+  constexpr int GR = G * R, DP = LANES * GR, COLS = kStepThreads / LANES, PASSES = 32 / GR < 8 ? 32 / GR : 8;
+  typedef float rows_t __attribute__((ext_vector_type(R)));
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kv = blockIdx.x, e = blockIdx.y;
+  const int dim = sh.dim, vdim = sh.vdim, group = sh.heads / sh.kv_heads, h0 = kv * group, cols = group * vdim;
+  const int nqk = sh.kv_heads * dim, nv = sh.heads * vdim, channels = 2 * nqk + nv, keep = sh.taps - 1;
+  float* const q = lds;                      // [DP], zeros from dim on
+  float* const k = q + DP;                   // [DP]
+  float* const g = k + DP;                   // [group][DP]
+  float* const v = g + group * DP;           // [cols]
+  float* const o = v + cols;                 // [cols]
+  float* const gate = o + cols;              // [cols]
+  int* const head = reinterpret_cast<int*>(gate + cols);      // [cols] a column's head
+  float* const beta = gate + 2 * cols;       // [group]
+  const int t = q_start[e];
+  float* const st = state + (size_t)state_slots[e] * state_stride;
+  float* const sp = st + s_offset + (size_t)h0 * vdim * dim;      // column f of the workgroup's: at f * dim
+  const int part = lane & (LANES - 1), i0 = part * GR, mine = tid / LANES;
+  float s[PASSES][GR];
+  auto load = [&](int f0) {
+    if (vec) {
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          const uint32_t at = (uint32_t)(min(f0 + p * COLS + mine, cols - 1) * dim + min(i0 + j * R, dim - R));
+          const rows_t x = *reinterpret_cast<const rows_t*>(sp + at);
+#pragma unroll
+          for (int r = 0; r < R; ++r) s[p][j * R + r] = x[r];
+        }
+    } else {
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+        for (int r = 0; r < GR; ++r) s[p][r] = sp[(uint32_t)(min(f0 + p * COLS + mine, cols - 1) * dim + min(i0 + r, dim - 1))];
+    }
+  };
+  auto store = [&](int f0) {
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int f = f0 + p * COLS + mine;
+      if (f >= cols) continue;
+      const uint32_t to = (uint32_t)(f * dim + i0);
+      if (vec) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+          rows_t x;
+#pragma unroll
+          for (int r = 0; r < R; ++r) x[r] = s[p][j * R + r];
+          if (i0 + j * R < dim) *reinterpret_cast<rows_t*>(sp + (to + j * R)) = x;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < GR; ++r)
+          if (i0 + r < dim) sp[to + r] = s[p][r];
+      }
+    }
+  };
+  load(0);
+  // the workgroup's channels: q, k, then v
+  const int own = 2 * dim + cols;
+  auto channel = [&](int i) { return i < dim ? kv * dim + i : i < 2 * dim ? nqk + kv * dim + i - dim : 2 * nqk + h0 * vdim + i - 2 * dim; };
+  auto input = [&](int i) {
+    return proj[(size_t)t * sh.ldp + (i < dim ? sh.off_q + kv * dim + i : i < 2 * dim ? sh.off_k + kv * dim + i - dim
+                                                                                     : sh.off_v + h0 * vdim + i - 2 * dim)];
+  };
+  float held[4], held_in = 0.f;              // of the thread's first channel: its earlier inputs and the token's
+  // (channels, decays and gates are different threads' where there are enough: each is a trip to memory of its own)
+  const int decays = own + group * DP, items = decays + cols;
+  for (int i = tid; i < items; i += kStepThreads) {
+    if (i < own) {
+      const int c = channel(i);
+      float x[4] = {0.f, 0.f, 0.f, 0.f};
+      const float in = input(i), y = convolve_one(st + c, taps_w + (size_t)c * sh.taps, keep, channels, in, 0.f, x);
+      if (i == tid) {
+        held_in = in;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) held[j] = x[j];
+      }
+      (i < dim ? q + i : i < 2 * dim ? k + i - dim : v + i - 2 * dim)[0] = y * sigmoidf_(y);
+    } else if (i < decays) {
+      const int hl = (i - own) / DP, h = h0 + hl, d = min((i - own) % DP, dim - 1);
+      const float pre = dt_pre[(size_t)t * ld_dt + (size_t)h * dim + d], bias = dt_bias[(size_t)h * dim + d], rate = expf(a_log[h]);
+      g[i - own] = expf(-rate * softplusf_(pre + bias));      // (beyond dim: never used)
+    } else {
+      const int f = i - decays, hl = f / vdim;
+      const float raw = gate_pre[(size_t)t * ld_gate + (size_t)h0 * vdim + f], b = proj[(size_t)t * sh.ldp + sh.off_b + h0 + hl];
+      gate[f] = sigmoidf_(raw);
+      head[f] = hl;
+      beta[hl] = sigmoidf_(b);                                // (the same by all of the head's columns)
+    }
+  }
+  for (int i = dim + tid; i < DP; i += kStepThreads) q[i] = k[i] = 0.f;
+  lds_barrier();
+  if (wave < 2) {
+    float* const x = wave == 0 ? q : k;
+    float ss = 0.f;
+    for (int i = lane; i < dim; i += 64) ss += x[i] * x[i];
+    ss = wave_sum(ss);
+    const float inv = (wave == 0 ? 1.0f / sqrtf((float)dim) : 1.0f) / sqrtf(ss + 1e-6f);
+    for (int i = lane; i < dim; i += 64) x[i] = x[i] * inv;
+  }
+  lds_barrier();
+  float kq = 0.f;                            // k . q
+  for (int i = lane; i < dim; i += 64) kq = fmaf(q[i], k[i], kq);
+  kq = wave_sum(kq);
+  float kr[GR], qr[GR];
+#pragma unroll
+  for (int r = 0; r < GR; ++r) kr[r] = k[i0 + r], qr[r] = q[i0 + r];
+  for (int f0 = 0; f0 < cols; f0 += PASSES * COLS) {
+    if (f0 > 0) load(f0);
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const int f = f0 + p * COLS + mine, there = min(f, cols - 1), hl = head[there];
+      float p1[G], p2[G];
+#pragma unroll
+      for (int j = 0; j < G; ++j) p1[j] = p2[j] = 0.f;
+#pragma unroll
+      for (int r = 0; r < GR; ++r) {
+        // (what was fetched for a row beyond dim is another row's; made zero here and not at the load, which would then stand
+        // under the condition and be waited for at once)
+        s[p][r] = i0 + r < dim ? s[p][r] * g[hl * DP + i0 + r] : 0.f;
+        p1[r / R] = fmaf(s[p][r], kr[r], p1[r / R]);
+        p2[r / R] = fmaf(s[p][r], qr[r], p2[r / R]);
+      }
+      const float d1 = column_sum<LANES>(p1), d2 = column_sum<LANES>(p2);
+      const float u = beta[hl] * (v[there] - d1);
+      if (part == 0 && f < cols) o[f] = fmaf(u, kq, d2);
+#pragma unroll
+      for (int r = 0; r < GR; ++r) s[p][r] = fmaf(kr[r], u, s[p][r]);
+    }
+    store(f0);
+  }
+  for (int i = tid; i < own; i += kStepThreads) push_inputs(st + channel(i), keep, channels, i == tid ? held_in : input(i), held, i == tid);
+  lds_barrier();
+  for (int hl = wave; hl < group; hl += kStepThreads / kWave) {
+    const float* const oh = o + hl * vdim;
+    float ss = 0.f;
+    for (int j = lane; j < vdim; j += 64) ss += oh[j] * oh[j];
+    ss = wave_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)vdim + eps);
+    for (int j = lane; j < vdim; j += 64)
+      out[((size_t)t * sh.heads + h0 + hl) * vdim + j] = from_f32<TO>(oh[j] * inv * norm_w[j] * gate[hl * vdim + j]);
+  }
+}
+
 // The second half of a low-rank map for few tokens: out[t, n] = sum_k x[t, k] * w[n, k], K small (the inner size of
 // the map).  A thread an output; the token's K inputs wait in LDS.  With many tokens the general product is the better
 // kernel (it reads a tile of w once for 64 tokens); the sums are added in its order (gemm_f32_tile.h), so that a token's
@@ -396,6 +559,53 @@ extern "C" int atoma_delta_out(const float* o, const float* gate_pre, int ld_gat
                        eps, (bf16_t*)out, heads, vdim);
   else
     return ATOMA_ERR_DTYPE;
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+static size_t step_lds_floats(const DeltaShape& sh, int dp) {
+  const size_t group = sh.heads / sh.kv_heads, cols = group * sh.vdim;
+  return 2 * dp + group * dp + 4 * cols + group;
+}
+static int padded_dim(int dim) { return dim <= 16 ? 16 : dim <= 32 ? 32 : dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
+
+// Whether delta_step_kernel takes heads of these sizes: its vectors fit LDS, and a workgroup's state is at most 256 KB, beyond which the
+// scan's many workgroups are the better split (four heads of 128 x 128 to a q/k head are the most that are measured).
+extern "C" int atoma_delta_step_fits(int heads, int kv_heads, int dim, int vdim, int taps) {
+  const DeltaShape sh{heads, kv_heads, dim, vdim, taps, 1, 0, 0, 0, 0};
+  return shape_ok(sh) && kv_heads <= 65535 && (size_t)(heads / kv_heads) * vdim * dim <= 65536 &&
+         step_lds_floats(sh, padded_dim(dim)) * sizeof(float) <= 60 * 1024;
+}
+
+// One token of every entry: what atoma_delta_prepare, atoma_delta_scan and atoma_delta_out do in turn.
+extern "C" int atoma_delta_step(const float* proj, int ldp, int off_q, int off_k, int off_v, int off_b, int heads, int kv_heads,
+                                int dim, int vdim, int taps, const int32_t* q_start, const int32_t* state_slots, float* state,
+                                size_t state_stride, const float* taps_w, const float* dt_pre, int ld_dt, const float* dt_bias,
+                                const float* a_log, const float* gate_pre, int ld_gate, const float* norm_w, float eps, void* out,
+                                int out_dtype, int n_entries, hipStream_t stream) {
+  if (n_entries <= 0) return 0;
+  const DeltaShape sh{heads, kv_heads, dim, vdim, taps, ldp, off_q, off_k, off_v, off_b};
+  if (!shape_ok(sh) || !atoma_delta_step_fits(heads, kv_heads, dim, vdim, taps) || n_entries > 65535) return ATOMA_ERR_SHAPE;
+  const size_t s_offset = (size_t)(taps - 1) * (2 * kv_heads * dim + heads * vdim);
+  const size_t lds = step_lds_floats(sh, padded_dim(dim)) * sizeof(float);
+  const bool vec = dim % 8 == 0 && s_offset % 8 == 0 && state_stride % 8 == 0 && (uintptr_t)state % 32 == 0;
+  const dim3 grid(kv_heads, n_entries), block(kStepThreads);
+#define ATOMA_STEP(R, G, LANES, TO)                                                                                              \
+  hipLaunchKernelGGL((delta_step_kernel<R, G, LANES, TO>), grid, block, lds, stream, proj, sh, q_start, state_slots, state,       \
+                     state_stride, s_offset, taps_w, dt_pre, ld_dt, dt_bias, a_log, gate_pre, ld_gate, norm_w, eps, (TO*)out, vec)
+#define ATOMA_STEP_BY_DIM(TO)                        \
+  do {                                               \
+    if (dim <= 16) ATOMA_STEP(1, 1, 16, TO);         \
+    else if (dim <= 32) ATOMA_STEP(1, 2, 16, TO);    \
+    else if (dim <= 64) ATOMA_STEP(2, 2, 16, TO);    \
+    else if (dim <= 128) ATOMA_STEP(4, 1, 32, TO);   \
+    else ATOMA_STEP(8, 1, 32, TO);                   \
+  } while (0)
+  if (out_dtype == kF32) ATOMA_STEP_BY_DIM(float);
+  else if (out_dtype == kBF16) ATOMA_STEP_BY_DIM(bf16_t);
+  else return ATOMA_ERR_DTYPE;
+#undef ATOMA_STEP_BY_DIM
+#undef ATOMA_STEP
   ATOMA_LAUNCH_CHECK();
   return 0;
 }

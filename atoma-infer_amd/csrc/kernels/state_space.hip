@@ -4,7 +4,7 @@
 //   S <- a S + dt B x^T;   y = S^T C + D x,        a = exp(-exp(A_log) dt),  dt = softplus(dt_raw + dt_bias),
 //
 // with x (vdim per head), B and C (n per group of heads) the token's projections after a short causal convolution over
-// time (with bias) and SiLU.  Everything here is float32.  Four kernels:
+// time (with bias) and SiLU.  Everything here is float32.  Its kernels:
 //   ssd_prepare      per token: the convolution (the taps - 1 inputs before an entry's first token come from the
 //                    request's state), bias and SiLU of the x, B, C channels; dt and the decay of every head;
 //   ssd_conv_state   per request: the last taps - 1 inputs of the convolution, for the request's next step;
@@ -13,6 +13,7 @@
 //                    16 neighbouring lanes (n / 16 rows each, rounded up); the tokens' inputs pass LDS in blocks;
 //   ssd_scores,      the same recurrence for entries of many tokens (prompts and their portions), 64 tokens at a time on
 //   ssd_chunk        the matrix cores in float32 (v_mfma_f32_16x16x4_f32), see below;
+//   ssd_step         prepare, conv_state and scan in one, for steps of single tokens;
 //   ssd_out          per token and norm group: y * silu(z), divided by the root mean square of its group, times the
 //                    weight, in the activation dtype.
 // The order of every sum depends on the sizes alone, so a token's result does not depend on how the request was cut
@@ -159,6 +160,88 @@ ssd_scan_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, con
       if (row < sh.n) s_ptr[row] = s[r];
     }
   }
+}
+
+// A step of single tokens (every entry has one): prepare, convolution state and scan in one launch, a workgroup a (request, head,
+// 16 * PASSES columns of S).  The columns are asked for before anything else and arrive while the workgroup makes the convolution of
+// its x and, as every head of a group does, of the group's B and C; the sums are added as above: the same bits.  x's part of the
+// convolution's state belongs to one workgroup, which replaces it; B's and C's, which all heads of the group read, are left to
+// ssd_out.  Bound by the state's bytes, from two trips to memory on.  Eight requests of 64 heads of 128 x 64 (34 MB
+// read and written): 10.3 us, where prepare, the convolution's state and the scan take 5.0 + 5.2 + 8.5; 21 with masks on the state at
+// its loads, which the compiler then waits for one by one.
+template <int R, int PASSES>
+__global__ void __launch_bounds__(256)
+ssd_step_kernel(const float* __restrict__ proj, SsdShape sh, const int32_t* __restrict__ q_start,
+                const int32_t* __restrict__ state_slots, float* __restrict__ state, size_t state_stride,
+                const float* __restrict__ taps_w, const float* __restrict__ conv_bias, const float* __restrict__ dt_bias,
+                const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ y) {
+  constexpr int COLS = 16 * PASSES;
+  __shared__ float sb[16 * R], sc[16 * R], sx[COLS], scalars[3];
+  const int e = blockIdx.z, h = blockIdx.y, v0 = blockIdx.x * COLS, tid = threadIdx.x;
+  const int inner = sh.heads * sh.vdim, gn = sh.groups * sh.n, channels = inner + 2 * gn, keep = sh.taps - 1;
+  const int g = h / (sh.heads / sh.groups), col = tid >> 4, l = tid & 15;
+  const int t = q_start[e];
+  float* const st = state + (size_t)state_slots[e] * state_stride;
+  float* const sp = st + (size_t)keep * channels + ((size_t)h * sh.vdim + v0) * sh.n;
+  const int live = min(COLS, sh.vdim - v0);         // columns that exist
+  float s[PASSES][R];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int v = p * 16 + col, row = l + 16 * r;
+      s[p][r] = sp[(uint32_t)(min(v, live - 1) * sh.n + min(row, sh.n - 1))];
+    }
+  auto input = [&](int c) { return proj[(size_t)t * sh.ldp + sh.off_x + c]; };
+  float held[4] = {0.f, 0.f, 0.f, 0.f}, held_in = 0.f;      // of the thread's column of x: the earlier inputs and the token's
+  static_assert(COLS <= 256, "x is everybody's first channel");
+  for (int i = tid; i < COLS + 32 * R; i += 256) {
+    const int j = (i - COLS) % (16 * R);
+    const bool of_c = i >= COLS + 16 * R, there = i < COLS ? i < live : j < sh.n;
+    float out = 0.f;
+    if (there) {
+      const int c = i < COLS ? h * sh.vdim + v0 + i : inner + (of_c ? gn : 0) + g * sh.n + j;
+      float x[4] = {0.f, 0.f, 0.f, 0.f};
+      const float in = input(c), z = convolve_one(st + c, taps_w + (size_t)c * sh.taps, keep, channels, in, conv_bias[c], x);
+      out = z * ssd_sigmoid(z);
+      if (i == tid) {
+        held_in = in;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) held[q] = x[q];
+      }
+    }
+    (i < COLS ? sx + i : of_c ? sc + j : sb + j)[0] = out;
+  }
+  // (one lane, of a wave whose others have no second channel: its trip to memory runs beside theirs)
+  if (tid == 255) {
+    const float rate = expf(a_log[h]), step = ssd_softplus(proj[(size_t)t * sh.ldp + sh.off_dt + h] + dt_bias[h]);
+    scalars[0] = step, scalars[1] = expf(-rate * step), scalars[2] = d_skip[h];
+  }
+  lds_barrier();
+  const float d = scalars[0], a = scalars[1], dh = scalars[2];
+  float b[R], cc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) b[r] = sb[l + 16 * r], cc[r] = sc[l + 16 * r];
+#pragma unroll
+  for (int p = 0; p < PASSES; ++p) {
+    const int v = p * 16 + col;
+    const float xv = sx[v], w = d * xv;
+    float acc = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      // (made zero here and not at the load, which would then stand under the condition and be waited for at once)
+      s[p][r] = l + 16 * r < sh.n ? fmaf(a, s[p][r], w * b[r]) : 0.f;
+      acc = fmaf(s[p][r], cc[r], acc);
+    }
+    acc = lanes16_sum(acc);
+    if (v < live) {
+      if (l == 0) y[(size_t)t * inner + (size_t)h * sh.vdim + v0 + v] = acc + dh * xv;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+        if (l + 16 * r < sh.n) sp[(size_t)v * sh.n + l + 16 * r] = s[p][r];
+    }
+  }
+  if (tid < live) push_inputs(st + h * sh.vdim + v0 + tid, keep, channels, held_in, held, true);
 }
 
 // The recurrence 64 tokens at a time.  With c_t the sum of the log decays of the chunk's tokens up to t (inclusive),
@@ -421,12 +504,30 @@ ssd_scores_kernel(const float* __restrict__ xbc, SsdShape sh, const int32_t* __r
 }
 
 // one workgroup per (token, norm group); parts of up to 4,096 columns wait in registers between the two passes
-template <typename TO, int PER>
-__global__ void __launch_bounds__(256)
+// What is left of the convolution's state after ssd_step_kernel (state: null elsewhere): channels from `first` on of the token's request
+struct SsdTail {
+  float* state;
+  const int32_t* state_slots;
+  size_t stride;
+  int off_x, first, channels, keep;
+};
+
+template <typename TO, int PER, int NT>
+__global__ void __launch_bounds__(NT)
 ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int ldp, int off_z,
-               const float* __restrict__ w, float eps, int inner, int part, TO* __restrict__ out) {
-  __shared__ float scratch[4];
+               const float* __restrict__ w, float eps, int inner, int part, TO* __restrict__ out, SsdTail tail) {
+  __shared__ float scratch[NT / 64];
   const int t = blockIdx.x, p0 = blockIdx.y * part;
+  if (tail.state != nullptr && blockIdx.y == 0) {
+    // (a step of single tokens: token t is entry t's)
+    float* const st = tail.state + (size_t)tail.state_slots[t] * tail.stride;
+    for (int c = tail.first + threadIdx.x; c < tail.channels; c += NT) {
+      float x[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = st[(size_t)min(r, tail.keep - 1) * tail.channels + c];
+      push_inputs(st + c, tail.keep, tail.channels, proj[(size_t)t * ldp + tail.off_x + c], x, true);
+    }
+  }
   const float* zp = proj + (size_t)t * ldp + off_z + p0;
   const float* yp = y + (size_t)t * inner + p0;
   float ss = 0.f;
@@ -435,7 +536,7 @@ ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int 
     float u[P], yv[P], zv[P];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = threadIdx.x + j * 256;
+      const int i = threadIdx.x + j * NT;
       yv[j] = i < part ? yp[i] : 0.f;
       zv[j] = i < part ? zp[i] : 0.f;
     }
@@ -444,23 +545,23 @@ ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int 
       u[j] = yv[j] * (zv[j] * ssd_sigmoid(zv[j]));
       ss = fmaf(u[j], u[j], ss);
     }
-    ss = block_sum<4>(ss, scratch);
+    ss = block_sum<NT / 64>(ss, scratch);
     const float inv = 1.0f / sqrtf(ss / (float)part + eps);
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int i = threadIdx.x + j * 256;
+      const int i = threadIdx.x + j * NT;
       if (i < part) out[(size_t)t * inner + p0 + i] = from_f32<TO>(u[j] * inv * w[p0 + i]);
     }
     return;
   }
-  for (int i = threadIdx.x; i < part; i += 256) {
+  for (int i = threadIdx.x; i < part; i += NT) {
     const float z = zp[i];
     const float u = yp[i] * (z * ssd_sigmoid(z));
     ss = fmaf(u, u, ss);
   }
-  ss = block_sum<4>(ss, scratch);
+  ss = block_sum<NT / 64>(ss, scratch);
   const float inv = 1.0f / sqrtf(ss / (float)part + eps);
-  for (int i = threadIdx.x; i < part; i += 256) {
+  for (int i = threadIdx.x; i < part; i += NT) {
     const float z = zp[i];
     const float u = yp[i] * (z * ssd_sigmoid(z));
     out[(size_t)t * inner + p0 + i] = from_f32<TO>(u * inv * w[p0 + i]);
@@ -600,25 +701,56 @@ extern "C" int atoma_ssd_chunk(const float* xbc, const float* dt, const float* a
 }
 
 extern "C" int atoma_ssd_out(const float* y, const float* proj, int ldp, int off_z, const float* w, float eps,
-                             int inner, int norm_groups, void* out, int out_dtype, int n_tokens, hipStream_t stream) {
+                             int inner, int norm_groups, void* out, int out_dtype, int n_tokens, float* state,
+                             const int32_t* state_slots, size_t state_stride, int off_x, int channels, int taps, hipStream_t stream) {
   if (n_tokens <= 0) return 0;
   if (inner <= 0 || norm_groups <= 0 || inner % norm_groups || norm_groups > 65535 || ldp < inner) return ATOMA_ERR_SHAPE;
   const int part = inner / norm_groups;
-  dim3 grid(n_tokens, norm_groups), block(256);
-#define ATOMA_SSD_OUT(TO, PER)                                                                                    \
-  hipLaunchKernelGGL((ssd_out_kernel<TO, PER>), grid, block, 0, stream, y, proj, ldp, off_z, w, eps, inner, part, \
-                     (TO*)out)
-#define ATOMA_SSD_OUT_BY_PART(TO)                 \
-  do {                                            \
-    if (part <= 1024) ATOMA_SSD_OUT(TO, 4);       \
-    else if (part <= 4096) ATOMA_SSD_OUT(TO, 16); \
-    else ATOMA_SSD_OUT(TO, 0);                    \
+  if (taps < 2) state = nullptr;
+  if (state != nullptr && (channels < inner || state_slots == nullptr || taps > 64)) return ATOMA_ERR_SHAPE;
+  const SsdTail tail{state, state_slots, state_stride, off_x, inner, channels, taps - 1};
+  const dim3 grid(n_tokens, norm_groups);
+#define ATOMA_SSD_OUT(TO, PER, NT)                                                                                       \
+  hipLaunchKernelGGL((ssd_out_kernel<TO, PER, NT>), grid, dim3(NT), 0, stream, y, proj, ldp, off_z, w, eps, inner, part, \
+                     (TO*)out, tail)
+  // (four values a thread: eight tokens of 4,096 take 7.6 us, 10.7 with sixteen)
+#define ATOMA_SSD_OUT_BY_PART(TO)                     \
+  do {                                                \
+    if (part <= 1024) ATOMA_SSD_OUT(TO, 4, 256);      \
+    else if (part <= 4096) ATOMA_SSD_OUT(TO, 4, 1024); \
+    else ATOMA_SSD_OUT(TO, 0, 1024);                  \
   } while (0)
   if (out_dtype == kF32) ATOMA_SSD_OUT_BY_PART(float);
   else if (out_dtype == kBF16) ATOMA_SSD_OUT_BY_PART(bf16_t);
   else return ATOMA_ERR_DTYPE;
 #undef ATOMA_SSD_OUT_BY_PART
 #undef ATOMA_SSD_OUT
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+// One token of every entry: what atoma_ssd_prepare, atoma_ssd_conv_state and atoma_ssd_scan do in turn, but for B's and C's part of the
+// convolution's state, which atoma_ssd_out replaces where it is given the state.
+extern "C" int atoma_ssd_step(const float* proj, int ldp, int off_x, int off_dt, int heads, int groups, int vdim, int n, int taps,
+                              const int32_t* q_start, const int32_t* state_slots, float* state, size_t state_stride,
+                              const float* taps_w, const float* conv_bias, const float* dt_bias, const float* a_log,
+                              const float* d_skip, float* y, int n_entries, hipStream_t stream) {
+  if (n_entries <= 0) return 0;
+  const SsdShape sh{heads, groups, vdim, n, taps, ldp, 0, off_x, off_dt};
+  if (!shape_ok(sh) || n_entries > 65535 || heads > 65535) return ATOMA_ERR_SHAPE;
+  const int rows = (n + 15) / 16;
+#define ATOMA_STEP(R, P)                                                                                                     \
+  hipLaunchKernelGGL((ssd_step_kernel<R, P>), dim3((vdim + 16 * P - 1) / (16 * P), heads, n_entries), dim3(256), 0, stream,  \
+                     proj, sh, q_start, state_slots, state, state_stride, taps_w, conv_bias, dt_bias, a_log, d_skip, y)
+  if (rows <= 1) ATOMA_STEP(1, 4);
+  else if (rows <= 2) ATOMA_STEP(2, 4);
+  else if (rows <= 3) ATOMA_STEP(3, 4);
+  else if (rows <= 4) ATOMA_STEP(4, 4);
+  else if (rows <= 6) ATOMA_STEP(6, 4);
+  else if (rows <= 8) ATOMA_STEP(8, 4);
+  else if (rows <= 12) ATOMA_STEP(12, 2);
+  else ATOMA_STEP(16, 2);
+#undef ATOMA_STEP
   ATOMA_LAUNCH_CHECK();
   return 0;
 }

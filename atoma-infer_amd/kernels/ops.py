@@ -533,6 +533,44 @@ def delta_out(o: torch.Tensor, gate_pre: torch.Tensor, w: torch.Tensor, eps: flo
     return out
 
 
+def delta_step_fits(heads: int, kv_heads: int, dim: int, vdim: int, taps: int) -> bool:
+    """Whether ``delta_step`` takes heads of these sizes."""
+    return bool(_module("delta_rule").atoma_delta_step_fits(heads, kv_heads, dim, vdim, taps))
+
+
+def delta_step(proj: torch.Tensor, offsets, heads: int, kv_heads: int, dim: int, vdim: int, taps: int, q_start: torch.Tensor,
+               state_slots: torch.Tensor, state: torch.Tensor, taps_w: torch.Tensor, dt_pre: torch.Tensor, dt_bias: torch.Tensor,
+               a_log: torch.Tensor, gate_pre: torch.Tensor, norm_w: torch.Tensor, eps: float, out_dtype: torch.dtype) -> torch.Tensor:
+    """``delta_prepare``, ``delta_scan`` and ``delta_out`` of a step whose entries have one token each, in one launch (the same
+    bits)."""
+    _dev(proj, q_start, state_slots, state, taps_w, dt_pre, dt_bias, a_log, gate_pre, norm_w)
+    t, s = proj.shape[0], state_slots.numel()
+    nqk, nv, nd = kv_heads * dim, heads * vdim, heads * dim
+    channels = 2 * nqk + nv
+    off_q, off_k, off_v, off_b = (int(o) for o in offsets)
+    _need(t == s, "one token an entry")
+    _need(proj.dtype is torch.float32 and proj.dim() == 2 and proj.stride(1) == 1, "proj must be float32 [T, ld]")
+    _need(max(off_q + nqk, off_k + nqk, off_v + nv, off_b + heads) <= proj.shape[1] and min(offsets) >= 0,
+          "the projections' columns do not fit proj")
+    _i32(q_start, "q_start", s + 1)
+    _i32(state_slots, "state_slots", s)
+    _need(state.dtype is torch.float32 and state.dim() == 2 and state.is_contiguous()
+          and state.shape[1] == (taps - 1) * channels + heads * vdim * dim, "state: bad shape")
+    _f32(taps_w, "taps", channels * taps)
+    for x, n, what in ((dt_pre, nd, "dt_pre"), (gate_pre, nv, "gate")):
+        _need(x.dtype is torch.float32 and x.stride(1) == 1 and tuple(x.shape) == (t, n), f"{what}: bad shape")
+    _f32(dt_bias, "dt_bias", nd)
+    _f32(a_log, "A_log", heads)
+    _f32(norm_w, "norm weight", vdim)
+    out = torch.empty((t, nv), dtype=out_dtype, device=proj.device)
+    _check(_module("delta_rule").atoma_delta_step(
+        _p(proj), proj.stride(0), off_q, off_k, off_v, off_b, heads, kv_heads, dim, vdim, taps, _p(q_start), _p(state_slots),
+        _p(state), ctypes.c_size_t(state.stride(0)), _p(taps_w), _p(dt_pre), dt_pre.stride(0) if t > 1 else nd, _p(dt_bias),
+        _p(a_log), _p(gate_pre), gate_pre.stride(0) if t > 1 else nv, _p(norm_w), ctypes.c_float(eps), _p(out), _code(out, "out"),
+        s, _stream()), "delta_step")
+    return out
+
+
 # ---- a state-space recurrence with a scalar decay per head (state_space.hip) ----------------------------------------
 
 def _ssd_state_ok(state, heads, groups, vdim, n, taps):
@@ -633,10 +671,39 @@ def ssd_scan(xbc: torch.Tensor, dt: torch.Tensor, decay: torch.Tensor, a_log: to
     return y
 
 
+def ssd_step(proj: torch.Tensor, offsets, heads: int, groups: int, vdim: int, n: int, taps: int, q_start: torch.Tensor,
+             state_slots: torch.Tensor, state: torch.Tensor, taps_w: torch.Tensor, conv_bias: torch.Tensor, dt_bias: torch.Tensor,
+             a_log: torch.Tensor, d_skip: torch.Tensor) -> torch.Tensor:
+    """``ssd_prepare``, ``ssd_conv_state`` and ``ssd_scan`` of a step whose entries have one token each, in one launch (the same
+    bits), but for B's and C's part of the convolution's state: ``ssd_out`` with ``tail`` replaces it."""
+    _dev(proj, q_start, state_slots, state, taps_w, conv_bias, dt_bias, a_log, d_skip)
+    t, s = proj.shape[0], state_slots.numel()
+    channels = _ssd_state_ok(state, heads, groups, vdim, n, taps)
+    off_z, off_x, off_dt = (int(o) for o in offsets)
+    _need(t == s, "one token an entry")
+    _need(proj.dtype is torch.float32 and proj.dim() == 2 and proj.stride(1) == 1, "proj must be float32 [T, ld]")
+    _need(min(off_z, off_x, off_dt) >= 0 and max(off_z + heads * vdim, off_x + channels, off_dt + heads) <= proj.shape[1],
+          "the projections' columns do not fit proj")
+    _i32(q_start, "q_start", s + 1)
+    _i32(state_slots, "state_slots", s)
+    _f32(taps_w, "taps", channels * taps)
+    _f32(conv_bias, "the convolution's bias", channels)
+    _f32(dt_bias, "dt_bias", heads)
+    _f32(a_log, "A_log", heads)
+    _f32(d_skip, "D", heads)
+    y = torch.empty((t, heads * vdim), dtype=torch.float32, device=proj.device)
+    _check(_module("state_space").atoma_ssd_step(
+        _p(proj), proj.stride(0), off_x, off_dt, heads, groups, vdim, n, taps, _p(q_start), _p(state_slots), _p(state),
+        ctypes.c_size_t(state.stride(0)), _p(taps_w), _p(conv_bias), _p(dt_bias), _p(a_log), _p(d_skip), _p(y), s, _stream()),
+        "ssd_step")
+    return y
+
+
 def ssd_out(y: torch.Tensor, proj: torch.Tensor, off_z: int, w: torch.Tensor, eps: float, norm_groups: int,
-            out_dtype: torch.dtype) -> torch.Tensor:
+            out_dtype: torch.dtype, tail=None) -> torch.Tensor:
     """u = y * silu(z) with z the columns of ``proj`` from ``off_z`` on; u divided by the root mean square of each of
-    its ``norm_groups`` equal parts, times w, in ``out_dtype``."""
+    its ``norm_groups`` equal parts, times w, in ``out_dtype``.  ``tail`` = (state, state_slots, off_x, channels, taps), behind
+    ``ssd_step``: the step's last inputs of the convolved channels behind x's go into the state."""
     _dev(y, proj, w)
     t, inner = y.shape
     _need(y.dtype is torch.float32 and y.is_contiguous(), "y: bad shape")
@@ -645,8 +712,18 @@ def ssd_out(y: torch.Tensor, proj: torch.Tensor, off_z: int, w: torch.Tensor, ep
     _need(norm_groups > 0 and inner % norm_groups == 0, "the norm's groups must divide the row")
     _f32(w, "norm weight", inner)
     out = torch.empty((t, inner), dtype=out_dtype, device=y.device)
+    state = slots = None
+    off_x = channels = taps = 0
+    if tail is not None:
+        state, slots, off_x, channels, taps = tail
+        _dev(state, slots)
+        _i32(slots, "state_slots", t)
+        _need(state.dtype is torch.float32 and state.dim() == 2 and state.is_contiguous() and channels >= inner
+              and state.shape[1] >= (taps - 1) * channels and 0 <= off_x and off_x + channels <= proj.shape[1], "state: bad shape")
     _check(_module("state_space").atoma_ssd_out(_p(y), _p(proj), proj.stride(0), int(off_z), _p(w), ctypes.c_float(eps),
-                                                inner, int(norm_groups), _p(out), _code(out, "out"), t, _stream()),
+                                                inner, int(norm_groups), _p(out), _code(out, "out"), t, _p(state), _p(slots),
+                                                ctypes.c_size_t(state.stride(0) if state is not None else 0), int(off_x),
+                                                int(channels), int(taps), _stream()),
            "ssd_out")
     return out
 

@@ -33,6 +33,11 @@ from .linear import linear, linear_delta
 from .position import rotation_frequencies
 
 
+def single_tokens(ctx) -> bool:
+    """Every entry of the step has one token: the recurrences' one-launch kernels take such steps."""
+    return ctx.n_tokens == ctx.n_entries and int(ctx.h_counts.max()) == 1
+
+
 class GatedDeltaRule(Mixer):
     def __init__(self, width: int, heads: int, kv_heads: int, dim: int, vdim: int, taps: int, norm_eps: float,
                  decay_rank: Optional[int] = None, gate_rank: Optional[int] = None):
@@ -119,6 +124,11 @@ class GatedDeltaRule(Mixer):
         pre = ops.lowrank_up(low, self.w_ag) if x.shape[0] <= ops.LOWRANK_UP_MAX_TOKENS else \
             linear(low, self.w_ag, torch.float32)
         dt_pre, gate_pre = pre[:, : self.nd], pre[:, self.nd:]
+        if single_tokens(ctx) and ops.delta_step_fits(self.heads, self.kv_heads, self.dim, self.vdim, self.taps):
+            y = ops.delta_step(proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim,
+                               self.vdim, self.taps, ctx.q_start, ctx.state_slots, state, self.taps_w, dt_pre, self.dt_bias,
+                               self.a_log, gate_pre, self.norm_w, self.norm_eps, x.dtype)
+            return linear_delta(y, self.w_o, None, self.w_o_tiled)
         qn, kn, vn, beta, decay, kq = ops.delta_prepare(
             proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim, self.vdim,
             self.taps, ctx.token_seq, ctx.q_start, ctx.state_slots, state, self.taps_w, dt_pre, self.dt_bias, self.a_log)
@@ -206,6 +216,12 @@ class StateSpaceDuality(Mixer):
         state = cache.state
         dims = (self.heads, self.groups, self.vdim, self.n, self.taps)
         proj = linear(x, self.w_in, torch.float32)
+        if single_tokens(ctx):
+            y = ops.ssd_step(proj, (self.off_z, self.off_x, self.off_dt), *dims, ctx.q_start, ctx.state_slots, state, self.taps_w,
+                             self.conv_b, self.dt_bias, self.a_log, self.d_skip)
+            u = ops.ssd_out(y, proj, self.off_z, self.norm_w, self.norm_eps, self.norm_groups, x.dtype,
+                            tail=(state, ctx.state_slots, self.off_x, self.channels, self.taps))
+            return linear_delta(u, self.w_o, sink, self.w_o_tiled)
         xbc, dt, decay = ops.ssd_prepare(proj, (self.off_z, self.off_x, self.off_dt), *dims, ctx.token_seq, ctx.q_start,
                                          ctx.state_slots, state, self.taps_w, self.conv_b, self.dt_bias, self.a_log)
         ops.ssd_conv_state(proj, self.off_x, *dims, ctx.q_start, ctx.state_slots, state)

@@ -144,6 +144,33 @@ def test_a_product_of_its_own_per_head(t, h, k, n, dtype):
 
 # ---- the recurrence alone ---------------------------------------------------------------------------------------------
 
+@pytest.mark.parametrize("heads, groups, vdim, n, taps, norm_groups, entries", [
+    (1, 1, 1, 1, 1, 1, 1), (4, 2, 24, 16, 2, 2, 3), (2, 1, 65, 33, 3, 1, 2), (6, 3, 100, 72, 4, 1, 5), (64, 1, 64, 128, 4, 1, 8),
+    (2, 2, 40, 200, 9, 1, 3), (3, 1, 50, 256, 4, 3, 2), (80, 1, 64, 16, 4, 1, 70)])
+def test_a_step_of_single_tokens_in_one_launch_is_the_same_bits(heads, groups, vdim, n, taps, norm_groups, entries):
+    """Outputs and state against the launches it stands for, over three steps; slots out of order, one of them untouched."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(heads + vdim + n)
+    r = lambda *size: torch.randn(*size, generator=g).to(DEV)
+    inner = heads * vdim
+    channels = inner + 2 * groups * n
+    offsets = (0, inner, inner + channels)
+    taps_w, conv_b, dt_bias, a_log, d_skip, norm_w = r(channels, taps), r(channels), r(heads), r(heads), r(heads), r(inner)
+    one = r(entries + 1, (taps - 1) * channels + heads * vdim * n)
+    four = one.clone()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slots, seq, q_start = i32([entries - i for i in range(entries)]), i32(list(range(entries))), i32(list(range(entries + 1)))
+    sizes = (heads, groups, vdim, n, taps)
+    for dtype in (torch.float32, torch.bfloat16, torch.float32):
+        proj = r(entries, inner + channels + heads + 3)
+        ins = ops.ssd_prepare(proj, offsets, *sizes, seq, q_start, slots, four, taps_w, conv_b, dt_bias, a_log)
+        ops.ssd_conv_state(proj, inner, *sizes, q_start, slots, four)
+        want = ops.ssd_out(ops.ssd_scan(*ins, a_log, d_skip, *sizes, q_start, slots, four), proj, 0, norm_w, 1e-5, norm_groups, dtype)
+        y = ops.ssd_step(proj, offsets, *sizes, q_start, slots, one, taps_w, conv_b, dt_bias, a_log, d_skip)
+        got = ops.ssd_out(y, proj, 0, norm_w, 1e-5, norm_groups, dtype, tail=(one, slots, inner, channels, taps))
+        assert torch.equal(got, want) and torch.equal(one, four)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads, groups, vdim, n, taps, parts", [(4, 2, 16, 16, 3, 2), (3, 1, 8, 12, 2, 1), (2, 2, 40, 100, 5, 5),
                                                                  (1, 1, 5, 1, 1, 5), (6, 3, 24, 200, 4, 3), (4, 4, 64, 48, 4, 2),

@@ -140,6 +140,33 @@ def test_the_recurrence_is_the_same_bits_however_it_is_cut(dim, vdim):
                                              state0[:, :(taps - 1) * (2 * kv * dim + heads * vdim)]).all())
 
 
+@pytest.mark.parametrize("dim, vdim, heads, kv, taps, n", [(12, 8, 4, 2, 3, 3), (30, 8, 2, 2, 1, 2), (64, 24, 4, 1, 4, 5), (72, 17, 4, 2, 2, 3),
+                                                           (128, 40, 6, 3, 9, 2), (200, 9, 2, 1, 4, 1), (128, 128, 8, 4, 4, 8),
+                                                           (256, 128, 2, 1, 4, 9), (16, 600, 2, 1, 4, 2), (1, 1, 1, 1, 2, 1), (64, 64, 4, 4, 4, 300)])
+def test_a_step_of_single_tokens_in_one_launch_is_the_same_bits(dim, vdim, heads, kv, taps, n):
+    """Outputs and state against the launches it stands for, over three steps; slots out of order, one of them untouched."""
+    from atoma_infer_amd.kernels import ops
+    assert ops.delta_step_fits(heads, kv, dim, vdim, taps)
+    g = torch.Generator().manual_seed(dim + vdim)
+    r = lambda *size: torch.randn(*size, generator=g).to(DEV)
+    nqk, nv, nd = kv * dim, heads * vdim, heads * dim
+    offsets = (0, nqk, 2 * nqk, 2 * nqk + nv)
+    ld = 2 * nqk + nv + heads + 5
+    taps_w, dt_bias, a_log, norm_w = r(2 * nqk + nv, taps), r(nd), r(heads), r(vdim)
+    one = r(n + 1, (taps - 1) * (2 * nqk + nv) + heads * vdim * dim)
+    four = one.clone()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slots, seq, q_start = i32([n - i for i in range(n)]), i32(list(range(n))), i32(list(range(n + 1)))
+    for dtype in (torch.float32, torch.bfloat16, torch.float32):
+        proj, pre = r(n, ld), r(n, nd + nv)
+        dt_pre, gate_pre = pre[:, :nd], pre[:, nd:]
+        sizes = (heads, kv, dim, vdim, taps)
+        ins = ops.delta_prepare(proj, offsets, *sizes, seq, q_start, slots, four, taps_w, dt_pre, dt_bias, a_log)
+        want = ops.delta_out(ops.delta_scan(*ins, *sizes, q_start, slots, four), gate_pre, norm_w, 1e-5, heads, vdim, dtype)
+        got = ops.delta_step(proj, offsets, *sizes, q_start, slots, one, taps_w, dt_pre, dt_bias, a_log, gate_pre, norm_w, 1e-5, dtype)
+        assert torch.equal(got, want) and torch.equal(one, four)
+
+
 def test_a_far_token_stays_in_the_recurrent_state():
     """Decays close to one and one early token whose value is large: hundreds of tokens later the read-out still
     holds it.  A state that is lost, cleared or carried by the wrong slot changes the late outputs entirely."""
