@@ -52,14 +52,22 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// Sum over a block of NWAVES*64 threads; every thread gets the result.  `scratch` holds NWAVES floats.
+// A barrier for what passes LDS: unlike __syncthreads it does not wait for the wave's loads from and stores to memory.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Sum over a block of NWAVES*64 threads; every thread gets the result.  `scratch` holds NWAVES floats.  What a thread has stored
+// to memory before is not waited for (the norms store the rows between their sums).
 template <int NWAVES> __device__ __forceinline__ float block_sum(float v, float* scratch) {
   v = wave_sum(v);
   if (NWAVES == 1) return v;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
+  lds_barrier();
   if (lane == 0) scratch[wave] = v;
-  __syncthreads();
+  lds_barrier();
   float t = 0.f;
 #pragma unroll
   for (int i = 0; i < NWAVES; ++i) t += scratch[i];
@@ -82,11 +90,51 @@ template <int NWAVES> __device__ __forceinline__ float block_max(float v, float*
 // Element type codes of the C interface.
 enum DType : int { kF32 = 0, kBF16 = 1 };
 
-// A barrier for what passes LDS: unlike __syncthreads it does not wait for the wave's loads from and stores to memory.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+// Four neighbouring values of a row as they come from memory (aligned to all four).  They become floats where they are used: a conversion
+// beside the load would make the wave wait for it before it asks for the next.
+template <typename T> struct Raw4 { float4 v; };
+template <> struct Raw4<bf16_t> { uint2 v; };
+__device__ __forceinline__ Raw4<float> fetch4(const float* p) { return {*reinterpret_cast<const float4*>(p)}; }
+__device__ __forceinline__ Raw4<bf16_t> fetch4(const bf16_t* p) { return {*reinterpret_cast<const uint2*>(p)}; }
+__device__ __forceinline__ float value4(const Raw4<float>& r, int i) { return i == 0 ? r.v.x : i == 1 ? r.v.y : i == 2 ? r.v.z : r.v.w; }
+__device__ __forceinline__ float value4(const Raw4<bf16_t>& r, int i) {
+  const uint32_t two = i < 2 ? r.v.x : r.v.y;
+  return __uint_as_float(i & 1 ? two & 0xffff0000u : two << 16);
+}
+
+// sum[j] += the sum over `planes` planes, in the order of their index, of the four values at column 4 * col[j] of p.  The loads of up to
+// eight planes are issued together (each is a trip to memory), and no more than there are planes, or the next of 1, 2, 4: repeats of the
+// last plane would cost the cache as much as others.
+template <int PB, int MAXJ, typename T, typename V>
+__device__ __forceinline__ void add_some_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, int n, const int (&col)[MAXJ]) {
+  Raw4<T> d[PB][MAXJ];
+#pragma unroll
+  for (int q = 0; q < PB; ++q) {
+    const T* const at = p + (size_t)min(q, n - 1) * stride;
+#pragma unroll
+    for (int j = 0; j < MAXJ; ++j) d[q][j] = fetch4(at + 4 * col[j]);
+  }
+#pragma unroll
+  for (int q = 0; q < PB; ++q) {
+    if (q >= n) break;
+#pragma unroll
+    for (int j = 0; j < MAXJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[j].v[i] += value4(d[q][j], i);
+  }
+}
+template <int MAXJ, typename T, typename V>
+__device__ __forceinline__ void add_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, int planes, const int (&col)[MAXJ]) {
+  constexpr int PB = MAXJ <= 2 ? 8 : 4;
+  if (planes == 1) {
+    add_some_planes<1, MAXJ>(sum, p, stride, 1, col);
+  } else if (planes == 2) {
+    add_some_planes<2, MAXJ>(sum, p, stride, 2, col);
+  } else if (planes <= 4) {
+    add_some_planes<4, MAXJ>(sum, p, stride, planes, col);
+  } else {
+    for (int p0 = 0; p0 < planes; p0 += PB) add_some_planes<PB, MAXJ>(sum, p + p0 * stride, stride, min(PB, planes - p0), col);
+  }
 }
 
 // One token of a causal convolution over time whose earlier inputs lie in the rows of `rows` (keep of them, `channels` apart), the

@@ -28,11 +28,15 @@ latent_prepare_kernel(const float* __restrict__ proj, int ldp, int off_q, int of
   __shared__ float scratch[4];
   const int t = blockIdx.x;
   const float* row = proj + (size_t)t * ldp;
+  // (what needs no sum goes first, a thread's loads of it together: behind the sum the queries were a trip to memory each)
+  const int slot = slot_mapping[t];
   float ss = 0.f;
   for (int i = threadIdx.x; i < rank; i += 256) ss = fmaf(row[off_c + i], row[off_c + i], ss);
+#pragma unroll 8
+  for (int i = threadIdx.x; i < nq; i += 256) q_out[(size_t)t * nq + i] = from_f32<TA>(row[off_q + i]);
+  for (int h = threadIdx.x; h < heads; h += 256) gate[(size_t)t * heads + h] = 1.0f / (1.0f + expf(-row[off_g + h]));
   ss = block_sum<4>(ss, scratch);
   const float inv = 1.0f / sqrtf(ss / (float)rank + eps);
-  const int slot = slot_mapping[t];
   if (slot >= 0) {
     const int page = slot / page_size, off = slot % page_size;
     TC* ktile = kcache + (size_t)page * page_size * rank_p;
@@ -43,8 +47,6 @@ latent_prepare_kernel(const float* __restrict__ proj, int ldp, int off_q, int of
       vtile[value_offset(i, off, rank_p, page_size)] = c;
     }
   }
-  for (int i = threadIdx.x; i < nq; i += 256) q_out[(size_t)t * nq + i] = from_f32<TA>(row[off_q + i]);
-  for (int h = threadIdx.x; h < heads; h += 256) gate[(size_t)t * heads + h] = 1.0f / (1.0f + expf(-row[off_g + h]));
 }
 
 // out[t, h * N + n] = (sum_k x[t, h * K + k] * w[(h * N + n) * K + k]) * (gate ? gate[t * H + h] : 1)

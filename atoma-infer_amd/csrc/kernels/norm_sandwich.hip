@@ -100,31 +100,13 @@ __device__ __forceinline__ void store4(bf16_t* p, const f4& x) {
   *reinterpret_cast<uint2*>(p) = o;
 }
 
-template <typename TD, int MAXJ>
-__device__ __forceinline__ void add_term(f4 (&d)[MAXJ], const Term& t, size_t base, int n4) {
-  const TD* p0 = (const TD*)t.data + base;
+template <int MAXJ>
+__device__ __forceinline__ void add_term(f4 (&d)[MAXJ], const Term& t, size_t base, const int (&col)[MAXJ]) {
   f4 sum[MAXJ];
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) sum[j] = f4{{0.f, 0.f, 0.f, 0.f}};
-  for (int s0 = 0; s0 < t.planes; s0 += 4) {
-    f4 x[4][MAXJ];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int s = s0 + q < t.planes ? s0 + q : t.planes - 1;
-#pragma unroll
-      for (int j = 0; j < MAXJ; ++j) {
-        const int c = threadIdx.x + j * 256;
-        if (c < n4) x[q][j] = load4(p0 + s * t.plane_stride + 4 * c);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (s0 + q < t.planes)
-#pragma unroll
-        for (int j = 0; j < MAXJ; ++j)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sum[j].v[i] += x[q][j].v[i];
-  }
+  if (t.dtype == kF32) add_planes(sum, (const float*)t.data + base, t.plane_stride, t.planes, col);
+  else add_planes(sum, (const bf16_t*)t.data + base, t.plane_stride, t.planes, col);
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j)
 #pragma unroll
@@ -139,20 +121,23 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   __shared__ float scratch[4];
   const size_t base = (size_t)blockIdx.x * width;
   const int n4 = width >> 2;
-  f4 d[MAXJ], x[MAXJ];
+  // (threads beyond the row's end fetch its last columns: no load stands under a condition.  Both norms' weights come with the
+  // rows: behind the sums they are two trips to memory more)
+  int col[MAXJ];
+  f4 d[MAXJ], x[MAXJ], wp[MAXJ], wn[MAXJ];
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) {
+    col[j] = min((int)threadIdx.x + j * 256, n4 - 1);
     d[j] = f4{{0.f, 0.f, 0.f, 0.f}};
-    const int c = threadIdx.x + j * 256;
-    if (c < n4) x[j] = load4(resid + base + 4 * c);
   }
-  const size_t base_a = row_of(a, base), base_b = row_of(b, base);
-  if (a.dtype == kF32) add_term<float, MAXJ>(d, a, base_a, n4);
-  else add_term<bf16_t, MAXJ>(d, a, base_a, n4);
-  if (n_terms > 1) {
-    if (b.dtype == kF32) add_term<float, MAXJ>(d, b, base_b, n4);
-    else add_term<bf16_t, MAXJ>(d, b, base_b, n4);
-  }
+#pragma unroll
+  for (int j = 0; j < MAXJ; ++j) x[j] = load4(resid + base + 4 * col[j]);
+  const float* const w1 = w_post != nullptr ? w_post : resid + base;       // (some row, where there is no such norm)
+  const float* const w2 = out != nullptr ? w_next : resid + base;
+#pragma unroll
+  for (int j = 0; j < MAXJ; ++j) wp[j] = load4(w1 + 4 * col[j]), wn[j] = load4(w2 + 4 * col[j]);
+  add_term(d, a, row_of(a, base), col);
+  if (n_terms > 1) add_term(d, b, row_of(b, base), col);
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j)
@@ -169,10 +154,9 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   for (int j = 0; j < MAXJ; ++j) {
     const int c = threadIdx.x + j * 256;
     if (c < n4) {
-      const f4 wp = w_post != nullptr ? load4(w_post + 4 * c) : f4{{1.f, 1.f, 1.f, 1.f}};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        x[j].v[i] += w_post != nullptr ? d[j].v[i] * inv * wp.v[i] : d[j].v[i];
+        x[j].v[i] += w_post != nullptr ? d[j].v[i] * inv * wp[j].v[i] : d[j].v[i];
         ss2 += x[j].v[i] * x[j].v[i];
       }
       store4(resid + base + 4 * c, x[j]);
@@ -185,10 +169,9 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   for (int j = 0; j < MAXJ; ++j) {
     const int c = threadIdx.x + j * 256;
     if (c < n4) {
-      const f4 wn = load4(w_next + 4 * c);
       f4 y;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y.v[i] = x[j].v[i] * inv2 * wn.v[i];
+      for (int i = 0; i < 4; ++i) y.v[i] = x[j].v[i] * inv2 * wn[j].v[i];
       store4(out + base + 4 * c, y);
     }
   }
@@ -302,12 +285,13 @@ depth_average_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms,
   const size_t base = (size_t)blockIdx.x * width;
   const int n4 = width >> 2;
   f4 d[MAXJ], x[MAXJ], acc[MAXJ];
+  int col[MAXJ];
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) {
+    col[j] = min((int)threadIdx.x + j * 256, n4 - 1);
     d[j] = f4{{0.f, 0.f, 0.f, 0.f}};
     acc[j] = f4{{0.f, 0.f, 0.f, 0.f}};
-    const int c = threadIdx.x + j * 256;
-    if (c < n4) x[j] = load4(resid + base + 4 * c);
+    x[j] = load4(resid + base + 4 * col[j]);
   }
   // sum_(j < n - 1) dw[j] * results[j], j ascending
   for (int s0 = 0; s0 < n - 1; s0 += 4) {
@@ -316,10 +300,7 @@ depth_average_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms,
     for (int q = 0; q < 4; ++q) {
       const int s = s0 + q < n - 1 ? s0 + q : n - 2;
 #pragma unroll
-      for (int j = 0; j < MAXJ; ++j) {
-        const int c = threadIdx.x + j * 256;
-        if (c < n4) r[q][j] = load4(earlier + (size_t)s * result_stride + base + 4 * c);
-      }
+      for (int j = 0; j < MAXJ; ++j) r[q][j] = load4(earlier + (size_t)s * result_stride + base + 4 * col[j]);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -331,12 +312,8 @@ depth_average_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms,
           for (int i = 0; i < 4; ++i) acc[j].v[i] += w * r[q][j].v[i];
       }
   }
-  if (a.dtype == kF32) add_term<float, MAXJ>(d, a, base, n4);
-  else add_term<bf16_t, MAXJ>(d, a, base, n4);
-  if (n_terms > 1) {
-    if (b.dtype == kF32) add_term<float, MAXJ>(d, b, base, n4);
-    else add_term<bf16_t, MAXJ>(d, b, base, n4);
-  }
+  add_term(d, a, base, col);
+  if (n_terms > 1) add_term(d, b, base, col);
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j)
