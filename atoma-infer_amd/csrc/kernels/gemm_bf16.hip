@@ -842,6 +842,7 @@ extern "C" int atoma_gemm_bf16_skinny_rope_tiled(const void* a, const void* w_ti
 // share, each fetching an eighth of the activations, where the product with the rotary epilogue has 192 that each
 // fetch all of them), summed here in the order of the planes, rotated and stored: a thread takes four outputs of a row.
 constexpr int kMaxPlanes = 8;
+template <int P>      // planes that are fetched (of more than there are, the first again)
 __global__ void __launch_bounds__(256)
 rope_from_planes_kernel(const float* __restrict__ planes, int slices, size_t plane, int M, int N, uint16_t* __restrict__ q_out,
                         int ldq, RopeArgs ra) {
@@ -850,12 +851,12 @@ rope_from_planes_kernel(const float* __restrict__ planes, int slices, size_t pla
   if (n0 + 3 >= N) return;
   const float* p = planes + (size_t)row * N + n0;
   // (all planes are asked for at once: each load is a trip to memory)
-  f32x4 v[kMaxPlanes];
+  f32x4 v[P];
 #pragma unroll
-  for (int s = 0; s < kMaxPlanes; ++s) v[s] = *reinterpret_cast<const f32x4*>(p + (size_t)(s < slices ? s : 0) * plane);
+  for (int s = 0; s < P; ++s) v[s] = *reinterpret_cast<const f32x4*>(p + (size_t)(s < slices ? s : 0) * plane);
   f32x4 sum = v[0];
 #pragma unroll
-  for (int s = 1; s < kMaxPlanes; ++s)
+  for (int s = 1; s < P; ++s)
     if (s < slices) sum[0] += v[s][0], sum[1] += v[s][1], sum[2] += v[s][2], sum[3] += v[s][3];
   rope_store4(sum[0], sum[1], sum[2], sum[3], row, n0, ra, q_out, ldq);
 }
@@ -874,8 +875,13 @@ extern "C" int atoma_rope_from_planes(const float* planes, int slices, int M, vo
     return ATOMA_ERR_SHAPE;
   const RopeArgs ra{positions, cos_t, sin_t, (uint16_t*)kcache, (uint16_t*)vcache, slot_mapping, page_size, nh, nkv, hd};
   dim3 grid(M, (N / 4 + 255) / 256);
-  hipLaunchKernelGGL(rope_from_planes_kernel, grid, dim3(256), 0, stream, planes, slices, (size_t)M * N, M, N,
-                     (uint16_t*)q_out, ldq, ra);
+#define ATOMA_ROPE_PLANES(P)                                                                                             \
+  hipLaunchKernelGGL((rope_from_planes_kernel<P>), grid, dim3(256), 0, stream, planes, slices, (size_t)M * N, M, N,      \
+                     (uint16_t*)q_out, ldq, ra)
+  if (slices <= 2) ATOMA_ROPE_PLANES(2);
+  else if (slices <= 4) ATOMA_ROPE_PLANES(4);
+  else ATOMA_ROPE_PLANES(kMaxPlanes);
+#undef ATOMA_ROPE_PLANES
   ATOMA_LAUNCH_CHECK();
   return 0;
 }

@@ -72,7 +72,9 @@ def linear_delta(x, w: torch.Tensor, sink: Optional[ResidualSink] = None, tiled=
     x = as_tensor(x)
     if x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16:
         from ..kernels import gemm_bf16
-        y = gemm_bf16.linear_planes(x, w, tiled.many if tiled is not None else None)
+        y = gemm_bf16.try_few_rows_planes(x, w)
+        if y is None:
+            y = gemm_bf16.linear_planes(x, w, tiled.many if tiled is not None else None)
         if y is not None:
             return y
         # many rows that the tile kernel has left: the library's product, its float32 sums handed to the residual stream

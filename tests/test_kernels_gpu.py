@@ -955,6 +955,51 @@ def test_gemm_tile(tile, m, n, k):
         assert bool(((c.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 32, 128), (41, 80, 192), (63, 544, 512), (64, 1056, 1024), (64, 2048, 8192), (1, 64, 128)])
+def test_gemm_tile_of_64_rows(m, n, k):
+    """The tiles for 33 to 64 rows, as test_gemm_tile holds the others; then what parts call with as many rows: 41 and more leave the
+    planned planes, 33 and more the fused SiLU."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    wide = rnd(m, k + 8, dtype=torch.bfloat16, seed=1)
+    x, w = wide[:, 8:], rnd(n, k, dtype=torch.bfloat16, seed=2)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    bound = k * 2.0 ** -24 * size
+    for tile in gb.FEW_ROWS_TILES:
+        for slices in (1, 2, 8):
+            if k % (64 * slices) == 0:
+                c = torch.full((slices, m, n), 7.0, device=DEV)
+                gb.tile_product(x, w, c, gb.TILE_F32, tile, slices)
+                assert bool(((c.double().sum(0) - want).abs() <= bound).all())
+    if n % 32 == 0:
+        z = want.view(m, n // 32, 2, 16)
+        ref = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(m, n // 2)
+        c = torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV)
+        gb.tile_product(x, w, c, gb.TILE_SILU, 6)
+        for got in (c, gb.try_linear_swiglu(x, w)) if m > 32 else (c,):
+            assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
+    if m > gb.FEW_ROWS_PLANES_MIN_M:
+        planes = gb.try_few_rows_planes(x, w)
+        assert planes.shape[0] == gb._few_rows_plan(m, n, k)[1] and bool(((planes.double().sum(0) - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("planes", [1, 2, 3, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("width", [4, 1028, 2048, 4096])
+def test_add_rmsnorm_planes(planes, width):
+    """Every number of planes: the sums in their order, bit for bit, and the norm of them (a float32 sum of `width` squares)."""
+    from atoma_infer_amd.kernels import ops
+    for ddt in (torch.float32, torch.bfloat16):
+        r0, d, w = rnd(5, width, seed=1), rnd(planes, 5, width, dtype=ddt, seed=2), rnd(width, dtype=torch.bfloat16, seed=3)
+        r = r0.clone()
+        out = ops.add_rmsnorm(r, d if planes > 1 else d[0], w, 1e-5, torch.float32)
+        want = r0.clone()
+        for p in range(planes):
+            want += d[p].float()
+        assert torch.equal(r, want)
+        x = want.double()
+        ref = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5) * w.double()
+        assert bool(((out.double() - ref).abs() <= width * 2.0 ** -24 * ref.abs() + 2.0 ** -22 * ref.abs()).all())
+
+
 def test_gemm_tile_silu_is_exact():
     """silu(gate) * up of the tile kernel, from gates and ups that are exact in float32: as few results as with the formula in
     float32 fall on the other side of a rounding to bfloat16 than the exact ones (an error of 2^-22 moves one in about 10,000),

@@ -167,6 +167,47 @@ def test_a_step_of_single_tokens_in_one_launch_is_the_same_bits(dim, vdim, heads
         assert torch.equal(got, want) and torch.equal(one, four)
 
 
+@pytest.mark.parametrize("nh, nkv, hd, hd_out, rot, ld_more", [(2, 1, 8, 8, 8, 0), (32, 8, 64, 64, 64, 2), (24, 8, 128, 128, 64, 0),
+                                                               (5, 5, 72, 80, 10, 4), (32, 8, 64, 64, 64, 1), (64, 8, 64, 64, 0, 0)])
+def test_q_k_norm_and_rotation_by_pairs(nh, nkv, hd, hd_out, rot, ld_more):
+    """Rows whose pairs stay in registers (few or many a thread), and odd strides and long rows, which the general kernel takes, against
+    64 bits: norms over the whole projections, pairs of neighbours turned, padded heads zero, keys and raw values in their tiles."""
+    from atoma_infer_amd.kernels import ops
+    from atoma_infer_amd.cache.layout import pack_keys, pack_values
+    t, page = 5, 16
+    g = torch.Generator().manual_seed(nh + hd)
+    nq, nk = nh * hd, nkv * hd
+    qk = torch.randn(t, nq + nk + ld_more, generator=g)
+    wq, wk, inv = torch.rand(nq, generator=g) + 0.5, torch.rand(nk, generator=g) + 0.5, torch.rand(rot // 2, generator=g)
+    pos, slots = torch.tensor([0, 3, 17, 900, 5], dtype=torch.int32), torch.tensor([5, 0, 31, 16, 40], dtype=torch.int32)
+    kc = torch.full((3, nkv, page * hd_out), 7.0, device=DEV)
+    vc = kc.clone()
+    q = torch.full((t, nh * hd_out), 7.0, device=DEV)
+    ops.qk_norm_rope(qk.to(DEV), pos.to(DEV), inv.to(DEV), rot, wq.to(DEV), wk.to(DEV), 1e-5, q, kc, vc, slots.to(DEV), page, nh, nkv, hd, hd_out)
+
+    def normed(x, w, heads):
+        x = x.double()
+        y = (x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5) * w.double()).view(t, heads, hd)
+        out = torch.zeros(t, heads, hd_out, dtype=torch.float64)
+        angle = (pos.float()[:, None] * inv[None]).double()
+        c, s = angle.cos()[:, None], angle.sin()[:, None]
+        u, v = y[..., 0:rot:2], y[..., 1:rot:2]
+        out[..., :hd] = y
+        out[..., 0:rot:2], out[..., 1:rot:2] = u * c - v * s, v * c + u * s
+        return out
+
+    want_q, want_k = normed(qk[:, :nq], wq, nh), normed(qk[:, nq:nq + nk], wk, nkv)
+    assert (q.cpu().double().view(t, nh, hd_out) - want_q).abs().max() <= 2e-6 * want_q.abs().max()
+    tiles_k, tiles_v = torch.full((3, nkv, hd_out, page), 7.0, dtype=torch.float64), torch.full((3, nkv, hd_out, page), 7.0, dtype=torch.float64)
+    raw = torch.zeros(t, nkv, hd_out, dtype=torch.float64)
+    raw[..., :hd] = qk[:, nq:nq + nk].double().view(t, nkv, hd)
+    for i, slot in enumerate(slots.tolist()):
+        tiles_k[slot // page, :, :, slot % page], tiles_v[slot // page, :, :, slot % page] = want_k[i], raw[i]
+    as_tokens = lambda x: x.permute(0, 1, 3, 2).contiguous()
+    assert (kc.cpu().double() - pack_keys(as_tokens(tiles_k)).view(kc.shape)).abs().max() <= 2e-6 * want_k.abs().max()
+    assert torch.equal(vc.cpu().double(), pack_values(tiles_v).view(vc.shape))
+
+
 def test_a_far_token_stays_in_the_recurrent_state():
     """Decays close to one and one early token whose value is large: hundreds of tokens later the read-out still
     holds it.  A state that is lost, cleared or carried by the wrong slot changes the late outputs entirely."""
