@@ -838,7 +838,7 @@ extern "C" int atoma_gemm_bf16_skinny_rope_tiled(const void* a, const void* w_ti
   return launch_rope<1, 2, 1, 4, 2>(a, w_tiled, c, M, N, K, lda, K, ldc, ra, fa, stream);
 }
 
-// The fused q, k, v projection of 17 to 64 rows as float32 planes of a K-split product (which about 256 workgroups
+// The fused q, k, v projection of 17 to some hundred rows as float32 planes of a K-split product (which about 256 workgroups
 // share, each fetching an eighth of the activations, where the product with the rotary epilogue has 192 that each
 // fetch all of them), summed here in the order of the planes, rotated and stored: a thread takes four outputs of a row.
 constexpr int kMaxPlanes = 8;
@@ -878,7 +878,8 @@ extern "C" int atoma_rope_from_planes(const float* planes, int slices, int M, vo
 #define ATOMA_ROPE_PLANES(P)                                                                                             \
   hipLaunchKernelGGL((rope_from_planes_kernel<P>), grid, dim3(256), 0, stream, planes, slices, (size_t)M * N, M, N,      \
                      (uint16_t*)q_out, ldq, ra)
-  if (slices <= 2) ATOMA_ROPE_PLANES(2);
+  if (slices <= 1) ATOMA_ROPE_PLANES(1);
+  else if (slices <= 2) ATOMA_ROPE_PLANES(2);
   else if (slices <= 4) ATOMA_ROPE_PLANES(4);
   else ATOMA_ROPE_PLANES(kMaxPlanes);
 #undef ATOMA_ROPE_PLANES

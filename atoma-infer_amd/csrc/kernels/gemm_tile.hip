@@ -409,7 +409,7 @@ static int pick(int tile, const void* x, const void* w, int M, int N, int K, int
     case 3: ATOMA_TILE(128, 64, 2, 2, 4);
     case 4: if constexpr (!GATED) ATOMA_TILE(256, 160, 4, 2, 3); break;     // (a wave's blocks are not in pairs)
     case 5: if constexpr (!GATED) ATOMA_TILE(256, 96, 4, 2, 3); break;
-    // 33 to 64 rows: bound by what a CU brings to LDS, so small tiles, two workgroups a CU, and K in slices.  64 rows, gate-up
+    // 33 to 64 rows, and q, k, v and small weights with some hundred: bound by what a CU brings to LDS, so small tiles, two workgroups a CU, and K in slices.  64 rows, gate-up
     // of 16,384 x 2,048 in 64 x 64 17.7 us with four buffers, 18.8 with three, 18.2 with eight (one workgroup a CU); 64 x 128 with three
     // 21.6.  Planes of 3,072 x 8,192 13.7 by 64 x 128 in eight slices, 15.4 by 64 x 64.
     case 6: if constexpr (EPI == kOutF32 || GATED) ATOMA_TILE(64, 64, 2, 2, 4); break;

@@ -92,7 +92,12 @@ class RMSNorm(Norm):
         if y is not None:
             y.norm = self
             return y
-        if gemm_bf16.try_add_resid(as_tensor(x), w, resid):
+        x = as_tensor(x)
+        # (small weights: planes of K slices, which the norm adds, fill more CUs than sums into the rows)
+        planes = gemm_bf16.try_few_rows_planes(x, w) if x.shape[0] > gemm_bf16.SKINNY_MAX_M else None
+        if planes is not None:
+            return Normed(self.add_norm(resid, planes), self)
+        if gemm_bf16.try_add_resid(x, w, resid):
             return Normed(self.add_norm(resid, None), self)
         return None
 

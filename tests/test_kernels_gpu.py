@@ -982,6 +982,24 @@ def test_gemm_tile_of_64_rows(m, n, k):
         assert planes.shape[0] == gb._few_rows_plan(m, n, k)[1] and bool(((planes.double().sum(0) - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 2048, 2048), (128, 512, 1024), (129, 1040, 4096), (256, 2048, 3072), (300, 96, 1024)])
+def test_small_weights_with_more_than_64_rows(m, n, k):
+    """Planes of K slices by tiles of 64 x 64 where their rule asks for them (sums within k 2^-24 of the absolute values'), the fused SiLU by
+    the same tiles where they are one round; and what both rules leave alone."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    planes = gb.try_few_rows_planes(x, w)
+    assert planes.shape == (gb._small_product_slices(m, n, k), m, n) and planes.shape[0] > 1
+    assert bool(((planes.double().sum(0) - want).abs() <= k * 2.0 ** -24 * size).all())
+    if n % 32 == 0 and gb._small_swiglu(m, n, k):
+        z = want.view(m, n // 32, 2, 16)
+        ref = (torch.nn.functional.silu(z[:, :, 0]) * z[:, :, 1]).reshape(m, n // 2)
+        got = gb.try_tile_swiglu(x, w)
+        assert bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
+    assert not gb._small_product_slices(64, n, k) and not gb._small_product_slices(m, 4096, 4096) and not gb._small_swiglu(2048, 2048, 512)
+
+
 @pytest.mark.parametrize("planes", [1, 2, 3, 4, 5, 8, 9, 17])
 @pytest.mark.parametrize("width", [4, 1028, 2048, 4096])
 def test_add_rmsnorm_planes(planes, width):
@@ -1049,6 +1067,28 @@ def test_gemm_tile_planned():
     assert gb.try_tile_swiglu(rnd(64, 256, dtype=torch.bfloat16), w) is None          # (few rows)
     assert gb.try_tile_swiglu(rnd(70, 96, dtype=torch.bfloat16), rnd(64, 96, dtype=torch.bfloat16)) is None   # (K % 64)
     assert gb.try_tile_swiglu(rnd(70, 264, dtype=torch.bfloat16)[:, 4:260], w) is None                       # (not aligned)
+
+
+@pytest.mark.parametrize("m,nh,nkv,hd,k,page", [(65, 16, 4, 64, 1024, 16), (130, 8, 2, 128, 2048, 32), (200, 32, 8, 64, 2048, 16), (400, 16, 4, 64, 1024, 5)])
+def test_q_k_v_of_some_hundred_rows_by_planes(m, nh, nkv, hd, k, page):
+    """The product that leaves float32 planes of K slices and the kernel that sums, rotates and stores them, where the rule for more than
+    64 rows asks for them, against the product and the rotary kernel apart in float32: the difference is the rounding to bfloat16."""
+    from atoma_infer_amd.kernels import gemm_bf16, ops
+    n, pages = (nh + 2 * nkv) * hd, -(-m // page) + 1
+    assert gemm_bf16._rope_planes_plan(m, n, k) is not None
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    pos = (torch.arange(m) * 7 % 90).int().to(DEV)
+    slots = (torch.randperm(pages * page, generator=torch.Generator().manual_seed(5))[:m]).int()
+    slots[2] = -1
+    slots = slots.to(DEV)
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    k1 = torch.full((pages, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
+    v1, kf, vf, q2 = k1.clone(), k1.float(), k1.float(), torch.empty(m, nh * hd, device=DEV)
+    ops.rope_cache_write(ops.gemm_generic(x, w, torch.float32), pos, cos, sin, hd, kf, vf, slots, page, nh, nkv, hd, q2)
+    q1 = gemm_bf16.try_tile_rope(x, w, pos, cos, sin, k1, v1, slots, page, nh, nkv, hd)
+    for got, want in ((q1, q2), (k1, kf), (v1, vf)):
+        assert bool(((got.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * want.abs().max()).all())
 
 
 @pytest.mark.parametrize("m", [65, 90, 300])
