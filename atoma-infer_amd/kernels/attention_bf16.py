@@ -462,6 +462,38 @@ def build_tasks(starts: np.ndarray, counts: np.ndarray, group: int, window: int,
     return arr, (len(head) + len(split), len(combine), n_part, waves, row_tiles if len(head) else 1, merge)
 
 
+def whole_waves(pairs: int, keys: int, head_size: int) -> int:
+    """The waves that share a decoded token's whole key range, up to ``MERGE_MAX_KEYS`` keys.  Eight shorten the walk where the pairs are
+    few; where they fill the GPU several times over, or have less than a block of 32 keys a wave, what counts are the workgroups that
+    run side by side (a CU holds two of eight waves, whatever few keys they have), and fewer waves a pair make more of them.
+    Measured with 17 to 256 requests of 8 and of 4 KV heads, contexts of one length and of lengths spread evenly up to it, us by
+    eight waves / as here, head size 64: 32 requests up to 256 keys 9.2 / 9.0, 64 up to 512 13.6 / 12.7, up to 2,048 34.7 /
+    33.0, 128 up to 256 17.7 / 13.1, 200 up to 256 27.8 / 18.4, up to 512 33.7 / 28.8; head size 128: 64 up to 256 22.9 /
+    15.4, up to 1,024 41.4 / 35.7, 128 up to 256 43.6 / 21.9, 200 up to 512 82.7 / 59.5, up to 1,024 111 / 104, 256 up
+    to 512 100 / 69.  Beyond these lines the counts are within 3 percent of each other, or eight win."""
+    if pairs < 256 or keys > MERGE_MAX_KEYS or head_size > 128:
+        return 8
+    if head_size <= 64:
+        if keys <= 256:
+            return 1 if pairs >= 1024 else 4
+        return 4 if keys <= 512 or 512 <= pairs < 768 else 8
+    if pairs >= 1024:
+        return 1 if keys <= 1024 else 4
+    return 4 if pairs >= 512 or keys <= 256 else 8
+
+
+def plan_step(starts: np.ndarray, counts: np.ndarray, group: int, window: int, bucket_keys: Optional[int] = None, *, kv_heads: int,
+              head_size: int = 64, keep: int = 0, **options) -> Tuple[np.ndarray, tuple]:
+    """``build_tasks`` as a step's launches want it: decode steps whose tasks are whole key ranges with the waves that
+    ``whole_waves`` names (a function of the entries and the bucket, as all of a decode step's plan is)."""
+    arr, meta = build_tasks(starts, counts, group, window, bucket_keys, kv_heads=kv_heads, head_size=head_size, keep=keep, **options)
+    n_main, n_comb, n_part, waves, pieces, merge = meta
+    if bucket_keys is not None and n_comb == 0 and n_part == 0 and waves == 8 and not keep and len(counts) and int(counts.max()) == 1:
+        keys = bucket_keys if window == 0 else min(bucket_keys, abs(window) + CHUNK)
+        meta = (n_main, 0, 0, whole_waves(n_main * kv_heads, keys, head_size), pieces, merge)
+    return arr, meta
+
+
 def _build_decode_tasks(starts: np.ndarray, group: int, window: int, bucket: int, kv_heads: int,
                         max_waves: int = 2, head_size: int = 64, keep: int = 0):
     """``build_tasks`` for a step in which every entry brings one token, without a Python loop over entries."""

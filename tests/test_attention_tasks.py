@@ -306,3 +306,16 @@ def test_four_waves_a_task_where_two_would_leave_half_of_the_gpu_idle():
     assert one(1024, max_waves=8, head_size=128)[3] == 2        # one workgroup a CU: 256 are a full round
     assert one(512, max_waves=8, head_size=128)[3] == 4
     assert one(100, max_waves=8)[3] == 1                        # short walks: a wave a task
+
+
+@pytest.mark.parametrize("s,keys,head_size,want", [(17, 256, 64, 8), (32, 256, 64, 4), (32, 768, 64, 8), (64, 2048, 64, 4), (128, 256, 64, 1),
+                                                   (128, 512, 64, 4), (128, 1024, 64, 8), (64, 2304, 128, 4), (128, 1024, 128, 1),
+                                                   (128, 1280, 128, 4), (32, 512, 128, 8), (200, 256, 160, 8), (64, 4096, 64, 8)])
+def test_waves_of_whole_ranges(s, keys, head_size, want):
+    """The steps' plans: the tasks of ``build_tasks``, shared by as many waves as the rule names; a plan hangs on entries and bucket alone."""
+    starts = np.random.default_rng(s).integers(0, keys, s).astype(np.int32)
+    counts = np.ones(s, dtype=np.int32)
+    for st in (starts, starts // 2):
+        arr, meta = A.plan_step(st, counts, 4, 0, keys, kv_heads=8, max_waves=8, head_size=head_size)
+        arr0, meta0 = A.build_tasks(st, counts, 4, 0, keys, kv_heads=8, max_waves=8, head_size=head_size)
+        assert (arr == arr0).all() and meta == meta0[:3] + (want,) + meta0[4:] and meta0[3] == 8

@@ -1296,6 +1296,29 @@ def test_tokens_outside_the_table_and_rows_of_nan_do_no_harm():
             assert tok[0] == int(torch.argmax(logits[0])) and tok[3] == 0
 
 
+@pytest.mark.parametrize("waves", [1, 2, 4, 8])
+@pytest.mark.parametrize("nh,nkv,hd,window,s", [(8, 2, 64, 0, 7), (4, 4, 128, 0, 6), (12, 2, 96, 300, 5), (40, 1, 64, 0, 3)])
+def test_attention_whole_ranges_by_any_number_of_waves(nh, nkv, hd, window, s, waves):
+    """Decoded tokens whose whole key ranges one, two, four or eight waves share, several requests' in a workgroup and the last one not
+    full; ranges from one key to 1,100, so that waves have none, part of a block, or several, and rows of more than one piece."""
+    from atoma_infer_amd.kernels import attention_bf16 as A
+    lens = [1, 1100, 33, 511, 64, 700, 257][:s]
+    ks, vs, kc, vc, bt = paged_setup(lens, nkv, hd, 16, torch.bfloat16, seed=hd + nh)
+    starts, counts = [n - 1 for n in lens], [1] * s
+    g = torch.Generator().manual_seed(2)
+    qkv = (torch.randn(s, (nh + 2 * nkv) * hd, generator=g) * 1.5).bfloat16().to(DEV)
+    out = torch.full((s, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ctx, cache = FakeCtx(starts, counts), FakeCache(bt, 16)
+    arr, meta = A.build_tasks(ctx.h_starts, ctx.h_counts, nh // nkv, window, 1280, kv_heads=64, max_waves=8, head_size=hd)
+    assert meta[1] == 0 and meta[3] == 8
+    ctx.plans = {A.plan_key(nh // nkv, window, nkv, hd, hd, 0): (torch.from_numpy(arr).to(DEV), meta[:3] + (waves,) + meta[4:])}
+    assert A.try_attention(qkv, kc, vc, out, ctx, cache, hd ** -0.5, window, nh, nkv, hd)
+    for e, n in enumerate(lens):
+        want = plain_attention(qkv[e:e + 1, : nh * hd].cpu().view(1, nh, hd), ks[e], vs[e], n - 1, hd ** -0.5, window, nh // nkv).reshape(nh * hd)
+        got = out[e].double().cpu()
+        assert bool(((got - want).abs() <= 2.0 ** -9 * want.abs() + 2.0 ** -9 * vs[e].abs().max()).all()), f"entry {e} ({n})"
+
+
 PLANS = ["chunks", "chunks, second kernel", "whole"]
 
 
