@@ -22,6 +22,8 @@ from .params import SamplingPlan
 _MASK = (1 << 64) - 1
 # vocabularies from which on the rows of a step that draws are cut into parts (a block walks fewer values quickly enough)
 SPLIT_MIN_VOCAB = 32768
+# rows up to which a step's parameters are written one by one (each of the lists below costs a microsecond or two whatever it holds)
+FEW_ROWS = 4
 
 
 def uniform(seed: int, counter: int) -> float:
@@ -117,11 +119,20 @@ class Sampler:
         meta = meta_pool.pop() if meta_pool else torch.empty((5, s), dtype=torch.float32, pin_memory=True)
         mn = meta.numpy()
         top_ks, top_ps = [pl.top_k for pl in plans], [pl.top_p for pl in plans]
-        mn[0] = [0.0 if pl.greedy else pl.temperature for pl in plans]
-        mn[1] = top_ps
-        mn[3] = penalties
-        mn[4].view(np.int32)[:] = top_ks
-        write_uniforms([pl.random_seed for pl in plans], steps, meta.data_ptr() + 8 * s)
+        if s <= FEW_ROWS:
+            ints = mn[4].view(np.int32)
+            for i, pl in enumerate(plans):
+                mn[0, i] = 0.0 if pl.greedy else pl.temperature
+                mn[1, i] = pl.top_p
+                mn[2, i] = 0.0 if pl.greedy else uniform(pl.random_seed, steps[i])
+                mn[3, i] = pl.repetition_penalty
+                ints[i] = pl.top_k
+        else:
+            mn[0] = [0.0 if pl.greedy else pl.temperature for pl in plans]
+            mn[1] = top_ps
+            mn[3] = penalties
+            mn[4].view(np.int32)[:] = top_ks
+            write_uniforms([pl.random_seed for pl in plans], steps, meta.data_ptr() + 8 * s)
         m = meta.to(self.device, non_blocking=True)
         if all_greedy:
             # (top_p, penalty and top_k of a greedy row are never read; the copy kept is this batch's)
