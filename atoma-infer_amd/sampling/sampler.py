@@ -143,7 +143,8 @@ class Sampler:
         # (rows that draw are shared by several blocks each: a block walks a row of a large vocabulary too slowly)
         if any([pl.greedy for pl in plans]):          # (what a greedy row's parameters say has no say in this)
             drawn = [i for i, pl in enumerate(plans) if not pl.greedy]
-            top_ks, top_ps = [top_ks[i] for i in drawn] or [0], [top_ps[i] for i in drawn] or [1.0]
+            top_ks, top_ps = [top_ks[i] for i in drawn], [top_ps[i] for i in drawn]
+        top_ks, top_ps = top_ks or [0], top_ps or [1.0]          # (no row draws, or there is none)
         cuts_p = min(top_ps) < 1.0
         out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2],
                                 split=not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB, cuts=cuts_p or max(top_ks) > 0,

@@ -384,6 +384,14 @@ def test_the_sampler_shares_the_rows_of_a_large_vocabulary():
     assert [kw.get("cuts") for kw in calls] == [True] * 3 + [False] * 3
 
 
+def test_a_step_of_no_rows_samples_nothing():
+    """Twice: the record that greedy batches keep of a size must not be what a second call lives on."""
+    from atoma_infer_amd.sampling import Sampler
+    sampler = Sampler(torch.device("cuda:0"))
+    for vocab in (128256, 64):
+        assert [sampler.sample(torch.empty(0, vocab, device="cuda:0"), [], [], []) for _ in range(2)] == [([], [])] * 2
+
+
 def test_repeat_penalty_kernel_and_temperature_limit():
     from atoma_infer_amd.kernels import ops
     from atoma_infer_amd.sampling import Sampler, validate, GenerateParameters
