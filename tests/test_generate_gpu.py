@@ -1,5 +1,6 @@
 """Generation through the entry points: greedy tokens against the plain implementation, sampling kernels against
 the plain sampling functions, the scheduler under page pressure on the GPU, and bin/trace_run as a program."""
+import dataclasses
 import json
 import os
 import subprocess
@@ -382,6 +383,44 @@ def test_the_sampler_shares_the_rows_of_a_large_vocabulary():
         ops.sample_packed = real
     assert all(kw.get("split") for kw in calls)
     assert [kw.get("cuts") for kw in calls] == [True] * 3 + [False] * 3
+
+
+@pytest.mark.parametrize("rows", [3, 4, 5, 12])         # (up to four rows' parameters are written one by one)
+def test_the_sampler_sends_steps_of_small_top_ks_to_the_lists(rows, monkeypatch):
+    """Which draw a step is sent to: the lists where every row that draws has a top-k of at most 128, their two launches where none
+    of those has a top-p, whatever greedy rows carry; the tokens are those of a block a row with the functions' uniform numbers."""
+    from atoma_infer_amd.kernels import ops
+    from atoma_infer_amd.sampling import Sampler, validate, GenerateParameters
+    from atoma_infer_amd.sampling.sampler import uniform
+    vocab = 128256
+    logits = (torch.randn(rows, vocab, generator=torch.Generator().manual_seed(rows)) * 2.5).cuda()
+    make = lambda **kw: validate(GenerateParameters(ignore_eos_token=True, **kw), 3, 100, 200)
+    draw = lambda **kw: make(temperature=0.8, **kw)
+    greedy = make(do_sample=False, temperature=0.7, top_p=0.5)            # (top_k 0 and a top_p, neither of them read)
+    assert greedy.greedy and greedy.top_k == 0 and greedy.top_p == 0.5
+    # (the rows' parameters, whether the lists take the step, whether they are told of a top-p cut)
+    steps = [([draw(top_k=50, top_p=0.9), draw(top_k=1)], True, True),
+             ([draw(top_k=50), draw(top_k=2)], True, False),
+             ([draw(top_k=50), greedy], True, False),
+             ([draw(top_k=50, top_p=0.3), greedy], True, True),
+             ([draw(top_k=128), draw(top_k=1)], True, False),
+             ([draw(top_k=129), draw(top_k=1)], False, False),
+             ([draw(top_k=50), draw()], False, False),
+             ([draw(top_k=50), draw(top_p=0.9)], False, True)]
+    calls, real = [], ops.sample_packed
+    monkeypatch.setattr(ops, "sample_packed", lambda *a, **kw: (calls.append(kw) if kw else None, real(*a, **kw))[1])
+    sampler = Sampler(torch.device("cuda:0"))
+    dev = lambda x, dt: torch.tensor(x, dtype=dt, device="cuda:0")
+    for kinds, few, top_p_cuts in steps:
+        plans = [dataclasses.replace(kinds[i % 2], random_seed=91 * i + 5) for i in range(rows)]
+        for step in (0, 7):
+            got = sampler.sample(logits.clone(), plans, [step + i for i in range(rows)], [()] * rows)
+            assert calls[-1]["split"] and calls[-1]["cuts"] and calls[-1]["few"] == few and calls[-1]["top_p_cuts"] == top_p_cuts
+            want, want_lg = ops.sample(logits, dev([0.0 if pl.greedy else pl.temperature for pl in plans], torch.float32),
+                                       dev([pl.top_k for pl in plans], torch.int32), dev([pl.top_p for pl in plans], torch.float32),
+                                       dev([uniform(pl.random_seed, step + i) for i, pl in enumerate(plans)], torch.float32))
+            assert got == (want.cpu().tolist(), want_lg.cpu().tolist())
+    assert len(calls) == 2 * len(steps)
 
 
 def test_a_step_of_no_rows_samples_nothing():
