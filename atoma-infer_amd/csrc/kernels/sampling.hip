@@ -1134,11 +1134,15 @@ split_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts
 // row's largest logit nor the temperature for its list.  What is left are the two walks that nothing can replace: the largest logit
 // (with the lists), then the mass of all weights where a top-p cut asks for a share of it.
 //   A part's list: the values not below a floor that at least k + kFewSpare threads' largest values reach, found by two levels of
-// histogram over those 1,024 values (not the part's 16,384).  The spare ones put the floor's weight below the k-th weight even if one
-// part holds all k; where it is not clearly below (values tied by the hundred, or a list that is too long, or values that are no
-// numbers) the block that draws takes the row by itself as sample_kernel does: the tokens are the same in every case.
-// 64 rows of 128,256 logits, top-k 50 and top-p 0.9: the three launches take 15 + 7.5 + 9.5 us, 30 with what lies between them, where
-// the search's six take 77.  The lists stop at a k of 128, which two weights a lane of the last launch hold.
+// histogram over those 1,024 values (not the part's 16,384).  Where that is more than a list holds (large logits side by side, values
+// tied by the hundred) the part's k + kFewSpare largest by value and index are found exactly, bit by bit.  The spare ones put the
+// weight of whatever is left out below the k-th weight even if one part holds all k; only where it is not clearly below (a row, or a
+// temperature, that makes all weights equal to within a millionth) does the block that draws take the row by itself as sample_kernel
+// does.  The tokens are the same in every case.
+// Rows of 128,256 logits, top-k 50 and top-p 0.9, us from the first launch's start to the last one's end, in a graph: the three launches
+// here / the search's six: 1 row 26.5 / 45.8, 64 rows 33.6 / 70.7, 200 rows 80 / 193.  64 rows, k 128, 600 large neighbours in a part 51 /
+// 72; constant rows 76 / 280; a NaN in every row 34 / 71 (where one block takes such a row by itself: 128, 1,060 and 133).  The lists stop
+// at a k of 128, which two weights a lane of the last launch hold.
 constexpr int kFewMaxK = 128, kFewSpare = 16;
 constexpr int kFewCap = 384;                      // of a part's list
 constexpr int kFewNear = 1024;                    // weights in the k-th one's bin or above
@@ -1147,8 +1151,9 @@ struct FewRow {
   u64 part_mass[kMaxParts];          // of a part: the mass of its weights (rows with a top-p cut)
   float part_max_v[kMaxParts];       // its largest logit and that one's index
   int32_t part_max_i[kMaxParts];
-  float part_floor[kMaxParts];       // every value that is not below this is in the list
+  float part_floor[kMaxParts];       // what the list leaves out and might still be drawn is at most this
   uint32_t part_count[kMaxParts];    // length of the list; kFewRefused: there is none
+  uint32_t part_nan[kMaxParts];      // values that are no numbers: they come first in the order of weights, and weigh nothing
   uint2 list[kMaxParts][kFewCap];    // (bits of the logit, index in the row), in no order
 };
 static_assert(sizeof(FewRow) % 16 == 0, "rows of scratch stay aligned");
@@ -1162,16 +1167,16 @@ __device__ __forceinline__ float from_rising(uint32_t u) {
   return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
 }
 
-// launch 1: a part's largest logit and its list
-__global__ void __launch_bounds__(kSampThreads)
+// launch 1: a part's largest logit and its list.  Two blocks a CU (64 registers): with one, 64 rows of 128,256 logits take 7 us more.
+__global__ void __launch_bounds__(kSampThreads, 8)
 few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __restrict__ rows, const int32_t* __restrict__ top_k,
                 const float* __restrict__ temperature) {
   __shared__ ArgMax am[kSampWaves];
   __shared__ uint32_t hist[2][kBins];
   __shared__ uint32_t wave_u32[kSampWaves];
   __shared__ int sel_s;
-  __shared__ uint32_t rest_s, count;
-  const int row = blockIdx.x, parts = gridDim.y, part = blockIdx.y, tid = threadIdx.x;
+  __shared__ uint32_t rest_s, count, nans;
+  const int row = blockIdx.x, parts = gridDim.y, part = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   FewRow& r = rows[row];
   int lo, hi;
   part_range(vocab, parts, part, lo, hi);
@@ -1181,12 +1186,12 @@ few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __r
   const float temp = temperature[row];
   hist[0][tid] = 0;
   hist[1][tid] = 0;
-  if (tid == 0) count = 0;
+  if (tid == 0) count = nans = 0;
   ArgMax a = {-INFINITY, 0x7fffffff};
   bool odd = false;
   for_part(pv, lo, hi, [&](float v, int i) {
     a = better(a, ArgMax{v, i});
-    odd |= !(v < INFINITY);
+    odd |= v != v;
   });
   const uint32_t top = rising(a.v);
   a = block_argmax(a, am);
@@ -1195,10 +1200,27 @@ few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __r
     r.part_max_i[part] = a.i;
   }
   if (!(temp > 0.f)) return;                       // (a greedy row needs no more)
-  if (__syncthreads_or(odd) || k <= 0 || k > kFewMaxK) {
+  if (k <= 0 || k > kFewMaxK) {
     if (tid == 0) r.part_count[part] = kFewRefused;
     return;
   }
+  // From here on the values are numbers in their order, 0 where there is none: beyond the part's end, and what is no number, which is
+  // counted
+  // (indexes and floats are made anew where they are written, which the empty asm statements say to the compiler: sixteen more of
+  // either would not fit)
+  int first = lo + tid * 4;
+  auto index = [&](int j, int e) { return first + j * kSampThreads * 4 + e; };
+  uint32_t u[kPartQuads][4], mine = 0;
+#pragma unroll
+  for (int j = 0; j < kPartQuads; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool there = index(j, e) < hi, number = pv.v[j][e] == pv.v[j][e];
+      u[j][e] = there && number ? rising(pv.v[j][e]) : 0u;
+      mine += there && !number;
+      asm volatile("" : "+v"(u[j][e]));
+    }
+  if (odd) atomicAdd(&nans, mine);
   int sel0, sel1;
   uint32_t want = (uint32_t)(k + kFewSpare);
   atomicAdd(&hist[0][top >> 22], 1u);
@@ -1209,19 +1231,129 @@ few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __r
   select_bin<uint32_t>(hist[1], want, sel1, want, wave_u32, &sel_s, &rest_s);
   const uint32_t least = rising(-INFINITY) + 1;    // (weights of zero are never drawn)
   uint32_t edge = ((uint32_t)sel0 << 22) | ((uint32_t)sel1 << 12);
-  const bool all = edge < least;
-  if (all) edge = least;
+  if (edge < least) edge = least;
+  // a wave's values take their places in one go: thousands of ties would queue at the counter
+  uint32_t below = least - 1;                      // the largest value that is left out
+  mine = 0;
   if (top >= edge) {
-    for_part(pv, lo, hi, [&](float v, int i) {
-      if (rising(v) < edge) return;
-      const uint32_t at = atomicAdd(&count, 1u);
-      if (at < kFewCap) r.list[part][at] = make_uint2(__float_as_uint(v), (uint32_t)i);
-    });
+#pragma unroll
+    for (int j = 0; j < kPartQuads; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        mine += u[j][e] >= edge;
+        if (u[j][e] < edge && u[j][e] > below) below = u[j][e];
+      }
+  } else if (top > below) {
+    below = top;
   }
+  if (__ballot(mine != 0)) {
+    const uint32_t incl = wave_prefix(mine);
+    uint32_t at = 0;
+    if (lane == 63) at = atomicAdd(&count, incl);
+    at = __shfl(at, 63, 64) + incl - mine;
+    if (mine) {
+      asm volatile("" : "+v"(first));
+#pragma unroll
+      for (int j = 0; j < kPartQuads; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (u[j][e] < edge) continue;
+          if (at < kFewCap) r.list[part][at] = make_uint2(__float_as_uint(from_rising(u[j][e])), (uint32_t)index(j, e));
+          ++at;
+        }
+    }
+  }
+  // the largest of `below` over the wave, to the block's array
+  auto share_below = [&]() {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t other = __shfl_xor(below, o, 64);
+      below = other > below ? other : below;
+    }
+    if (lane == 0) wave_u32[wave] = below;
+  };
+  share_below();
   __syncthreads();
+  uint32_t listed = count, bound = 0;
+  if (tid == 0)
+    for (int w2 = 0; w2 < kSampWaves; ++w2) bound = wave_u32[w2] > bound ? wave_u32[w2] : bound;
+  if (listed > kFewCap) {
+    // More than a list holds: the `want` largest, ties towards the lower index.  The smallest of them is found a bit at a time (a
+    // histogram would queue at one bin where the values are ties), with a counter a bit, so that a bit costs one barrier.
+    want = (uint32_t)(k + kFewSpare);
+    asm volatile("" : "+v"(first));
+    __syncthreads();                               // (`count` is read)
+    hist[0][tid] = 0;
+    if (tid == 0) count = 0;
+    __syncthreads();
+    uint32_t last = 0;
+#pragma unroll 1
+    for (int bit = 31; bit >= 0; --bit) {
+      const uint32_t next = last | 1u << bit;
+      uint32_t n = 0;
+#pragma unroll
+      for (int j = 0; j < kPartQuads; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) n += __popcll(__ballot(u[j][e] >= next));
+      if (lane == 0 && n) atomicAdd(&hist[0][bit], n);
+      __syncthreads();
+      if (hist[0][bit] >= want) last = next;
+    }
+    uint32_t before[kPartQuads], next = rising(INFINITY);
+    below = least - 1;
+#pragma unroll
+    for (int j = 0; j < kPartQuads; ++j) {
+      uint32_t n = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        n += u[j][e] == last;
+        if (u[j][e] < last && u[j][e] > below) below = u[j][e];
+        if (u[j][e] > last) {
+          if (u[j][e] < next) next = u[j][e];
+          r.list[part][atomicAdd(&count, 1u)] = make_uint2(__float_as_uint(from_rising(u[j][e])), (uint32_t)index(j, e));      // (fewer than `want`)
+        }
+      }
+      before[j] = wave_prefix(n);
+      if (lane == 63) hist[1][j * kSampWaves + wave] = before[j];
+      before[j] -= n;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t higher = __shfl_xor(next, o, 64);
+      next = higher < next ? higher : next;
+    }
+    if (lane == 0) hist[0][kBins - 1 - wave] = next;      // (the bits' counters are the first 32)
+    share_below();
+    __syncthreads();
+    const uint32_t above = count;
+#pragma unroll
+    for (int j = 0; j < kPartQuads; ++j) {
+      uint32_t at = above + before[j];
+      for (int q = 0; q < j * kSampWaves + wave; ++q) at += hist[1][q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (u[j][e] != last) continue;
+        if (at < want) r.list[part][at] = make_uint2(__float_as_uint(from_rising(last)), (uint32_t)index(j, e));
+        ++at;
+      }
+    }
+    uint32_t ties = 0;
+    for (int q = 0; q < kPartQuads * kSampWaves; ++q) ties += hist[1][q];
+    bound = 0;
+    for (int w2 = 0; w2 < kSampWaves; ++w2) {
+      bound = wave_u32[w2] > bound ? wave_u32[w2] : bound;
+      next = hist[0][kBins - 1 - w2] < next ? hist[0][kBins - 1 - w2] : next;
+    }
+    // Ties that are left out come behind the listed ones, unless a larger value's weight is rounded to theirs: then an index says which
+    // comes first, and the floor is the tie itself.  (An exponent is at most 41 here, and off by less than 2^-17.)
+    const bool apart = (from_rising(next) - from_rising(last)) * (1.4426950408889634f / temp) > 0x1p-16f;
+    if (above + ties > want && !apart) bound = last;
+    listed = want;
+  }
   if (tid == 0) {
-    r.part_floor[part] = all ? -INFINITY : from_rising(edge);
-    r.part_count[part] = count <= kFewCap ? count : kFewRefused;
+    r.part_floor[part] = from_rising(bound);
+    r.part_count[part] = listed;
+    r.part_nan[part] = nans;
   }
 }
 
@@ -1275,6 +1407,7 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
   // a wave takes a part's list, its length and its floor in one trip to memory
   const int mine = wave < parts ? wave : 0;
   uint2 got[kPerLane];
+  int nans = 0;
 #pragma unroll
   for (int j = 0; j < kPerLane; ++j) got[j] = r.list[mine][j * kWave + lane];
   const uint32_t listed = r.part_count[mine];
@@ -1283,7 +1416,11 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
   const int k = top_k[row];
   const float* lr = logits + (size_t)row * ld;
   const ArgMax a = row_max(r, parts, vocab);
-  if (!(temp > 0.f)) {
+  const bool in_range = k > 0 && k <= kFewMaxK;
+  for (int q = 0; q < parts; ++q) nans += (int)r.part_nan[q];      // (of use where there are lists)
+  const int k_left = k - nans;                     // of the k largest weights, those that are numbers
+  // (beside an infinite logit all weights are zero or no numbers; nothing but infinities below zero: likewise)
+  if (!(temp > 0.f) || !(fabsf(a.v) < INFINITY) || (in_range && k_left <= 0)) {
     if (tid == 0) out_token[row] = a.i, out_logit[row] = lr[a.i];
     return;
   }
@@ -1292,9 +1429,8 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
   auto from_lists = [&]() -> bool {
     sh.hist_k[tid] = 0;
     if (tid == 0) n_near = 0;
-    // (the longest list there is fits: counts beyond it are refusals)
-    if (__syncthreads_or(wave < parts && listed > kFewCap) || !(a.v > -INFINITY) || !(inv_t < INFINITY) || k <= 0 || k > kFewMaxK)
-      return false;
+    __syncthreads();
+    if (!(inv_t < INFINITY) || !in_range) return false;
     const int n = wave < parts ? (int)listed : 0;
     uint32_t bits[kPerLane];
 #pragma unroll
@@ -1305,7 +1441,7 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
     __syncthreads();
     int sel;
     uint32_t rest;
-    select_bin<uint32_t>(sh.hist_k, (uint32_t)k, sel, rest, sh.wave_u32, &sh.sel_s, &sh.rest_u32);
+    select_bin<uint32_t>(sh.hist_k, (uint32_t)k_left, sel, rest, sh.wave_u32, &sh.sel_s, &sh.rest_u32);
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
       if (j * kWave + lane < n && (int)(bits[j] >> 20) >= sel) {          // (sel < 0: fewer than k weights above zero, all kept)
@@ -1314,9 +1450,34 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
       }
     }
     __syncthreads();
-    const int m = (int)n_near;
-    if (m > kFewNear) return false;
-    const int n_k = m < k ? m : k;
+    int m = (int)n_near;
+    if (m > kFewNear) {
+      // (ties in many lists) only the k_left first, whose last one is found a bit at a time as in the lists' launch; no two keys
+      // are equal
+      __syncthreads();
+      sh.hist_k[tid] = 0;
+      if (tid == 0) n_near = 0;
+      __syncthreads();
+      u64 keys[kPerLane], last_key = 0;
+#pragma unroll
+      for (int j = 0; j < kPerLane; ++j) keys[j] = j * kWave + lane < n ? ((u64)bits[j] << 32) | (uint32_t)~got[j].y : 0;
+#pragma unroll 1
+      for (int bit = 61; bit >= 0; --bit) {
+        const u64 next = last_key | 1ull << bit;
+        uint32_t c = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) c += __popcll(__ballot(keys[j] >= next));
+        if (lane == 0 && c) atomicAdd(&sh.hist_k[bit], c);
+        __syncthreads();
+        if (sh.hist_k[bit] >= (uint32_t)k_left) last_key = next;
+      }
+#pragma unroll
+      for (int j = 0; j < kPerLane; ++j)
+        if (keys[j] >= last_key) near[atomicAdd(&n_near, 1u)] = keys[j];
+      __syncthreads();
+      m = (int)n_near;
+    }
+    const int n_k = m < k_left ? m : k_left;
     if (tid < m) {
       const u64 key = near[tid];
       int rank = 0;
@@ -1329,7 +1490,7 @@ few_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts, 
     __syncthreads();
     // Nothing that the lists leave out may weigh as much as the k-th weight: the weight of a part's floor must lie below it by more than
     // exp2 can be off, or be too small to be drawn.
-    const float last = m < k ? 0.f : __uint_as_float((uint32_t)(kept_key[k - 1] >> 32));
+    const float last = m < k_left ? 0.f : __uint_as_float((uint32_t)(kept_key[k_left - 1] >> 32));
     const float edge = __builtin_amdgcn_exp2f((floor_v - a.v) * inv_t);
     const bool below = edge < 0x1p-41f || edge * (1.0f + 0x1p-20f) < last;
     if (__syncthreads_or(wave < parts && !below)) return false;

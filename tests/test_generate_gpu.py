@@ -343,6 +343,49 @@ def test_rows_that_keep_few_weights_draw_the_same_tokens(rows, vocab):
     assert same(ops.sample_packed(lg, t, k, no_p, uu), ops.sample_packed(lg, t, k, p, uu, split=True, few=True, top_p_cuts=False))
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 128256), (10, 128256), (64, 128256), (30, 33333), (20, 700)])
+def test_lists_settle_ties_clusters_and_values_that_are_no_numbers(rows, vocab):
+    """Rows whose parts hold more large logits than a list does: neighbours by the hundred, ties by the thousand (more of them than k,
+    on both sides of the k-th weight), constant rows, zeros of both signs, NaN, infinities: the tokens of a block a row, bit for bit,
+    and without its walks but for the two kinds whose choice hangs on the last bits of the weights."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + vocab)
+    base = torch.randn(vocab, generator=g) * 3.0
+    n = min(600, vocab // 2)
+
+    def near(at, count, by):
+        x = base.clone()
+        x[at:at + count] += by
+        return x
+    tied = base.clone()
+    tied[torch.randperm(vocab, generator=g)[:vocab // 3]] = float(base.topk(20)[0][-1])
+    nan, inf, few_nan = base.clone(), base.clone(), base.clone()
+    nan[torch.randperm(vocab, generator=g)[:n // 2]] = float("nan")
+    few_nan[[3, vocab - 2]] = float("nan")
+    inf[vocab // 2] = float("inf")
+    zeros = torch.zeros(vocab)
+    zeros[::3] = -0.0
+    kinds = [near(vocab // 3, n, 14.0), near(0, min(1500, vocab), 14.0), tied, torch.zeros(vocab), base.round(), (base * 0.1).round(),
+             nan, few_nan, inf, torch.full((vocab,), -float("inf")), torch.full((vocab,), float("nan")), zeros, 2.0 + 1e-6 * base]
+    settled = len(kinds) - 2
+    pick = [i % len(kinds) for i in range(rows)]
+    dev = lambda x, dt: torch.tensor(x, dtype=dt, device="cuda:0")
+    same = lambda a, b: (torch.equal(a[0].view(torch.int32), b[0].view(torch.int32)) and torch.equal(a[1].isnan(), b[1].isnan())
+                         and torch.equal(a[1].nan_to_num(), b[1].nan_to_num()))
+    lg = torch.stack([kinds[i] for i in pick]).cuda()
+    for kt in (1, 20, 50, ops.FEW_MAX_K):
+        for pt, temp in ((0.9, 0.8), (1.0, 0.8), (0.5, 30.0)):
+            k, p, t = dev([max(1, kt - i % 3) for i in range(rows)], torch.int32), dev([pt] * rows, torch.float32), dev([temp] * rows, torch.float32)
+            for u in (0.0, 0.37, 0.999):
+                uu = dev([(u + 0.37 * i) % 1.0 for i in range(rows)], torch.float32)
+                assert same(ops.sample_packed(lg, t, k, p, uu), ops.sample_packed(lg, t, k, p, uu, split=True, few=True)), (kt, pt, temp, u)
+    # the draw of a block a row leaves the row's weights in the workspace; the lists' leaves it alone
+    ws = torch.full((rows, vocab), 7.0, device="cuda:0")
+    ops.sample_packed(lg, dev([0.8] * rows, torch.float32), dev([50] * rows, torch.int32), p, uu, ws, split=True, few=True)
+    for i, kind in enumerate(pick):
+        assert kind >= settled or bool((ws[i] == 7.0).all()), f"row {i} (kind {kind}) was drawn by one block"
+
+
 def test_the_sampler_shares_the_rows_of_a_large_vocabulary():
     """Through the engine's sampler: a step whose rows draw from 128k logits goes to the launches that share every
     row among several blocks, with the search left out when no row has a cut; the tokens are those of a block a row
