@@ -342,6 +342,7 @@ extern "C" int atoma_add_rmsnorm(float* resid, const void* delta, int delta_dtyp
                                  void* out, int out_dtype, const int32_t* rows, int n_rows, int width, float eps,
                                  int planes, size_t plane_stride, hipStream_t stream) {
   if (n_rows <= 0) return 0;
+  if (planes <= 0) delta = nullptr;        // nothing to add (the vector kernel fetches its first plane before it counts them)
   if (delta_dtype == kF32)
     return add_rmsnorm_w<float>(resid, (const float*)delta, w, w_dtype, out, out_dtype, rows, n_rows, width, eps,
                                 planes, plane_stride, stream);

@@ -1018,6 +1018,19 @@ def test_add_rmsnorm_planes(planes, width):
         assert bool(((out.double() - ref).abs() <= width * 2.0 ** -24 * ref.abs() + 2.0 ** -22 * ref.abs()).all())
 
 
+@pytest.mark.parametrize("width", [8, 2048, 4097])
+def test_add_rmsnorm_of_no_planes(width):
+    """The C entry with a delta of no planes adds nothing, as without one."""
+    import ctypes
+    from atoma_infer_amd.kernels import ops
+    r, d, w = rnd(5, width, seed=1), rnd(5, width, seed=2), rnd(width, seed=3)
+    r0, out = r.clone(), torch.empty(5, width, device=DEV)
+    p = lambda x: ctypes.c_void_p(x.data_ptr())
+    assert ops.core().atoma_add_rmsnorm(p(r), p(d), ops.F32, p(w), ops.F32, p(out), ops.F32, None, 5, width, ctypes.c_float(1e-5), 0,
+                                        ctypes.c_size_t(5 * width), ops._stream()) == 0
+    assert torch.equal(r, r0) and torch.equal(out, ops.add_rmsnorm(r0, None, w, 1e-5, torch.float32))
+
+
 def test_gemm_tile_silu_is_exact():
     """silu(gate) * up of the tile kernel, from gates and ups that are exact in float32: as few results as with the formula in
     float32 fall on the other side of a rounding to bfloat16 than the exact ones (an error of 2^-22 moves one in about 10,000),
