@@ -107,3 +107,20 @@ TILES_QUICKER = [(T_SILU, 2048, 16384, 2048, 127.5, 114.8), (T_SILU, 200, 16384,
 def test_tile_rule_where_one_side_is_much_the_quicker():
     for kind, m, n, k, lib, tiles in LIBRARY_QUICKER + TILES_QUICKER:
         assert gemm_bf16._tile_wins(m, n, k, kind) == (tiles < lib), (kind, m, n, k)
+
+
+def test_few_rows_plans_count_what_their_reader_pays_for_a_plane():
+    """41 to 64 rows: sizes where more planes were measured slower than fewer, or than the streaming kernel's (None), and sizes where
+    they are the quicker ones; beyond 64 rows no slice of more than 1,536 values of K."""
+    plan = gemm_bf16._few_rows_plan
+    for (m, n, k), slices in {(48, 2048, 2048): 4, (41, 1024, 1024): 2, (48, 512, 1024): 4, (56, 1536, 1536): 4, (41, 4096, 1024): 2,
+                              (64, 2048, 8192): 8, (48, 1024, 4096): 4}.items():
+        assert plan(m, n, k) == (6, slices), (m, n, k)
+    for m, n, k in ((48, 5120, 3072), (41, 6144, 4096), (64, 4096, 8192), (40, 2048, 2048), (65, 2048, 2048)):
+        assert plan(m, n, k) is None, (m, n, k)
+    assert plan(41, 5120, 3072, True) == (7, 4) and plan(64, 3072, 2048, True) == (6, 4) and plan(48, 6144, 4096, True) == (7, 4)
+    assert plan(41, 768, 512, True) is None and plan(64, 768, 512, True) is not None and plan(64, 8192, 8192, True) is None
+    for m, n, k in ((320, 1024, 8192), (200, 2048, 4096), (160, 1536, 6144), (1000, 512, 11008)):
+        assert gemm_bf16._small_product_slices(m, n, k) == 0, (m, n, k)
+    for (m, n, k), slices in {(200, 2048, 2048): 2, (65, 2048, 4096): 4, (128, 1024, 4096): 8, (160, 1024, 4096): 4, (128, 3072, 3072): 2}.items():
+        assert gemm_bf16._small_product_slices(m, n, k) == slices, (m, n, k)
