@@ -497,6 +497,11 @@ static bool shape_ok(const DeltaShape& sh) {
          sh.taps >= 1 && sh.taps <= 64 && sh.ldp > 0;
 }
 
+// Whether a token's q, k and v channels fit the LDS that delta_prepare keeps them in
+static bool channels_fit(const DeltaShape& sh) {
+  return (2 * (size_t)sh.kv_heads * sh.dim + (size_t)sh.heads * sh.vdim) * sizeof(float) <= 60 * 1024;
+}
+
 extern "C" int atoma_delta_prepare(const float* proj, int ldp, int off_q, int off_k, int off_v, int off_b, int heads,
                                    int kv_heads, int dim, int vdim, int taps, const int32_t* token_seq,
                                    const int32_t* q_start, const int32_t* state_slots, float* state,
@@ -509,7 +514,7 @@ extern "C" int atoma_delta_prepare(const float* proj, int ldp, int off_q, int of
   if (!shape_ok(sh) || n_entries <= 0 || n_entries > 65535) return ATOMA_ERR_SHAPE;
   // (a token has two workgroups: convolution, SiLU and unit lengths; beta and decay)
   const int channels = 2 * kv_heads * dim + heads * vdim;
-  if ((size_t)channels * sizeof(float) > 60 * 1024) return ATOMA_ERR_SHAPE;
+  if (!channels_fit(sh)) return ATOMA_ERR_SHAPE;
   hipLaunchKernelGGL(delta_prepare_kernel, dim3(n_tokens, 2), dim3(256), channels * sizeof(float), stream, proj, sh,
                      token_seq, q_start, state_slots, state, state_stride, taps_w, dt_pre, ld_dt, dt_bias, a_log, qn, kn, vn,
                      beta, decay, kq);
@@ -571,9 +576,11 @@ static int padded_dim(int dim) { return dim <= 16 ? 16 : dim <= 32 ? 32 : dim <=
 
 // Whether delta_step_kernel takes heads of these sizes: its vectors fit LDS, and a workgroup's state is at most 256 KB, beyond which the
 // scan's many workgroups are the better split (four heads of 128 x 128 to a q/k head are the most that are measured).
+// It takes none that atoma_delta_prepare refuses, whose rows of channels wait in LDS: a layer's prompts and its decoded tokens are
+// refused alike.
 extern "C" int atoma_delta_step_fits(int heads, int kv_heads, int dim, int vdim, int taps) {
   const DeltaShape sh{heads, kv_heads, dim, vdim, taps, 1, 0, 0, 0, 0};
-  return shape_ok(sh) && kv_heads <= 65535 && (size_t)(heads / kv_heads) * vdim * dim <= 65536 &&
+  return shape_ok(sh) && kv_heads <= 65535 && channels_fit(sh) && (size_t)(heads / kv_heads) * vdim * dim <= 65536 &&
          step_lds_floats(sh, padded_dim(dim)) * sizeof(float) <= 60 * 1024;
 }
 

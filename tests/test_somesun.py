@@ -77,6 +77,14 @@ def test_the_planner_s_first_key_under_windows_and_chunks():
     assert sorted(zip(live[:, 0].tolist(), live[:, 4].tolist(), live[:, 5].tolist())) == [(0, 32, 100), (1, 96, 101), (2, 0, 8)]
 
 
+@pytest.mark.parametrize("heads, kv, dim, vdim, fits", [(8, 4, 128, 128, True), (24, 24, 192, 128, True), (32, 32, 192, 128, False),
+                                                       (50, 25, 256, 64, False), (60, 60, 64, 128, True), (61, 61, 64, 128, False)])
+def test_single_tokens_are_refused_where_prompts_are(heads, kv, dim, vdim, fits):
+    """A token's 2 kv dim + heads vdim channels must fit 60 KB of LDS, whichever launches take it."""
+    from atoma_infer_amd.kernels import ops
+    assert (2 * kv * dim + heads * vdim <= 15360) == fits and ops.delta_step_fits(heads, kv, dim, vdim, 4) == fits
+
+
 # ---- what pins the plain implementation -------------------------------------------------------------------------
 
 def test_plain_rotation_is_a_turn_of_neighbouring_pairs():
