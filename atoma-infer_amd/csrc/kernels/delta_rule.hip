@@ -281,6 +281,8 @@ delta_out_kernel(const float* __restrict__ o, const float* __restrict__ gate_pre
 // Bound by its trips to memory (the slot, then the state) and by what a CU moves of the state, 256 KB for two heads of 128 x 128: with
 // eight requests of 8 heads over 4 q/k heads 32 workgroups, 12.6 us for the launch, where the four take 29.5 (prepare 11.7, the
 // convolution's state 5.1, scan 8.2, output 5.2).  (With the loads of the state, the taps and the gates each waited for by itself: 15.8.)
+// A CU has one such workgroup at a time (heads of 64 and 128 take all 128 registers a thread may have, and three values spill around
+// the passes), so steps of many small heads keep the four launches: delta_step_pays in ops.py.
 template <int R, int G, int LANES, typename TO>
 __global__ void __launch_bounds__(kStepThreads)
 delta_step_kernel(const float* __restrict__ proj, DeltaShape sh, const int32_t* __restrict__ q_start,
@@ -575,7 +577,8 @@ static size_t step_lds_floats(const DeltaShape& sh, int dp) {
 static int padded_dim(int dim) { return dim <= 16 ? 16 : dim <= 32 ? 32 : dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
 
 // Whether delta_step_kernel takes heads of these sizes: its vectors fit LDS, and a workgroup's state is at most 256 KB, beyond which the
-// scan's many workgroups are the better split (four heads of 128 x 128 to a q/k head are the most that are measured).
+// scan's many workgroups are the better split (at 256 KB, four heads of 128 x 128 to a q/k head, one request takes 14.9 us here and 16.3
+// by the four launches, 64 requests 27.6 and 54.5).
 // It takes none that atoma_delta_prepare refuses, whose rows of channels wait in LDS: a layer's prompts and its decoded tokens are
 // refused alike.
 extern "C" int atoma_delta_step_fits(int heads, int kv_heads, int dim, int vdim, int taps) {

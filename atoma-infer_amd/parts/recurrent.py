@@ -124,7 +124,8 @@ class GatedDeltaRule(Mixer):
         pre = ops.lowrank_up(low, self.w_ag) if x.shape[0] <= ops.LOWRANK_UP_MAX_TOKENS else \
             linear(low, self.w_ag, torch.float32)
         dt_pre, gate_pre = pre[:, : self.nd], pre[:, self.nd:]
-        if single_tokens(ctx) and ops.delta_step_fits(self.heads, self.kv_heads, self.dim, self.vdim, self.taps):
+        if (single_tokens(ctx) and ops.delta_step_pays(self.heads, self.kv_heads, self.dim, self.vdim, ctx.n_entries)
+                and ops.delta_step_fits(self.heads, self.kv_heads, self.dim, self.vdim, self.taps)):
             y = ops.delta_step(proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim,
                                self.vdim, self.taps, ctx.q_start, ctx.state_slots, state, self.taps_w, dt_pre, self.dt_bias,
                                self.a_log, gate_pre, self.norm_w, self.norm_eps, x.dtype)

@@ -85,6 +85,15 @@ def test_single_tokens_are_refused_where_prompts_are(heads, kv, dim, vdim, fits)
     assert (2 * kv * dim + heads * vdim <= 15360) == fits and ops.delta_step_fits(heads, kv, dim, vdim, 4) == fits
 
 
+def test_steps_of_many_small_heads_keep_the_four_launches():
+    """(heads, q/k heads, dim, vdim, entries) that were measured slower in one launch, and some that were the quicker ones."""
+    from atoma_infer_amd.kernels import ops
+    for sizes in ((16, 16, 64, 64, 200), (32, 32, 16, 16, 64), (4, 4, 64, 64, 200), (16, 8, 32, 32, 128), (32, 32, 64, 128, 200)):
+        assert not ops.delta_step_pays(*sizes), sizes
+    for sizes in ((8, 4, 128, 128, 8), (8, 8, 128, 128, 256), (16, 16, 64, 64, 32), (32, 32, 128, 64, 256), (32, 8, 64, 64, 256), (1, 1, 16, 16, 256)):
+        assert ops.delta_step_pays(*sizes), sizes
+
+
 # ---- what pins the plain implementation -------------------------------------------------------------------------
 
 def test_plain_rotation_is_a_turn_of_neighbouring_pairs():
