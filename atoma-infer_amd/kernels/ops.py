@@ -681,6 +681,16 @@ def ssd_scan(xbc: torch.Tensor, dt: torch.Tensor, decay: torch.Tensor, a_log: to
     return y
 
 
+def ssd_step_pays(heads: int, groups: int, vdim: int, n: int, entries: int) -> bool:
+    """Whether ``ssd_step`` is quicker than the launches it stands for.  Every head's workgroup makes its group's B and C anew, which
+    heads of few columns and long rows do not pay for, and one workgroup a token replaces all groups' part of the convolution's state.
+    Measured over 552 sizes (4 to 128 heads of 8 to 128 columns, rows of 16 to 256, 1 to 24 groups, 1 to 200 requests): within this rule
+    0.73 of the four launches' time in the geometric mean and none slower; without it up to 1.97 (8 requests, 24 heads of 256 x 16 in
+    24 groups: 15.7 -> 31.0 us; 200 requests, 128 heads of 128 x 8 in one: 86 -> 123)."""
+    shared = 2 * groups * n
+    return shared <= 4096 and (vdim >= 32 or n <= 64 or (shared <= 2048 and heads * entries <= 1024))
+
+
 def ssd_step(proj: torch.Tensor, offsets, heads: int, groups: int, vdim: int, n: int, taps: int, q_start: torch.Tensor,
              state_slots: torch.Tensor, state: torch.Tensor, taps_w: torch.Tensor, conv_bias: torch.Tensor, dt_bias: torch.Tensor,
              a_log: torch.Tensor, d_skip: torch.Tensor) -> torch.Tensor:

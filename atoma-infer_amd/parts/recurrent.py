@@ -217,7 +217,7 @@ class StateSpaceDuality(Mixer):
         state = cache.state
         dims = (self.heads, self.groups, self.vdim, self.n, self.taps)
         proj = linear(x, self.w_in, torch.float32)
-        if single_tokens(ctx):
+        if single_tokens(ctx) and ops.ssd_step_pays(self.heads, self.groups, self.vdim, self.n, ctx.n_entries):
             y = ops.ssd_step(proj, (self.off_z, self.off_x, self.off_dt), *dims, ctx.q_start, ctx.state_slots, state, self.taps_w,
                              self.conv_b, self.dt_bias, self.a_log, self.d_skip)
             u = ops.ssd_out(y, proj, self.off_z, self.norm_w, self.norm_eps, self.norm_groups, x.dtype,

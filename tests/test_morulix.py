@@ -243,3 +243,12 @@ def test_plain_model_does_not_look_ahead():
     a = pm.forward([1, 2, 3, 4, 5, 6, 7, 8], w, MOR_A)
     b = pm.forward([1, 2, 3, 4, 5, 9, 9, 9], w, MOR_A)
     assert torch.allclose(a[:5], b[:5]) and not torch.allclose(a[5], b[5])
+
+
+def test_steps_whose_heads_do_not_pay_for_their_groups_inputs_keep_the_four_launches():
+    """(heads, groups, vdim, n, entries) that were measured slower with prepare, state and scan in one launch, and some quicker ones."""
+    from atoma_infer_amd.kernels import ops
+    for sizes in ((24, 24, 16, 256, 8), (128, 1, 8, 128, 200), (64, 8, 16, 128, 200), (24, 24, 64, 256, 1), (64, 8, 8, 256, 1)):
+        assert not ops.ssd_step_pays(*sizes), sizes
+    for sizes in ((64, 1, 64, 128, 8), (64, 8, 64, 128, 200), (128, 1, 16, 64, 200), (16, 1, 8, 128, 8), (24, 24, 8, 64, 64), (96, 1, 64, 256, 64)):
+        assert ops.ssd_step_pays(*sizes), sizes
