@@ -503,7 +503,6 @@ ssd_scores_kernel(const float* __restrict__ xbc, SsdShape sh, const int32_t* __r
   }
 }
 
-// one workgroup per (token, norm group); parts of up to 4,096 columns wait in registers between the two passes
 // What is left of the convolution's state after ssd_step_kernel (state: null elsewhere): channels from `first` on of the token's request
 struct SsdTail {
   float* state;
@@ -512,6 +511,7 @@ struct SsdTail {
   int off_x, first, channels, keep;
 };
 
+// one workgroup per (token, norm group); parts of up to 4,096 columns wait in registers between the two passes
 template <typename TO, int PER, int NT>
 __global__ void __launch_bounds__(NT)
 ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int ldp, int off_z,
