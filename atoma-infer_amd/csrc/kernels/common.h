@@ -103,38 +103,30 @@ __device__ __forceinline__ float value4(const Raw4<bf16_t>& r, int i) {
 }
 
 // sum[j] += the sum over `planes` planes, in the order of their index, of the four values at column 4 * col[j] of p.  The loads of up to
-// eight planes are issued together (each is a trip to memory), and no more than there are planes, or the next of 1, 2, 4: repeats of the
-// last plane would cost the cache as much as others.
+// eight planes are issued together (each is a trip to memory), in whole batches of 8, 4, 2 and 1: no load and no sum stands under a
+// condition, which the compiler would take the loads along to, one by one (64 rows of 2,048 with eight planes and their norm 6.4 us then,
+// 4.9 so).
 template <int PB, int MAXJ, typename T, typename V>
-__device__ __forceinline__ void add_some_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, int n, const int (&col)[MAXJ]) {
+__device__ __forceinline__ void add_some_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, const int (&col)[MAXJ]) {
   Raw4<T> d[PB][MAXJ];
 #pragma unroll
-  for (int q = 0; q < PB; ++q) {
-    const T* const at = p + (size_t)min(q, n - 1) * stride;
+  for (int q = 0; q < PB; ++q)
 #pragma unroll
-    for (int j = 0; j < MAXJ; ++j) d[q][j] = fetch4(at + 4 * col[j]);
-  }
+    for (int j = 0; j < MAXJ; ++j) d[q][j] = fetch4(p + q * stride + 4 * col[j]);
 #pragma unroll
-  for (int q = 0; q < PB; ++q) {
-    if (q >= n) break;
+  for (int q = 0; q < PB; ++q)
 #pragma unroll
     for (int j = 0; j < MAXJ; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum[j].v[i] += value4(d[q][j], i);
-  }
 }
 template <int MAXJ, typename T, typename V>
 __device__ __forceinline__ void add_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, int planes, const int (&col)[MAXJ]) {
   constexpr int PB = MAXJ <= 2 ? 8 : 4;
-  if (planes == 1) {
-    add_some_planes<1, MAXJ>(sum, p, stride, 1, col);
-  } else if (planes == 2) {
-    add_some_planes<2, MAXJ>(sum, p, stride, 2, col);
-  } else if (planes <= 4) {
-    add_some_planes<4, MAXJ>(sum, p, stride, planes, col);
-  } else {
-    for (int p0 = 0; p0 < planes; p0 += PB) add_some_planes<PB, MAXJ>(sum, p + p0 * stride, stride, min(PB, planes - p0), col);
-  }
+  for (; planes >= PB; planes -= PB, p += PB * stride) add_some_planes<PB, MAXJ>(sum, p, stride, col);
+  if (PB > 4 && planes & 4) add_some_planes<4, MAXJ>(sum, p, stride, col), p += 4 * stride;
+  if (planes & 2) add_some_planes<2, MAXJ>(sum, p, stride, col), p += 2 * stride;
+  if (planes & 1) add_some_planes<1, MAXJ>(sum, p, stride, col);
 }
 
 // One token of a causal convolution over time whose earlier inputs lie in the rows of `rows` (keep of them, `channels` apart), the
