@@ -103,7 +103,7 @@ __device__ __forceinline__ float value4(const Raw4<bf16_t>& r, int i) {
 }
 
 // sum[j] += the sum over `planes` planes, in the order of their index, of the four values at column 4 * col[j] of p.  The loads of up to
-// eight planes are issued together (each is a trip to memory), in whole batches of 8, 4, 2 and 1: no load and no sum stands under a
+// PB planes are issued together (each is a trip to memory), in whole batches of PB, 4, 2 and 1: no load and no sum stands under a
 // condition, which the compiler would take the loads along to, one by one (64 rows of 2,048 with eight planes and their norm 6.4 us then,
 // 4.9 so).
 template <int PB, int MAXJ, typename T, typename V>
@@ -120,9 +120,9 @@ __device__ __forceinline__ void add_some_planes(V (&sum)[MAXJ], const T* __restr
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum[j].v[i] += value4(d[q][j], i);
 }
-template <int MAXJ, typename T, typename V>
+template <int PB, int MAXJ, typename T, typename V>
 __device__ __forceinline__ void add_planes(V (&sum)[MAXJ], const T* __restrict__ p, size_t stride, int planes, const int (&col)[MAXJ]) {
-  constexpr int PB = MAXJ <= 2 ? 8 : 4;
+  static_assert(PB == 4 || PB == 8, "the batches of what is left are 4, 2 and 1");
   for (; planes >= PB; planes -= PB, p += PB * stride) add_some_planes<PB, MAXJ>(sum, p, stride, col);
   if (PB > 4 && planes & 4) add_some_planes<4, MAXJ>(sum, p, stride, col), p += 4 * stride;
   if (planes & 2) add_some_planes<2, MAXJ>(sum, p, stride, col), p += 2 * stride;

@@ -265,7 +265,7 @@ add_rmsnorm_vec_kernel(float* __restrict__ resid, const TD* __restrict__ delta, 
   for (int j = 0; j < MAXJ; ++j) v[j] = load4(resid + src + 4 * col[j]);
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) wv[j] = fetch4(w + 4 * col[j]);
-  if (delta) add_planes(v, delta + src, plane_stride, planes, col);
+  if (delta) add_planes<(MAXJ <= 2 ? 8 : 4)>(v, delta + src, plane_stride, planes, col);
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) {
     if (threadIdx.x + j * 256 >= n4) continue;

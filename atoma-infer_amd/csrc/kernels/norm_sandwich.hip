@@ -105,8 +105,8 @@ __device__ __forceinline__ void add_term(f4 (&d)[MAXJ], const Term& t, size_t ba
   f4 sum[MAXJ];
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j) sum[j] = f4{{0.f, 0.f, 0.f, 0.f}};
-  if (t.dtype == kF32) add_planes(sum, (const float*)t.data + base, t.plane_stride, t.planes, col);
-  else add_planes(sum, (const bf16_t*)t.data + base, t.plane_stride, t.planes, col);
+  if (t.dtype == kF32) add_planes<4>(sum, (const float*)t.data + base, t.plane_stride, t.planes, col);
+  else add_planes<4>(sum, (const bf16_t*)t.data + base, t.plane_stride, t.planes, col);
 #pragma unroll
   for (int j = 0; j < MAXJ; ++j)
 #pragma unroll
@@ -122,7 +122,9 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   const size_t base = (size_t)blockIdx.x * width;
   const int n4 = width >> 2;
   // (threads beyond the row's end fetch its last columns: no load stands under a condition.  Both norms' weights come with the
-  // rows: behind the sums they are two trips to memory more)
+  // rows: behind the sums they are two trips to memory more.  Rows of more than 4,096 columns have no registers left for them: 332 a
+  // thread halved the rows that a CU has on their way, 4,096 rows of 5,120 75 -> 96 us)
+  constexpr bool EARLY = MAXJ <= 4;
   int col[MAXJ];
   f4 d[MAXJ], x[MAXJ], wp[MAXJ], wn[MAXJ];
 #pragma unroll
@@ -134,8 +136,10 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   for (int j = 0; j < MAXJ; ++j) x[j] = load4(resid + base + 4 * col[j]);
   const float* const w1 = w_post != nullptr ? w_post : resid + base;       // (some row, where there is no such norm)
   const float* const w2 = out != nullptr ? w_next : resid + base;
+  if constexpr (EARLY) {
 #pragma unroll
-  for (int j = 0; j < MAXJ; ++j) wp[j] = load4(w1 + 4 * col[j]), wn[j] = load4(w2 + 4 * col[j]);
+    for (int j = 0; j < MAXJ; ++j) wp[j] = load4(w1 + 4 * col[j]), wn[j] = load4(w2 + 4 * col[j]);
+  }
   add_term(d, a, row_of(a, base), col);
   if (n_terms > 1) add_term(d, b, row_of(b, base), col);
   float ss = 0.f;
@@ -154,6 +158,7 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   for (int j = 0; j < MAXJ; ++j) {
     const int c = threadIdx.x + j * 256;
     if (c < n4) {
+      if constexpr (!EARLY) wp[j] = load4(w1 + 4 * c);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         x[j].v[i] += w_post != nullptr ? d[j].v[i] * inv * wp[j].v[i] : d[j].v[i];
@@ -169,6 +174,7 @@ add_normed_vec_kernel(float* __restrict__ resid, Term a, Term b, int n_terms, co
   for (int j = 0; j < MAXJ; ++j) {
     const int c = threadIdx.x + j * 256;
     if (c < n4) {
+      if constexpr (!EARLY) wn[j] = load4(w2 + 4 * c);
       f4 y;
 #pragma unroll
       for (int i = 0; i < 4; ++i) y.v[i] = x[j].v[i] * inv2 * wn[j].v[i];
@@ -181,7 +187,10 @@ template <typename TO>
 static void launch_vec(dim3 grid, hipStream_t stream, float* resid, const Term& a, const Term& b, int n_terms,
                        const float* w_post, const float* w_next, void* out, int width, float eps_post, float eps_next) {
   const dim3 block(256);
-  if (width <= 2048)
+  if (width <= 1024)
+    hipLaunchKernelGGL((add_normed_vec_kernel<TO, 1>), grid, block, 0, stream, resid, a, b, n_terms, w_post, w_next,
+                       (TO*)out, width, eps_post, eps_next);
+  else if (width <= 2048)
     hipLaunchKernelGGL((add_normed_vec_kernel<TO, 2>), grid, block, 0, stream, resid, a, b, n_terms, w_post, w_next,
                        (TO*)out, width, eps_post, eps_next);
   else if (width <= 4096)

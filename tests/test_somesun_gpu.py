@@ -27,6 +27,21 @@ def oracle(path, toks):
 
 # ---- mechanisms alone -----------------------------------------------------------------------------------------
 
+@pytest.mark.parametrize("planes", [1, 2, 3, 4, 7, 8, 9])
+@pytest.mark.parametrize("width", [4, 1020, 1024, 1028, 2052, 4096, 4100, 8192])
+def test_sum_and_norm_at_the_widths_that_change_kernel(width, planes):
+    """Against 64 bits; a float32 sum of `planes` numbers and of at most `width` squares, twice."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + planes)
+    resid, d = torch.randn(3, width, generator=g), torch.randn(planes, 3, width, generator=g)
+    wp, wn = torch.rand(width, generator=g) + 0.5, torch.rand(width, generator=g) + 0.5
+    want = resid.double() + ps.rms_norm(d.double().sum(0), wp.double(), 1e-5)
+    r = resid.to(DEV)
+    out = ops.add_normed(r, [((d if planes > 1 else d[0]).to(DEV), 1.0)], wp.to(DEV), 1e-5, wn.to(DEV), 2e-6, torch.float32)
+    bound = (width ** 0.5 + planes + 16) * 2.0 ** -23 * want.abs().max()
+    assert (r.cpu().double() - want).abs().max() <= bound and (out.cpu().double() - ps.rms_norm(want, wn.double(), 2e-6)).abs().max() <= 2 * bound
+
+
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width, planes", [(64, (1, 1)), (200, (2, 3)), (4100, (1, 0))])
 def test_sum_and_norm_behind_a_sublayer(width, planes, out_dtype):
