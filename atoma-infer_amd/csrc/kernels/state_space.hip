@@ -511,14 +511,17 @@ struct SsdTail {
   int off_x, first, channels, keep;
 };
 
-// one workgroup per (token, norm group); parts of up to 4,096 columns wait in registers between the two passes
-template <typename TO, int PER, int NT>
+// one workgroup per (token, norm group); parts of up to 4,096 columns wait in registers between the two passes.  A thread does the work
+// of V threads of a block of V * NT, sums apart, so that a row's result is the same whatever V: few rows want many threads (eight tokens of
+// 4,096 columns 5.1 us with 1,024 threads, 6.8 with 256), many rows fewer, since a CU then has more rows on their way.
+template <typename TO, int PER, int NT, int V, bool TAIL>
 __global__ void __launch_bounds__(NT)
 ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int ldp, int off_z,
                const float* __restrict__ w, float eps, int inner, int part, TO* __restrict__ out, SsdTail tail) {
-  __shared__ float scratch[NT / 64];
+  constexpr int WAVES = NT / 64;
+  __shared__ float scratch[WAVES * V];
   const int t = blockIdx.x, p0 = blockIdx.y * part;
-  if (tail.state != nullptr && blockIdx.y == 0) {
+  if (TAIL && blockIdx.y == 0) {
     // (a step of single tokens: token t is entry t's)
     float* const st = tail.state + (size_t)tail.state_slots[t] * tail.stride;
     for (int c = tail.first + threadIdx.x; c < tail.channels; c += NT) {
@@ -530,37 +533,53 @@ ssd_out_kernel(const float* __restrict__ y, const float* __restrict__ proj, int 
   }
   const float* zp = proj + (size_t)t * ldp + off_z + p0;
   const float* yp = y + (size_t)t * inner + p0;
-  float ss = 0.f;
+  float ss[V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) ss[q] = 0.f;
+  // over the threads of the block of V * NT, in their order
+  auto sum = [&]() {
+    if constexpr (V == 1) return block_sum<WAVES>(ss[0], scratch);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const float all = wave_sum(ss[q]);
+      if (lane == 0) scratch[q * WAVES + wave] = all;
+    }
+    lds_barrier();
+    float total = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES * V; ++i) total += scratch[i];
+    return total;
+  };
   if constexpr (PER > 0) {
-    constexpr int P = PER > 0 ? PER : 1;
+    constexpr int P = PER * V;
     float u[P], yv[P], zv[P];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
+    for (int j = 0; j < P; ++j) {
       const int i = threadIdx.x + j * NT;
       yv[j] = i < part ? yp[i] : 0.f;
       zv[j] = i < part ? zp[i] : 0.f;
     }
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
+    for (int j = 0; j < P; ++j) {
       u[j] = yv[j] * (zv[j] * ssd_sigmoid(zv[j]));
-      ss = fmaf(u[j], u[j], ss);
+      ss[j % V] = fmaf(u[j], u[j], ss[j % V]);
     }
-    ss = block_sum<NT / 64>(ss, scratch);
-    const float inv = 1.0f / sqrtf(ss / (float)part + eps);
+    const float inv = 1.0f / sqrtf(sum() / (float)part + eps);
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
+    for (int j = 0; j < P; ++j) {
       const int i = threadIdx.x + j * NT;
       if (i < part) out[(size_t)t * inner + p0 + i] = from_f32<TO>(u[j] * inv * w[p0 + i]);
     }
     return;
   }
+  static_assert(PER > 0 || V == 1, "a row that is walked twice: a thread an own sum");
   for (int i = threadIdx.x; i < part; i += NT) {
     const float z = zp[i];
     const float u = yp[i] * (z * ssd_sigmoid(z));
-    ss = fmaf(u, u, ss);
+    ss[0] = fmaf(u, u, ss[0]);
   }
-  ss = block_sum<NT / 64>(ss, scratch);
-  const float inv = 1.0f / sqrtf(ss / (float)part + eps);
+  const float inv = 1.0f / sqrtf(sum() / (float)part + eps);
   for (int i = threadIdx.x; i < part; i += NT) {
     const float z = zp[i];
     const float u = yp[i] * (z * ssd_sigmoid(z));
@@ -710,21 +729,31 @@ extern "C" int atoma_ssd_out(const float* y, const float* proj, int ldp, int off
   if (state != nullptr && (channels < inner || state_slots == nullptr || taps > 64)) return ATOMA_ERR_SHAPE;
   const SsdTail tail{state, state_slots, state_stride, off_x, inner, channels, taps - 1};
   const dim3 grid(n_tokens, norm_groups);
-#define ATOMA_SSD_OUT(TO, PER, NT)                                                                                       \
-  hipLaunchKernelGGL((ssd_out_kernel<TO, PER, NT>), grid, dim3(NT), 0, stream, y, proj, ldp, off_z, w, eps, inner, part, \
+#define ATOMA_SSD_OUT_AS(TO, PER, NT, V, TAIL)                                                                                     \
+  hipLaunchKernelGGL((ssd_out_kernel<TO, PER, NT, V, TAIL>), grid, dim3(NT), 0, stream, y, proj, ldp, off_z, w, eps, inner, part, \
                      (TO*)out, tail)
-  // (four values a thread: eight tokens of 4,096 take 7.6 us, 10.7 with sixteen)
-#define ATOMA_SSD_OUT_BY_PART(TO)                     \
-  do {                                                \
-    if (part <= 1024) ATOMA_SSD_OUT(TO, 4, 256);      \
-    else if (part <= 4096) ATOMA_SSD_OUT(TO, 4, 1024); \
-    else ATOMA_SSD_OUT(TO, 0, 1024);                  \
+#define ATOMA_SSD_OUT(TO, PER, NT, V)                                    \
+  do {                                                                   \
+    if (state != nullptr) ATOMA_SSD_OUT_AS(TO, PER, NT, V, true);        \
+    else ATOMA_SSD_OUT_AS(TO, PER, NT, V, false);                        \
+  } while (0)
+  // (rows from which on 256 threads are the quicker ones, us by 1,024 / by 256: of 2,048 columns 1,000 10.1 / 10.5, 1,400 13.2 / 12.7,
+  // 4,096 31.6 / 25.7; of 3,072 1,400 14.8 / 15.1, 2,048 19.5 / 19.3, 4,096 36.2 / 32.0; longer ones walk the row twice, where 1,024 win or
+  // are as quick: of 8,192 512 15.2 / 29.7, 4,096 111 / 113)
+  const bool many = (size_t)n_tokens * norm_groups > (part <= 2048 ? 1280 : 1792);
+#define ATOMA_SSD_OUT_BY_PART(TO)                                \
+  do {                                                           \
+    if (part <= 1024) ATOMA_SSD_OUT(TO, 4, 256, 1);              \
+    else if (part <= 4096 && many) ATOMA_SSD_OUT(TO, 4, 256, 4); \
+    else if (part <= 4096) ATOMA_SSD_OUT(TO, 4, 1024, 1);        \
+    else ATOMA_SSD_OUT(TO, 0, 1024, 1);                          \
   } while (0)
   if (out_dtype == kF32) ATOMA_SSD_OUT_BY_PART(float);
   else if (out_dtype == kBF16) ATOMA_SSD_OUT_BY_PART(bf16_t);
   else return ATOMA_ERR_DTYPE;
 #undef ATOMA_SSD_OUT_BY_PART
 #undef ATOMA_SSD_OUT
+#undef ATOMA_SSD_OUT_AS
   ATOMA_LAUNCH_CHECK();
   return 0;
 }

@@ -144,6 +144,20 @@ def test_a_product_of_its_own_per_head(t, h, k, n, dtype):
 
 # ---- the recurrence alone ---------------------------------------------------------------------------------------------
 
+@pytest.mark.parametrize("inner, groups, rows", [(1030, 1, 1281), (2048, 1, 1300), (2048, 2, 700), (4096, 1, 1793), (6000, 2, 900), (4000, 1, 1792)])
+def test_a_row_s_gated_norm_does_not_hang_on_how_many_rows_there_are(inner, groups, rows):
+    """The same bits with the threads that few rows want and with those of many, on both sides of the line; against 64 bits."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(inner)
+    y, proj, w = (torch.randn(*s, generator=g).to(DEV) for s in ((rows, inner), (rows, inner + 3), (inner,)))
+    out = ops.ssd_out(y, proj, 0, w, 1e-5, groups, torch.float32)
+    assert torch.equal(out[:7], ops.ssd_out(y[:7], proj[:7], 0, w, 1e-5, groups, torch.float32))
+    u = (y.double() * torch.nn.functional.silu(proj[:, :inner].double())).view(rows, groups, -1)
+    ref = (u / torch.sqrt((u * u).mean(-1, keepdim=True) + 1e-5)).view(rows, inner) * w.double()
+    # (a float32 sum of at most inner / groups squares, a sigmoid and three products)
+    assert bool(((out.double() - ref).abs() <= (inner // groups + 32) * 2.0 ** -24 * ref.abs() + 1e-12).all())
+
+
 @pytest.mark.parametrize("heads, groups, vdim, n, taps, norm_groups, entries", [
     (1, 1, 1, 1, 1, 1, 1), (4, 2, 24, 16, 2, 2, 3), (2, 1, 65, 33, 3, 1, 2), (6, 3, 100, 72, 4, 1, 5), (64, 1, 64, 128, 4, 1, 8),
     (2, 2, 40, 200, 9, 1, 3), (3, 1, 50, 256, 4, 3, 2), (80, 1, 64, 16, 4, 1, 70)])
