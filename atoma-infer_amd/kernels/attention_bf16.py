@@ -463,32 +463,49 @@ def build_tasks(starts: np.ndarray, counts: np.ndarray, group: int, window: int,
 
 
 def whole_waves(pairs: int, keys: int, head_size: int) -> int:
-    """The waves that share a decoded token's whole key range, up to ``MERGE_MAX_KEYS`` keys.  Eight shorten the walk where the pairs are
-    few; where they fill the GPU several times over, or have less than a block of 32 keys a wave, what counts are the workgroups that
-    run side by side (a CU holds two of eight waves, whatever few keys they have), and fewer waves a pair make more of them.
-    Measured with 17 to 256 requests of 8 and of 4 KV heads, contexts of one length and of lengths spread evenly up to it, us by
-    eight waves / as here, head size 64: 32 requests up to 256 keys 9.2 / 9.0, 64 up to 512 13.6 / 12.7, up to 2,048 34.7 /
-    33.0, 128 up to 256 17.7 / 13.1, 200 up to 256 27.8 / 18.4, up to 512 33.7 / 28.8; head size 128: 64 up to 256 22.9 /
-    15.4, up to 1,024 41.4 / 35.7, 128 up to 256 43.6 / 21.9, 200 up to 512 82.7 / 59.5, up to 1,024 111 / 104, 256 up
-    to 512 100 / 69.  Beyond these lines the counts are within 3 percent of each other, or eight win."""
+    """The waves that share a decoded token's whole key range, up to ``MERGE_MAX_KEYS`` keys.  Eight shorten a walk most; fewer waves a
+    pair make more of the workgroups that run side by side (of eight waves, a CU holds two for heads of up to 64 columns and one for
+    wider ones, whatever few keys they have), which counts where the pairs need several rounds over the CUs, or have less than a
+    block of 32 keys a wave.  Up to 512 pairs four waves are one round (two pairs a workgroup).
+
+    Measured with 32 to 384 requests of 8 KV heads and 64 to 384 of 4, contexts of one length and of lengths spread evenly up to it,
+    256 to 2,304 keys, head sizes 32 to 128, KV caches out of the caches.  Over the 464 cases of head sizes 64 and 128 what the rule
+    names takes 0.91 of eight waves' time in the geometric mean and nowhere more than 1.015; times by one / two / four / eight waves are given as
+    shares of eight waves', spread lengths and then one length.  Head size 64: 64 requests up to 2,048 keys 1.63 / 1.26 / 0.96, 1.29 /
+    1.08 / 0.96 (four); 80 requests, 640 pairs, 1.42 / 1.15 / 1.24, 1.08 / 0.98 / 1.12 (eight); 128 up to 256 0.75 / 0.77 / 0.78, 0.83 /
+    0.84 / 0.81 (one); 200 up to 512 0.88 / 0.93 / 0.86, 0.95 / 0.98 / 0.99 (four), up to 2,048 1.14 / 1.15 / 1.05, 0.99 / 1.03 /
+    1.06 (eight).  Head size 128: 64 up to 256 0.69 / 0.77 / 0.68, 0.78 / 0.84 / 0.72 (four); 128 up to 512 0.65 / 0.70 / 0.74, 0.74 /
+    0.76 / 0.81 (one), up to 2,048 0.99 / 0.99 / 0.99, 0.95 / 0.96 / 0.97 (four); 160 up to 2,048 1.19 / 1.21 / 1.04, 1.12 / 1.13 / 1.00
+    and 200 1.07 / 1.08 / 0.97, 0.94 / 0.96 / 1.01 (eight)."""
     if pairs < 256 or keys > MERGE_MAX_KEYS or head_size > 128:
         return 8
+    if keys <= 256:
+        if head_size > 64:
+            return 1 if pairs > 512 else 4
+        if pairs >= 1024:
+            return 1
+        return 4 if pairs > 256 or head_size > 32 else 8
+    if pairs <= 256:
+        return 8
     if head_size <= 64:
-        if keys <= 256:
-            return 1 if pairs >= 1024 else 4
-        return 4 if keys <= 512 or 512 <= pairs < 768 else 8
-    if pairs >= 1024:
-        return 1 if keys <= 1024 else 4
-    return 4 if pairs >= 512 or keys <= 256 else 8
+        return 4 if keys <= 512 or (pairs <= 512 and head_size > 32) else 8
+    if keys <= 512:
+        return 1 if pairs > 512 else 4
+    if keys <= 1024:
+        return 1 if 512 < pairs <= 1024 else 4
+    if keys <= 1536:
+        return 8 if 512 < pairs <= 768 else 4
+    return 4 if pairs <= 512 or 768 < pairs <= 1024 else 8
 
 
 def plan_step(starts: np.ndarray, counts: np.ndarray, group: int, window: int, bucket_keys: Optional[int] = None, *, kv_heads: int,
-              head_size: int = 64, keep: int = 0, **options) -> Tuple[np.ndarray, tuple]:
+              head_size: int = 64, keep: int = 0, plain: bool = True, **options) -> Tuple[np.ndarray, tuple]:
     """``build_tasks`` as a step's launches want it: decode steps whose tasks are whole key ranges with the waves that
-    ``whole_waves`` names (a function of the entries and the bucket, as all of a decode step's plan is)."""
+    ``whole_waves`` names (a function of the entries and the bucket, as all of a decode step's plan is).  ``plain``: values are as
+    wide as keys and the scores have no bias; other layers, which take other registers and LDS, keep eight waves."""
     arr, meta = build_tasks(starts, counts, group, window, bucket_keys, kv_heads=kv_heads, head_size=head_size, keep=keep, **options)
     n_main, n_comb, n_part, waves, pieces, merge = meta
-    if bucket_keys is not None and n_comb == 0 and n_part == 0 and waves == 8 and not keep and len(counts) and int(counts.max()) == 1:
+    if plain and bucket_keys is not None and n_comb == 0 and n_part == 0 and waves == 8 and not keep and len(counts) and int(counts.max()) == 1:
         keys = bucket_keys if window == 0 else min(bucket_keys, abs(window) + CHUNK)
         meta = (n_main, 0, 0, whole_waves(n_main * kv_heads, keys, head_size), pieces, merge)
     return arr, meta

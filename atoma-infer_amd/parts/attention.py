@@ -149,13 +149,14 @@ class PagedAttention(Mixer):
             return None
         group, window, nkv, vd, keep = self.nh // self.nkv, self.span, self.nkv, self.value_hd, self.keep_first
         cus = torch.cuda.get_device_properties(self.w_o.device).multi_processor_count
-        shares = attention_bf16.shares_keys(self.hd, vd, biased=bool(keep) or self.slopes is not None)
+        biased = bool(keep) or self.slopes is not None
+        shares, plain = attention_bf16.shares_keys(self.hd, vd, biased), vd == self.hd and not biased
         return (attention_bf16.plan_key(group, window, nkv, self.hd, vd, keep),
                 lambda starts, counts, bucket: attention_bf16.plan_step(
                     starts, counts, group, window, bucket, kv_heads=nkv,
                     max_waves=attention_bf16.max_waves_for(self.hd, vd),
                     row_tiles=1 if shares else attention_bf16.max_row_tiles_for(self.hd, vd), head_size=self.hd, compute_units=cus,
-                    keep=keep))
+                    keep=keep, plain=plain))
 
     @property
     def span(self) -> int:

@@ -319,3 +319,15 @@ def test_waves_of_whole_ranges(s, keys, head_size, want):
         arr, meta = A.plan_step(st, counts, 4, 0, keys, kv_heads=8, max_waves=8, head_size=head_size)
         arr0, meta0 = A.build_tasks(st, counts, 4, 0, keys, kv_heads=8, max_waves=8, head_size=head_size)
         assert (arr == arr0).all() and meta == meta0[:3] + (want,) + meta0[4:] and meta0[3] == 8
+
+
+# (requests, KV heads, keys, head size, waves): where the counts were measured more than two percent apart, on both sides of each line
+@pytest.mark.parametrize("s,kv_heads,keys,head_size,want", [
+    (80, 8, 2048, 64, 8), (160, 4, 1536, 64, 8), (48, 8, 2304, 64, 4), (112, 4, 1024, 64, 4), (32, 8, 512, 64, 8), (33, 8, 512, 64, 4),
+    (32, 8, 256, 32, 8), (64, 8, 2048, 32, 8), (48, 8, 512, 128, 4), (80, 8, 2304, 128, 8), (80, 8, 512, 128, 1), (96, 8, 1024, 128, 1),
+    (160, 8, 1024, 128, 4), (160, 8, 2048, 128, 8), (200, 8, 2048, 128, 8), (112, 8, 2304, 128, 4), (64, 8, 2048, 96, 4)])
+def test_waves_of_whole_ranges_at_the_lines(s, kv_heads, keys, head_size, want):
+    assert A.whole_waves(s * kv_heads, keys, head_size) == want
+    starts, counts = np.arange(s, dtype=np.int32) % keys, np.ones(s, dtype=np.int32)
+    # layers whose values are wider than their keys, or whose scores have a bias, keep eight
+    assert A.plan_step(starts, counts, 4, 0, keys, kv_heads=kv_heads, max_waves=8, head_size=head_size, plain=False)[1][3] == 8
