@@ -3,6 +3,7 @@ name a kernel that exists and sizes that the kernel accepts (no GPU needed)."""
 import random
 
 import pytest
+import torch
 
 from atoma_infer_amd.kernels import gemm_bf16
 
@@ -124,3 +125,14 @@ def test_few_rows_plans_count_what_their_reader_pays_for_a_plane():
         assert gemm_bf16._small_product_slices(m, n, k) == 0, (m, n, k)
     for (m, n, k), slices in {(200, 2048, 2048): 2, (65, 2048, 4096): 4, (128, 1024, 4096): 8, (160, 1024, 4096): 4, (128, 3072, 3072): 2}.items():
         assert gemm_bf16._small_product_slices(m, n, k) == slices, (m, n, k)
+
+
+@pytest.mark.parametrize("n, k, made", [(3072, 2048, False), (5120, 3072, False), (6144, 4096, False), (7168, 5120, True)])
+def test_the_planes_copy_of_q_k_v_is_made_only_where_it_is_read(n, k, made, monkeypatch):
+    """Llama 1B, 3B, 8B: 41 to 64 rows all go to the tile kernel; wider and larger ones stay with the kernel that reads the copy."""
+    monkeypatch.setattr(gemm_bf16, "tile_weight_rope", lambda w: "few")
+    monkeypatch.setattr(gemm_bf16, "tile_weight_planes", lambda w: "many")
+    w = torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+    assert gemm_bf16.tile_copies_rope(w).many == ("many" if made else None)
+    left = [m for m in range(41, 65) if gemm_bf16._few_rows_plan(m, n, k, True) is None]
+    assert bool(left) == made
