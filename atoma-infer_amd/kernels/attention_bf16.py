@@ -622,7 +622,8 @@ def try_attention(q, k_cache, v_cache, out, ctx, cache, scale, window, nh, nkv, 
     group = nh // nkv
     plan = getattr(ctx, "plans", {}).get(plan_key(group, window, nkv, hd, vd, keep))
     if plan is None:
-        # a caller without a step planner (a kernel test): plan here and now
+        # a caller without a step planner (a kernel test): plan here and now, with two pieces a wave wherever the kernel has them
+        # (steps of layers that share keys plan one, see shares_keys)
         key = ("attention_tasks_adhoc", group, window, nkv, hd, vd, keep)
         plan = ctx.scratch.get(key)
         if plan is None:

@@ -127,12 +127,13 @@ def test_few_rows_plans_count_what_their_reader_pays_for_a_plane():
         assert gemm_bf16._small_product_slices(m, n, k) == slices, (m, n, k)
 
 
-@pytest.mark.parametrize("n, k, made", [(3072, 2048, False), (5120, 3072, False), (6144, 4096, False), (7168, 5120, True)])
+@pytest.mark.parametrize("n, k, made", [(3072, 2048, False), (5120, 3072, False), (6144, 4096, False), (7168, 5120, False), (768, 512, True)])
 def test_the_planes_copy_of_q_k_v_is_made_only_where_it_is_read(n, k, made, monkeypatch):
-    """Llama 1B, 3B, 8B: 41 to 64 rows all go to the tile kernel; wider and larger ones stay with the kernel that reads the copy."""
+    """Llama 1B, 3B, 8B and larger: 41 to 64 rows all go to the tile kernel or the library; very small ones to the kernel that reads it."""
     monkeypatch.setattr(gemm_bf16, "tile_weight_rope", lambda w: "few")
     monkeypatch.setattr(gemm_bf16, "tile_weight_planes", lambda w: "many")
     w = torch.empty(n, k, dtype=torch.bfloat16, device="meta")
     assert gemm_bf16.tile_copies_rope(w).many == ("many" if made else None)
-    left = [m for m in range(41, 65) if gemm_bf16._few_rows_plan(m, n, k, True) is None]
+    left = [m for m in range(41, 65) if gemm_bf16._few_rows_plan(m, n, k, True) is None
+            and not gemm_bf16._library_wins(m, n, k, torch.bfloat16)]
     assert bool(left) == made
