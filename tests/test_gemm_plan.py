@@ -137,3 +137,19 @@ def test_the_planes_copy_of_q_k_v_is_made_only_where_it_is_read(n, k, made, monk
     left = [m for m in range(41, 65) if gemm_bf16._few_rows_plan(m, n, k, True) is None
             and not gemm_bf16._library_wins(m, n, k, torch.bfloat16)]
     assert bool(left) == made
+
+
+def test_products_that_small_tiles_and_planes_were_measured_slower_at():
+    """What three rules leave to the kernels and the library that were there before them, and neighbours that they take."""
+    for m, n, k in ((64, 28672, 5120), (40, 16384, 8192), (64, 22016, 5120)):
+        assert not gemm_bf16._few_rows_swiglu(m, n, k), (m, n, k)
+    for m, n, k in ((64, 28672, 4096), (40, 16384, 5120), (64, 16384, 2048), (33, 16384, 3072)):
+        assert gemm_bf16._few_rows_swiglu(m, n, k), (m, n, k)
+    for m, n, k in ((65, 2048, 4096), (96, 2048, 5120), (128, 2048, 5120), (256, 2048, 8192)):
+        assert not gemm_bf16._small_swiglu(m, n, k), (m, n, k)
+    for m, n, k in ((200, 2048, 4096), (128, 8192, 1024), (65, 4096, 512), (200, 4096, 8192)):
+        assert gemm_bf16._small_swiglu(m, n, k), (m, n, k)
+    for m, n, k in ((160, 6144, 2048), (320, 5120, 3072), (200, 12288, 4096), (320, 10240, 8192)):
+        assert gemm_bf16._rope_planes_plan(m, n, k) is None, (m, n, k)
+    for m, n, k in ((200, 3072, 2048), (128, 5120, 3072), (65, 6144, 4096), (400, 1536, 1024)):
+        assert gemm_bf16._rope_planes_plan(m, n, k) is not None, (m, n, k)
