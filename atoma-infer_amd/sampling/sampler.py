@@ -118,7 +118,9 @@ class Sampler:
         meta_pool = self._meta_pool.setdefault(s, [])
         meta = meta_pool.pop() if meta_pool else torch.empty((5, s), dtype=torch.float32, pin_memory=True)
         mn = meta.numpy()
-        top_ks, top_ps = [pl.top_k for pl in plans], [pl.top_p for pl in plans]
+        top_ks = top_ps = ()
+        if s > FEW_ROWS or logits.shape[1] >= SPLIT_MIN_VOCAB:
+            top_ks, top_ps = [pl.top_k for pl in plans], [pl.top_p for pl in plans]
         if s <= FEW_ROWS:
             ints = mn[4].view(np.int32)
             for i, pl in enumerate(plans):
@@ -141,14 +143,14 @@ class Sampler:
             pen = torch.tensor([pen_rows, pen_toks], dtype=torch.int32).to(self.device)
             ops.repeat_penalty(logits, pen[0], pen[1], m[3])
         # (rows that draw are shared by several blocks each: a block walks a row of a large vocabulary too slowly)
-        if any([pl.greedy for pl in plans]):          # (what a greedy row's parameters say has no say in this)
-            drawn = [i for i, pl in enumerate(plans) if not pl.greedy]
-            top_ks, top_ps = [top_ks[i] for i in drawn], [top_ps[i] for i in drawn]
-        top_ks, top_ps = top_ks or [0], top_ps or [1.0]          # (no row draws, or there is none)
-        cuts_p = min(top_ps) < 1.0
-        out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2],
-                                split=not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB, cuts=cuts_p or max(top_ks) > 0,
-                                few=0 < min(top_ks) and max(top_ks) <= ops.FEW_MAX_K, top_p_cuts=cuts_p)
+        how = {}
+        if not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB:
+            if any([pl.greedy for pl in plans]):          # (what a greedy row's parameters say has no say in this)
+                drawn = [i for i, pl in enumerate(plans) if not pl.greedy]
+                top_ks, top_ps = [top_ks[i] for i in drawn] or [0], [top_ps[i] for i in drawn] or [1.0]
+            cuts_p, least, most = min(top_ps) < 1.0, min(top_ks), max(top_ks)
+            how = dict(split=True, cuts=cuts_p or most > 0, few=0 < least and most <= ops.FEW_MAX_K, top_p_cuts=cuts_p)
+        out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2], **how)
         tok, lg = out[0].view(torch.int32), out[1]
         host, pool = self._host_buffer(s)
         host.copy_(out, non_blocking=True)
