@@ -476,15 +476,56 @@ lowrank_up_kernel(const float* __restrict__ x, int ldx, const TW* __restrict__ w
   out[(size_t)t * ldo + n] = total;
 }
 
+// The same against a bfloat16 weight, on the matrix cores as the general product does it: a wave takes sixteen tokens against
+// sixteen rows of the weight.
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+lowrank_split_kernel(const float* __restrict__ x, const bf16_t* __restrict__ w, float* __restrict__ out, int T, int N, int K, int ldx,
+                     int ldo) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * 64 + (threadIdx.x >> 6) * 16, t = blockIdx.y * 16 + r16;
+  if (n0 >= N) return;
+  const float* const xr = x + (size_t)min(t, T - 1) * ldx;             // (rows past the end: the last, never stored)
+  const bf16_t* const wr = w + (size_t)min(n0 + r16, N - 1) * K;
+  const int steps = (K + kF32Step - 1) / kF32Step, bits = f32_part_bits(N);
+  f32x4_t total = {0.f, 0.f, 0.f, 0.f}, acc = total;
+  int part = 0, next = f32_part_begin(steps, 1, bits);
+  for (int s = 0; s < steps; ++s) {
+    if (s == next) {
+      total += acc;
+      acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      do next = f32_part_begin(steps, ++part + 1, bits);
+      while (next == s);
+    }
+    f32x4_t xv[2];
+    uint4 wv;
+    split_load<VEC>(xr, s * kF32Step + kg * 8, K, xv);
+    split_load<VEC>(wr, s * kF32Step + kg * 8, K, wv);
+    const Split8 p = split_of(xv);
+    const bf16x8_t whole = __builtin_bit_cast(bf16x8_t, wv), finite = split_weight(whole);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q == 0 ? whole : finite, p.p[q], acc, 0, 0, 0);
+  }
+  total += acc;
+  if (t >= T) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n0 + kg * 4 + e < N) out[(size_t)t * ldo + n0 + kg * 4 + e] = total[e];
+}
+
 extern "C" int atoma_lowrank_up(const float* x, int ldx, const void* w, int w_dtype, float* out, int ldo, int n_tokens,
                                 int N, int K, hipStream_t stream) {
   if (n_tokens <= 0 || N <= 0) return 0;
   if (K <= 0 || K > 8192 || ldx < K || ldo < N || n_tokens > 65535) return ATOMA_ERR_SHAPE;
   const size_t lds = (size_t)(K + kF32Step - 1) / kF32Step * kF32Step * sizeof(float);
   dim3 grid((N + 255) / 256, n_tokens), block(256);
-  if (w_dtype == kBF16)
-    hipLaunchKernelGGL((lowrank_up_kernel<bf16_t>), grid, block, lds, stream, x, ldx, (const bf16_t*)w,
-                       out, ldo, N, K);
+  if (w_dtype == kBF16 && split_product(N, K)) {
+    const bool vec = K % kF32Step == 0 && ldx % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    grid = dim3((N + 63) / 64, (n_tokens + 15) / 16);
+    if (vec) hipLaunchKernelGGL((lowrank_split_kernel<true>), grid, block, 0, stream, x, (const bf16_t*)w, out, n_tokens, N, K, ldx, ldo);
+    else hipLaunchKernelGGL((lowrank_split_kernel<false>), grid, block, 0, stream, x, (const bf16_t*)w, out, n_tokens, N, K, ldx, ldo);
+  } else if (w_dtype == kBF16)
+    hipLaunchKernelGGL((lowrank_up_kernel<bf16_t>), grid, block, lds, stream, x, ldx, (const bf16_t*)w, out, ldo, N, K);
   else if (w_dtype == kF32)
     hipLaunchKernelGGL((lowrank_up_kernel<float>), grid, block, lds, stream, x, ldx, (const float*)w, out,
                        ldo, N, K);

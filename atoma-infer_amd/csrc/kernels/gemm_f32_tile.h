@@ -145,4 +145,184 @@ __device__ __forceinline__ void f32_tile(float* __restrict__ lds, int K, int bit
     for (int j = 0; j < TM / 32; ++j) total[i][j] = SPLIT ? total[i][j] + acc[i][j] : acc[i][j];
 }
 
+// ---- float32 rows against a bfloat16 weight -----------------------------------------------------------------------------
+// A float32 number is the sum of three bfloat16 numbers of its sign (24 bits of significand, eight at a time), so a product of
+// float32 rows and a bfloat16 weight is three bfloat16 ones, whose products float32 holds exactly and whose sums the matrix cores
+// keep in float32: nothing is rounded that the float32 instruction would not round, and 32 values of K take three instructions
+// where they took eight of twice the length.  A step of 32 values is added as the weight times the first, the second and the third
+// bfloat16 of each value, by v_mfma_f32_16x16x32_bf16 with lane group g holding values 8 g .. 8 g + 7; the parts of K are
+// those above.  Every kernel of the general product keeps to that.
+// Its error against 64-bit results is 0.6 of the float32 instruction's (200 rows, K of 2,048: 1.8e-7 and 2.9e-7 of the result, K of
+// 8,192 3.5e-7 and 5.7e-7, over normal, one-sided and heavy-tailed values).  What the matrix cores drop below a sum's last bit
+// counts against it only where all products have one sign and a part's sum outgrows them by far: in parts of 1,280 values the two are
+// even, in parts of 2,560 it is 1.9e-6 against 3.9e-7.  So parts longer than 1,024 values keep the float32 instruction.
+__host__ __device__ __forceinline__ constexpr bool split_product(int N, int K) { return K <= 1024 << f32_part_bits(N); }
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+
+struct Split8 { bf16x8_t p[3]; };
+
+__device__ __forceinline__ uint32_t high_halves(float lo, float hi) {      // the upper sixteen bits of both
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302);
+}
+// Exact but for what lies below 2^-133 (bfloat16's smallest number).  An infinite value's second and third number are those of
+// the largest finite one, so that its products stay infinities.
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  u32x4 h[3];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    float r[2], t[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float v = __builtin_amdgcn_fmed3f(x[i + e], -3.402823466e38f, 3.402823466e38f);
+      r[e] = v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
+      t[e] = r[e] - __uint_as_float(__float_as_uint(r[e]) & 0xffff0000u);
+    }
+    h[0][i / 2] = high_halves(x[i], x[i + 1]);
+    h[1][i / 2] = high_halves(r[0], r[1]);
+    h[2][i / 2] = high_halves(t[0], t[1]);
+  }
+  Split8 s;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) s.p[q] = __builtin_bit_cast(bf16x8_t, h[q]);
+  return s;
+}
+
+// The weight as the second and third numbers meet it: its infinities and NaN made the largest finite numbers (those numbers may
+// be zero, and the first one's product has said what the sum is).
+__device__ __forceinline__ bf16x8_t split_weight(bf16x8_t w) {
+  typedef __attribute__((ext_vector_type(8))) short i16x8;
+  typedef __attribute__((ext_vector_type(8))) unsigned short u16x8;
+  const i16x8 a = __builtin_elementwise_min(__builtin_bit_cast(i16x8, w), (i16x8)(short)0x7f7f);
+  return __builtin_bit_cast(bf16x8_t, __builtin_elementwise_min(__builtin_bit_cast(u16x8, a), (u16x8)(unsigned short)0xff7f));
+}
+
+// eight neighbouring values of K of one row, from k on; zeros from K on.  VEC: as in f32_load4, and the rows are aligned to 16 bytes
+template <bool VEC>
+__device__ __forceinline__ void split_load(const float* __restrict__ row, int k, int K, f32x4_t (&v)[2]) {
+  if constexpr (VEC) {
+    v[0] = *reinterpret_cast<const f32x4_t*>(row + k), v[1] = *reinterpret_cast<const f32x4_t*>(row + k + 4);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = k + i < K ? row[k + i] : 0.f;
+  }
+}
+template <bool VEC>
+__device__ __forceinline__ void split_load(const bf16_t* __restrict__ row, int k, int K, uint4& v) {
+  if constexpr (VEC) {
+    v = *reinterpret_cast<const uint4*>(row + k);
+  } else {
+    uint16_t* const e = reinterpret_cast<uint16_t*>(&v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) e[i] = k + i < K ? __builtin_bit_cast(uint16_t, row[k + i]) : (uint16_t)0;
+  }
+}
+__device__ __forceinline__ Split8 split_of(const f32x4_t (&v)[2]) {
+  const float x[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
+  return split8(x);
+}
+
+// A row of a step in LDS: 64 bytes, 80 apart, so that the sixteen rows of a load fall on different banks.
+constexpr int kSplitRow = 80;
+// TM rows of A against TN rows of W by WM x WN waves; bytes of LDS: two buffers of A's three planes and W's rows
+template <int TM_, int TN_, int WM_, int WN_, int ST_>
+struct SplitTile {
+  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, ST = ST_, THREADS = 64 * WM * WN;
+  static constexpr int BM = TM / WM / 16, BN = TN / WN / 16;             // blocks of 16 of a wave
+  static constexpr int PLANE = TM * kSplitRow, BUF = (3 * TM + TN) * kSplitRow, LDS = 2 * BUF;
+  static_assert(TM * 4 % THREADS == 0 && TN * 4 % THREADS == 0 && LDS <= 160 * 1024, "");
+};
+
+// As f32_tile with SPLIT and no scale: total[i][j] of this wave's share (wave / WN of A's rows, wave % WN of W's).  A step's values
+// are asked for three steps ahead, wait in registers in two sets in turn, and are split and written to LDS beside the products of the
+// step before theirs: one barrier a step.
+template <typename C, bool VEC, typename RowA, typename RowW>
+__device__ __forceinline__ void split_tile(char* __restrict__ lds, int K, int bits, RowA row_a, RowW row_w,
+                                           f32x4_t (&total)[C::BN][C::BM]) {
+  constexpr int PA = C::TM * 4 / C::THREADS, PW = C::TN * 4 / C::THREADS, RP = C::THREADS / 4;      // pieces of eight a thread moves
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int k8 = (tid & 3) * 8, r0 = tid >> 2;             // four threads a row of the step
+  const float* pa[PA];
+  const bf16_t* pw[PW];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) pa[i] = row_a(r0 + i * RP);
+#pragma unroll
+  for (int i = 0; i < PW; ++i) pw[i] = row_w(r0 + i * RP);
+  struct Stage { f32x4_t a[PA][2]; uint4 w[PW]; };
+  const int steps = (K + kF32Step - 1) / kF32Step;
+  auto fetch = [&](Stage& st, int s) {                     // (steps past the end: the last one again, which nobody multiplies)
+    const int k = min(s, steps - 1) * kF32Step + k8;
+#pragma unroll
+    for (int i = 0; i < PA; ++i) split_load<VEC>(pa[i], k, K, st.a[i]);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) split_load<VEC>(pw[i], k, K, st.w[i]);
+  };
+  auto put = [&](char* buf, const Stage& st) {
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+      const Split8 x = split_of(st.a[i]);
+      bf16x8_t* const to = reinterpret_cast<bf16x8_t*>(buf + (r0 + i * RP) * kSplitRow + k8 * 2);
+      to[0] = x.p[0], to[C::PLANE / 16] = x.p[1], to[2 * C::PLANE / 16] = x.p[2];
+    }
+#pragma unroll
+    for (int i = 0; i < PW; ++i) *reinterpret_cast<uint4*>(buf + 3 * C::PLANE + (r0 + i * RP) * kSplitRow + k8 * 2) = st.w[i];
+  };
+  f32x4_t acc[C::BN][C::BM];
+#pragma unroll
+  for (int i = 0; i < C::BN; ++i)
+#pragma unroll
+    for (int j = 0; j < C::BM; ++j) total[i][j] = acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int part = 0, next = f32_part_begin(steps, 1, bits);
+  const int aw = (wave / C::WN * (C::TM / C::WM) + r16) * kSplitRow + kg * 16;
+  const int ww = 3 * C::PLANE + (wave % C::WN * (C::TN / C::WN) + r16) * kSplitRow + kg * 16;
+  // step s: its values lie in `now`; those of step s + 1 come in `st` and go to `then`
+  auto step = [&](int s, const char* now, char* then, Stage& st) {
+    if (s == next) {
+#pragma unroll
+      for (int i = 0; i < C::BN; ++i)
+#pragma unroll
+        for (int j = 0; j < C::BM; ++j) total[i][j] += acc[i][j], acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // (parts without a step add nothing)
+      do next = f32_part_begin(steps, ++part + 1, bits);
+      while (next == s);
+    }
+    // (everybody has written this step's values and read those of the step before)
+    lds_barrier();
+    bf16x8_t fw[C::BN];
+#pragma unroll
+    for (int i = 0; i < C::BN; ++i) fw[i] = *reinterpret_cast<const bf16x8_t*>(now + ww + i * 16 * kSplitRow);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      bf16x8_t fa[C::BM];
+#pragma unroll
+      for (int j = 0; j < C::BM; ++j) fa[j] = *reinterpret_cast<const bf16x8_t*>(now + aw + q * C::PLANE + j * 16 * kSplitRow);
+      if (q == 1) {
+#pragma unroll
+        for (int i = 0; i < C::BN; ++i) fw[i] = split_weight(fw[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < C::BN; ++i)
+#pragma unroll
+        for (int j = 0; j < C::BM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[i], fa[j], acc[i][j], 0, 0, 0);
+    }
+    put(then, st);
+    fetch(st, s + C::ST + 1);
+  };
+  Stage st[C::ST];
+#pragma unroll
+  for (int i = 0; i < C::ST; ++i) fetch(st[i], i);
+  put(lds, st[0]);
+  fetch(st[0], C::ST);
+  for (int s = 0; s < steps; s += C::ST) {
+#pragma unroll
+    for (int i = 0; i < C::ST; ++i)
+      if (s + i < steps) step(s + i, lds + (i & 1) * C::BUF, lds + (~i & 1) * C::BUF, st[(i + 1) % C::ST]);
+  }
+#pragma unroll
+  for (int i = 0; i < C::BN; ++i)
+#pragma unroll
+    for (int j = 0; j < C::BM; ++j) total[i][j] += acc[i][j];
+}
+
 }  // namespace atoma

@@ -4,23 +4,31 @@
 // bfloat16 kernels refuse.
 //
 // Weights are [out, in] row-major as checkpoints store them (models/src/llama.rs:322-325), so both operands
-// are contiguous along K.  Two kernels:
+// are contiguous along K.  Two kernels, each in two kinds:
 //
 //   f32_tile_kernel    tiles of 128 x 128 (64 x 64 where those would leave CUs idle) through LDS, see gemm_f32_tile.h.
 //                      Bound by the matrix cores (a float32 MFMA has a sixteenth of the bfloat16 rate);
 //   f32_stream_kernel  up to 64 rows of A a workgroup against 16 rows of W, which come straight from memory, once: K is
 //                      split over the workgroup's waves, whose sums meet in LDS.  Bound by W's bytes up to 16 rows of A.
 //                      It also takes more rows where tiles of 64 x 64 would be fewer than the CUs (four waves of a tile
-//                      walk all of K, eight of a streaming workgroup an eighth of it each).
+//                      walk all of K, eight of a streaming workgroup an eighth of it each);
+//   split_tile_kernel, split_stream_kernel
+//                      the same for float32 rows against a bfloat16 weight, which is the 32-bit path of a bfloat16 checkpoint:
+//                      every float32 value as three bfloat16 ones (gemm_f32_tile.h), at three bfloat16 MFMAs for 32 values of K.
+//                      Tiles are bound by what a step costs beside its MFMAs (splitting A, a trip through LDS, a barrier: 1.4 us for
+//                      128 x 256, of which the MFMAs are 0.7), streaming workgroups by W's bytes and the splitting.
 //
-// Measured on MI355X, float32 rows against bfloat16 weights, beside the one kernel of vector multiply-adds before (a tile
-// of 64 x 64 a workgroup, 4 x 4 outputs a thread): the four layers of Llama 1B sizes and its head, 836 rows in one step
-// and 16 steps of 4 rows, 106.5 -> 9.8 ms in all; gate-up (16,384 x 2,048) with 836 rows 569 us (99 TFLOP/s; the
-// card's float32 product of 8,192^3 reaches 153), with 4 rows 18 us (22.7 with one batch of loads in flight); the head
-// (128,256 x 2,048) with 4 rows 124 us.
+// Measured on MI355X, float32 rows against bfloat16 weights, us by the float32 MFMA / by three bfloat16 ones: gate-up of Llama 1B
+// (16,384 x 2,048) with 836 rows 568 / 175, with 64 rows 73 / 32, with 4 rows 17.4 / 15.3; its down product (2,048 x 8,192) with 836
+// rows 317 / 155; q, k, v (3,072 x 2,048) with 836 rows 123 / 60; the head (128,256 x 2,048) with 4 rows 115 / 99, with 64
+// rows 557 / 153.
 //
-// Both kernels sum an output's K products in the order that gemm_f32_tile.h states, a function of (N, K) alone: a row's
+// All sum an output's K products in the order that gemm_f32_tile.h states, a function of (N, K) alone: a row's
 // result depends neither on its place nor on the rows beside it.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "gemm_f32_tile.h"
 
 using namespace atoma;
@@ -70,6 +78,31 @@ f32_tile_kernel(const TA* __restrict__ a, const TW* __restrict__ w, TC* __restri
 #pragma unroll
     for (int i = 0; i < T / 32; ++i) {
       const int n = n0 + (wave & 1) * (T / 2) + i * 16 + (lane >> 4) * 4;
+      put4(c + (size_t)m * ldc, n, N, aligned, acc[i][j]);
+    }
+  }
+}
+
+// the same for float32 rows against a bfloat16 weight
+template <typename C, bool VEC, typename TC>
+__global__ void __launch_bounds__(C::THREADS, 2)
+split_tile_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* __restrict__ c, int M, int N, int K, int lda,
+                  int ldw, int ldc) {
+  extern __shared__ __attribute__((aligned(16))) char split_lds[];
+  const int m0 = blockIdx.y * C::TM, n0 = blockIdx.x * C::TN;
+  f32x4_t acc[C::BN][C::BM];
+  split_tile<C, VEC>(
+      split_lds, K, f32_part_bits(N), [&](int r) { return a + (size_t)min(m0 + r, M - 1) * lda; },
+      [&](int r) { return w + (size_t)min(n0 + r, N - 1) * ldw; }, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool aligned = aligned4(c, ldc);
+#pragma unroll
+  for (int j = 0; j < C::BM; ++j) {
+    const int m = m0 + wave / C::WN * (C::TM / C::WM) + j * 16 + (lane & 15);
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < C::BN; ++i) {
+      const int n = n0 + wave % C::WN * (C::TN / C::WN) + i * 16 + (lane >> 4) * 4;
       put4(c + (size_t)m * ldc, n, N, aligned, acc[i][j]);
     }
   }
@@ -167,6 +200,101 @@ f32_stream_kernel(const TA* __restrict__ a, const TW* __restrict__ w, TC* __rest
   }
 }
 
+// The same for float32 rows against a bfloat16 weight: a step is 32 values of K, three instructions for each block of 16 rows of A
+// and of W.  RT blocks of W a wave share the split of A's values, which takes as long as four blocks' instructions.
+template <int MT, int RT, int WK, typename TC>
+__global__ void __launch_bounds__(64 * WK)
+split_stream_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* __restrict__ c, int M, int N, int K, int lda,
+                    int ldw, int ldc) {
+  constexpr int BITS = WK == 8 ? 3 : 2;
+  static_assert(WK == 1 << BITS, "a wave a part of K");
+  constexpr int U = MT == 1 && RT == 1 ? 4 : 2;       // steps whose loads are in flight together
+  __shared__ f32x4_t red[WK - 1][RT][MT][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * (16 * RT), m0 = blockIdx.y * (16 * MT);
+  const int steps = K / 32, begin = f32_part_begin(steps, wave, BITS), end = f32_part_begin(steps, wave + 1, BITS);
+  const bf16_t* wp[RT];                                    // (rows past the end: the last, never stored)
+#pragma unroll
+  for (int i = 0; i < RT; ++i) wp[i] = w + (size_t)min(n0 + i * 16 + r16, N - 1) * ldw + kg * 8;
+  const float* ap[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) ap[m] = a + (size_t)min(m0 + m * 16 + r16, M - 1) * lda + kg * 8;
+  f32x4_t acc[RT][MT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[i][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  struct Step { bf16x8_t w[RT]; f32x4_t a[MT][2]; };
+  auto load = [&](Step& x, int s) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) x.w[i] = *reinterpret_cast<const bf16x8_t*>(wp[i] + s * 32);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) split_load<true>(ap[m], s * 32, K, x.a[m]);
+  };
+  auto multiply = [&](Step& x) {
+    Split8 p[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) p[m] = split_of(x.a[m]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if (q == 1) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) x.w[i] = split_weight(x.w[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.w[i], p[m].p[q], acc[i][m], 0, 0, 0);
+    }
+  };
+  // two batches of U steps in turn: while the MFMAs of one run, the loads of the other are on their way
+  Step x[2][U];
+  const int batches = (end - begin) / U;
+  auto fetch = [&](int buf, int b) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(x[buf][u], begin + b * U + u);
+  };
+  auto take = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) multiply(x[buf][u]);
+  };
+  if (batches > 0) fetch(0, 0);
+  int b = 0;
+  for (; b + 2 <= batches; b += 2) {
+    fetch(1, b + 1);
+    take(0);
+    if (b + 2 < batches) fetch(0, b + 2);
+    take(1);
+  }
+  if (b < batches) take(0);
+  for (int s = begin + batches * U; s < end; ++s) {
+    load(x[0][0], s);
+    multiply(x[0][0]);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) red[wave - 1][i][m][lane] = acc[i][m];
+  }
+  __syncthreads();
+  // (a part's sums are added in the parts' order; the waves share the blocks)
+  const bool aligned = aligned4(c, ldc);
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    if (wave > 0) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int q = 0; q < WK - 1; ++q) acc[i][m] += red[q][i][m][lane];
+      const int row = m0 + m * 16 + r16, n = n0 + i * 16 + kg * 4;
+      if (row >= M) continue;
+      put4(c + (size_t)row * ldc, n, N, aligned, acc[i][m]);
+    }
+  }
+}
+
 constexpr int kStreamRows = 64;       // rows of A that one streaming workgroup takes
 constexpr int kCUs = 256;
 
@@ -184,10 +312,94 @@ static void launch_stream(const TA* a, const TW* w, TC* c, int M, int N, int K, 
 #undef ATOMA_STREAM
 }
 
+template <int MT, int RT, typename TC>
+static int launch_split_stream(const float* a, const bf16_t* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc,
+                               hipStream_t stream) {
+  const dim3 grid(ceil_div(N, 16 * RT), ceil_div(M, 16 * MT));
+  // (a wave a part of K)
+  if constexpr (RT <= 2) {
+    if (f32_part_bits(N) == 3) {
+      hipLaunchKernelGGL((split_stream_kernel<MT, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+      ATOMA_LAUNCH_CHECK();
+      return 0;
+    }
+  }
+  hipLaunchKernelGGL((split_stream_kernel<MT, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename C, bool VEC, typename TC>
+static int launch_split_tile(const float* a, const bf16_t* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
+  if (ceil_div(M, C::TM) > 65535) return ATOMA_ERR_SHAPE;
+  // (every device that the kernel is launched on has its own setting)
+  const hipError_t e = hipFuncSetAttribute((const void*)split_tile_kernel<C, VEC, TC>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL((split_tile_kernel<C, VEC, TC>), dim3(ceil_div(N, C::TN), ceil_div(M, C::TM)), dim3(C::THREADS), C::LDS, stream,
+                     a, w, c, M, N, K, lda, ldw, ldc);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+// microseconds that tiles of C take: a step with one of them a CU, a round over the CUs, and as many as there are (fitted to 420
+// products of 17 to 2,048 rows, 512 to 128,256 columns and K of 1,024 to 8,192, each tile within a quarter)
+template <typename C>
+static float split_tile_us(int M, int N, int K, float fixed, float one, float round, float each) {
+  const float tiles = (float)ceil_div(M, C::TM) * ceil_div(N, C::TN) / kCUs;
+  return fixed + ceil_div(K, kF32Step) * std::max({one, round * std::ceil(tiles), each * tiles});
+}
+
+// Which kernel takes float32 rows against a bfloat16 weight; whichever does, the results are the same bits.  Streaming workgroups of
+// few blocks are the quickest as long as each has a CU (64 rows, 2,048 x 2,048: 10.3 us by one block of rows and two of the weight,
+// 14.4 by two and two, 20.4 by four and one, 29.4 by tiles), so the first of the combinations below that is one round over
+// the CUs; with more than 4,096 columns a workgroup has four waves and takes up to four blocks of each.  Beyond, tiles.
+template <typename TC>
+static int launch_split(const float* a, const bf16_t* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc, bool aligned,
+                        hipStream_t stream) {
+  const bool vec = aligned && K % kF32Step == 0, wide = f32_part_bits(N) == 2;
+#define ATOMA_STREAM(MT, RT) return launch_split_stream<MT, RT>(a, w, c, M, N, K, lda, ldw, ldc, stream)
+  if (vec) {
+    auto round = [&](int mt, int rt, int most) { return (int64_t)ceil_div(N, 16 * rt) * ceil_div(M, 16 * mt) <= most; };
+    if (!wide) {
+      if (round(1, 1, kCUs)) ATOMA_STREAM(1, 1);
+      if (M <= 20 && round(2, 1, kCUs)) ATOMA_STREAM(2, 1);
+      if (round(1, 2, kCUs)) ATOMA_STREAM(1, 2);
+      if (round(2, 2, 320)) ATOMA_STREAM(2, 2);
+      if (round(4, 2, kCUs)) ATOMA_STREAM(4, 2);
+    } else if (M <= 16) {
+      // (what a wave splits of A weighs less the fewer rows there are: 1 row, 28,672 x 4,096: one block 44.9 us, four 49.0; 16 rows 78 and 58)
+      if (M <= 4 && N <= (M == 1 ? 32768 : 8192)) ATOMA_STREAM(1, 1);
+      if (N <= 8192 || (M <= 4 && N > 32768)) ATOMA_STREAM(1, 2);
+      ATOMA_STREAM(1, 4);
+    } else {
+      if (round(2, 2, kCUs)) ATOMA_STREAM(2, 2);
+      if (round(1, 4, kCUs)) ATOMA_STREAM(1, 4);
+      if (round(2, 4, kCUs) || (M <= 32 && N <= 65536)) ATOMA_STREAM(2, 4);
+      if (round(4, 4, kCUs)) ATOMA_STREAM(4, 4);
+    }
+  }
+#undef ATOMA_STREAM
+  using Large = SplitTile<128, 256, 2, 4, 2>;
+  using Middle = SplitTile<64, 128, 2, 2, 4>;
+  using Small = SplitTile<64, 64, 2, 2, 2>;
+#define ATOMA_TILE(C)                                                                                  \
+  return vec ? launch_split_tile<C, true>(a, w, c, M, N, K, lda, ldw, ldc, stream)                    \
+             : launch_split_tile<C, false>(a, w, c, M, N, K, lda, ldw, ldc, stream)
+  const float large = split_tile_us<Large>(M, N, K, 7.17f, 1.03f, 0.3f, 1.58f), middle = split_tile_us<Middle>(M, N, K, 3.79f, 0.57f, 0.44f, 0.51f),
+              small = split_tile_us<Small>(M, N, K, 2.7f, 0.43f, 0.31f, 0.2f);
+  if (large <= std::min(middle, small)) ATOMA_TILE(Large);
+  if (middle <= small) ATOMA_TILE(Middle);
+  ATOMA_TILE(Small);
+#undef ATOMA_TILE
+}
+
 template <typename TA, typename TW, typename TC>
 static int launch(const TA* a, const TW* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
   auto rows16 = [](const void* p, int ld, size_t size) { return ((uintptr_t)p | (ld * size)) % 16 == 0; };
   const bool aligned = rows16(a, lda, sizeof(TA)) && rows16(w, ldw, sizeof(TW));
+  if constexpr (std::is_same_v<TA, float> && std::is_same_v<TW, bf16_t>) {
+    if (split_product(N, K)) return launch_split(a, w, c, M, N, K, lda, ldw, ldc, aligned, stream);
+  }
   const int small = ceil_div(M, 64) * ceil_div(N, 64), large = ceil_div(M, 128) * ceil_div(N, 128);
   if (aligned && K % 32 == 0 && (M <= kStreamRows || small < kCUs)) {
     // (a wave a part of K)

@@ -144,6 +144,32 @@ def test_gemm_generic_row_alone(n, k, wdt):
                 assert bool((c[:, :off] == 7.0).all()) and bool((c[:, off + n:] == 7.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 48, 96), (20, 4000, 64), (48, 2050, 544), (65, 3000, 32), (130, 2500, 96), (300, 4090, 100),
+                                   (1, 5000, 64), (1, 40000, 32), (5, 5003, 96), (7, 9000, 64), (17, 4112, 288), (33, 5120, 64),
+                                   (70, 5200, 96), (130, 5100, 160), (140, 20000, 64), (1100, 8200, 352), (200, 130, 8192),
+                                   (70, 4100, 4096), (3, 4100, 4128)])
+def test_gemm_float32_by_bfloat16_thirds(m, n, k):
+    """float32 rows against a bfloat16 weight: every number of blocks a streaming workgroup takes, every tile, and both sides of the
+    longest part of K that goes to the bfloat16 instruction.  The three numbers that a value is cut into hold all of it, so the bound is
+    that of any float32 sum, three additions a product.  Infinities, NaN and large numbers stay what they are."""
+    from atoma_infer_amd.kernels import ops
+    a, w = rnd(m, k, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    c = ops.gemm_generic(a, w, torch.float32)
+    want = a.double() @ w.double().T
+    assert bool(((c.double() - want).abs() <= 3 * k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
+    assert (c.double() - want).norm() <= 1e-6 * want.norm()
+    w[0, 5], w[1 % n, 6] = math.inf, math.nan
+    a[m // 3, 7] = 1e37
+    a[-1] = 1.0             # (the second and third numbers are zero)
+    a[-1, 3] = math.inf
+    a[m // 2, 9] = -math.inf
+    a[0, 11] = math.nan
+    got, want = ops.gemm_generic(a, w, torch.float32), a @ w.float().T
+    assert torch.equal(got.isnan(), want.isnan())
+    bad = want.isinf() & (want.double() - (a.double() @ w.double().T)).isnan()        # (infinite in 64 bits too)
+    assert torch.equal(got[bad], want[bad])
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 48, 64])
 @pytest.mark.parametrize("n,k", [(16, 32), (100, 64), (3072, 2048), (2048, 8192), (1000, 96), (40000, 128),
                                  (70000, 64)])
