@@ -12,15 +12,15 @@
 //                      split over the workgroup's waves, whose sums meet in LDS.  Bound by W's bytes up to 16 rows of A.
 //                      It also takes more rows where tiles of 64 x 64 would be fewer than the CUs (four waves of a tile
 //                      walk all of K, eight of a streaming workgroup an eighth of it each);
-//   split_tile_kernel, split_stream_kernel
+//   split_tile_kernel, split_stream_kernel, split_few_kernel (up to eight rows)
 //                      the same for float32 rows against a bfloat16 weight, which is the 32-bit path of a bfloat16 checkpoint:
 //                      every float32 value as three bfloat16 ones (gemm_f32_tile.h), at three bfloat16 MFMAs for 32 values of K.
 //                      Tiles are bound by what a step costs beside its MFMAs (splitting A, a trip through LDS, a barrier: 1.4 us for
 //                      128 x 256, of which the MFMAs are 0.7), streaming workgroups by W's bytes and the splitting.
 //
 // Measured on MI355X, float32 rows against bfloat16 weights, us by the float32 MFMA / by three bfloat16 ones: gate-up of Llama 1B
-// (16,384 x 2,048) with 836 rows 568 / 175, with 64 rows 73 / 32, with 4 rows 17.4 / 15.3; its down product (2,048 x 8,192) with 836
-// rows 317 / 155; q, k, v (3,072 x 2,048) with 836 rows 123 / 60; the head (128,256 x 2,048) with 4 rows 115 / 99, with 64
+// (16,384 x 2,048) with 836 rows 568 / 175, with 64 rows 73 / 32, with 4 rows 17.3 / 13.4; its down product (2,048 x 8,192) with 836
+// rows 317 / 155, with 4 rows 16.4 / 11.4; q, k, v (3,072 x 2,048) with 836 rows 123 / 60; the head (128,256 x 2,048) with 4 rows 114 / 87, with 64
 // rows 557 / 153.
 //
 // All sum an output's K products in the order that gemm_f32_tile.h states, a function of (N, K) alone: a row's
@@ -279,11 +279,10 @@ split_stream_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, T
       for (int m = 0; m < MT; ++m) red[wave - 1][i][m][lane] = acc[i][m];
   }
   __syncthreads();
-  // (a part's sums are added in the parts' order; the waves share the blocks)
+  if (wave > 0) return;
   const bool aligned = aligned4(c, ldc);
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
-    if (wave > 0) return;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
 #pragma unroll
@@ -292,6 +291,101 @@ split_stream_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, T
       if (row >= M) continue;
       put4(c + (size_t)row * ldc, n, N, aligned, acc[i][m]);
     }
+  }
+}
+
+// The same for up to 4 RW rows of A, 4 or 8: sixteen lanes split a row's values of four steps and hand them to the others through LDS,
+// so that no lane splits what another splits too (every wave has its own corner of LDS, which it fills and reads in order).
+template <int RW, int RT, int WK, typename TC>
+__global__ void __launch_bounds__(64 * WK)
+split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* __restrict__ c, int M, int N, int K, int lda,
+                 int ldw, int ldc) {
+  constexpr int BITS = WK == 8 ? 3 : 2, U = 4;             // steps of a batch
+  static_assert(WK == 1 << BITS, "a wave a part of K");
+  __shared__ f32x4_t red[WK - 1][RT][64];
+  __shared__ bf16x8_t thirds[WK][3][RW * 4][U * 4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r16 = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * (16 * RT);
+  const int steps = K / 32, begin = f32_part_begin(steps, wave, BITS), end = f32_part_begin(steps, wave + 1, BITS);
+  const bf16_t* wp[RT];                                    // (rows past the end: the last, never stored)
+#pragma unroll
+  for (int i = 0; i < RT; ++i) wp[i] = w + (size_t)min(n0 + i * 16 + r16, N - 1) * ldw + kg * 8;
+  const float* ap[RW];                                     // lane l splits values 8 (l % 16) .. + 7 of a batch, of rows l / 16 + 4 r
+#pragma unroll
+  for (int r = 0; r < RW; ++r) ap[r] = a + (size_t)min(kg + r * 4, M - 1) * lda + r16 * 8;
+  f32x4_t acc[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  struct Batch { bf16x8_t w[U][RT]; f32x4_t a[RW][2]; };
+  auto fetch = [&](Batch& x, int s) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) split_load<true>(ap[r], s * 32, K, x.a[r]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) x.w[u][i] = *reinterpret_cast<const bf16x8_t*>(wp[i] + (s + u) * 32);
+  };
+  const int row = r16 % (RW * 4);
+  auto add = [&](bf16x8_t (&wv)[RT], const bf16x8_t (&p)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if (q == 1) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) wv[i] = split_weight(wv[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], p[q], acc[i], 0, 0, 0);
+    }
+  };
+  auto take = [&](Batch& x) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+      const Split8 t = split_of(x.a[r]);
+      thirds[wave][0][kg + r * 4][r16] = t.p[0], thirds[wave][1][kg + r * 4][r16] = t.p[1], thirds[wave][2][kg + r * 4][r16] = t.p[2];
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bf16x8_t p[3] = {thirds[wave][0][row][u * 4 + kg], thirds[wave][1][row][u * 4 + kg], thirds[wave][2][row][u * 4 + kg]};
+      add(x.w[u], p);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  // two batches in turn: while the MFMAs of one run, the loads of the other are on their way
+  Batch x[2];
+  const int batches = (end - begin) / U;
+  if (batches > 0) fetch(x[0], begin);
+  int b = 0;
+  for (; b + 2 <= batches; b += 2) {
+    fetch(x[1], begin + (b + 1) * U);
+    take(x[0]);
+    if (b + 2 < batches) fetch(x[0], begin + (b + 2) * U);
+    take(x[1]);
+  }
+  if (b < batches) take(x[0]);
+  const float* const own = a + (size_t)min(r16, M - 1) * lda + kg * 8;
+  for (int s = begin + batches * U; s < end; ++s) {        // (steps that fill no batch: every lane its own)
+    f32x4_t v[2];
+    split_load<true>(own, s * 32, K, v);
+    bf16x8_t wv[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) wv[i] = *reinterpret_cast<const bf16x8_t*>(wp[i] + s * 32);
+    const Split8 t = split_of(v);
+    add(wv, t.p);
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) red[wave - 1][i][lane] = acc[i];
+  }
+  __syncthreads();
+  if (wave > 0 || r16 >= M) return;
+  const bool aligned = aligned4(c, ldc);
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+#pragma unroll
+    for (int q = 0; q < WK - 1; ++q) acc[i] += red[q][i][lane];
+    put4(c + (size_t)r16 * ldc, n0 + i * 16 + kg * 4, N, aligned, acc[i]);
   }
 }
 
@@ -310,6 +404,22 @@ static void launch_stream(const TA* a, const TW* w, TC* c, int M, int N, int K, 
   else if (M <= 32) ATOMA_STREAM(2);
   else ATOMA_STREAM(4);
 #undef ATOMA_STREAM
+}
+
+template <int RW, int RT, typename TC>
+static int launch_split_few(const float* a, const bf16_t* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
+  const dim3 grid(ceil_div(N, 16 * RT));
+  // (a wave a part of K)
+  if constexpr (RT == 1) {
+    if (f32_part_bits(N) == 3) {
+      hipLaunchKernelGGL((split_few_kernel<RW, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+      ATOMA_LAUNCH_CHECK();
+      return 0;
+    }
+  }
+  hipLaunchKernelGGL((split_few_kernel<RW, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
 }
 
 template <int MT, int RT, typename TC>
@@ -360,6 +470,16 @@ static int launch_split(const float* a, const bf16_t* w, TC* c, int M, int N, in
 #define ATOMA_STREAM(MT, RT) return launch_split_stream<MT, RT>(a, w, c, M, N, K, lda, ldw, ldc, stream)
   if (vec) {
     auto round = [&](int mt, int rt, int most) { return (int64_t)ceil_div(N, 16 * rt) * ceil_div(M, 16 * mt) <= most; };
+    // (up to eight rows the splitting is shared: 4 rows, 2,048 x 8,192 16.5 -> 11.4 us, 28,672 x 4,096 53 -> 41, the head of Llama 1B 101 -> 87;
+    // two blocks of the weight against one, 4 rows: 5,120 x 3,072 9.3 and 10.0, 28,672 x 4,096 43.6 and 41.1)
+#define ATOMA_FEW(RW, RT) return launch_split_few<RW, RT>(a, w, c, M, N, K, lda, ldw, ldc, stream)
+    if (M <= 4) {
+      if (!wide || (N > 16384 && N < 65536)) ATOMA_FEW(1, 1);
+      ATOMA_FEW(1, 2);
+    }
+    if (M <= 8 && wide) ATOMA_FEW(2, 2);
+    if (M <= 8 && (M > 6 || K > 4096)) ATOMA_FEW(2, 1);      // (5 rows, 2,048 x 2,048: 6.0 against 5.5 by the kernel below)
+#undef ATOMA_FEW
     if (!wide) {
       if (round(1, 1, kCUs)) ATOMA_STREAM(1, 1);
       if (M <= 20 && round(2, 1, kCUs)) ATOMA_STREAM(2, 1);
@@ -367,9 +487,7 @@ static int launch_split(const float* a, const bf16_t* w, TC* c, int M, int N, in
       if (round(2, 2, 320)) ATOMA_STREAM(2, 2);
       if (round(4, 2, kCUs)) ATOMA_STREAM(4, 2);
     } else if (M <= 16) {
-      // (what a wave splits of A weighs less the fewer rows there are: 1 row, 28,672 x 4,096: one block 44.9 us, four 49.0; 16 rows 78 and 58)
-      if (M <= 4 && N <= (M == 1 ? 32768 : 8192)) ATOMA_STREAM(1, 1);
-      if (N <= 8192 || (M <= 4 && N > 32768)) ATOMA_STREAM(1, 2);
+      if (N <= 8192) ATOMA_STREAM(1, 2);      // (16 rows, 8,192 x 4,096: 18.8 us, 26.9 by four blocks; 28,672 x 4,096: 65.7 and 57.8)
       ATOMA_STREAM(1, 4);
     } else {
       if (round(2, 2, kCUs)) ATOMA_STREAM(2, 2);

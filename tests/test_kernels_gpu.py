@@ -147,7 +147,8 @@ def test_gemm_generic_row_alone(n, k, wdt):
 @pytest.mark.parametrize("m,n,k", [(16, 48, 96), (20, 4000, 64), (48, 2050, 544), (65, 3000, 32), (130, 2500, 96), (300, 4090, 100),
                                    (1, 5000, 64), (1, 40000, 32), (5, 5003, 96), (7, 9000, 64), (17, 4112, 288), (33, 5120, 64),
                                    (70, 5200, 96), (130, 5100, 160), (140, 20000, 64), (1100, 8200, 352), (200, 130, 8192),
-                                   (70, 4100, 4096), (3, 4100, 4128)])
+                                   (70, 4100, 4096), (3, 4100, 4128), (3, 2050, 1696), (8, 1000, 1184), (4, 20000, 544), (5, 5003, 608),
+                                   (2, 70000, 544)])
 def test_gemm_float32_by_bfloat16_thirds(m, n, k):
     """float32 rows against a bfloat16 weight: every number of blocks a streaming workgroup takes, every tile, and both sides of the
     longest part of K that goes to the bfloat16 instruction.  The three numbers that a value is cut into hold all of it, so the bound is
