@@ -1,5 +1,8 @@
 // The numbers that a step's draws take, one per (request seed, counter): splitmix64's finaliser, 24 random bits in [0, 1),
 // as sampler.py: uniform() states them.
+//
+// And the parameters of a step's rows, from the plans' own packed form (params.py: SamplingPlan.packed): lists of attributes cost
+// 64 rows 10 us a step in Python, their numbers another 5, and the GPU waits for both.
 #include <cstdint>
 
 extern "C" void sampling_uniforms(const uint64_t* seeds, const uint64_t* counters, int n, float* out) {
@@ -10,4 +13,38 @@ extern "C" void sampling_uniforms(const uint64_t* seeds, const uint64_t* counter
     z ^= z >> 31;
     out[i] = (float)(z >> 40) * 0x1p-24f;
   }
+}
+
+namespace {
+struct PlanRow {               // as SamplingPlan.packed writes it
+  float temperature, top_p, penalty;
+  int32_t top_k;
+  uint64_t seed;
+  int32_t greedy, penalised;
+};
+static_assert(sizeof(PlanRow) == 32, "a plan's bytes");
+enum Found : int { kAllGreedy = 1, kPenalised = 2, kTopP = 4, kTopK = 8, kFewK = 16 };
+}  // namespace
+
+// meta [5][n]: temperature (0: greedy), top_p, uniform, penalty, top_k (int32 bits).  What the rows that draw ask for, as bits: a
+// top-p cut, a top-k cut, top-k cuts of at most few_max all of them.
+extern "C" int sampling_pack(const void* plans, const uint64_t* counters, int n, int few_max, float* meta) {
+  const PlanRow* const rows = static_cast<const PlanRow*>(plans);
+  int32_t* const top_k = reinterpret_cast<int32_t*>(meta + 4 * (long)n);
+  int found = kAllGreedy | kFewK;
+  for (int i = 0; i < n; ++i) {
+    const PlanRow& r = rows[i];
+    meta[i] = r.greedy ? 0.f : r.temperature;
+    meta[n + i] = r.top_p;
+    meta[3 * (long)n + i] = r.penalty;
+    top_k[i] = r.top_k;
+    sampling_uniforms(&r.seed, counters + i, 1, meta + 2 * (long)n + i);
+    if (r.penalised) found |= kPenalised;
+    if (r.greedy) continue;
+    found &= ~kAllGreedy;
+    if (r.top_p < 1.0f) found |= kTopP;
+    if (r.top_k > 0) found |= kTopK;
+    if (r.top_k <= 0 || r.top_k > few_max) found &= ~kFewK;
+  }
+  return found;
 }

@@ -1598,11 +1598,11 @@ def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
     s, v = logits.shape
     for name, x, dt in (("temperature", temperature, torch.float32), ("top_k", top_k, torch.int32),
                         ("top_p", top_p, torch.float32), ("uniform", uniform, torch.float32)):
-        _need(x.dtype is dt and x.is_contiguous() and x.numel() == s, f"{name} must be {dt} [S]")
-    if workspace is None:
-        workspace = torch.empty((s, v), dtype=torch.float32, device=logits.device)
-    _need(workspace.dtype is torch.float32 and workspace.is_contiguous() and workspace.numel() >= s * v,
-          "sample: workspace too small")
+        if not (x.dtype is dt and x.is_contiguous() and x.numel() == s):
+            _need(False, f"{name} must be {dt} [S]")
+    if workspace is not None:
+        _need(workspace.dtype is torch.float32 and workspace.is_contiguous() and workspace.numel() >= s * v,
+              "sample: workspace too small")
     out = torch.empty((2, s), dtype=torch.float32, device=logits.device)
     ld = logits.stride(0) if s > 1 else v
     if split and v <= SPLIT_MAX_VOCAB:
@@ -1613,15 +1613,18 @@ def sample_packed(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.
             i, ptr = ctypes.c_int, ctypes.c_void_p
             # (with the types of its arguments known, a call takes plain numbers: 8 us less a step)
             lib.atoma_sample_split.argtypes = [ptr, i, i, i] + [ptr] * 6 + [i, ptr, ptr, ptr]
-            _split = lib.atoma_sample_split, lib.atoma_sample_split_scratch_bytes
-        draw, scratch_bytes = _split
-        scratch = torch.empty((scratch_bytes(s) + 3) // 4, dtype=torch.int32, device=logits.device)
-        at = out.data_ptr()
+            _split = lib.atoma_sample_split, lib.atoma_sample_split_scratch_bytes(1)
+        draw, row_bytes = _split               # (a row's scratch: a multiple of 16 bytes)
+        scratch = torch.empty(row_bytes // 4 * s + (s * v if workspace is None else 0), dtype=torch.int32, device=logits.device)
+        at, scratch_at = out.data_ptr(), scratch.data_ptr()
+        weights_at = scratch_at + row_bytes * s if workspace is None else workspace.data_ptr()
         _check(draw(logits.data_ptr(), ld, s, v, temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), uniform.data_ptr(),
-                    workspace.data_ptr(), scratch.data_ptr(), (3 if top_p_cuts else 2) if few and cuts else 1 if cuts else 0,
+                    weights_at, scratch_at, (3 if top_p_cuts else 2) if few and cuts else 1 if cuts else 0,
                     at, at + 4 * s, _stream()),
                "sample (split)")
         return out
+    if workspace is None:
+        workspace = torch.empty((s, v), dtype=torch.float32, device=logits.device)
     _check(core().atoma_sample(_p(logits), ld, s, v, _p(temperature), _p(top_k),
                                _p(top_p), _p(uniform), _p(workspace), _p(out[0]), _p(out[1]), _stream()), "sample")
     return out

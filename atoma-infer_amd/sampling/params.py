@@ -11,9 +11,19 @@ validation.rs:358) that benchmarks need.
 from __future__ import annotations
 
 import dataclasses
+import functools
+import struct
 from typing import List, Optional
 
+import numpy as np
+
 DEFAULT_RANDOM_SEED = 1_283_768_955  # backends/vllm/src/validation.rs:11
+
+
+# a plan as the sampler's native packing reads it (csrc/host/uniforms.cpp: PlanRow)
+_PACKED = np.dtype([("temperature", "<f4"), ("top_p", "<f4"), ("penalty", "<f4"), ("top_k", "<i4"), ("seed", "<u8"), ("greedy", "<i4"),
+                    ("penalised", "<i4")])
+_PACK = struct.Struct("<fffiQii").pack
 
 
 class ValidationError(ValueError):
@@ -42,7 +52,7 @@ class GenerateParameters:
     ignore_eos_token: bool = False
 
 
-@dataclasses.dataclass(frozen=True)
+@dataclasses.dataclass(frozen=True, init=False)
 class SamplingPlan:
     """What the sampler needs for one request, after validation."""
     greedy: bool
@@ -56,6 +66,28 @@ class SamplingPlan:
     stop: tuple
     ignore_eos_token: bool
     return_full_text: bool
+
+    def __init__(self, greedy: bool, temperature: float, top_k: int, top_p: float, repetition_penalty: float, repeat_last_n: int,
+                 random_seed: int, max_new_tokens: int, stop: tuple, ignore_eos_token: bool, return_full_text: bool):
+        # (the fields in one go: with the packed form still quicker than a frozen dataclass's own, field by field)
+        own = self.__dict__
+        own.update(greedy=greedy, temperature=temperature, top_k=top_k, top_p=top_p, repetition_penalty=repetition_penalty,
+                   repeat_last_n=repeat_last_n, random_seed=random_seed, max_new_tokens=max_new_tokens, stop=stop,
+                   ignore_eos_token=ignore_eos_token, return_full_text=return_full_text)
+        try:
+            own["packed"] = _PACK(temperature, top_p, repetition_penalty, top_k, random_seed & 0xFFFFFFFFFFFFFFFF, greedy,
+                                  repetition_penalty != 1.0 and repeat_last_n > 0)
+        except (struct.error, OverflowError, TypeError):
+            pass              # (numbers beyond 32 bits: made below, if ever)
+
+    @functools.cached_property
+    def packed(self) -> bytes:
+        """What a step writes of this plan, as the sampler's native packing reads it; made once a plan."""
+        row = np.zeros((), _PACKED)
+        row["temperature"], row["top_p"], row["penalty"] = self.temperature, self.top_p, self.repetition_penalty
+        row["top_k"], row["seed"], row["greedy"] = np.array(self.top_k).astype(np.int32), int(self.random_seed) & (1 << 64) - 1, self.greedy
+        row["penalised"] = self.repetition_penalty != 1.0 and self.repeat_last_n > 0
+        return row.tobytes()
 
     @property
     def mode(self) -> str:

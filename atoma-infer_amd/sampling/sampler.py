@@ -40,7 +40,19 @@ def _native() -> ctypes.CDLL:
     lib = load_host_library()
     ptr = ctypes.c_void_p
     lib.sampling_uniforms.argtypes, lib.sampling_uniforms.restype = [ptr, ptr, ctypes.c_int, ptr], None
+    lib.sampling_pack.argtypes = [ctypes.c_char_p, ptr, ctypes.c_int, ctypes.c_int, ptr]
     return lib
+
+
+# what ``sampling_pack`` finds in a step's plans (csrc/host/uniforms.cpp: Found)
+_ALL_GREEDY, _PENALISED, _TOP_P, _TOP_K, _FEW_K = 1, 2, 4, 8, 16
+
+
+def _counters(steps: Sequence[int]) -> array:
+    try:
+        return array("q", steps)
+    except OverflowError:
+        return array("Q", [x & _MASK for x in steps])
 
 
 def write_uniforms(seeds: Sequence[int], counters: Sequence[int], address: int) -> None:
@@ -48,6 +60,23 @@ def write_uniforms(seeds: Sequence[int], counters: Sequence[int], address: int) 
     function above, more than the GPU on its draws."""
     s, c = array("Q", [x & _MASK for x in seeds]), array("Q", [x & _MASK for x in counters])
     _native().sampling_uniforms(s.buffer_info()[0], c.buffer_info()[0], len(s), address)
+
+
+def _found(plans: Sequence[SamplingPlan]) -> int:
+    """What ``sampling_pack`` finds, for the few rows that are written one by one."""
+    drawn = [pl for pl in plans if not pl.greedy]
+    found = 0 if drawn else _ALL_GREEDY
+    for pl in plans:
+        if pl.repetition_penalty != 1.0 and pl.repeat_last_n > 0:
+            found |= _PENALISED
+    few = True
+    for pl in drawn:
+        if pl.top_p < 1.0:
+            found |= _TOP_P
+        if pl.top_k > 0:
+            found |= _TOP_K
+        few = few and 0 < pl.top_k <= ops.FEW_MAX_K
+    return found | _FEW_K if few else found
 
 
 class Pending:
@@ -61,8 +90,8 @@ class Pending:
     def result(self) -> Tuple[List[int], List[float]]:
         """Wait for the copy and return (tokens, logits of the chosen tokens)."""
         self.event.synchronize()
-        n = self.tokens.numel()
-        got = self._host[0, :n].view(torch.int32).tolist(), self._host[1, :n].tolist()
+        host = self._host.numpy()
+        got = host[0].view(np.int32).tolist(), host[1].tolist()
         if self._pool is not None:            # the pinned buffer serves a later step
             self._pool.append(self._host)
             self._pool = None
@@ -86,6 +115,10 @@ class Sampler:
         host = pool.pop() if pool else torch.empty((2, s), dtype=torch.float32, pin_memory=True)
         return host, pool
 
+    def _meta_buffer(self, s: int):
+        pool = self._meta_pool.setdefault(s, [])
+        return pool, pool.pop() if pool else torch.empty((5, s), dtype=torch.float32, pin_memory=True)
+
     def launch(self, logits: torch.Tensor, plans: Sequence[SamplingPlan], steps: Sequence[int],
                contexts: Sequence[Sequence[int]]) -> Pending:
         """Start sampling one token per row of ``logits`` [S, V]; nothing waits for the GPU.
@@ -96,32 +129,39 @@ class Sampler:
         """
         s = logits.shape[0]
         assert len(plans) == s and len(steps) == s
+        meta_pool = meta = None
+        if s <= FEW_ROWS:
+            found = _found(plans)
+        else:
+            # one packed upload: temperature, top_p, uniform, penalty (float32) and top_k (int32 bits)
+            meta_pool, meta = self._meta_buffer(s)
+            counters = _counters(steps)
+            found = _native().sampling_pack(b"".join([pl.packed for pl in plans]), counters.buffer_info()[0], s, ops.FEW_MAX_K,
+                                            meta.data_ptr())
         pen_rows, pen_toks = [], []
-        penalties = [pl.repetition_penalty for pl in plans]
-        if penalties.count(1.0) < s:
+        if found & _PENALISED:
             for i, pl in enumerate(plans):
                 if pl.repetition_penalty != 1.0 and pl.repeat_last_n > 0:
                     uniq = set(contexts[i][-pl.repeat_last_n:])
                     pen_rows += [i] * len(uniq)
                     pen_toks += list(uniq)
         # rows that all take the largest logit need no parameters of their own: one upload per batch size, ever
-        all_greedy = not pen_rows and all(pl.greedy for pl in plans)
+        all_greedy = not pen_rows and bool(found & _ALL_GREEDY)
         if all_greedy and s in self._greedy_meta:
+            if meta is not None:
+                meta_pool.append(meta)
             m = self._greedy_meta[s]
-            out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2])
+            temperature, top_p, numbers, _, top_k = m.unbind(0)
+            out = ops.sample_packed(logits, temperature, top_k.view(torch.int32), top_p, numbers)
             host, pool = self._host_buffer(s)
             host.copy_(out, non_blocking=True)
             ev = torch.cuda.Event()
             ev.record()
-            return Pending(out[0].view(torch.int32), out[1], host, ev, pool)
-        # one packed upload: temperature, top_p, uniform, penalty (float32) and top_k (int32 bits)
-        meta_pool = self._meta_pool.setdefault(s, [])
-        meta = meta_pool.pop() if meta_pool else torch.empty((5, s), dtype=torch.float32, pin_memory=True)
-        mn = meta.numpy()
-        top_ks = top_ps = ()
-        if s > FEW_ROWS or logits.shape[1] >= SPLIT_MIN_VOCAB:
-            top_ks, top_ps = [pl.top_k for pl in plans], [pl.top_p for pl in plans]
-        if s <= FEW_ROWS:
+            tok, lg = out.unbind(0)
+            return Pending(tok.view(torch.int32), lg, host, ev, pool)
+        if meta is None:
+            meta_pool, meta = self._meta_buffer(s)
+            mn = meta.numpy()
             ints = mn[4].view(np.int32)
             for i, pl in enumerate(plans):
                 mn[0, i] = 0.0 if pl.greedy else pl.temperature
@@ -129,12 +169,6 @@ class Sampler:
                 mn[2, i] = 0.0 if pl.greedy else uniform(pl.random_seed, steps[i])
                 mn[3, i] = pl.repetition_penalty
                 ints[i] = pl.top_k
-        else:
-            mn[0] = [0.0 if pl.greedy else pl.temperature for pl in plans]
-            mn[1] = top_ps
-            mn[3] = penalties
-            mn[4].view(np.int32)[:] = top_ks
-            write_uniforms([pl.random_seed for pl in plans], steps, meta.data_ptr() + 8 * s)
         m = meta.to(self.device, non_blocking=True)
         if all_greedy:
             # (top_p, penalty and top_k of a greedy row are never read; the copy kept is this batch's)
@@ -145,18 +179,17 @@ class Sampler:
         # (rows that draw are shared by several blocks each: a block walks a row of a large vocabulary too slowly)
         how = {}
         if not all_greedy and logits.shape[1] >= SPLIT_MIN_VOCAB:
-            if any([pl.greedy for pl in plans]):          # (what a greedy row's parameters say has no say in this)
-                drawn = [i for i, pl in enumerate(plans) if not pl.greedy]
-                top_ks, top_ps = [top_ks[i] for i in drawn] or [0], [top_ps[i] for i in drawn] or [1.0]
-            cuts_p, least, most = min(top_ps) < 1.0, min(top_ks), max(top_ks)
-            how = dict(split=True, cuts=cuts_p or most > 0, few=0 < least and most <= ops.FEW_MAX_K, top_p_cuts=cuts_p)
-        out = ops.sample_packed(logits, m[0], m[4].view(torch.int32), m[1], m[2], **how)
-        tok, lg = out[0].view(torch.int32), out[1]
+            # (what a greedy row's parameters say has no say in this)
+            cuts_p = bool(found & _TOP_P)
+            how = dict(split=True, cuts=cuts_p or bool(found & _TOP_K), few=bool(found & _FEW_K), top_p_cuts=cuts_p)
+        temperature, top_p, numbers, _, top_k = m.unbind(0)
+        out = ops.sample_packed(logits, temperature, top_k.view(torch.int32), top_p, numbers, **how)
+        tok, lg = out.unbind(0)
         host, pool = self._host_buffer(s)
         host.copy_(out, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
-        pending = Pending(tok, lg, host, ev, pool)
+        pending = Pending(tok.view(torch.int32), lg, host, ev, pool)
         # (pinned memory must outlive the copy that reads it; a greedy batch's copy is kept, and its buffer with it)
         pending._meta, pending._meta_pool = meta, (None if all_greedy else meta_pool)
         return pending

@@ -63,3 +63,32 @@ def test_a_steps_uniform_numbers_written_natively_are_the_functions():
     got = (ctypes.c_float * len(seeds))()
     write_uniforms(seeds, counters, ctypes.addressof(got))
     assert list(got) == [uniform(s, c) for s, c in zip(seeds, counters)]
+
+
+def test_a_steps_parameters_packed_natively_are_the_plans():
+    """What the native packing writes and finds against the plans' own attributes, over greedy rows, cuts on both sides of the lists'
+    largest, penalties and seeds beyond 64 bits."""
+    import random
+
+    import numpy as np
+    import torch
+
+    from atoma_infer_amd.kernels import ops
+    from atoma_infer_amd.sampling import sampler
+    pick = random.Random(5)
+    for rows in (1, 5, 64, 65):
+        for _ in range(40):
+            plans = [validate(GenerateParameters(do_sample=pick.random() < 0.7, temperature=pick.choice([None, 0.7, 1.0, 2.0]),
+                                                 top_k=pick.choice([None, 1, 128, 129]), top_p=pick.choice([None, 0.3]),
+                                                 random_seed=pick.choice([None, -5, 2 ** 64 + 7, pick.randrange(2 ** 64)]),
+                                                 repetition_penalty=pick.choice([None, None, 1.3]), repeat_last_n=4,
+                                                 max_new_tokens=4), 3, 100, 200) for _ in range(rows)]
+            steps = [pick.randrange(1000) for _ in plans]
+            meta, counters = torch.zeros(5, rows), sampler._counters(steps)
+            found = sampler._native().sampling_pack(b"".join([p.packed for p in plans]), counters.buffer_info()[0], rows,
+                                                    ops.FEW_MAX_K, meta.data_ptr())
+            assert found == sampler._found(plans)
+            want = np.array([[0.0 if p.greedy else p.temperature for p in plans], [p.top_p for p in plans],
+                             [uniform(p.random_seed, c) for p, c in zip(plans, steps)],
+                             [p.repetition_penalty for p in plans]], np.float32)
+            assert (meta.numpy()[:4] == want).all() and meta.numpy()[4].view(np.int32).tolist() == [p.top_k for p in plans]
