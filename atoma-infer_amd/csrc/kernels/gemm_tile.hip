@@ -22,6 +22,8 @@
 // bfloat16, or q rotated in bfloat16 and k, v in the paged cache.
 //
 // Needs K % 64 == 0, N % 16 == 0 and 16-byte aligned rows; the host wrapper checks and otherwise refuses.
+#include <type_traits>
+
 #include "common.h"
 #include "rope_store.h"
 
@@ -240,6 +242,57 @@ __device__ __forceinline__ void meet() {
 }
 #endif
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// What leaves of row m: NB blocks of 16 columns from column nw on, of which this lane has columns 4 kg .. + 3.
+template <int EPI, bool GROUPED, int NB>
+__device__ __forceinline__ void put_row(const f32x4 (&v)[NB], int m, int nw, int N, int kg, const TileOut& out, const Groups& groups) {
+  size_t to_row = 0;
+  float to_scale = 1.f;
+  if constexpr (EPI == kOutF32 && GROUPED) {
+    const int slot = groups.perm[m];
+    to_row = (size_t)(slot % groups.top) * groups.plane_rows + slot / groups.top;
+    if (groups.scale) to_scale = groups.scale[slot];
+  }
+  if constexpr (EPI == kOutSilu) {
+    uint16_t* const row = (uint16_t*)out.c + (size_t)m * out.ldc;
+#pragma unroll
+    for (int i = 0; i + 1 < NB; i += 2) {         // blocks of 16 gate rows, then the 16 up rows of the same outputs
+      if (nw + i * 16 >= N) continue;
+      const int n = (nw + i * 16) / 2 + kg * 4;
+      uint2 r;
+      __bf16* const o = reinterpret_cast<__bf16*>(&r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (__bf16)silu_times(v[i][e], v[i + 1][e]);
+      *reinterpret_cast<uint2*>(row + n) = r;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int n = nw + i * 16 + kg * 4;
+      if (nw + i * 16 >= N) continue;                // (N is a multiple of 16: a block is there or is not)
+      if constexpr (EPI == kOutF32 && GROUPED) {
+        *reinterpret_cast<f32x4*>((float*)out.c + to_row * out.ldc + n) = v[i] * to_scale;
+      } else if constexpr (EPI == kOutF32) {
+        *reinterpret_cast<f32x4*>((float*)out.c + blockIdx.y * out.plane + (size_t)m * out.ldc + n) = v[i];
+      } else {
+        f32x4* const p = reinterpret_cast<f32x4*>((float*)out.c + (size_t)m * out.ldc + n);
+        *p = *p + v[i];
+      }
+    }
+  }
+}
+
+// The workgroup's tile: this XCD's run of the order, patches of kPatch rows of tiles, column by column.
+template <typename C>
+__device__ __forceinline__ void tile_of(int rows, int N, int& mi, int& n0) {
+  const int mt = (rows + C::BM - 1) / C::BM, nt = (N + C::BN - 1) / C::BN;
+  const int share = (mt * nt) >> 3, rest = (mt * nt) & 7, xcd = blockIdx.x & 7;
+  const int id = xcd * share + min(xcd, rest) + (blockIdx.x >> 3);
+  const int patch = id / (kPatch * nt), pm = min(kPatch, mt - patch * kPatch), in = id - patch * kPatch * nt;
+  mi = patch * kPatch + in % pm, n0 = (in / pm) * C::BN;
+}
+#endif
+
 // (rows: M of X, or the entries of the groups' list times BM)
 template <typename C, int EPI, bool GROUPED>
 __global__ void __launch_bounds__(64 * C::NW, C::NW >= 8 ? 2 : 1)
@@ -249,12 +302,8 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
-  // the tile: this XCD's run of the order, patches of kPatch rows of tiles, column by column
-  const int mt = (rows + C::BM - 1) / C::BM, nt = (N + C::BN - 1) / C::BN;
-  const int share = (mt * nt) >> 3, rest = (mt * nt) & 7, xcd = blockIdx.x & 7;
-  const int id = xcd * share + min(xcd, rest) + (blockIdx.x >> 3);
-  const int patch = id / (kPatch * nt), pm = min(kPatch, mt - patch * kPatch), in = id - patch * kPatch * nt;
-  const int mi = patch * kPatch + in % pm, n0 = (in / pm) * C::BN;
+  int mi, n0;
+  tile_of<C>(rows, N, mi, n0);
   const int k0 = blockIdx.y * k_len;
   int m0 = mi * C::BM, M = rows;
   if constexpr (GROUPED) {
@@ -340,47 +389,208 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 #pragma unroll
   for (int j = 0; j < C::TM; ++j) {
     const int m = m0 + wm * (C::BM / C::WM) + j * 16 + r16;
-    const int nw = n0 + wn * (C::BN / C::WN);
     if (m >= M) continue;
-    size_t to_row = 0;
-    float to_scale = 1.f;
-    if constexpr (EPI == kOutF32 && GROUPED) {
-      const int slot = groups.perm[m];
-      to_row = (size_t)(slot % groups.top) * groups.plane_rows + slot / groups.top;
-      if (groups.scale) to_scale = groups.scale[slot];
-    }
-    if constexpr (EPI == kOutSilu) {
-      uint16_t* const row = (uint16_t*)out.c + (size_t)m * out.ldc;
+    f32x4 v[C::TN];
 #pragma unroll
-      for (int i = 0; i + 1 < C::TN; i += 2) {         // blocks of 16 gate rows, then the 16 up rows of the same outputs
-        if (nw + i * 16 >= N) continue;
-        const int n = (nw + i * 16) / 2 + kg * 4;
-        uint2 v;
-        __bf16* const o = reinterpret_cast<__bf16*>(&v);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (__bf16)silu_times(acc[i][j][e], acc[i + 1][j][e]);
-        *reinterpret_cast<uint2*>(row + n) = v;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < C::TN; ++i) {
-        const int n = nw + i * 16 + kg * 4;
-        if (nw + i * 16 >= N) continue;                // (N is a multiple of 16: a block is there or is not)
-        const f32x4 v = acc[i][j];
-        if constexpr (EPI == kOutF32 && GROUPED) {
-          *reinterpret_cast<f32x4*>((float*)out.c + to_row * out.ldc + n) = v * to_scale;
-        } else if constexpr (EPI == kOutF32) {
-          *reinterpret_cast<f32x4*>((float*)out.c + blockIdx.y * out.plane + (size_t)m * out.ldc + n) = v;
-        } else {
-          f32x4* const p = reinterpret_cast<f32x4*>((float*)out.c + (size_t)m * out.ldc + n);
-          *p = *p + v;
-        }
-      }
-    }
+    for (int i = 0; i < C::TN; ++i) v[i] = acc[i][j];
+    put_row<EPI, GROUPED>(v, m, n0 + wn * (C::BN / C::WN), N, kg, out, groups);
   }
 #endif
 }
 
+// ---- tiles of 256 x 256 ---------------------------------------------------------------------------------------------------
+// With one barrier a step a buffer is free, and the loads for the step after next can start, only when all of its fragments have been
+// read, and those loads must be there a step later: 64 KB of a burst and the latency behind it, 1.27 us a step on their own, about what
+// a step's MFMAs take.  Here a step is multiplied in four phases, half of X's rows by half of W's at a time, and a phase's fragments
+// are read under the MFMAs of the one before:
+//   X0 W0 (W1 is read), X0 W1 (X1), X1 W1 (the next step's X0, into the registers of this one's), X1 W0 (its W0, into W1's)
+// So X0 and W0 of a step are read before the step begins, W1 and X1 by its middle, and with a barrier at either place the halves are
+// loaded anew a step and a half before they are read again, 32 KB at a time: the loads alone take 0.95 us a step.
+// us, before / now: gate-up with SiLU, 2,048 rows against 16,384 x 2,048 116 / 111, 16,384 x 3,072 164 / 156, 28,672 x 4,096 391 / 370;
+// float32 sums of 8,192^3 800 / 763.  What is left is power: the MFMAs alone would take 555 of the 763 and the loads alone 486, with all of them
+// served by the L2 the product still takes 735, and the clock is at 1.85 GHz; priorities for the MFMAs (s_setprio) cost 2 %.
+template <int BM_, int BN_, int WM_, int WN_>
+struct Phased {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM * WN;
+  static constexpr int XH = BM / 2, WH = BN / 2;                              // rows of a half
+  static constexpr int JX = XH / WM / 16, JW = WH / WN / 16;                  // blocks of 16 of a wave in a half
+  static constexpr int QX = XH / 8, XI = (QX + NW - 1) / NW;                  // loads of eight rows: a half's, a wave's
+  static constexpr int QW = WH / 8, WI = (QW + NW - 1) / NW;
+  static constexpr int PAIR = XI + WI;                                        // of a wave for a half of X and one of W
+  static constexpr int X0 = 0, X1 = XH * 128, W0 = BM * 128, W1 = W0 + WH * 128;      // bytes: the halves of a buffer
+  static constexpr int BUF = (BM + BN) * 128, LDS = 2 * BUF;
+  static_assert(XH % (16 * WM) == 0 && WH % (16 * WN) == 0 && LDS <= 160 * 1024 && 4 * PAIR < 64, "");
+};
+
+#if defined(__HIP_DEVICE_COMPILE__)
+template <int NB>
+__device__ __forceinline__ void read_half(const char* __restrict__ p, uint32_t row, int lane, bf16x8 (&f)[NB][2]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t col = (uint32_t)((h * 4 + (lane >> 4)) ^ (lane & 7)) * 16;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) f[i][h] = *reinterpret_cast<const bf16x8*>(p + row + i * 2048 + col);
+  }
+}
+// READS reads of LDS spread over the MFMAs
+template <int READS, int JW, int JX>
+__device__ __forceinline__ void phase(const bf16x8 (&w)[JW][2], const bf16x8 (&x)[JX][2], f32x4 (&acc)[JW][JX]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < JX; ++j)
+#pragma unroll
+      for (int i = 0; i < JW; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][h], x[j][h], acc[i][j], 0, 0, 0);
+  constexpr int all = 2 * JW * JX, per = all / READS > 0 ? all / READS : 1;
+#pragma unroll
+  for (int i = 0; i < READS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, per, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(0x8, all, 0);
+  __builtin_amdgcn_sched_barrier(0);
+}
+#endif
+
+// Two steps or more; ODD: their number is (a kernel that takes either spills registers).
+template <typename C, int EPI, bool GROUPED, bool ODD>
+__global__ void __launch_bounds__(64 * C::NW, 2)
+gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int rows, int N, int ldx, int ldw, int k_len,
+                   TileOut out, Groups groups) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, kg = lane >> 4;
+  int mi, n0;
+  tile_of<C>(rows, N, mi, n0);
+  const int k0 = blockIdx.y * k_len;
+  int m0 = mi * C::BM, M = rows;
+  if constexpr (GROUPED) {
+    const int g = groups.tiles[2 * mi];
+    if (g < 0) return;
+    m0 = groups.tiles[2 * mi + 1], M = groups.offsets[g + 1];
+    w += (size_t)g * N * ldw;
+  }
+  const int rows_x = min(C::BM, M - m0), rows_w = min(C::BN, N - n0);
+  // a half's rows through a buffer of its own: what lies past the last row is out of its range, reads as zero and is never stored
+  const int lr = lane >> 3;
+  const uint32_t piece = ((lane & 7) ^ lr) * 16;
+  uint32_t xo[C::XI], wo[C::WI];
+#pragma unroll
+  for (int i = 0; i < C::XI; ++i) xo[i] = (uint32_t)(min(i * C::NW + wave, C::QX - 1) * 8 + lr) * ldx * 2 + piece;
+#pragma unroll
+  for (int i = 0; i < C::WI; ++i) wo[i] = (uint32_t)(min(i * C::NW + wave, C::QW - 1) * 8 + lr) * ldw * 2 + piece;
+  auto half = [&](const uint16_t* p, int ld, int there) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, there <= 0 ? 0 : ((there - 1) * ld + k_len) * 2, 0x00027000);
+  };
+  const uint16_t* const xp = x + (size_t)m0 * ldx + k0;
+  const uint16_t* const wp = w + (size_t)n0 * ldw + k0;
+  const rsrc_t xb0 = half(xp, ldx, min(rows_x, C::XH)), xb1 = half(xp + (size_t)C::XH * ldx, ldx, rows_x - C::XH);
+  const rsrc_t wb0 = half(wp, ldw, min(rows_w, C::WH)), wb1 = half(wp + (size_t)C::WH * ldw, ldw, rows_w - C::WH);
+
+  f32x4 acc[2][2][C::JW][C::JX];          // by half of W, half of X
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < C::JW; ++i)
+#pragma unroll
+        for (int j = 0; j < C::JX; ++j) acc[g][h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const uint32_t xr = (wm * (C::XH / C::WM) + r16) * 128, wr = (wn * (C::WH / C::WN) + r16) * 128;
+
+  const int steps = k_len / 64;
+  auto load_first = [&](char* __restrict__ buf, int s) {
+    issue<C::QX, C::XI, C::NW>(buf + C::X0, xb0, s * 128, xo, wave);
+    issue<C::QW, C::WI, C::NW>(buf + C::W0, wb0, s * 128, wo, wave);
+  };
+  auto load_second = [&](char* __restrict__ buf, int s) {
+    issue<C::QW, C::WI, C::NW>(buf + C::W1, wb1, s * 128, wo, wave);
+    issue<C::QX, C::XI, C::NW>(buf + C::X1, xb1, s * 128, xo, wave);
+  };
+  char* const b0 = lds;
+  char* const b1 = lds + C::BUF;
+  load_first(b0, 0);
+  load_second(b0, 0);
+  load_first(b1, 1);
+  load_second(b1, 1);
+  wait<3 * C::PAIR, false>();
+  meet();
+  bf16x8 fx0[C::JX][2], fx1[C::JX][2], fa[C::JW][2], fb[C::JW][2];
+  read_half(b0 + C::X0, xr, lane, fx0);
+  read_half(b0 + C::W0, wr, lane, fa);
+  // Step s, whose X0 and W0 are in fx0 and w0.  REST: how many steps are behind it (2: two or more).  (now and own are the same buffer,
+  // then the other one: that they promise not to overlap keeps the compiler from waiting for the loads before the reads.)
+  auto step = [&](auto rest, int s, const char* __restrict__ now, char* __restrict__ own, const char* __restrict__ then,
+                  bf16x8 (&w0)[C::JW][2], bf16x8 (&w1)[C::JW][2]) {
+    constexpr int REST = decltype(rest)::value;
+    // everybody has read X0 and W0, and this step's W1 and X1 have landed
+    if constexpr (REST > 0) wait<2 * C::PAIR, true>();
+    else wait<0, true>();
+    meet();
+    read_half(now + C::W1, wr, lane, w1);
+    if constexpr (REST == 2) load_first(own, s + 2);
+    phase<2 * C::JW>(w0, fx0, acc[0][0]);
+    read_half(now + C::X1, xr, lane, fx1);
+    phase<2 * C::JX>(w1, fx0, acc[1][0]);
+    // everybody has read W1 and X1, and the next step's X0 and W0 have landed
+    if constexpr (REST > 0) {
+      wait<(REST == 2 ? 2 : 1) * C::PAIR, true>();
+      meet();
+      read_half(then + C::X0, xr, lane, fx0);
+    }
+    if constexpr (REST == 2) load_second(own, s + 2);
+    phase<2 * C::JX>(w1, fx1, acc[1][1]);
+    if constexpr (REST > 0) read_half(then + C::W0, wr, lane, w1);
+    phase<2 * C::JW>(w0, fx1, acc[0][1]);
+  };
+  constexpr std::integral_constant<int, 0> none{};
+  constexpr std::integral_constant<int, 1> one{};
+  constexpr std::integral_constant<int, 2> more{};
+  int s = 0;
+  for (; s + 2 + ODD < steps; s += 2) {
+    step(more, s, b0, b0, b1, fa, fb);
+    step(more, s + 1, b1, b1, b0, fb, fa);
+  }
+  if constexpr (ODD) {
+    step(more, s, b0, b0, b1, fa, fb);
+    step(one, s + 1, b1, b1, b0, fb, fa);
+    step(none, s + 2, b0, b0, b1, fa, fb);
+  } else {
+    step(one, s, b0, b0, b1, fa, fb);
+    step(none, s + 1, b1, b1, b0, fb, fa);
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < C::JX; ++j) {
+      const int m = m0 + h * C::XH + wm * (C::XH / C::WM) + j * 16 + r16;
+      if (m >= M) continue;
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        f32x4 v[C::JW];
+#pragma unroll
+        for (int i = 0; i < C::JW; ++i) v[i] = acc[g][h][i][j];
+        put_row<EPI, GROUPED>(v, m, n0 + g * C::WH + wn * (C::WH / C::WN), N, kg, out, groups);
+      }
+    }
+#endif
+}
+
+template <typename C, int EPI, bool GROUPED, bool ODD>
+static int launch_phased(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
+                         hipStream_t stream, const Groups& groups) {
+  // (every device that the kernel is launched on has its own setting)
+  const hipError_t e = hipFuncSetAttribute((const void*)gemm_phased_kernel<C, EPI, GROUPED, ODD>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+  if (e != hipSuccess) return (int)e;
+  const int64_t tiles = (int64_t)((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
+  if (tiles > 0x7fffffff) return ATOMA_ERR_SHAPE;
+  hipLaunchKernelGGL((gemm_phased_kernel<C, EPI, GROUPED, ODD>), dim3((int)tiles, slices), dim3(64 * C::NW), C::LDS, stream,
+                     (const uint16_t*)x, (const uint16_t*)w, M, N, ldx, ldw, K / slices, out, groups);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
 template <typename C, int EPI, bool GROUPED = false>
 static int launch(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
                   hipStream_t stream, const Groups& groups = Groups{}) {
@@ -396,6 +606,16 @@ static int launch(const void* x, const void* w, int M, int N, int K, int ldx, in
   return 0;
 }
 
+// (one step: by tiles of as many rows and half the columns)
+template <typename C, int EPI, bool GROUPED = false>
+static int launch_phased(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
+                         hipStream_t stream, const Groups& groups = Groups{}) {
+  const int steps = K / slices / 64;
+  if (steps == 1) return launch<Tile<256, 128, 4, 2, 3>, EPI, GROUPED>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups);
+  return steps % 2 ? launch_phased<C, EPI, GROUPED, true>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups)
+                   : launch_phased<C, EPI, GROUPED, false>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups);
+}
+
 template <int EPI>
 static int pick(int tile, const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
                 hipStream_t stream) {
@@ -403,7 +623,10 @@ static int pick(int tile, const void* x, const void* w, int M, int N, int K, int
   (void)GATED;
 #define ATOMA_TILE(...) return launch<Tile<__VA_ARGS__>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream)
   switch (tile) {
-    case 0: if constexpr (EPI != kOutRope) ATOMA_TILE(256, 256, 2, 4, 2); break;      // (its sums do not fit LDS)
+    case 0:
+      if constexpr (EPI != kOutRope)                  // (its sums do not fit LDS)
+        return launch_phased<Phased<256, 256, 2, 4>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream);
+      break;
     case 1: ATOMA_TILE(256, 128, 4, 2, 3);
     case 2: ATOMA_TILE(128, 128, 2, 4, 4);
     case 3: ATOMA_TILE(128, 64, 2, 2, 4);
@@ -467,7 +690,12 @@ extern "C" int atoma_gemm_tile_groups(const void* x, const void* w, void* c, int
       return launch<Tile<BM, __VA_ARGS__>, kOutF32, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);      \
   } while (0)
   switch (tile) {
-    case 0: ATOMA_TILE(256, 256, 2, 4, 2); break;
+    case 0:
+      if (kind == kOutSilu)
+        return launch_phased<Phased<256, 256, 2, 4>, kOutSilu, true>(x, w, max_tiles * 256, N, K, K, K, 1, out, stream, groups);
+      if (kind == kOutF32)
+        return launch_phased<Phased<256, 256, 2, 4>, kOutF32, true>(x, w, max_tiles * 256, N, K, K, K, 1, out, stream, groups);
+      break;
     case 1: ATOMA_TILE(256, 128, 4, 2, 3); break;
     case 2: ATOMA_TILE(128, 128, 2, 4, 4); break;
     case 3: ATOMA_TILE(128, 64, 2, 2, 4); break;

@@ -982,6 +982,29 @@ def test_gemm_tile(tile, m, n, k):
         assert bool(((c.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (128, 128, 128), (129, 160, 192), (255, 96, 256), (385, 416, 320), (513, 800, 448), (300, 272, 640)])
+def test_gemm_tile_in_phases_equals_the_one_by_steps(m, n, k):
+    """The tiles of 256 x 256 sum in the order of the others, so the bits are theirs: 1 to 7 and 10 steps, in slices too (5 steps), with rows
+    that end in a tile's first or second half."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    for slices in (1, 2):
+        if k % (64 * slices) == 0:
+            c = torch.full((2, slices, m, n), 7.0, device=DEV)
+            for i in range(2):
+                gb.tile_product(x, w, c[i], gb.TILE_F32, i, slices)
+            assert torch.equal(c[0], c[1])
+    r = rnd(m, n, seed=3)[None].repeat(2, 1, 1)
+    for i in range(2):
+        gb.tile_product(x, w, r[i], gb.TILE_RESID, i)
+    assert torch.equal(r[0], r[1])
+    if n % 32 == 0:
+        g = torch.empty(2, m, n // 2, dtype=torch.bfloat16, device=DEV)
+        for i in range(2):
+            gb.tile_product(x, w, g[i], gb.TILE_SILU, i)
+        assert torch.equal(g[0], g[1])
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 32, 128), (41, 80, 192), (63, 544, 512), (64, 1056, 1024), (64, 2048, 8192), (1, 64, 128)])
 def test_gemm_tile_of_64_rows(m, n, k):
     """The tiles for 33 to 64 rows, as test_gemm_tile holds the others; then what parts call with as many rows: 41 and more leave the
