@@ -10,7 +10,7 @@
 //   delta_scan         per (request, head, 8 or 16 columns of S): the recurrence over the entry's tokens in order, S read
 //                      from the request's state slot before and written back after.  A column of S lives in the registers
 //                      of 32 or 16 neighbouring lanes, so a token costs a lane a dozen or two multiply-adds and one
-//                      exchange of four or five steps among those lanes; the tokens' inputs pass LDS in blocks, fetched a
+//                      exchange of four or six steps among those lanes; the tokens' inputs pass LDS in blocks, fetched a
 //                      block ahead;
 //   delta_out          per token and head: o / sqrt(mean(o^2) + eps) * w * sigmoid(gate), in the activation dtype.
 // The order of every sum depends on the sizes alone, so from the same projections a token's result does not depend on how
@@ -18,6 +18,8 @@
 // bfloat16 come from a kernel that the step's row count chooses.)
 //
 // State of a request (float32, one row of the state tensor):  [taps - 1][conv channels]  then  [heads][vdim][dim].
+#include <algorithm>
+
 #include "gemm_f32_tile.h"
 
 using namespace atoma;
@@ -134,82 +136,153 @@ __device__ __forceinline__ float column_sum(const float (&x)[1]) {
 template <int LANES>
 __device__ __forceinline__ float column_sum(const float (&x)[2]) { return row_sum(x[0] + x[1]); }
 
+// d1, d2: a column's sums of x1 and x2.  Where a column has two rows of 16 lanes, the swap that adds their neighbours (what a lane of 16
+// adds by itself) leaves x1 in the first row and x2 in the second, so that the other four steps serve both.
+template <int LANES, int G>
+__device__ __forceinline__ void column_sums(const float (&x1)[G], const float (&x2)[G], float& d1, float& d2) {
+  if constexpr (LANES == 32) {
+    const auto half = __builtin_amdgcn_permlane16_swap(__float_as_uint(x1[0]), __float_as_uint(x2[0]), false, false);
+    const uint32_t y = __float_as_uint(row_sum(__uint_as_float(half[0]) + __uint_as_float(half[1])));
+    const auto both = __builtin_amdgcn_permlane16_swap(y, y, false, false);
+    d1 = __uint_as_float(both[0]), d2 = __uint_as_float(both[1]);
+  } else {
+    d1 = column_sum<LANES>(x1), d2 = column_sum<LANES>(x2);
+  }
+}
+
 // LANES (32 or 16) lanes share a column of S and hold G groups of R rows of it each, up to dim rows; a workgroup of four
 // waves holds COLS columns.  The tokens' q, k, decay (for the head), v (for the columns), beta and k . q pass LDS in blocks
-// of TB tokens: the next block is fetched from memory while this one is worked on, and the next token's rows are read from
-// LDS while this one's are worked on.
-// Bound by a wave's instructions for a token, one after the other, and where the workgroups fill the CUs by all of them, of
-// which 16 lanes a column have fewer (half the exchanges and loads of v, beta and k . q).  So 16 lanes, with two exceptions:
-// dim beyond 128, whose rows then fill the registers (256 x 256, 8 heads, 300 tokens: 157 us against 93 with 32 lanes, with
-// eight such entries 534 against 409); and dim beyond 64 where an entry has fewer than 16 tokens on average, whose time is
-// that of fetching the state (128 x 128, 8 heads, 8 / 64 decoded tokens 8.8 / 40.6 against 7.7 / 33.3).  Elsewhere
-// (128 x 128, 8 heads) one entry of 300 tokens takes 67 us, 71 with 32 lanes, eight 92 and 139; 64 x 64, 64 decoded tokens
-// 9.2 and 11.4.  The sums are the same bits either way.
+// of TB tokens: the next block is fetched from memory while this one is worked on, W values at a time (4 where dim allows it), and the
+// next token's rows are read from LDS while this one's are worked on.
+// Bound by a wave's instructions for a token, one after the other, and where the workgroups fill the CUs by all of them.  So a whole
+// block is written out with every place in LDS a constant, and a lane keeps the output of one of its tokens for one store at the end: 36
+// instructions a token with 32 lanes a column, where addresses, a branch and a store for each were as many as the arithmetic.
+// us, before / now: one entry of 2,048 tokens, 8 heads of 128 x 128 433 / 248, of 64 x 64 339 / 206, of 256 x 128 593 / 407; 300
+// tokens of 128 x 128 67 / 40, eight entries of 256 76 / 63; 8 and 64 single tokens beside each other 6.0 / 4.5 and 30.7 / 18.6 (their time
+// is that of the state's way, four values a load where dim and the row allow it).
+// 16 lanes a column need fewer instructions in all, 32 fewer in a row.  dim beyond 128 takes 32, whose rows would fill the registers
+// otherwise; dim from 65 on takes 32 for entries long enough to leave CUs idle else (scan_wide); up to 64 rows 32 lanes give 2 percent to
+// such entries and take up to 40 from others, so they take 16.  The sums are the same bits either way.
+
+struct ScanArgs {
+  const float *qn, *kn, *vn, *beta, *decay, *kq;
+  DeltaShape sh;
+  const int32_t *q_start, *state_slots;
+  float* state;
+  size_t state_stride, s_offset;
+  float* o;
+  int n_tokens;
+};
+
+// An entry's columns take 32 lanes each where as many workgroups as the step's tokens would make of such entries are about one a CU or fewer
+// (a sixteenth more leaves an entry beside single tokens in).  us with 32 / 16 lanes, heads of 128 x 128: 8 heads, one entry of 2,048 (128
+// workgroups) 249 / 300, the same beside 63 single tokens 242 / 294, two of 1,024 (256) 128 / 151; 16 heads, 2,041 tokens and seven single ones
+// (257) 251 / 303.  Beyond: 12 heads, 1,400 and 640 tokens (280) 211 / 208; 16 heads, the same (373) 213 / 209; 8 heads, three of 682 (384)
+// 107 / 103, four of 512 82 / 78.  (Some counts there leave 16 lanes the worse split, 12 heads, four of 512 107 / 119, but no rule tells them.)
+constexpr int kScanGroups = 272;
+__host__ __device__ __forceinline__ bool scan_wide(const DeltaShape& sh, int count, int n_tokens) {
+  return (int64_t)sh.heads * ((sh.vdim + 7) / 8) * n_tokens <= (int64_t)kScanGroups * count;
+}
 template <int R, int G, int LANES>
-__global__ void __launch_bounds__(256)
-delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vn,
-                  const float* __restrict__ beta, const float* __restrict__ decay, const float* __restrict__ kq,
-                  DeltaShape sh, const int32_t* __restrict__ q_start, const int32_t* __restrict__ state_slots,
-                  float* __restrict__ state, size_t state_stride, size_t s_offset, float* __restrict__ o) {
-  constexpr int DP = LANES * G * R;            // dim rounded up; rows beyond dim hold zeros
-  constexpr int TB = R <= 4 ? 16 : 8;          // tokens a block
-  constexpr int COLS = 256 / LANES;
-  constexpr int PER = TB * DP / 256;           // elements of q (k, decay) a thread fetches a block
-  __shared__ __attribute__((aligned(16))) float sq[2][TB][DP], sk[2][TB][DP], sg[2][TB][DP];
-  __shared__ float sv[2][TB][COLS], sb[2][TB], skq[2][TB];
+struct ScanBlock {
+  static constexpr int DP = LANES * G * R;            // dim rounded up; rows beyond dim hold zeros
+  static constexpr int TB = R <= 4 ? 16 : 8;          // tokens a block
+  static constexpr int COLS = 256 / LANES;
+  static constexpr int FLOATS = 2 * TB * (3 * DP + COLS + 2);       // of LDS
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+// columns group * COLS and on of a head's state, for tokens first .. first + count - 1
+template <int R, int G, int LANES, int W>
+__device__ __forceinline__ void scan_columns(const ScanArgs& a, int group, int h, int e, int first, int count, float* __restrict__ lds) {
+  using C = ScanBlock<R, G, LANES>;
+  constexpr int DP = C::DP, TB = C::TB, COLS = C::COLS;
+  constexpr int PER = (TB * DP / W + 255) / 256;       // pieces of W values of q (k, decay) a thread fetches a block
+  constexpr int RW = W < R ? W : R;                    // rows of the state a load takes
+  static_assert((LANES == 16 || G == 1) && R % RW == 0, "");
+  typedef float piece_t __attribute__((ext_vector_type(W)));
+  typedef float four_t __attribute__((ext_vector_type(4)));
+  typedef float rows_t __attribute__((ext_vector_type(RW)));
+  const DeltaShape& sh = a.sh;
+  auto& sq = *reinterpret_cast<float(*)[2][TB][DP]>(lds);
+  auto& sk = *reinterpret_cast<float(*)[2][TB][DP]>(lds + 2 * TB * DP);
+  auto& sg = *reinterpret_cast<float(*)[2][TB][DP]>(lds + 4 * TB * DP);
+  auto& sv = *reinterpret_cast<float(*)[2][COLS][TB]>(lds + 6 * TB * DP);
+  auto& sb = *reinterpret_cast<float(*)[2][TB]>(lds + 6 * TB * DP + 2 * TB * COLS);
+  auto& skq = *reinterpret_cast<float(*)[2][TB]>(lds + 6 * TB * DP + 2 * TB * COLS + 2 * TB);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int part = lane & (LANES - 1);
   const int col_local = wave * (64 / LANES) + lane / LANES;
-  const int col = blockIdx.x * COLS + col_local;
-  const int h = blockIdx.y, e = blockIdx.z;
+  const int col = group * COLS + col_local;
   const int kv = h / (sh.heads / sh.kv_heads);
   const int dim = sh.dim, vdim = sh.vdim;
   const bool col_ok = col < vdim;
-  const int i0 = part * G * R;
-  const int first = q_start[e], count = q_start[e + 1] - first;
-  float* sp = state + (size_t)state_slots[e] * state_stride + s_offset +
+  const int i0 = (LANES == 32 ? (part & 15) * 2 + (part >> 4) : part) * G * R;      // (neighbouring groups in the two rows)
+  float* sp = a.state + (size_t)a.state_slots[e] * a.state_stride + a.s_offset +
               ((size_t)h * vdim + (col_ok ? col : 0)) * dim + i0;
   float s[G * R];
 #pragma unroll
-  for (int r = 0; r < G * R; ++r) s[r] = (col_ok && i0 + r < dim) ? sp[r] : 0.f;
+  for (int r = 0; r < G * R; r += RW) {
+    const rows_t x = col_ok && i0 + r < dim ? *reinterpret_cast<const rows_t*>(sp + r) : rows_t(0.f);
+#pragma unroll
+    for (int i = 0; i < RW; ++i) s[r + i] = x[i];
+  }
 
   const int nqk = sh.kv_heads * dim, nd = sh.heads * dim, nv = sh.heads * vdim;
-  float pq[PER], pk[PER], pg[PER], pv = 0.f, pb = 0.f, pkq = 0.f;
-  // block b's share of this thread: element idx = tid + j * 256 of [TB][DP]; v: thread tid of [TB][COLS]; beta, k . q: tid < TB
-  // (No load stands under a condition, which the compiler would wait for where the branches meet: what lies beyond the
-  // entry's tokens is fetched from the last one and never used, what lies beyond dim or vdim becomes zero on the way to LDS.)
-  auto fetch = [&](int b) {
+  // block b's share of this thread: piece idx = tid + j * 256 of [TB][DP / W]; v: thread tid of [TB][COLS]; beta, k . q: tid < TB.
+  // (Loads stand under no condition, which the compiler would wait for where the branches meet: what lies beyond the entry's tokens, dim
+  // or vdim is out of the buffer's range and comes as zero.)
+  constexpr uint32_t kOutside = 0x80000000u;
+  uint32_t to_qk[PER], to_g[PER];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int idx = tid + j * 256, tok = idx / DP, i = min(idx % DP, dim - 1);
-      const size_t t = (size_t)(first + min(b * TB + tok, count - 1));
-      pq[j] = qn[t * nqk + (size_t)kv * dim + i];
-      pk[j] = kn[t * nqk + (size_t)kv * dim + i];
-      pg[j] = decay[t * nd + (size_t)h * dim + i];
-    }
-    const size_t tv = (size_t)(first + min(b * TB + tid / COLS, count - 1)), tb = (size_t)(first + min(b * TB + tid, count - 1));
-    pv = vn[tv * nv + (size_t)h * vdim + min((int)blockIdx.x * COLS + tid % COLS, vdim - 1)];
-    pb = beta[tb * sh.heads + h];
-    pkq = kq[tb * sh.kv_heads + kv];
+  for (int j = 0; j < PER; ++j) {
+    const int idx = tid + j * 256, tok = idx / (DP / W), i = idx % (DP / W) * W;
+    const bool there = idx < TB * DP / W && i < dim;
+    to_qk[j] = there ? (uint32_t)(tok * nqk + i) * 4 : kOutside;
+    to_g[j] = there ? (uint32_t)(tok * nd + i) * 4 : kOutside;
+  }
+  const int cols = min(COLS, vdim - group * COLS);
+  const uint32_t to_v = tid < TB * COLS && tid % COLS < cols ? (uint32_t)(tid / COLS * nv + tid % COLS) * 4 : kOutside;
+  const uint32_t to_b = tid < TB ? (uint32_t)(tid * sh.heads) * 4 : kOutside, to_kq = tid < TB ? (uint32_t)(tid * sh.kv_heads) * 4 : kOutside;
+  piece_t pq[PER], pk[PER], pg[PER];
+  float pv = 0.f, pb = 0.f, pkq = 0.f;
+  auto fetch = [&](int b) {
+    const size_t t = (size_t)(first + b * TB);
+    const int rows = min(TB, count - b * TB);
+    auto some = [&](const float* p, int ld, int width) {
+      return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, ((rows - 1) * ld + width) * 4, 0x00027000);
+    };
+    const auto q_b = some(a.qn + t * nqk + (size_t)kv * dim, nqk, dim), k_b = some(a.kn + t * nqk + (size_t)kv * dim, nqk, dim);
+    const auto g_b = some(a.decay + t * nd + (size_t)h * dim, nd, dim);
+    auto piece = [&](auto from, uint32_t at) {
+      if constexpr (W == 4) return __builtin_bit_cast(piece_t, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
+      else return __builtin_bit_cast(piece_t, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
+    };
+#pragma unroll
+    for (int j = 0; j < PER; ++j) pq[j] = piece(q_b, to_qk[j]), pk[j] = piece(k_b, to_qk[j]), pg[j] = piece(g_b, to_g[j]);
+    auto one = [&](auto from, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0)); };
+    pv = one(some(a.vn + t * nv + (size_t)h * vdim + (size_t)group * COLS, nv, cols), to_v);
+    pb = one(some(a.beta + t * sh.heads + h, sh.heads, 1), to_b);
+    pkq = one(some(a.kq + t * sh.kv_heads + kv, sh.kv_heads, 1), to_kq);
   };
   auto stash = [&](int buf) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const int idx = tid + j * 256, tok = idx / DP, i = idx % DP;
-      sq[buf][tok][i] = i < dim ? pq[j] : 0.f;
-      sk[buf][tok][i] = i < dim ? pk[j] : 0.f;
-      sg[buf][tok][i] = i < dim ? pg[j] : 0.f;
+      const int idx = tid + j * 256;
+      if (TB * DP / W % 256 != 0 && idx >= TB * DP / W) continue;
+      *reinterpret_cast<piece_t*>(&sq[buf][0][0] + idx * W) = pq[j];
+      *reinterpret_cast<piece_t*>(&sk[buf][0][0] + idx * W) = pk[j];
+      *reinterpret_cast<piece_t*>(&sg[buf][0][0] + idx * W) = pg[j];
     }
-    if (tid < TB * COLS) sv[buf][tid / COLS][tid % COLS] = pv;
+    if (tid < TB * COLS) sv[buf][tid % COLS][tid / COLS] = pv;
     if (tid < TB) sb[buf][tid] = pb, skq[buf][tid] = pkq;
   };
-  struct Rows { float k[G * R], g[G * R], q[G * R], v, b, kq; };
+  struct Rows { float k[G * R], g[G * R], q[G * R]; };
   auto load = [&](Rows& x, int buf, int tok) {
 #pragma unroll
     for (int r = 0; r < G * R; ++r) x.k[r] = sk[buf][tok][i0 + r], x.g[r] = sg[buf][tok][i0 + r], x.q[r] = sq[buf][tok][i0 + r];
-    x.v = sv[buf][tok][col_local], x.b = sb[buf][tok], x.kq = skq[buf][tok];
   };
-  auto token = [&](const Rows& x, int n) {
+  float out = 0.f;       // of the block's token `part`
+  auto token = [&](const Rows& x, float v, float b, float kq_, int tok) {
     float p1[G], p2[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) p1[g] = p2[g] = 0.f;
@@ -219,10 +292,11 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn, co
       p1[r / R] = fmaf(s[r], x.k[r], p1[r / R]);
       p2[r / R] = fmaf(s[r], x.q[r], p2[r / R]);
     }
-    const float d1 = column_sum<LANES>(p1), d2 = column_sum<LANES>(p2);
-    const float u = x.b * (x.v - d1);
+    float d1, d2;
+    column_sums<LANES>(p1, p2, d1, d2);
+    const float u = b * (v - d1);
     // o = S_new^T q with S_new = diag(g) S + k u^T
-    if (part == 0 && col_ok) o[(size_t)(first + n) * nv + (size_t)h * vdim + col] = fmaf(u, x.kq, d2);
+    out = part == tok ? fmaf(u, kq_, d2) : out;
 #pragma unroll
     for (int r = 0; r < G * R; ++r) s[r] = fmaf(x.k[r], u, s[r]);
   };
@@ -239,22 +313,96 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn, co
     const int buf = b & 1;
     if (b + 1 < blocks) fetch(b + 1);
     const int n_tok = min(TB, count - b * TB);
-    Rows x, y;
-    load(x, buf, 0);
-    for (int tok = 0; tok < n_tok; tok += 2) {
-      load(y, buf, min(tok + 1, TB - 1));
-      token(x, b * TB + tok);
-      load(x, buf, min(tok + 2, TB - 1));
-      if (tok + 1 < n_tok) token(y, b * TB + tok + 1);
+    if (n_tok == TB) {
+      // the rows are read two tokens before their turn, what every lane of a column needs by fours
+      Rows x[3];
+      four_t v[2], be[2], kq4[2];
+      auto load_four = [&](int tok) {
+        const int i = (tok >> 2) & 1;
+        v[i] = *reinterpret_cast<const four_t*>(&sv[buf][col_local][tok]);
+        be[i] = *reinterpret_cast<const four_t*>(&sb[buf][tok]);
+        kq4[i] = *reinterpret_cast<const four_t*>(&skq[buf][tok]);
+      };
+      load(x[0], buf, 0);
+      load_four(0);
+      load(x[1], buf, 1);
+#pragma unroll
+      for (int tok = 0; tok < TB; ++tok) {
+        __builtin_amdgcn_sched_barrier(0);       // (the compiler would read them when it needs them)
+        if (tok + 2 < TB) load(x[(tok + 2) % 3], buf, tok + 2);
+        if (tok % 4 == 2 && tok + 2 < TB) load_four(tok + 2);
+        const int i = (tok >> 2) & 1, at = tok & 3;
+        token(x[tok % 3], v[i][at], be[i][at], kq4[i][at], tok);
+      }
+    } else {
+      Rows x, y;
+      float v = sv[buf][col_local][0], be = sb[buf][0], kq1 = skq[buf][0];
+      load(x, buf, 0);
+#pragma unroll 1
+      for (int tok = 0; tok < n_tok; ++tok) {
+        load(y, buf, tok + 1);      // (there is one: n_tok < TB)
+        const float next_v = sv[buf][col_local][tok + 1], next_b = sb[buf][tok + 1], next_kq = skq[buf][tok + 1];
+        token(x, v, be, kq1, tok);
+        x = y, v = next_v, be = next_b, kq1 = next_kq;
+      }
     }
+    if (part < n_tok && col_ok) a.o[(size_t)(first + b * TB + part) * nv + (size_t)h * vdim + col] = out;
     if (b + 1 < blocks) stash(buf ^ 1);
     __syncthreads();
   }
   if (col_ok) {
 #pragma unroll
-    for (int r = 0; r < G * R; ++r)
-      if (i0 + r < dim) sp[r] = s[r];
+    for (int r = 0; r < G * R; r += RW) {
+      rows_t x;
+#pragma unroll
+      for (int i = 0; i < RW; ++i) x[i] = s[r + i];
+      if (i0 + r < dim) *reinterpret_cast<rows_t*>(sp + r) = x;
+    }
   }
+}
+#endif
+
+template <int R, int G, int LANES, int W>
+__global__ void __launch_bounds__(256) delta_scan_kernel(ScanArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(16))) float lds[ScanBlock<R, G, LANES>::FLOATS];
+  // (a step's portions of prompts come behind its single tokens: begun first, they have the CUs for themselves.  Portions that are in front all
+  // the same begin late: 32 heads of 128 x 128, 2,041 tokens and seven single ones 491 us, and 305 the other way round)
+  const int e = (int)gridDim.z - 1 - (int)blockIdx.z, first = a.q_start[e];
+  scan_columns<R, G, LANES, W>(a, blockIdx.x, blockIdx.y, e, first, a.q_start[e + 1] - first, lds);
+#endif
+}
+// 32 lanes a column for the entries that have most of the step's tokens, 16 for the others.  The first `extra` of blockIdx.z count the
+// former's, for the columns that 16 lanes would leave no workgroup; then all entries follow.
+// (With workgroups without work between those with it, every second CU stayed idle: four entries of 512 tokens 118 us against 78.)
+template <int R, int W>
+__global__ void __launch_bounds__(256) delta_scan_long_kernel(ScanArgs a, int n_entries) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(16))) float lds[ScanBlock<R, 2, 16>::FLOATS];
+  const int extra = (int)gridDim.z - n_entries;
+  const bool more = (int)blockIdx.z < extra;
+  int e = (int)gridDim.z - 1 - (int)blockIdx.z;      // (see delta_scan_kernel)
+  if (more) {
+    int nth = blockIdx.z;
+    e = -1;
+    for (int from = 0; from < n_entries; from += 64) {
+      const int i = min(from + (int)(threadIdx.x & 63), n_entries - 1);
+      unsigned long long wide = __ballot(from + (int)(threadIdx.x & 63) < n_entries && scan_wide(a.sh, a.q_start[i + 1] - a.q_start[i], a.n_tokens));
+      for (; wide != 0 && nth > 0; --nth) wide &= wide - 1;
+      if (wide != 0) {
+        e = from + __builtin_ctzll(wide);
+        break;
+      }
+    }
+    if (e < 0) return;
+  }
+  const int first = a.q_start[e], count = a.q_start[e + 1] - first, group = blockIdx.x + (more ? gridDim.x : 0);
+  if (scan_wide(a.sh, count, a.n_tokens)) {
+    if (group * 8 < a.sh.vdim) scan_columns<R, 1, 32, W>(a, group, blockIdx.y, e, first, count, lds);
+  } else {
+    scan_columns<R, 2, 16, W>(a, group, blockIdx.y, e, first, count, lds);
+  }
+#endif
 }
 
 template <typename TO>
@@ -279,8 +427,9 @@ delta_out_kernel(const float* __restrict__ o, const float* __restrict__ gate_pre
 // columns, `PASSES` a thread at a time, are asked for before anything else and arrive while convolution, unit lengths and decays are
 // made; the heads' outputs are normed from LDS.  Every sum is added in the order of the kernels above: the same bits.
 // Bound by its trips to memory (the slot, then the state) and by what a CU moves of the state, 256 KB for two heads of 128 x 128: with
-// eight requests of 8 heads over 4 q/k heads 32 workgroups, 12.6 us for the launch, where the four take 29.5 (prepare 11.7, the
-// convolution's state 5.1, scan 8.2, output 5.2).  (With the loads of the state, the taps and the gates each waited for by itself: 15.8.)
+// eight requests of 8 heads over 4 q/k heads 32 workgroups, 12.6 us for the launch, where the four took 29.5 (prepare 11.7, the
+// convolution's state 5.1, scan 8.2, since then 1.5 less, output 5.2).  (With the loads of the state, the taps and the gates each waited for
+// by itself: 15.8.)
 // A CU has one such workgroup at a time (heads of 64 and 128 take all 128 registers a thread may have, and three values spill around
 // the passes), so steps of many small heads keep the four launches: delta_step_pays in ops.py.
 template <int R, int G, int LANES, typename TO>
@@ -578,17 +727,26 @@ extern "C" int atoma_delta_scan(const float* qn, const float* kn, const float* v
   DeltaShape sh{heads, kv_heads, dim, vdim, taps, 1, 0, 0, 0, 0};
   if (!shape_ok(sh) || n_entries > 65535 || heads > 65535) return ATOMA_ERR_SHAPE;
   const size_t s_offset = (size_t)(taps - 1) * (2 * kv_heads * dim + heads * vdim);
-  const bool wide = dim > 128 || (dim > 64 && n_tokens < (int64_t)16 * n_entries);      // (see the kernel)
-  const int cols = wide ? 8 : 16;
-  const dim3 grid((vdim + cols - 1) / cols, heads, n_entries), block(256);
-#define ATOMA_SCAN(R, G, LANES)                                                                                         \
-  hipLaunchKernelGGL((delta_scan_kernel<R, G, LANES>), grid, block, 0, stream, qn, kn, vn, beta, decay, kq, sh, q_start, \
-                     state_slots, state, state_stride, s_offset, o)
+  // (the longest entry there can be)
+  const bool mixed = dim > 64 && dim <= 128 && n_entries < 32768 && scan_wide(sh, n_tokens - n_entries + 1, n_tokens);
+  const int cols = dim > 128 ? 8 : 16;
+  // (as many entries can have 32 lanes a column at most)
+  const int extra = mixed ? std::min(n_entries, kScanGroups / (heads * ((vdim + 7) / 8))) : 0;
+  const dim3 grid((vdim + cols - 1) / cols, heads, n_entries + extra), block(256);
+  const bool four = dim % 4 == 0 && s_offset % 4 == 0 && state_stride % 4 == 0 &&
+                    ((uintptr_t)qn | (uintptr_t)kn | (uintptr_t)decay | (uintptr_t)state) % 16 == 0;
+  const ScanArgs args{qn, kn, vn, beta, decay, kq, sh, q_start, state_slots, state, state_stride, s_offset, o, n_tokens};
+#define ATOMA_SCAN(...)                                                                                                   \
+  do {                                                                                                                    \
+    if (four) hipLaunchKernelGGL((delta_scan_kernel<__VA_ARGS__, 4>), grid, block, 0, stream, args);                      \
+    else hipLaunchKernelGGL((delta_scan_kernel<__VA_ARGS__, 1>), grid, block, 0, stream, args);                           \
+  } while (0)
   if (dim <= 16) ATOMA_SCAN(1, 1, 16);
   else if (dim <= 32) ATOMA_SCAN(1, 2, 16);
   else if (dim <= 64) ATOMA_SCAN(2, 2, 16);
-  else if (dim <= 128 && !wide) ATOMA_SCAN(4, 2, 16);
-  else if (dim <= 128) ATOMA_SCAN(4, 1, 32);
+  else if (mixed && four) hipLaunchKernelGGL((delta_scan_long_kernel<4, 4>), grid, block, 0, stream, args, n_entries);
+  else if (mixed) hipLaunchKernelGGL((delta_scan_long_kernel<4, 1>), grid, block, 0, stream, args, n_entries);
+  else if (dim <= 128) ATOMA_SCAN(4, 2, 16);
   else ATOMA_SCAN(8, 1, 32);
 #undef ATOMA_SCAN
   ATOMA_LAUNCH_CHECK();

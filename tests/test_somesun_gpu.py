@@ -155,6 +155,45 @@ def test_the_recurrence_is_the_same_bits_however_it_is_cut(dim, vdim):
                                              state0[:, :(taps - 1) * (2 * kv * dim + heads * vdim)]).all())
 
 
+@pytest.mark.parametrize("heads, kv, dim, vdim, taps", [(8, 4, 128, 128, 4), (6, 3, 70, 33, 3), (4, 2, 96, 24, 2), (2, 1, 66, 130, 1), (2, 2, 64, 20, 2),
+                                                        (2, 1, 200, 9, 3), (3, 3, 30, 16, 4), (2, 2, 16, 40, 2)])
+def test_the_recurrence_is_the_same_bits_whatever_is_beside_it(heads, kv, dim, vdim, taps):
+    """Entries of 0 to 100 tokens, whole blocks of 16 and rests, alone (where long ones have 32 lanes a column) and all in one step, the long
+    ones first, last and in the middle; and against 64 bits."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dim)
+    r = lambda *n: torch.randn(*n, generator=g).to(DEV)
+    for counts in ([100, 1, 1, 0, 2], [1, 16, 17, 15, 1, 64, 33], [1] * 70 + [95, 80], [32, 31, 48, 7] * 6):
+        t, n = sum(counts), len(counts)
+        unit = lambda x: torch.nn.functional.normalize(x.view(t, kv, dim), dim=-1).reshape(t, -1)
+        qn, kn, vn = unit(r(t, kv * dim)), unit(r(t, kv * dim)), r(t, heads * vdim)
+        kq = (qn * kn).view(t, kv, dim).sum(-1)
+        beta, decay = torch.sigmoid(r(t, heads)), torch.exp(-torch.exp(r(t, heads * dim)))
+        ins, sizes = (qn, kn, vn, beta, decay, kq), (heads, kv, dim, vdim, taps)
+        at = [sum(counts[:i]) for i in range(n + 1)]
+        conv = (taps - 1) * (2 * kv * dim + heads * vdim)
+        state0 = r(n, conv + heads * vdim * dim)
+        slots = torch.randperm(n, generator=g).to(DEV, torch.int32)
+        state, alone = state0.clone(), state0.clone()
+        out = ops.delta_scan(*ins, *sizes, torch.tensor(at, dtype=torch.int32, device=DEV), slots, state)
+        for i in range(n):
+            if counts[i]:
+                one = ops.delta_scan(*(x[at[i]: at[i + 1]].contiguous() for x in ins), *sizes,
+                                     torch.tensor([0, counts[i]], dtype=torch.int32, device=DEV), slots[i: i + 1], alone)
+                assert torch.equal(one, out[at[i]: at[i + 1]]), (counts, i)
+        assert torch.equal(state, alone)
+        i = max(range(n), key=lambda j: counts[j])
+        s = state0[slots[i].long(), conv:].view(heads, vdim, dim).double()
+        for j in range(at[i], at[i + 1]):
+            k, q = (x[j].view(kv, dim).double().repeat_interleave(heads // kv, 0) for x in (kn, qn))
+            s = s * decay[j].view(heads, 1, dim).double()
+            u = beta[j].double()[:, None] * (vn[j].view(heads, vdim).double() - (s * k[:, None]).sum(-1))
+            s = s + u[..., None] * k[:, None]
+            want = (s * q[:, None]).sum(-1).reshape(-1)
+            # a sum of dim products, and the state's own error, which decays
+            assert (out[j].double() - want).norm() <= 8 * dim ** 0.5 * 2.0 ** -24 * max(float(want.norm()), float(s.norm()) / dim ** 0.5)
+
+
 @pytest.mark.parametrize("dim, vdim, heads, kv, taps, n", [(12, 8, 4, 2, 3, 3), (30, 8, 2, 2, 1, 2), (64, 24, 4, 1, 4, 5), (72, 17, 4, 2, 2, 3),
                                                            (128, 40, 6, 3, 9, 2), (200, 9, 2, 1, 4, 1), (128, 128, 8, 4, 4, 8),
                                                            (256, 128, 2, 1, 4, 9), (16, 600, 2, 1, 4, 2), (1, 1, 1, 1, 2, 1), (64, 64, 4, 4, 4, 300)])
