@@ -249,218 +249,237 @@ ssd_step_kernel(const float* __restrict__ proj, SsdShape sh, const int32_t* __re
 //   S_64 = exp(c_63) S_0 + sum_s exp(c_63 - c_s) dt_s B_s x_s^T,
 // every exponent at most zero.  The products C_t . B_s are the same for all heads of a group and all columns of S: a
 // first kernel (ssd_scores) makes them once per (chunk, group).  Then a workgroup owns (entry, head, 16 columns of S)
-// and walks the entry's chunks in order; per chunk its four waves make M[t][s] = (C_t . B_s) exp(c_t - c_s) dt_s for
-// s <= t (ten tiles of 16 x 16 shared out among them, into LDS), then each takes 16 tokens of
-// y = M X + diag(exp(c)) C S, then each its share of the rows of S.
+// and walks the entry's chunks in order; per chunk each of its four waves takes 16 tokens of y = M X + diag(exp(c)) C S, with
+// M[t][s] = (C_t . B_s) exp(c_t - c_s) dt_s for s <= t, then its share of the rows of S.
 // All products are float32 MFMAs of 16 x 16 x 4 (result D[4 (l / 16) + i][l % 16] in lane l).  The sum over k of a
-// block of 16 is taken in the order that lets a lane fetch its four values with one 16-byte load from LDS: in the
-// block's MFMA j, lane l gives A[l % 16][4 (l / 16) + j] and B[4 (l / 16) + j][l % 16]; tiles whose k runs along their
-// rows in memory (x and S) are kept transposed in LDS for it.  The next chunk's B, C, x and dt are asked for while this
-// one is worked on.  An entry's result depends on its own length and sizes alone.
+// block of 16 is taken in the order that lets a lane have its four values as one 16-byte piece: in the block's MFMA j, lane l
+// gives A[l % 16][4 (l / 16) + j] and B[4 (l / 16) + j][l % 16].  C's and B's rows and the tiles of scores come from memory as
+// the operands that they are, each of them to the one wave that multiplies it, and M is made of the scores in registers; a wave's
+// rows of S stay in its registers too.  What the waves share passes LDS, transposed for the pieces, in two buffers that take turns:
+// x, and S for y.  So a chunk has one barrier, and each operand is asked for as soon as the one before it has been used.
+// Bound by a wave's way through a chunk, 3.7 us with a state of 128, of which its 36 to 48 MFMAs for y and 32 for S are 1.1, and where
+// entries are many by all waves' instructions; it was 6 us, with five barriers and all operands through 108 KB of LDS, one workgroup a CU.
+// us with the scores, before / now: 64 heads of 64 x 128, one entry of 2,048 tokens 202 / 129, 1,400 and 640 207 / 111, eight of 256 229 / 114,
+// 64 of 32 599 / 223; 32 heads of 64 x 64, one of 2,048 142 / 96.  The results' bits are the same.  (The next chunk's sums of decays made
+// between this one's MFMAs, or B's rows by pairs, gave nothing: 139 and 135 against 136 at that point.)
 constexpr int kChunk = 64;
-constexpr int kChunkLdt = kChunk + 4;      // row stride of the tiles whose rows are 64 tokens long (M, x transposed)
+constexpr int kChunkLdt = kChunk + 4;      // row stride of x transposed
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
-
-__host__ __device__ constexpr int chunk_lds_floats(int nb) {
-  return 2 * kChunk * (16 * nb + 4) + kChunk * kChunkLdt + 16 * kChunkLdt + 16 * (16 * nb + 4) + 4 * kChunk;
-}
 
 __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
-// VEC: B and C rows are fetched and put into LDS 16 bytes at a time (state size, channel counts and the first column
-// of the group's B all multiples of 4)
+// VEC: C and S are fetched 16 bytes at a time (state size, channel counts and the state's rows all multiples of 4)
 template <int NB, bool VEC>      // NB: blocks of 16 rows of S (the state size rounded up)
 __global__ void __launch_bounds__(256)
 ssd_chunk_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, const float* __restrict__ a_log,
                  const float* __restrict__ d_skip, SsdShape sh, const int32_t* __restrict__ q_start,
                  const int32_t* __restrict__ state_slots, float* __restrict__ state, size_t state_stride,
                  float* __restrict__ y, int at_least, const float* __restrict__ scores, int max_chunks) {
-  constexpr int NP = 16 * NB, LDN = NP + 4;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* Bs = lds;                         // [kChunk][LDN]   B of the chunk's tokens
-  float* Cs = Bs + kChunk * LDN;           // [kChunk][LDN]   C
-  float* Ms = Cs + kChunk * LDN;           // [kChunk][kChunkLdt]   M[t][s]
-  float* Xt = Ms + kChunk * kChunkLdt;     // [16][kChunkLdt]  x transposed: [column][token]
-  float* St = Xt + 16 * kChunkLdt;         // [16][LDN]        S transposed: [column][row], as the state keeps it
-  float* cum = St + 16 * LDN;              // [kChunk] log decays summed up to each token
-  float* dts = cum + kChunk;               // [kChunk]
-  float* wts = dts + kChunk;               // [kChunk] exp(c_last - c_s) dt_s
-  float* ect = wts + kChunk;               // [kChunk] exp(c_t)
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int NP = 16 * NB, LDN = NP + 4, MINE = (NB + 3) / 4;      // MINE: blocks of 16 rows of S of a wave
+  constexpr uint32_t kOutside = 0x80000000u;                          // (out of any buffer's range: comes as zero)
+  __shared__ __attribute__((aligned(16))) float St[2][16 * LDN];          // S transposed: [column][row], as the state keeps it
+  __shared__ __attribute__((aligned(16))) float Xt[2][16 * kChunkLdt];    // x transposed: [column][token]
+  __shared__ __attribute__((aligned(16))) float own[4][3][kChunk];        // of a wave: log decays summed up to a token, dt, and
+                                                                          // exp(c_last - c_s) dt_s
   const int e = blockIdx.z, h = blockIdx.y, v0 = blockIdx.x * 16;
   const int first = q_start[e], count = q_start[e + 1] - first;
   if (count < at_least) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kg = lane >> 4;
   const int inner = sh.heads * sh.vdim, gn = sh.groups * sh.n, channels = inner + 2 * gn;
   const int g = h / (sh.heads / sh.groups);
   const int vlive = min(16, sh.vdim - v0);
-  float* s_ptr = state + (size_t)state_slots[e] * state_stride + (size_t)(sh.taps - 1) * channels +
-                 ((size_t)h * sh.vdim + v0) * sh.n;
-  for (int idx = tid; idx < NP * 16; idx += 256) {
-    const int v = idx / NP, n = idx % NP;
-    St[v * LDN + n] = (v < vlive && n < sh.n) ? s_ptr[(size_t)v * sh.n + n] : 0.f;
-  }
   const float rate = expf(a_log[h]), dh = d_skip[h];
-  // A chunk's B, C, x and dt are asked for while the chunk before is worked on, and wait in registers meanwhile.
-  constexpr int PER = kChunk * NP / 256;        // elements of a [64][NP] tile a thread moves
-  float rb[PER], rc[PER], rx[4], rdt = 0.f;
-  f32x4 mt[3];       // the wave's tiles of C . B of the chunk, as the scores kernel left them
-  auto fetch = [&](int t0) {
-    const int nt = min(kChunk, count - t0);
-    const size_t tok0 = (size_t)(first + t0);
-    const float* sc = scores + (((size_t)e * max_chunks + t0 / kChunk) * sh.groups + g) * (10 * 256);
-#pragma unroll
-    for (int m = 0; m < 3; ++m)      // tile wave + 4 m is the wave's m-th
-      if (wave + 4 * m < 10) mt[m] = *reinterpret_cast<const f32x4*>(sc + ((wave + 4 * m) * 64 + lane) * 4);
-    if constexpr (VEC) {
-#pragma unroll
-      for (int i = 0; i < PER / 4; ++i) {
-        const int idx = tid + i * 256, tt = idx / (NP / 4), n = (idx % (NP / 4)) * 4;
-        const bool in = tt < nt && n < sh.n;
-        const size_t base = (tok0 + tt) * channels + inner + (size_t)g * sh.n + n;
-        const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-        const f32x4 b4 = in ? *reinterpret_cast<const f32x4*>(xbc + base) : zero;
-        const f32x4 c4 = in ? *reinterpret_cast<const f32x4*>(xbc + base + gn) : zero;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          rb[4 * i + q] = b4[q];
-          rc[4 * i + q] = c4[q];
-        }
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int idx = tid + i * 256, tt = idx / NP, n = idx % NP;
-        const bool in = tt < nt && n < sh.n;
-        const size_t base = (tok0 + tt) * channels + inner + (size_t)g * sh.n + n;
-        rb[i] = in ? xbc[base] : 0.f;
-        rc[i] = in ? xbc[base + gn] : 0.f;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = tid + i * 256, tt = idx >> 4, v = idx & 15;
-      rx[i] = (tt < nt && v < vlive) ? xbc[(tok0 + tt) * channels + (size_t)h * sh.vdim + v0 + v] : 0.f;
-    }
-    if (tid < kChunk) rdt = tid < nt ? dt[(tok0 + tid) * sh.heads + h] : 0.f;
+  float* const cum = own[wave][0];
+  float* const dts = own[wave][1];
+  float* const wts = own[wave][2];
+
+  // a chunk's rows of xbc, of dt and of scores; past the last chunk nothing is in range.  (No load stands under a condition, which the
+  // compiler would wait for where the branches meet.)
+  auto buffer = [&](const float* p, int floats) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, __builtin_amdgcn_readfirstlane(floats * 4), 0x00027000);
   };
-  fetch(0);
-  for (int t0 = 0; t0 < count; t0 += kChunk) {
-    const int nt = min(kChunk, count - t0);
-    const size_t tok0 = (size_t)(first + t0);
-    __syncthreads();       // the chunk before is done with every tile
-    if constexpr (VEC) {
+  auto rows_of = [&](int t0) { return max(0, min(kChunk, count - t0)); };
+  auto inputs = [&](int t0) { return buffer(xbc + (size_t)(first + t0) * channels, rows_of(t0) * channels); };
+  auto one = [&](auto from, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0)); };
+  auto four = [&](auto from, uint32_t at) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0)); };
+  // (places that are out of range stay values of a register: known to be constants, they become branches around the loads)
+  auto place = [&](bool in, int at) {
+    uint32_t x = in ? (uint32_t)at * 4 : kOutside;
+    asm("" : "+v"(x));
+    return x;
+  };
+  const uint32_t x_at = place((tid & 15) < vlive, (tid >> 4) * channels + h * sh.vdim + v0 + (tid & 15));
+  const uint32_t y_at = place(r16 < vlive, (wave * 16 + 4 * kg) * inner + r16);
+  const int c_row = (wave * 16 + r16) * channels + inner + gn + g * sh.n + 4 * kg;
+  uint32_t c_last[4], b_at[MINE], mt_at[4];      // (of C's blocks of 16 columns only the last one can end early)
 #pragma unroll
-      for (int i = 0; i < PER / 4; ++i) {
-        const int idx = tid + i * 256, tt = idx / (NP / 4), n = (idx % (NP / 4)) * 4;
-        *reinterpret_cast<f32x4*>(Bs + tt * LDN + n) = f32x4{rb[4 * i], rb[4 * i + 1], rb[4 * i + 2], rb[4 * i + 3]};
-        *reinterpret_cast<f32x4*>(Cs + tt * LDN + n) = f32x4{rc[4 * i], rc[4 * i + 1], rc[4 * i + 2], rc[4 * i + 3]};
-      }
-    } else {
+  for (int q = 0; q < (VEC ? 1 : 4); ++q) c_last[q] = place((NB - 1) * 16 + 4 * kg + q < sh.n, c_row + (NB - 1) * 16 + q);
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int idx = tid + i * 256, tt = idx / NP, n = idx % NP;
-        Bs[tt * LDN + n] = rb[i];
-        Cs[tt * LDN + n] = rc[i];
+  for (int m = 0; m < MINE; ++m) {
+    const int n = (wave + 4 * m) * 16 + r16;
+    b_at[m] = place(n < sh.n, 4 * kg * channels + inner + g * sh.n + n);
+  }
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) mt_at[sb] = place(sb <= wave, ((wave * (wave + 1) / 2 + sb) * 64 + lane) * 4);
+  f32x4 cc[NB], mt[4];
+  float bb[MINE][4][4], rx[4], rdt;
+  auto fetch_x = [&](int t0) {
+    const auto from = inputs(t0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rx[i] = one(from, x_at + (uint32_t)(i * 16 * channels) * 4);
+    const int rows = rows_of(t0);
+    rdt = one(buffer(dt + (size_t)(first + t0) * sh.heads + h, rows > 0 ? (rows - 1) * sh.heads + 1 : 0), (uint32_t)(lane * sh.heads) * 4);
+  };
+  // C's rows of the wave's 16 tokens, and its tiles of scores
+  auto fetch_c = [&](int t0) {
+    const auto from = inputs(t0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if constexpr (VEC) {
+        cc[b] = four(from, b < NB - 1 ? (uint32_t)(c_row + b * 16) * 4 : c_last[0]);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cc[b][q] = one(from, b < NB - 1 ? (uint32_t)(c_row + b * 16 + q) * 4 : c_last[q]);
       }
     }
+    const auto tiles = buffer(scores + (((size_t)e * max_chunks + t0 / kChunk) * sh.groups + g) * (10 * 256), rows_of(t0) > 0 ? 10 * 256 : 0);
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+      mt[sb] = four(tiles, mt_at[sb]);
+  };
+  // B's columns that are the wave's rows of S
+  auto fetch_b = [&](int t0) {
+    const auto from = inputs(t0);
+#pragma unroll
+    for (int m = 0; m < MINE; ++m)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) bb[m][k][q] = one(from, b_at[m] + (uint32_t)((k * 16 + q) * channels) * 4);
+  };
+  auto stash_x = [&](float* xt) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int idx = tid + i * 256;
-      Xt[(idx & 15) * kChunkLdt + (idx >> 4)] = rx[i];
+      xt[(idx & 15) * kChunkLdt + (idx >> 4)] = rx[i];
     }
-    if (tid < kChunk) dts[tid] = rdt;
-    __syncthreads();
-    if (wave == 0) {
-      // inclusive sums of the log decays over the 64 lanes
-      float c = -rate * dts[lane];
+  };
+
+  fetch_x(0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_c(0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_b(0);
+  __builtin_amdgcn_sched_barrier(0);
+  // lane: rows (wave + 4 m) 16 + 4 (l / 16) .. + 3 of S, column l % 16
+  float* const s_ptr = state + (size_t)state_slots[e] * state_stride + (size_t)(sh.taps - 1) * channels +
+                       ((size_t)h * sh.vdim + v0 + min(r16, vlive - 1)) * sh.n;
+  f32x4 s[MINE];
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const float up = __shfl_up(c, o, 64);
-        if (lane >= o) c += up;
-      }
-      cum[lane] = c;
-      const float last = __shfl(c, 63, 64);
-      wts[lane] = expf(last - c) * dts[lane];
-      ect[lane] = expf(c);
+  for (int m = 0; m < MINE; ++m) {
+    const int n = (wave + 4 * m) * 16 + 4 * kg;
+    s[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (VEC) {
+      if (r16 < vlive && n < sh.n) s[m] = *reinterpret_cast<const f32x4*>(s_ptr + n);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (r16 < vlive && n + q < sh.n) s[m][q] = s_ptr[n + q];
     }
-    // (the chunk after this one is fetched further down, when this chunk's tiles of scores have been used)
-    __syncthreads();       // the sums of the log decays are there
+    if (wave + 4 * m < NB) *reinterpret_cast<f32x4*>(St[0] + r16 * LDN + n) = s[m];
+  }
+  stash_x(Xt[0]);
+  __syncthreads();
+  for (int t0 = 0; t0 < count; t0 += kChunk) {
+    const int nt = min(kChunk, count - t0), buf = (t0 / kChunk) & 1;
+    const size_t tok0 = (size_t)(first + t0);
+    // inclusive sums of the log decays over the 64 lanes
+    float c = -rate * rdt;
 #pragma unroll
-    for (int j = 0; j < 10; ++j) {
-      const int tb = j >= 6 ? 3 : j >= 3 ? 2 : j >= 1 ? 1 : 0, sb = j - tb * (tb + 1) / 2;
-      if ((j & 3) == wave) {
-        const f32x4 acc = mt[j >> 2];
-        const int s = sb * 16 + r16;
-        const float cs = cum[s], ds = dts[s];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = tb * 16 + 4 * kg + i;
-          Ms[t * kChunkLdt + s] = s <= t ? acc[i] * expf(cum[t] - cs) * ds : 0.f;
-        }
-      }
+    for (int o = 1; o < 64; o <<= 1) {
+      const float up = __shfl_up(c, o, 64);
+      if (lane >= o) c += up;
     }
-    if (t0 + kChunk < count) fetch(t0 + kChunk);
-    __syncthreads();
+    const float last = __shfl(c, 63, 64), ec = expf(c);
+    cum[lane] = c;
+    dts[lane] = rdt;
+    wts[lane] = expf(last - c) * rdt;
+    const float keep = __shfl(ec, 63, 64), et = __shfl(ec, wave * 16 + r16, 64), ct = __shfl(c, wave * 16 + r16, 64);
+    __builtin_amdgcn_wave_barrier();      // (what is read of it below was written by this wave)
+    const float* const xp = Xt[buf] + r16 * kChunkLdt + 4 * kg;
+    fetch_x(t0 + kChunk);
+    __builtin_amdgcn_sched_barrier(0);
     // y of the wave's 16 tokens
     if (wave * 16 < nt) {
       f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int tb = wave;
-      const float* mp = Ms + (tb * 16 + r16) * kChunkLdt + 4 * kg;
-      const float* xp = Xt + r16 * kChunkLdt + 4 * kg;
-      for (int k = 0; k < (tb + 1) * 16; k += 16) {
-        const f32x4 a4 = lds4(mp + k), b4 = lds4(xp + k);
+      const f32x4 x4 = lds4(xp + wave * 16);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[q], b4[q], acc, 0, 0, 0);
-      }
-      const float et = ect[tb * 16 + r16];
-      const float* cp = Cs + (tb * 16 + r16) * LDN + 4 * kg;
-      const float* sp = St + r16 * LDN + 4 * kg;
+      for (int sb = 0; sb < 4; ++sb) {
+        if (sb > wave) continue;
+        const f32x4 cs = lds4(cum + sb * 16 + 4 * kg), ds = lds4(dts + sb * 16 + 4 * kg), b4 = lds4(xp + sb * 16);
 #pragma unroll
-      for (int k = 0; k < NP; k += 16) {
-        const f32x4 a4 = lds4(cp + k), b4 = lds4(sp + k);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(et * a4[q], b4[q], acc, 0, 0, 0);
-      }
-      if (r16 < vlive) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = tb * 16 + 4 * kg + i;
-          if (t < nt) y[(tok0 + t) * inner + (size_t)h * sh.vdim + v0 + r16] = acc[i] + dh * Xt[r16 * kChunkLdt + t];
+        for (int q = 0; q < 4; ++q) {
+          float m = mt[sb][q] * expf(ct - cs[q]) * ds[q];
+          asm("" : "+v"(m));      // (it is not worth a branch)
+          if (sb == wave && 4 * kg + q > r16) m = 0.f;
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(m, b4[q], acc, 0, 0, 0);
         }
       }
-    }
-    __syncthreads();       // every wave has read S
-    {
-      const float keep = ect[kChunk - 1];
-      for (int nb = wave; nb < NB; nb += 4) {
-        // lane: rows nb * 16 + 4 (l / 16) .. + 3 of S, column l % 16: four neighbours of the transposed tile
-        float* sp = St + r16 * LDN + nb * 16 + 4 * kg;
-        f32x4 acc = lds4(sp);
+      const float* const sp = St[buf] + r16 * LDN + 4 * kg;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] *= keep;
-        const float* bp = Bs + (4 * kg) * LDN + nb * 16 + r16;
-        const float* xp = Xt + r16 * kChunkLdt + 4 * kg;
+      for (int b = 0; b < NB; ++b) {
+        const f32x4 b4 = lds4(sp + b * 16);
 #pragma unroll
-        for (int k = 0; k < kChunk; k += 16) {
-          const f32x4 w4 = lds4(wts + k + 4 * kg), b4 = lds4(xp + k);
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bp[(k + q) * LDN] * w4[q], b4[q], acc, 0, 0, 0);
-        }
-        *reinterpret_cast<f32x4*>(sp) = acc;
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(et * cc[b][q], b4[q], acc, 0, 0, 0);
       }
+      const auto to = buffer(y + tok0 * inner + (size_t)h * sh.vdim + v0, (nt - 1) * inner + vlive);      // (what is out of range stays unwritten)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i] + dh * x4[i]), to, y_at + (uint32_t)(i * inner) * 4, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // (the loads arrive in the order in which they are asked for)
+    fetch_c(t0 + kChunk);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MINE; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[m][i] *= keep;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const f32x4 w4 = lds4(wts + k * 16 + 4 * kg), b4 = lds4(xp + k * 16);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int m = 0; m < MINE; ++m) s[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(bb[m][k][q] * w4[q], b4[q], s[m], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_b(t0 + kChunk);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < MINE; ++m)
+      if (wave + 4 * m < NB) *reinterpret_cast<f32x4*>(St[buf ^ 1] + r16 * LDN + (wave + 4 * m) * 16 + 4 * kg) = s[m];
+    stash_x(Xt[buf ^ 1]);
+    __syncthreads();       // the next chunk's x and S are there, and everybody is done with this one's
+  }
+#pragma unroll
+  for (int m = 0; m < MINE; ++m) {
+    const int n = (wave + 4 * m) * 16 + 4 * kg;
+    if constexpr (VEC) {
+      if (r16 < vlive && n < sh.n) *reinterpret_cast<f32x4*>(s_ptr + n) = s[m];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (r16 < vlive && n + q < sh.n) s_ptr[n + q] = s[m][q];
     }
   }
-  __syncthreads();
-  for (int idx = tid; idx < NP * 16; idx += 256) {
-    const int v = idx / NP, n = idx % NP;
-    if (v < vlive && n < sh.n) s_ptr[(size_t)v * sh.n + n] = St[v * LDN + n];
-  }
+#endif
 }
 
 // C_t . B_s of every chunk of 64 tokens, once per group of heads: the ten 16 x 16 tiles on and below the diagonal, each
-// as its 64 lanes' four numbers (lane l: rows 4 (l / 16) .. + 3, column l % 16 of the tile), [entry][chunk][group][10][64][4].
+// as its 64 lanes' four numbers (lane l: t = l % 16, s = 4 (l / 16) .. + 3 of the tile, as M's operand wants them),
+// [entry][chunk][group][10][64][4].
 template <int NB>
 __global__ void __launch_bounds__(256)
 ssd_scores_kernel(const float* __restrict__ xbc, SsdShape sh, const int32_t* __restrict__ q_start, int at_least,
@@ -496,7 +515,7 @@ ssd_scores_kernel(const float* __restrict__ xbc, SsdShape sh, const int32_t* __r
       for (int k = 0; k < NP; k += 16) {
         const f32x4 a4 = lds4(cp + k), b4 = lds4(bp + k);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[q], b4[q], acc, 0, 0, 0);
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[q], a4[q], acc, 0, 0, 0);
       }
       *reinterpret_cast<f32x4*>(out + (j * 64 + lane) * 4) = acc;
     }
@@ -655,15 +674,9 @@ template <int NB, bool VEC>
 static int launch_chunk(dim3 grid, hipStream_t stream, const float* xbc, const float* dt, const float* a_log,
                         const float* d_skip, const SsdShape& sh, const int32_t* q_start, const int32_t* state_slots,
                         float* state, size_t state_stride, float* y, int at_least, float* scores, int max_chunks) {
-  const size_t bytes = (size_t)chunk_lds_floats(NB) * sizeof(float);
   const size_t sbytes = (size_t)2 * kChunk * (16 * NB + 4) * sizeof(float);
   static bool asked = false;      // (per instantiation) more than the default 64 KB of LDS
   if (!asked) {
-    if (bytes > 64 * 1024) {
-      hipError_t err = hipFuncSetAttribute((const void*)ssd_chunk_kernel<NB, VEC>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-      if (err != hipSuccess) return (int)err;
-    }
     if (sbytes > 64 * 1024) {
       hipError_t err = hipFuncSetAttribute((const void*)ssd_scores_kernel<NB>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbytes);
@@ -673,7 +686,7 @@ static int launch_chunk(dim3 grid, hipStream_t stream, const float* xbc, const f
   }
   hipLaunchKernelGGL((ssd_scores_kernel<NB>), dim3(max_chunks, sh.groups, grid.z), dim3(256), sbytes, stream, xbc, sh,
                      q_start, at_least, scores, max_chunks);
-  hipLaunchKernelGGL((ssd_chunk_kernel<NB, VEC>), grid, dim3(256), bytes, stream, xbc, dt, a_log, d_skip, sh, q_start,
+  hipLaunchKernelGGL((ssd_chunk_kernel<NB, VEC>), grid, dim3(256), 0, stream, xbc, dt, a_log, d_skip, sh, q_start,
                      state_slots, state, state_stride, y, at_least, scores, max_chunks);
   return 0;
 }
@@ -697,7 +710,7 @@ extern "C" int atoma_ssd_chunk(const float* xbc, const float* dt, const float* a
   dim3 grid((vdim + 15) / 16, heads, n_entries);
   int rc;
   // (a state size that is a multiple of 4 is then also a whole number of 16-byte pieces of its NB blocks' row)
-  const bool vec = n % 4 == 0 && (heads * vdim) % 4 == 0 && ((uintptr_t)xbc & 15) == 0;
+  const bool vec = n % 4 == 0 && (heads * vdim) % 4 == 0 && state_stride % 4 == 0 && (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0;
 #define ATOMA_CHUNK(NB_)                                                                                            \
   rc = vec ? launch_chunk<NB_, true>(grid, stream, xbc, dt, a_log, d_skip, sh, q_start, state_slots, state,        \
                                      state_stride, y, at_least, scores, max_chunks)                               \

@@ -185,6 +185,50 @@ def test_a_step_of_single_tokens_in_one_launch_is_the_same_bits(heads, groups, v
         assert torch.equal(got, want) and torch.equal(one, four)
 
 
+@pytest.mark.parametrize("heads, groups, vdim, n, taps", [(2, 2, 16, 5, 2), (3, 1, 17, 30, 3), (2, 1, 32, 36, 4), (4, 2, 9, 64, 1), (2, 1, 16, 65, 2),
+                                                          (2, 2, 20, 88, 4), (1, 1, 33, 100, 3), (4, 1, 64, 128, 4), (3, 3, 16, 127, 2)])
+def test_the_recurrence_by_chunks_and_token_by_token(heads, groups, vdim, n, taps):
+    """Entries at the edges of a chunk of 64 tokens and of its quarters beside single tokens, every number of blocks of 16 rows of the state,
+    rows that are and are not whole pieces of 16 bytes; against 64 bits.  A chunk sums n and 64 products, and an exponent's error is that of
+    the sum of up to 64 decays; a result carries at most four chunks' errors, all of the sizes that the absolute values' recurrence has."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(n)
+    r = lambda *k: torch.randn(*k, generator=g).to(DEV)
+    counts = [64, 1, 65, 128, 16, 17, 200, 1, 63]
+    t, inner = sum(counts), heads * vdim
+    channels, conv = inner + 2 * groups * n, (taps - 1) * (inner + 2 * groups * n)
+    xbc, dt = r(t, channels), torch.nn.functional.softplus(r(t, heads) - 1)
+    a_log, d_skip = r(heads) * 0.5, r(heads)
+    decay = torch.exp(-torch.exp(a_log) * dt)
+    state0 = r(len(counts) + 1, conv + inner * n)
+    slots = torch.randperm(len(counts) + 1, generator=g)[: len(counts)].to(DEV, torch.int32)
+    q_start = torch.tensor([sum(counts[:i]) for i in range(len(counts) + 1)], dtype=torch.int32, device=DEV)
+
+    def plain(absolute):
+        f = (lambda x: x.double().cpu().abs()) if absolute else (lambda x: x.double().cpu())
+        y, state = torch.empty(t, inner, dtype=torch.float64), f(state0)
+        rate, b_all = torch.exp(a_log.double().cpu()), f(xbc)
+        for e, c in enumerate(counts):
+            s = state[int(slots[e]), conv:].view(heads, vdim, n)
+            for j in range(int(q_start[e]), int(q_start[e]) + c):
+                x = b_all[j, :inner].view(heads, vdim)
+                bb, cc = (z.view(groups, n).repeat_interleave(heads // groups, 0) for z in b_all[j, inner:].split(groups * n))
+                d = dt[j].double().cpu()
+                s.copy_(torch.exp(-rate * d)[:, None, None] * s + (d[:, None] * x)[..., None] * bb[:, None])
+                y[j] = ((s * cc[:, None]).sum(-1) + f(d_skip)[:, None] * x).reshape(-1)
+        return y, state
+
+    (want, want_state), (size, size_state) = plain(False), plain(True)
+    sums = max(float((torch.exp(a_log) * dt[lo: lo + 64].sum(0)).max()) for lo in range(t))
+    bound = 4 * (n + 128 + 4 * sums) * 2.0 ** -24
+    for c in (counts, None):
+        state = state0.clone()
+        y = ops.ssd_scan(xbc, dt, decay, a_log, d_skip, heads, groups, vdim, n, taps, q_start, slots, state, c)
+        assert bool(((y.double().cpu() - want).abs() <= bound * size).all())
+        assert bool(((state.double().cpu() - want_state).abs() <= bound * size_state).all())
+        assert torch.equal(state[:, :conv], state0[:, :conv])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads, groups, vdim, n, taps, parts", [(4, 2, 16, 16, 3, 2), (3, 1, 8, 12, 2, 1), (2, 2, 40, 100, 5, 5),
                                                                  (1, 1, 5, 1, 1, 5), (6, 3, 24, 200, 4, 3), (4, 4, 64, 48, 4, 2),
