@@ -185,6 +185,40 @@ def test_a_step_of_single_tokens_in_one_launch_is_the_same_bits(heads, groups, v
         assert torch.equal(got, want) and torch.equal(one, four)
 
 
+@pytest.mark.parametrize("heads, groups, vdim, n, taps", [(4, 2, 33, 9, 4), (3, 1, 64, 32, 3), (2, 1, 100, 30, 2), (2, 2, 16, 4, 1), (2, 1, 24, 8, 5)])
+def test_the_convolution_of_many_tokens_at_a_time(heads, groups, vdim, n, taps):
+    """128 tokens and more go four to a workgroup, fewer one by one: entries that begin, end and lie inside a workgroup's four, a rest of one to
+    three tokens; the same bits as a step of each entry's own, and the closed form in 64 bits (five products, a sigmoid, an exponential)."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(taps)
+    r = lambda *k: torch.randn(*k, generator=g).to(DEV)
+    inner, keep = heads * vdim, taps - 1
+    channels = inner + 2 * groups * n
+    for counts in ([1, 2, 3, 4, 5, 1, 100, 1, 1, 10], [131], [1] * 130, [4, 125]):
+        t, e = sum(counts), len(counts)
+        q_start = [sum(counts[:i]) for i in range(e + 1)]
+        ends = torch.tensor(q_start, dtype=torch.int32, device=DEV)
+        seq = torch.repeat_interleave(torch.arange(e), torch.tensor(counts)).to(DEV, torch.int32)
+        slots = torch.randperm(e, generator=g).to(DEV, torch.int32)
+        ldp = inner + channels + heads + 3
+        proj, state = r(t, ldp), r(e, keep * channels + inner * n)
+        taps_w, conv_b, dt_bias, a_log = r(channels, taps), r(channels), r(heads), r(heads) * 0.5
+        run = lambda p, sq, qs, sl: ops.ssd_prepare(p, (0, inner, inner + channels), heads, groups, vdim, n, taps, sq, qs, sl, state, taps_w, conv_b,
+                                                    dt_bias, a_log)
+        got = run(proj, seq, ends, slots)
+        for i in range(e):
+            for lo in range(q_start[i], q_start[i + 1], 100):
+                if lo == q_start[i]:
+                    m = min(counts[i], 100)
+                    one = run(proj[lo: lo + m], torch.zeros_like(seq[:m]), torch.tensor([0, m], dtype=torch.int32, device=DEV), slots[i: i + 1])
+                    assert all(torch.equal(x, y[lo: lo + m]) for x, y in zip(one, got)), (counts, i)
+            before = state[slots[i].long(), : keep * channels].view(keep, channels).double()
+            x = torch.cat([before, proj[q_start[i]: q_start[i + 1], inner: inner + channels].double()])
+            terms = torch.stack([x[j: j + counts[i]] * taps_w[:, j].double() for j in range(taps)] + [conv_b.double().expand(counts[i], -1)])
+            y, size = terms.sum(0), terms.abs().sum(0)
+            assert bool(((got[0][q_start[i]: q_start[i + 1]].double() - y * torch.sigmoid(y)).abs() <= 32 * 2.0 ** -24 * size * (1 + size)).all())
+
+
 @pytest.mark.parametrize("heads, groups, vdim, n, taps", [(2, 2, 16, 5, 2), (3, 1, 17, 30, 3), (2, 1, 32, 36, 4), (4, 2, 9, 64, 1), (2, 1, 16, 65, 2),
                                                           (2, 2, 20, 88, 4), (1, 1, 33, 100, 3), (4, 1, 64, 128, 4), (3, 3, 16, 127, 2)])
 def test_the_recurrence_by_chunks_and_token_by_token(heads, groups, vdim, n, taps):
