@@ -294,14 +294,54 @@ ssd_step_kernel(const float* __restrict__ proj, SsdShape sh, const int32_t* __re
 // x, and S for y.  So a chunk has one barrier, and each operand is asked for as soon as the one before it has been used.
 // Bound by a wave's way through a chunk, 3.7 us with a state of 128, of which its 36 to 48 MFMAs for y and 32 for S are 1.1, and where
 // entries are many by all waves' instructions; it was 6 us, with five barriers and all operands through 108 KB of LDS, one workgroup a CU.
-// us with the scores, before / now: 64 heads of 64 x 128, one entry of 2,048 tokens 202 / 129, 1,400 and 640 207 / 111, eight of 256 229 / 114,
-// 64 of 32 599 / 223; 32 heads of 64 x 64, one of 2,048 142 / 96.  The results' bits are the same.  (The next chunk's sums of decays made
+// us with the scores, before / now: 64 heads of 64 x 128, one entry of 2,048 tokens 202 / 114, 1,400 and 640 206 / 95, eight of 256 229 / 98,
+// 64 of 32 598 / 212; 32 heads of 64 x 64, one of 2,048 143 / 87.  The results' bits are the same.  (The next chunk's sums of decays made
 // between this one's MFMAs, or B's rows by pairs, gave nothing: 139 and 135 against 136 at that point.)
 constexpr int kChunk = 64;
 constexpr int kChunkLdt = kChunk + 4;      // row stride of x transposed
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ auto buffer(const float* p, int floats) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, __builtin_amdgcn_readfirstlane(floats * 4), 0x00027000);
+}
+template <typename B>
+__device__ __forceinline__ float one(B from, uint32_t at) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
+}
+template <typename B>
+__device__ __forceinline__ f32x4 four(B from, uint32_t at) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0));
+}
+// the place of float `at`, or one that is out of any buffer's range and comes as zero (which stays a value of a register: known to be a
+// constant, it becomes a branch around the load)
+__device__ __forceinline__ uint32_t place(bool in, int at) {
+  uint32_t x = in ? (uint32_t)at * 4 : 0x80000000u;
+  asm("" : "+v"(x));
+  return x;
+}
+// a row's NB blocks of 16 columns from `row` on, of which the lane has 4 (l / 16) .. + 3; `last`: the places in the last block, which alone
+// can end early
+template <int NB, bool VEC, typename B>
+__device__ __forceinline__ void operand(B from, int row, const uint32_t (&last)[4], f32x4 (&x)[NB]) {
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if constexpr (VEC) {
+      x[b] = four(from, b < NB - 1 ? (uint32_t)(row + b * 16) * 4 : last[0]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[b][q] = one(from, b < NB - 1 ? (uint32_t)(row + b * 16 + q) * 4 : last[q]);
+    }
+  }
+}
+template <int NB, bool VEC>
+__device__ __forceinline__ void last_places(int row, int column, int n, uint32_t (&last)[4]) {
+#pragma unroll
+  for (int q = 0; q < (VEC ? 1 : 4); ++q) last[q] = place((NB - 1) * 16 + column + q < n, row + (NB - 1) * 16 + q);
+}
+#endif
 
 // VEC: C and S are fetched 16 bytes at a time (state size, channel counts and the state's rows all multiples of 4)
 template <int NB, bool VEC>      // NB: blocks of 16 rows of S (the state size rounded up)
@@ -312,7 +352,6 @@ ssd_chunk_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, co
                  float* __restrict__ y, int at_least, const float* __restrict__ scores, int max_chunks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int NP = 16 * NB, LDN = NP + 4, MINE = (NB + 3) / 4;      // MINE: blocks of 16 rows of S of a wave
-  constexpr uint32_t kOutside = 0x80000000u;                          // (out of any buffer's range: comes as zero)
   __shared__ __attribute__((aligned(16))) float St[2][16 * LDN];          // S transposed: [column][row], as the state keeps it
   __shared__ __attribute__((aligned(16))) float Xt[2][16 * kChunkLdt];    // x transposed: [column][token]
   __shared__ __attribute__((aligned(16))) float own[4][3][kChunk];        // of a wave: log decays summed up to a token, dt, and
@@ -332,25 +371,13 @@ ssd_chunk_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, co
 
   // a chunk's rows of xbc, of dt and of scores; past the last chunk nothing is in range.  (No load stands under a condition, which the
   // compiler would wait for where the branches meet.)
-  auto buffer = [&](const float* p, int floats) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, __builtin_amdgcn_readfirstlane(floats * 4), 0x00027000);
-  };
   auto rows_of = [&](int t0) { return max(0, min(kChunk, count - t0)); };
   auto inputs = [&](int t0) { return buffer(xbc + (size_t)(first + t0) * channels, rows_of(t0) * channels); };
-  auto one = [&](auto from, uint32_t at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0)); };
-  auto four = [&](auto from, uint32_t at) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0)); };
-  // (places that are out of range stay values of a register: known to be constants, they become branches around the loads)
-  auto place = [&](bool in, int at) {
-    uint32_t x = in ? (uint32_t)at * 4 : kOutside;
-    asm("" : "+v"(x));
-    return x;
-  };
   const uint32_t x_at = place((tid & 15) < vlive, (tid >> 4) * channels + h * sh.vdim + v0 + (tid & 15));
   const uint32_t y_at = place(r16 < vlive, (wave * 16 + 4 * kg) * inner + r16);
   const int c_row = (wave * 16 + r16) * channels + inner + gn + g * sh.n + 4 * kg;
-  uint32_t c_last[4], b_at[MINE], mt_at[4];      // (of C's blocks of 16 columns only the last one can end early)
-#pragma unroll
-  for (int q = 0; q < (VEC ? 1 : 4); ++q) c_last[q] = place((NB - 1) * 16 + 4 * kg + q < sh.n, c_row + (NB - 1) * 16 + q);
+  uint32_t c_last[4], b_at[MINE], mt_at[4];
+  last_places<NB, VEC>(c_row, 4 * kg, sh.n, c_last);
 #pragma unroll
   for (int m = 0; m < MINE; ++m) {
     const int n = (wave + 4 * m) * 16 + r16;
@@ -369,16 +396,7 @@ ssd_chunk_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, co
   };
   // C's rows of the wave's 16 tokens, and its tiles of scores
   auto fetch_c = [&](int t0) {
-    const auto from = inputs(t0);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if constexpr (VEC) {
-        cc[b] = four(from, b < NB - 1 ? (uint32_t)(c_row + b * 16) * 4 : c_last[0]);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cc[b][q] = one(from, b < NB - 1 ? (uint32_t)(c_row + b * 16 + q) * 4 : c_last[q]);
-      }
-    }
+    operand<NB, VEC>(inputs(t0), c_row, c_last, cc);
     const auto tiles = buffer(scores + (((size_t)e * max_chunks + t0 / kChunk) * sh.groups + g) * (10 * 256), rows_of(t0) > 0 ? 10 * 256 : 0);
 #pragma unroll
     for (int sb = 0; sb < 4; ++sb)
@@ -514,47 +532,33 @@ ssd_chunk_kernel(const float* __restrict__ xbc, const float* __restrict__ dt, co
 
 // C_t . B_s of every chunk of 64 tokens, once per group of heads: the ten 16 x 16 tiles on and below the diagonal, each
 // as its 64 lanes' four numbers (lane l: t = l % 16, s = 4 (l / 16) .. + 3 of the tile, as M's operand wants them),
-// [entry][chunk][group][10][64][4].
-template <int NB>
+// [entry][chunk][group][10][64][4].  A wave a tile, its operands straight from memory: one trip there and 4 NB MFMAs.  (2,048 tokens, a
+// state of 128: some 5 us; a workgroup a chunk, which took B and C to LDS first, 20.)
+template <int NB, bool VEC>
 __global__ void __launch_bounds__(256)
 ssd_scores_kernel(const float* __restrict__ xbc, SsdShape sh, const int32_t* __restrict__ q_start, int at_least,
                   float* __restrict__ scores, int max_chunks) {
-  constexpr int NP = 16 * NB, LDN = NP + 4;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* Bs = lds;
-  float* Cs = Bs + kChunk * LDN;
-  const int e = blockIdx.z, g = blockIdx.y, t0 = blockIdx.x * kChunk;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, kg = lane >> 4;
+  const int chunk = blockIdx.x / 3, j = blockIdx.x % 3 * 4 + wave, e = blockIdx.z, g = blockIdx.y, t0 = chunk * kChunk;
   const int first = q_start[e], count = q_start[e + 1] - first;
-  if (count < at_least || t0 >= count) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r16 = lane & 15, kg = lane >> 4;
+  if (count < at_least || t0 >= count || j >= 10) return;
+  const int tb = j >= 6 ? 3 : j >= 3 ? 2 : j >= 1 ? 1 : 0, sb = j - tb * (tb + 1) / 2;
   const int inner = sh.heads * sh.vdim, gn = sh.groups * sh.n, channels = inner + 2 * gn;
-  const int nt = min(kChunk, count - t0);
-  for (int idx = tid; idx < kChunk * NP; idx += 256) {
-    const int tt = idx / NP, n = idx % NP;
-    const bool in = tt < nt && n < sh.n;
-    const size_t base = ((size_t)(first + t0) + tt) * channels + inner + (size_t)g * sh.n + n;
-    Bs[tt * LDN + n] = in ? xbc[base] : 0.f;
-    Cs[tt * LDN + n] = in ? xbc[base + gn] : 0.f;
-  }
-  __syncthreads();
-  float* out = scores + (((size_t)e * max_chunks + blockIdx.x) * sh.groups + g) * (10 * 256);
+  const auto from = buffer(xbc + (size_t)(first + t0) * channels, min(kChunk, count - t0) * channels);
+  const int b_row = (sb * 16 + r16) * channels + inner + g * sh.n + 4 * kg, c_row = (tb * 16 + r16) * channels + inner + gn + g * sh.n + 4 * kg;
+  uint32_t b_last[4], c_last[4];
+  last_places<NB, VEC>(b_row, 4 * kg, sh.n, b_last);
+  last_places<NB, VEC>(c_row, 4 * kg, sh.n, c_last);
+  f32x4 bb[NB], cc[NB], acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  operand<NB, VEC>(from, b_row, b_last, bb);
+  operand<NB, VEC>(from, c_row, c_last, cc);
 #pragma unroll
-  for (int j = 0; j < 10; ++j) {
-    const int tb = j >= 6 ? 3 : j >= 3 ? 2 : j >= 1 ? 1 : 0, sb = j - tb * (tb + 1) / 2;
-    if ((j & 3) == wave) {
-      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      const float* cp = Cs + (tb * 16 + r16) * LDN + 4 * kg;
-      const float* bp = Bs + (sb * 16 + r16) * LDN + 4 * kg;
+  for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int k = 0; k < NP; k += 16) {
-        const f32x4 a4 = lds4(cp + k), b4 = lds4(bp + k);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[q], a4[q], acc, 0, 0, 0);
-      }
-      *reinterpret_cast<f32x4*>(out + (j * 64 + lane) * 4) = acc;
-    }
-  }
+    for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bb[b][q], cc[b][q], acc, 0, 0, 0);
+  *reinterpret_cast<f32x4*>(scores + ((((size_t)e * max_chunks + chunk) * sh.groups + g) * 10 + j) * 256 + lane * 4) = acc;
+#endif
 }
 
 // What is left of the convolution's state after ssd_step_kernel (state: null elsewhere): channels from `first` on of the token's request
@@ -714,17 +718,7 @@ template <int NB, bool VEC>
 static int launch_chunk(dim3 grid, hipStream_t stream, const float* xbc, const float* dt, const float* a_log,
                         const float* d_skip, const SsdShape& sh, const int32_t* q_start, const int32_t* state_slots,
                         float* state, size_t state_stride, float* y, int at_least, float* scores, int max_chunks) {
-  const size_t sbytes = (size_t)2 * kChunk * (16 * NB + 4) * sizeof(float);
-  static bool asked = false;      // (per instantiation) more than the default 64 KB of LDS
-  if (!asked) {
-    if (sbytes > 64 * 1024) {
-      hipError_t err = hipFuncSetAttribute((const void*)ssd_scores_kernel<NB>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)sbytes);
-      if (err != hipSuccess) return (int)err;
-    }
-    asked = true;
-  }
-  hipLaunchKernelGGL((ssd_scores_kernel<NB>), dim3(max_chunks, sh.groups, grid.z), dim3(256), sbytes, stream, xbc, sh,
+  hipLaunchKernelGGL((ssd_scores_kernel<NB, VEC>), dim3(3 * max_chunks, sh.groups, grid.z), dim3(256), 0, stream, xbc, sh,
                      q_start, at_least, scores, max_chunks);
   hipLaunchKernelGGL((ssd_chunk_kernel<NB, VEC>), grid, dim3(256), 0, stream, xbc, dt, a_log, d_skip, sh, q_start,
                      state_slots, state, state_stride, y, at_least, scores, max_chunks);
