@@ -500,6 +500,18 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   const int wm = wave / C::WN, wn = wave % C::WN;
   const uint32_t xr = (wm * (C::XH / C::WM) + r16) * 128, wr = (wn * (C::WH / C::WN) + r16) * 128;
 
+  // lanes 0 .. 31: the wave's rows of X's first half, 32 .. 63: of the second
+  int pos_of = 0, page_of = -1, off_of = 0;
+  if constexpr (EPI == kOutRope) {
+    static_assert(C::XH / C::WM == 32, "");
+    const int row = m0 + (lane >> 5) * C::XH + wm * 32 + (lane & 31);
+    if (row < M) {
+      const int slot = out.rope.slot_mapping[row];
+      pos_of = out.rope.positions[row];
+      if (slot >= 0) page_of = slot / out.rope.page_size, off_of = slot - page_of * out.rope.page_size;
+    }
+  }
+
   const int steps = k_len / 64;
   auto load_first = [&](char* __restrict__ buf, int s) {
     issue<C::QX, C::XI, C::NW>(buf + C::X0, xb0, s * 128, xo, wave);
@@ -560,6 +572,32 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   } else {
     step(one, s, b0, b0, b1, fa, fb);
     step(none, s + 1, b1, b1, b0, fb, fa);
+  }
+  if constexpr (EPI == kOutRope) {
+    // (all sums at once do not fit LDS: a half of X's rows by a half of W's at a time.  2,048 rows against 6,144 x 4,096: 256 tiles of 256 x
+    // 192, 86 us; by 256 x 96 103, by the library with the rotation's kernel behind it 93)
+    constexpr int COLS = C::WH / C::WN;
+    meet();                  // everybody's reads of the last step are done
+    float* const sums = reinterpret_cast<float*>(lds) + wave * (32 * COLS);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int from = h * 32 + (lane & 31), pos = __shfl(pos_of, from, 64), page = __shfl(page_of, from, 64), off = __shfl(off_of, from, 64);
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+#pragma unroll
+        for (int j = 0; j < C::JX; ++j)
+#pragma unroll
+          for (int i = 0; i < C::JW; ++i)
+            *reinterpret_cast<f32x4*>(sums + (j * 16 + r16) * COLS + i * 16 + kg * 4) = acc[g][h][i][j];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        const int nw = n0 + g * C::WH + wn * COLS;
+        if (nw < N) rope_tile<32, COLS>(sums, m0 + h * C::XH + wm * 32, M, nw, N, pos, page, off, out.rope, (uint16_t*)out.c, out.ldc, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    return;
   }
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -637,6 +675,9 @@ static int pick(int tile, const void* x, const void* w, int M, int N, int K, int
     // 21.6.  Planes of 3,072 x 8,192 13.7 by 64 x 128 in eight slices, 15.4 by 64 x 64.
     case 6: if constexpr (EPI == kOutF32 || GATED) ATOMA_TILE(64, 64, 2, 2, 4); break;
     case 7: if constexpr (EPI == kOutF32) ATOMA_TILE(64, 128, 2, 2, 3); break;
+    case 8:
+      if constexpr (EPI == kOutRope) return launch_phased<Phased<256, 192, 4, 2>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream);
+      break;
   }
 #undef ATOMA_TILE
   return ATOMA_ERR_SHAPE;
