@@ -24,6 +24,7 @@ DEFAULT_RANDOM_SEED = 1_283_768_955  # backends/vllm/src/validation.rs:11
 _PACKED = np.dtype([("temperature", "<f4"), ("top_p", "<f4"), ("penalty", "<f4"), ("top_k", "<i4"), ("seed", "<u8"), ("greedy", "<i4"),
                     ("penalised", "<i4")])
 _PACK = struct.Struct("<fffiQii").pack
+MAX_TOP_K = (1 << 31) - 1            # what a step's parameters hold; no vocabulary is as large, so a larger cut is this one: none
 
 
 class ValidationError(ValueError):
@@ -85,7 +86,8 @@ class SamplingPlan:
         """What a step writes of this plan, as the sampler's native packing reads it; made once a plan."""
         row = np.zeros((), _PACKED)
         row["temperature"], row["top_p"], row["penalty"] = self.temperature, self.top_p, self.repetition_penalty
-        row["top_k"], row["seed"], row["greedy"] = np.array(self.top_k).astype(np.int32), int(self.random_seed) & (1 << 64) - 1, self.greedy
+        row["top_k"] = min(int(self.top_k), MAX_TOP_K)
+        row["seed"], row["greedy"] = int(self.random_seed) & (1 << 64) - 1, self.greedy
         row["penalised"] = self.repetition_penalty != 1.0 and self.repeat_last_n > 0
         return row.tobytes()
 

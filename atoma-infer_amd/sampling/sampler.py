@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from ..kernels import load_host_library, ops
-from .params import SamplingPlan
+from .params import MAX_TOP_K, SamplingPlan
 
 _MASK = (1 << 64) - 1
 # vocabularies from which on the rows of a step that draws are cut into parts (a block walks fewer values quickly enough)
@@ -168,7 +168,7 @@ class Sampler:
                 mn[1, i] = pl.top_p
                 mn[2, i] = 0.0 if pl.greedy else uniform(pl.random_seed, steps[i])
                 mn[3, i] = pl.repetition_penalty
-                ints[i] = pl.top_k
+                ints[i] = pl.top_k if pl.top_k <= MAX_TOP_K else MAX_TOP_K
         m = meta.to(self.device, non_blocking=True)
         if all_greedy:
             # (top_p, penalty and top_k of a greedy row are never read; the copy kept is this batch's)

@@ -92,3 +92,26 @@ def test_a_steps_parameters_packed_natively_are_the_plans():
                              [uniform(p.random_seed, c) for p, c in zip(plans, steps)],
                              [p.repetition_penalty for p in plans]], np.float32)
             assert (meta.numpy()[:4] == want).all() and meta.numpy()[4].view(np.int32).tolist() == [p.top_k for p in plans]
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 64])
+@pytest.mark.parametrize("top_k", [2 ** 31 - 1, 2 ** 31, 2 ** 32 + 1, 2 ** 32 + 40, 2 ** 64])
+def test_a_top_k_beyond_32_bits_is_no_cut_beside_any_number_of_rows(monkeypatch, rows, top_k):
+    """No vocabulary is as large as the largest number that a step's parameters hold, so that is what such a cut becomes: in the rows that
+    are written one by one and in those that are packed natively, which also count it as a cut beyond the lists."""
+    import torch
+
+    from atoma_infer_amd.kernels import ops
+    from atoma_infer_amd.sampling import Sampler, sampler
+    empty, seen = torch.empty, {}
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))
+    monkeypatch.setattr(torch.cuda, "Event", lambda: type("E", (), {"record": lambda self: None, "synchronize": lambda self: None})())
+
+    def draw(logits, temperature, top_k, top_p, uniform, **how):
+        seen.update(top_k=top_k.tolist(), how=how)
+        return torch.zeros(2, logits.shape[0])
+    monkeypatch.setattr(ops, "sample_packed", draw)
+    plans = [plan(do_sample=True, temperature=0.7, top_k=40) for _ in range(rows - 1)] + [plan(do_sample=True, temperature=0.7, top_k=top_k)]
+    Sampler(torch.device("cpu")).launch(torch.zeros(rows, sampler.SPLIT_MIN_VOCAB), plans, [0] * rows, [()] * rows)
+    assert seen["top_k"] == [40] * (rows - 1) + [2 ** 31 - 1]
+    assert seen["how"] == dict(split=True, cuts=True, few=False, top_p_cuts=False)
