@@ -165,16 +165,20 @@ __device__ __forceinline__ uint32_t high_halves(float lo, float hi) {      // th
   return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302);
 }
 // Exact but for what lies below 2^-133 (bfloat16's smallest number).  An infinite value's second and third number are those of
-// the largest finite one, so that its products stay infinities.
+// the largest finite one, so that its products stay infinities.  What is no number stays none: a payload in the lower half alone, which
+// the first number loses, is that of a signalling one, and v_med3_f32, which is the least of its operands then, passes on such a one as
+// the last of them (the test of these products holds it to that; with the value in front it would be the largest number's negative).
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
   u32x4 h[3];
+  float most = 3.402823466e38f;
+  asm("" : "+s"(most));      // (constants would be moved behind the value)
 #pragma unroll
   for (int i = 0; i < 8; i += 2) {
     float r[2], t[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const float v = __builtin_amdgcn_fmed3f(x[i + e], -3.402823466e38f, 3.402823466e38f);
+      const float v = __builtin_amdgcn_fmed3f(-most, most, x[i + e]);
       r[e] = v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
       t[e] = r[e] - __uint_as_float(__float_as_uint(r[e]) & 0xffff0000u);
     }

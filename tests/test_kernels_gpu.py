@@ -152,7 +152,8 @@ def test_gemm_generic_row_alone(n, k, wdt):
 def test_gemm_float32_by_bfloat16_thirds(m, n, k):
     """float32 rows against a bfloat16 weight: every number of blocks a streaming workgroup takes, every tile, and both sides of the
     longest part of K that goes to the bfloat16 instruction.  The three numbers that a value is cut into hold all of it, so the bound is
-    that of any float32 sum, three additions a product.  Infinities, NaN and large numbers stay what they are."""
+    that of any float32 sum, three additions a product.  Infinities, NaN (those with all of their payload in the lower sixteen bits too) and
+    large numbers stay what they are."""
     from atoma_infer_amd.kernels import ops
     a, w = rnd(m, k, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
     c = ops.gemm_generic(a, w, torch.float32)
@@ -169,6 +170,9 @@ def test_gemm_float32_by_bfloat16_thirds(m, n, k):
     assert torch.equal(got.isnan(), want.isnan())
     bad = want.isinf() & (want.double() - (a.double() @ w.double().T)).isnan()        # (infinite in 64 bits too)
     assert torch.equal(got[bad], want[bad])
+    rows = [m // 4, m - 1 - m // 4]
+    a[rows[0]].view(torch.int32)[13], a[rows[1]].view(torch.int32)[k - 1] = 0x7f800001, -0x7fffff      # (0x7f800001, 0xff800001)
+    assert bool(ops.gemm_generic(a, w, torch.float32)[rows].isnan().all())
 
 
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 48, 64])
