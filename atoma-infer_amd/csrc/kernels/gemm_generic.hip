@@ -12,7 +12,7 @@
 //                      split over the workgroup's waves, whose sums meet in LDS.  Bound by W's bytes up to 16 rows of A.
 //                      It also takes more rows where tiles of 64 x 64 would be fewer than the CUs (four waves of a tile
 //                      walk all of K, eight of a streaming workgroup an eighth of it each);
-//   split_tile_kernel, split_stream_kernel, split_few_kernel (up to eight rows)
+//   split_tile_kernel, split_stream_kernel, split_few_kernel (up to 24 rows)
 //                      the same for float32 rows against a bfloat16 weight, which is the 32-bit path of a bfloat16 checkpoint:
 //                      every float32 value as three bfloat16 ones (gemm_f32_tile.h), at three bfloat16 MFMAs for 32 values of K.
 //                      Tiles are bound by what a step costs beside its MFMAs (splitting A, a trip through LDS, a barrier: 1.4 us for
@@ -294,16 +294,17 @@ split_stream_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, T
   }
 }
 
-// The same for up to 4 RW rows of A, 4 or 8: sixteen lanes split a row's values of four steps and hand them to the others through LDS,
-// so that no lane splits what another splits too (every wave has its own corner of LDS, which it fills and reads in order).
-template <int RW, int RT, int WK, typename TC>
+// The same for up to 4 RW rows of A, 4 to 16, behind FULL blocks of 16 (none or one): sixteen lanes split a row's values of four steps and
+// hand them to the others through LDS, so that no lane splits what another splits too (every wave has its own corner of LDS, which it
+// fills and reads in order, with more than eight rows half a batch at a time).  A full block's rows are each lane's own.
+template <int FULL, int RW, int RT, int WK, typename TC>
 __global__ void __launch_bounds__(64 * WK)
 split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* __restrict__ c, int M, int N, int K, int lda,
                  int ldw, int ldc) {
-  constexpr int BITS = WK == 8 ? 3 : 2, U = 4;             // steps of a batch
+  constexpr int BITS = WK == 8 ? 3 : 2, U = 4, H = RW > 2 ? U / 2 : U;      // steps of a batch, and at a time in LDS
   static_assert(WK == 1 << BITS, "a wave a part of K");
-  __shared__ f32x4_t red[WK - 1][RT][64];
-  __shared__ bf16x8_t thirds[WK][3][RW * 4][U * 4];
+  __shared__ f32x4_t red[WK - 1][FULL + 1][RT][64];
+  __shared__ bf16x8_t thirds[WK][3][RW * 4][H * 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r16 = lane & 15, kg = lane >> 4;
   const int n0 = blockIdx.x * (16 * RT);
@@ -313,21 +314,29 @@ split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* 
   for (int i = 0; i < RT; ++i) wp[i] = w + (size_t)min(n0 + i * 16 + r16, N - 1) * ldw + kg * 8;
   const float* ap[RW];                                     // lane l splits values 8 (l % 16) .. + 7 of a batch, of rows l / 16 + 4 r
 #pragma unroll
-  for (int r = 0; r < RW; ++r) ap[r] = a + (size_t)min(kg + r * 4, M - 1) * lda + r16 * 8;
-  f32x4_t acc[RT];
+  for (int r = 0; r < RW; ++r) ap[r] = a + (size_t)min(FULL * 16 + kg + r * 4, M - 1) * lda + r16 * 8;
+  const float* own[FULL + 1];                              // its own values of a step
 #pragma unroll
-  for (int i = 0; i < RT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  struct Batch { bf16x8_t w[U][RT]; f32x4_t a[RW][2]; };
+  for (int m = 0; m <= FULL; ++m) own[m] = a + (size_t)min(m * 16 + r16, M - 1) * lda + kg * 8;
+  f32x4_t acc[FULL + 1][RT];
+#pragma unroll
+  for (int m = 0; m <= FULL; ++m)
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[m][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  struct Batch { bf16x8_t w[U][RT]; f32x4_t full[U][FULL + 1][2], a[RW][2]; };
   auto fetch = [&](Batch& x, int s) {
 #pragma unroll
     for (int r = 0; r < RW; ++r) split_load<true>(ap[r], s * 32, K, x.a[r]);
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int i = 0; i < RT; ++i) x.w[u][i] = *reinterpret_cast<const bf16x8_t*>(wp[i] + (s + u) * 32);
+#pragma unroll
+      for (int m = 0; m < FULL; ++m) split_load<true>(own[m], (s + u) * 32, K, x.full[u][m]);
+    }
   };
   const int row = r16 % (RW * 4);
-  auto add = [&](bf16x8_t (&wv)[RT], const bf16x8_t (&p)[3]) {
+  auto add = [&](bf16x8_t (&wv)[RT], const Split8 (&p)[FULL + 1]) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       if (q == 1) {
@@ -335,22 +344,40 @@ split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* 
         for (int i = 0; i < RT; ++i) wv[i] = split_weight(wv[i]);
       }
 #pragma unroll
-      for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], p[q], acc[i], 0, 0, 0);
+      for (int m = 0; m <= FULL; ++m)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], p[m].p[q], acc[m][i], 0, 0, 0);
     }
   };
   auto take = [&](Batch& x) {
+    Split8 t[H < U ? RW : 1];
+    auto put = [&](const Split8& v, int r) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) thirds[wave][q][kg + r * 4][r16 % (H * 4)] = v.p[q];
+    };
 #pragma unroll
     for (int r = 0; r < RW; ++r) {
-      const Split8 t = split_of(x.a[r]);
-      thirds[wave][0][kg + r * 4][r16] = t.p[0], thirds[wave][1][kg + r * 4][r16] = t.p[1], thirds[wave][2][kg + r * 4][r16] = t.p[2];
+      if constexpr (H < U) t[r] = split_of(x.a[r]);
+      else put(split_of(x.a[r]), r);
     }
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bf16x8_t p[3] = {thirds[wave][0][row][u * 4 + kg], thirds[wave][1][row][u * 4 + kg], thirds[wave][2][row][u * 4 + kg]};
-      add(x.w[u], p);
+    for (int h = 0; h < U; h += H) {
+      if (H < U && r16 / (H * 4) == h / H) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r) put(t[r], r);
+      }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = h; u < h + H; ++u) {
+        Split8 p[FULL + 1];
+#pragma unroll
+        for (int m = 0; m < FULL; ++m) p[m] = split_of(x.full[u][m]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) p[FULL].p[q] = thirds[wave][q][row][(u - h) * 4 + kg];
+        add(x.w[u], p);
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-    __builtin_amdgcn_wave_barrier();
   };
   // two batches in turn: while the MFMAs of one run, the loads of the other are on their way
   Batch x[2];
@@ -364,28 +391,36 @@ split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* 
     take(x[1]);
   }
   if (b < batches) take(x[0]);
-  const float* const own = a + (size_t)min(r16, M - 1) * lda + kg * 8;
   for (int s = begin + batches * U; s < end; ++s) {        // (steps that fill no batch: every lane its own)
-    f32x4_t v[2];
-    split_load<true>(own, s * 32, K, v);
+    f32x4_t v[FULL + 1][2];
     bf16x8_t wv[RT];
 #pragma unroll
+    for (int m = 0; m <= FULL; ++m) split_load<true>(own[m], s * 32, K, v[m]);
+#pragma unroll
     for (int i = 0; i < RT; ++i) wv[i] = *reinterpret_cast<const bf16x8_t*>(wp[i] + s * 32);
-    const Split8 t = split_of(v);
-    add(wv, t.p);
+    Split8 p[FULL + 1];
+#pragma unroll
+    for (int m = 0; m <= FULL; ++m) p[m] = split_of(v[m]);
+    add(wv, p);
   }
   if (wave > 0) {
 #pragma unroll
-    for (int i = 0; i < RT; ++i) red[wave - 1][i][lane] = acc[i];
+    for (int m = 0; m <= FULL; ++m)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) red[wave - 1][m][i][lane] = acc[m][i];
   }
   __syncthreads();
-  if (wave > 0 || r16 >= M) return;
+  if (wave > 0) return;
   const bool aligned = aligned4(c, ldc);
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
+  for (int m = 0; m <= FULL; ++m) {
+    if (m * 16 + r16 >= M) continue;
 #pragma unroll
-    for (int q = 0; q < WK - 1; ++q) acc[i] += red[q][i][lane];
-    put4(c + (size_t)r16 * ldc, n0 + i * 16 + kg * 4, N, aligned, acc[i]);
+    for (int i = 0; i < RT; ++i) {
+#pragma unroll
+      for (int q = 0; q < WK - 1; ++q) acc[m][i] += red[q][m][i][lane];
+      put4(c + (size_t)(m * 16 + r16) * ldc, n0 + i * 16 + kg * 4, N, aligned, acc[m][i]);
+    }
   }
 }
 
@@ -406,19 +441,21 @@ static void launch_stream(const TA* a, const TW* w, TC* c, int M, int N, int K, 
 #undef ATOMA_STREAM
 }
 
-template <int RW, int RT, typename TC>
+template <int FULL, int RW, int RT, typename TC>
 static int launch_split_few(const float* a, const bf16_t* w, TC* c, int M, int N, int K, int lda, int ldw, int ldc, hipStream_t stream) {
   const dim3 grid(ceil_div(N, 16 * RT));
   // (a wave a part of K)
   if constexpr (RT == 1) {
-    if (f32_part_bits(N) == 3) {
-      hipLaunchKernelGGL((split_few_kernel<RW, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+    if (FULL > 0 || RW > 2 || f32_part_bits(N) == 3) {      // (of many columns only up to eight rows come here)
+      hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
       ATOMA_LAUNCH_CHECK();
       return 0;
     }
   }
-  hipLaunchKernelGGL((split_few_kernel<RW, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
-  ATOMA_LAUNCH_CHECK();
+  if constexpr (FULL == 0 && RW <= 2) {
+    hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+    ATOMA_LAUNCH_CHECK();
+  }
   return 0;
 }
 
@@ -472,20 +509,28 @@ static int launch_split(const float* a, const bf16_t* w, TC* c, int M, int N, in
     auto round = [&](int mt, int rt, int most) { return (int64_t)ceil_div(N, 16 * rt) * ceil_div(M, 16 * mt) <= most; };
     // (up to eight rows the splitting is shared: 4 rows, 2,048 x 8,192 16.5 -> 11.4 us, 28,672 x 4,096 53 -> 41, the head of Llama 1B 101 -> 87;
     // two blocks of the weight against one, 4 rows: 5,120 x 3,072 9.3 and 10.0, 28,672 x 4,096 43.6 and 41.1)
-#define ATOMA_FEW(RW, RT) return launch_split_few<RW, RT>(a, w, c, M, N, K, lda, ldw, ldc, stream)
+#define ATOMA_FEW(FULL, RW, RT) return launch_split_few<FULL, RW, RT>(a, w, c, M, N, K, lda, ldw, ldc, stream)
     if (M <= 4) {
-      if (!wide || (N > 16384 && N < 65536)) ATOMA_FEW(1, 1);
-      ATOMA_FEW(1, 2);
+      if (!wide || (N > 16384 && N < 65536)) ATOMA_FEW(0, 1, 1);
+      ATOMA_FEW(0, 1, 2);
     }
-    if (M <= 8 && wide) ATOMA_FEW(2, 2);
-    if (M <= 8 && (M > 6 || K > 4096)) ATOMA_FEW(2, 1);      // (5 rows, 2,048 x 2,048: 6.0 against 5.5 by the kernel below)
-#undef ATOMA_FEW
+    if (M <= 8 && wide) ATOMA_FEW(0, 2, 2);
+    if (M <= 8 && (M > 6 || K > 4096)) ATOMA_FEW(0, 2, 1);      // (5 rows, 2,048 x 2,048: 6.0 against 5.5 by the kernel below)
     if (!wide) {
+      // (up to sixteen rows of long K likewise: 9 rows, 4,096 x 8,192 21.1 -> 18.8 us, x 4,096 11.5 -> 11.1, but x 3,584 10.3 -> 11.2; 16 rows,
+      // x 8,192 24.9 -> 22.6, 13 of x 5,120 16.2 -> 16.1, but of x 4,096 12.8 -> 13.1)
+      if (M <= 12 && K >= 4096) ATOMA_FEW(0, 3, 1);
+      if (M <= 16 && K >= 5120) ATOMA_FEW(0, 4, 1);
       if (round(1, 1, kCUs)) ATOMA_STREAM(1, 1);
-      if (M <= 20 && round(2, 1, kCUs)) ATOMA_STREAM(2, 1);
+      // (a block of sixteen rows and up to eight behind it, against two blocks: 17 rows, 4,096 x 8,192 25.9 and 29.3 us, x 3,072 11.9 and 13.7, x
+      // 1,024 5.35 and 5.65, x 768 4.94 and 4.67; 24 rows, against one block and two of the weight: 29.3 and 31.3, 13.5 and 13.7, 5.74 and 5.84)
+      if (M <= 20 && K >= 1024) ATOMA_FEW(1, 1, 1);
+      if (M <= 24 && K >= 1024) ATOMA_FEW(1, 2, 1);
+      if (M <= 20) ATOMA_STREAM(2, 1);
       if (round(1, 2, kCUs)) ATOMA_STREAM(1, 2);
       if (round(2, 2, 320)) ATOMA_STREAM(2, 2);
       if (round(4, 2, kCUs)) ATOMA_STREAM(4, 2);
+#undef ATOMA_FEW
     } else if (M <= 16) {
       if (N <= 8192) ATOMA_STREAM(1, 2);      // (16 rows, 8,192 x 4,096: 18.8 us, 26.9 by four blocks; 28,672 x 4,096: 65.7 and 57.8)
       ATOMA_STREAM(1, 4);

@@ -117,17 +117,18 @@ def test_gemm_generic_kernels(m, n, k, wdt):
     assert bool(((c.double() - want).abs() <= k * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)).all())
 
 
-@pytest.mark.parametrize("n,k", [(2048, 2048), (4112, 544), (100, 100), (4096, 36), (130, 4128), (16384, 96), (7, 1003)])
+@pytest.mark.parametrize("n,k", [(2048, 2048), (4112, 544), (100, 100), (4096, 36), (130, 4128), (16384, 96), (7, 1003), (2500, 1184)])
 @pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
 def test_gemm_generic_row_alone(n, k, wdt):
     """A row's float32 results are the same bits with 1 row and with thousands beside it, wherever it lies among them: by the
-    streaming kernel (four or eight parts of K, some of them empty), by either tile, with rows that are not aligned, and by the
-    low-rank kernel, whose multiply-adds are written one after the other."""
+    streaming kernel (four or eight parts of K, some of them empty), by those of few rows (whole batches of steps with and without a
+    rest behind them), by either tile, with rows that are not aligned, and by the low-rank kernel."""
     from atoma_infer_amd.kernels import ops
     wide = rnd(2200, k + 8, seed=1)
     a, w = wide[:, 4:4 + k], rnd(n, k, dtype=wdt, seed=2)
     full = ops.gemm_generic(a, w, torch.float32)
-    for m, at in ((1, 0), (1, 2199), (16, 3), (17, 100), (64, 0), (65, 7), (200, 1900), (836, 1000)):
+    for m, at in ((1, 0), (1, 2199), (2, 9), (4, 2000), (5, 1), (7, 300), (8, 77), (9, 1500), (12, 6), (13, 700), (16, 3), (17, 100), (20, 5),
+                  (21, 64), (24, 1111), (64, 0), (65, 7), (200, 1900), (836, 1000)):
         assert torch.equal(ops.gemm_generic(a[at:at + m], w, torch.float32), full[at:at + m])
     odd = torch.empty(2200, k + 1, device=DEV)[:, 1:]
     odd.copy_(a)
@@ -148,7 +149,8 @@ def test_gemm_generic_row_alone(n, k, wdt):
                                    (1, 5000, 64), (1, 40000, 32), (5, 5003, 96), (7, 9000, 64), (17, 4112, 288), (33, 5120, 64),
                                    (70, 5200, 96), (130, 5100, 160), (140, 20000, 64), (1100, 8200, 352), (200, 130, 8192),
                                    (70, 4100, 4096), (3, 4100, 4128), (3, 2050, 1696), (8, 1000, 1184), (4, 20000, 544), (5, 5003, 608),
-                                   (2, 70000, 544)])
+                                   (2, 70000, 544), (9, 2050, 4160), (12, 1000, 4096), (13, 500, 5152), (16, 4090, 8192), (17, 2500, 1184),
+                                   (20, 4096, 32), (20, 4096, 1056), (21, 3000, 96), (24, 4090, 1696)])
 def test_gemm_float32_by_bfloat16_thirds(m, n, k):
     """float32 rows against a bfloat16 weight: every number of blocks a streaming workgroup takes, every tile, and both sides of the
     longest part of K that goes to the bfloat16 instruction.  The three numbers that a value is cut into hold all of it, so the bound is
