@@ -472,7 +472,8 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
     w += (size_t)g * N * ldw;
   }
   const int rows_x = min(C::BM, M - m0), rows_w = min(C::BN, N - n0);
-  // a half's rows through a buffer of its own: what lies past the last row is out of its range, reads as zero and is never stored
+  // a half's rows through a buffer of its own: what lies past the last row is out of its range, reads as zero and is never stored.  A second
+  // half without a row is the first one again: no load has a place in K beyond the end of its buffer.
   const int lr = lane >> 3;
   const uint32_t piece = ((lane & 7) ^ lr) * 16;
   uint32_t xo[C::XI], wo[C::WI];
@@ -481,12 +482,13 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
 #pragma unroll
   for (int i = 0; i < C::WI; ++i) wo[i] = (uint32_t)(min(i * C::NW + wave, C::QW - 1) * 8 + lr) * ldw * 2 + piece;
   auto half = [&](const uint16_t* p, int ld, int there) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, there <= 0 ? 0 : ((there - 1) * ld + k_len) * 2, 0x00027000);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, ((there - 1) * ld + k_len) * 2, 0x00027000);
   };
   const uint16_t* const xp = x + (size_t)m0 * ldx + k0;
   const uint16_t* const wp = w + (size_t)n0 * ldw + k0;
-  const rsrc_t xb0 = half(xp, ldx, min(rows_x, C::XH)), xb1 = half(xp + (size_t)C::XH * ldx, ldx, rows_x - C::XH);
-  const rsrc_t wb0 = half(wp, ldw, min(rows_w, C::WH)), wb1 = half(wp + (size_t)C::WH * ldw, ldw, rows_w - C::WH);
+  const int x1 = rows_x > C::XH ? C::XH : 0, w1 = rows_w > C::WH ? C::WH : 0;
+  const rsrc_t xb0 = half(xp, ldx, min(rows_x, C::XH)), xb1 = half(xp + (size_t)x1 * ldx, ldx, min(rows_x - x1, C::XH));
+  const rsrc_t wb0 = half(wp, ldw, min(rows_w, C::WH)), wb1 = half(wp + (size_t)w1 * ldw, ldw, min(rows_w - w1, C::WH));
 
   f32x4 acc[2][2][C::JW][C::JX];          // by half of W, half of X
 #pragma unroll
@@ -577,6 +579,7 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
     // (all sums at once do not fit LDS: a half of X's rows by a half of W's at a time.  2,048 rows against 6,144 x 4,096: 256 tiles of 256 x
     // 192, 86 us; by 256 x 96 103, by the library with the rotation's kernel behind it 93)
     constexpr int COLS = C::WH / C::WN;
+    wait<0, true>();
     meet();                  // everybody's reads of the last step are done
     float* const sums = reinterpret_cast<float*>(lds) + wave * (32 * COLS);
 #pragma unroll

@@ -1192,6 +1192,34 @@ def test_gemm_tile_rope(m, nh, nkv, hd, k, page):
     assert gemm_bf16.try_tile_rope(x[:64], w, pos, cos, sin, kc, vc, slots, page, nh, nkv, hd) is None       # (few rows)
 
 
+@pytest.mark.parametrize("m,nh,nkv,hd,k", [(300, 6, 2, 64, 256), (385, 8, 2, 64, 320), (129, 4, 1, 128, 384), (641, 6, 2, 48, 448), (256, 5, 1, 64, 640),
+                                           (513, 24, 8, 128, 704)])
+def test_gemm_tile_rope_in_phases_equals_the_one_by_steps(m, nh, nkv, hd, k):
+    """The tile of 256 x 192 sums as the others do, so q, k and v are theirs bit for bit: 4 to 7, 10 and 11 steps of K (none to four turns of
+    its loop behind an even and an odd number), rows that end in a tile's first and second half, columns that do and do not fill the
+    last tile, a padding row, and caches that keep what no token writes."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    page, n = 16, (nh + 2 * nkv) * hd
+    pages = -(-m // page) + 2
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    g = torch.Generator().manual_seed(5)
+    pos = torch.randint(0, 90, (m,), generator=g).int().to(DEV)
+    slots = (torch.arange(m) + 5).int()
+    slots[: m // 3] = slots[: m // 3][torch.randperm(m // 3, generator=g)]
+    slots[2] = -1
+    slots = slots.to(DEV)
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    out = []
+    for tile in (1, 8):
+        q = torch.full((m, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+        kc = torch.full((pages, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
+        vc = kc.clone()
+        gb.tile_product(x, w, q, gb.TILE_ROPE, tile, rope=(pos, cos, sin, kc, vc, slots, page, nh, nkv, hd))
+        out.append((q, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 def _rms(x, g, eps):
     x = x.double()
     return x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps) * g.double()
