@@ -100,14 +100,28 @@ LIBRARY_QUICKER = [(T_RESID, 65, 5120, 5120, 35.2, 48.1), (T_RESID, 80, 8192, 81
                    (T_RESID, 640, 8192, 28672, 298.6, 394.1), (T_RESID, 1536, 8192, 8192, 185.2, 257.3),
                    (T_RESID, 3000, 4096, 14336, 291.1, 355.3), (T_RESID, 4096, 3072, 3072, 85.3, 105.3),
                    (T_SILU, 1300, 27648, 5120, 337.9, 382.5), (T_ROPE, 65, 2048, 1536, 13.1, 14.8), (T_SILU, 640, 16384, 3072, 70.5, 77.5),
-                   (T_ROPE, 160, 3072, 2048, 15.9, 17.2), (T_RESID, 3333, 3584, 18944, 372.7, 459.4)]
+                   (T_ROPE, 160, 3072, 2048, 15.9, 17.2), (T_RESID, 3333, 3584, 18944, 372.7, 459.4),
+                   (T_SILU, 512, 28672, 8192, 187.3, 197.4), (T_SILU, 3072, 16384, 8192, 556.6, 585.8), (T_SILU, 3072, 4096, 5120, 103.0, 107.4),
+                   (T_RESID, 2048, 6144, 2048, 76.2, 82.2), (T_RESID, 4096, 6144, 11008, 453.2, 519.4), (T_F32, 640, 8192, 3072, 68.4, 71.8),
+                   (T_F32, 4096, 3072, 1792, 68.4, 73.0)]
 TILES_QUICKER = [(T_SILU, 2048, 16384, 2048, 127.5, 114.8), (T_SILU, 200, 16384, 2048, 33.9, 24.9), (T_ROPE, 2048, 3072, 2048, 38.1, 32.8),
-                 (T_RESID, 128, 4096, 14336, 80.9, 37.8), (T_RESID, 200, 3072, 8192, 42.6, 29.5), (T_F32, 128, 4096, 4096, 30.3, 18.4)]
+                 (T_RESID, 128, 4096, 14336, 80.9, 37.8), (T_RESID, 200, 3072, 8192, 42.6, 29.5), (T_F32, 128, 4096, 4096, 30.3, 18.4),
+                 (T_SILU, 2600, 16384, 4096, 410.4, 276.0), (T_RESID, 2048, 3584, 18944, 365.7, 222.8), (T_F32, 2048, 4096, 11008, 178.9, 158.1),
+                 (T_RESID, 2048, 4096, 14336, 217.5, 195.9)]
 
 
 def test_tile_rule_where_one_side_is_much_the_quicker():
     for kind, m, n, k, lib, tiles in LIBRARY_QUICKER + TILES_QUICKER:
         assert gemm_bf16._tile_wins(m, n, k, kind) == (tiles < lib), (kind, m, n, k)
+
+
+# the same, us by the tiles of 256 x 256 and by others: (kind, rows, N, K, their slices, the others' tile and slices)
+@pytest.mark.parametrize("kind, m, n, k, wide_us, slices, other, other_us", [
+    (T_F32, 836, 8192, 4096, 92.5, 2, (1, 1), 85.3), (T_RESID, 1024, 8192, 8192, 143.4, 2, (1, 1), 136.3),
+    (T_RESID, 160, 8192, 28672, 179.1, 8, (1, 4), 163.4), (T_RESID, 2048, 4096, 14336, 195.9, 2, (1, 1), 200.2),
+    (T_F32, 2048, 3584, 18944, 222.8, 2, (1, 1), 280.4)])
+def test_tiles_of_256_by_256_where_they_are_the_quicker_ones(kind, m, n, k, wide_us, slices, other, other_us):
+    assert gemm_bf16.tile_plan(m, n, k, kind, True)[:2] == ((0, slices) if wide_us < other_us else other)
 
 
 def test_few_rows_plans_count_what_their_reader_pays_for_a_plane():
