@@ -171,7 +171,8 @@ struct ScanArgs {
   float* state;
   size_t state_stride, s_offset;
   float* o;
-  int n_tokens;
+  int n_tokens, n_entries;
+  int long_from;      // entries of so many tokens and more are begun before the others
 };
 
 // An entry's columns take 32 lanes each where as many workgroups as the step's tokens would make of such entries are about one a CU or fewer
@@ -362,45 +363,103 @@ __device__ __forceinline__ void scan_columns(const ScanArgs& a, int group, int h
 }
 #endif
 
-template <int R, int G, int LANES, int W>
+// A step's portions of prompts begin before its single tokens, wherever they lie among them (ORDERED): one that begins late has a CU for itself
+// only by chance.  Up to 64 entries are put in order; of more, those that end in a portion are taken from the last on, as steps are that have no
+// portion, those that begin with one from the first on, and up to 256 others are put in order.  us in the entries' order, by the kernel whose
+// blocks were not written out / from the last on / now: 32 heads of 128 x 128, 2,041 tokens behind seven single ones 452 / 305 / 302, in front of
+// them 442 / 490 / 303; 8 heads, 1,985 in front of 63 432 / 308 / 242, 700 among 200 196 / 128 / 93, in front of them 153 / 148 / 93.
+// Steps without a long entry lose by it (16 entries of three tokens 7.3 -> 7.8): those that can have none of kScanLong tokens are not looked at.
+constexpr int kScanOrdered = 256, kScanLong = 128;
+#if defined(__HIP_DEVICE_COMPILE__)
+struct ScanEntry { int e, first, count; };
+// The zth entry, long ones first.  Every wave looks at all of them, 64 at a time in one trip to memory, which tells it the entry's first token
+// as well.
+template <int CHUNKS>
+__device__ __forceinline__ ScanEntry entry_among(const ScanArgs& a, int z) {
+  const int lane = threadIdx.x & 63;
+  int first[CHUNKS], count[CHUNKS], n_long = 0, n_short = 0;
+  unsigned long long longs[CHUNKS], shorts[CHUNKS];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = min(c * 64 + lane, a.n_entries - 1);
+    first[c] = a.q_start[i], count[c] = a.q_start[i + 1];
+  }
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    count[c] -= first[c];
+    const bool there = c * 64 + lane < a.n_entries;
+    longs[c] = __ballot(there && count[c] >= a.long_from), shorts[c] = __ballot(there && count[c] < a.long_from);
+    n_short += __popcll(longs[c]);      // (short ones come behind all long ones)
+  }
+  auto before = [&](unsigned long long m) { return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0)); };
+  ScanEntry found{0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const bool is_long = count[c] >= a.long_from;
+    const int place = is_long ? n_long + before(longs[c]) : n_short + before(shorts[c]);
+    const unsigned long long hit = __ballot(c * 64 + lane < a.n_entries && place == z);
+    if (hit != 0) {
+      const int at = __builtin_ctzll(hit);
+      found = ScanEntry{c * 64 + at, __builtin_amdgcn_readlane(first[c], at), __builtin_amdgcn_readlane(count[c], at)};
+    }
+    n_long += __popcll(longs[c]), n_short += __popcll(shorts[c]);
+  }
+  return found;
+}
+template <bool ORDERED>
+__device__ __forceinline__ ScanEntry entry_at(const ScanArgs& a, int z) {
+  const int n = a.n_entries, e = n - 1 - z, first = a.q_start[e], end = a.q_start[e + 1];
+  if constexpr (ORDERED) {
+    if (n <= 64) return entry_among<1>(a, z);
+    const int z_first = a.q_start[z], z_end = a.q_start[z + 1];
+    if (a.q_start[n] - a.q_start[n - 1] < a.long_from) {
+      if (a.q_start[1] - a.q_start[0] >= a.long_from) return ScanEntry{z, z_first, z_end - z_first};
+      if (n <= kScanOrdered) return entry_among<kScanOrdered / 64>(a, z);
+    }
+  }
+  return ScanEntry{e, first, end - first};
+}
+#endif
+
+template <int R, int G, int LANES, int W, bool ORDERED>
 __global__ void __launch_bounds__(256) delta_scan_kernel(ScanArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(16))) float lds[ScanBlock<R, G, LANES>::FLOATS];
-  // (a step's portions of prompts come behind its single tokens: begun first, they have the CUs for themselves.  Portions that are in front all
-  // the same begin late: 32 heads of 128 x 128, 2,041 tokens and seven single ones 491 us, and 305 the other way round)
-  const int e = (int)gridDim.z - 1 - (int)blockIdx.z, first = a.q_start[e];
-  scan_columns<R, G, LANES, W>(a, blockIdx.x, blockIdx.y, e, first, a.q_start[e + 1] - first, lds);
+  const ScanEntry at = entry_at<ORDERED>(a, blockIdx.z);
+  scan_columns<R, G, LANES, W>(a, blockIdx.x, blockIdx.y, at.e, at.first, at.count, lds);
 #endif
 }
 // 32 lanes a column for the entries that have most of the step's tokens, 16 for the others.  The first `extra` of blockIdx.z count the
 // former's, for the columns that 16 lanes would leave no workgroup; then all entries follow.
 // (With workgroups without work between those with it, every second CU stayed idle: four entries of 512 tokens 118 us against 78.)
-template <int R, int W>
-__global__ void __launch_bounds__(256) delta_scan_long_kernel(ScanArgs a, int n_entries) {
+template <int R, int W, bool ORDERED>
+__global__ void __launch_bounds__(256) delta_scan_long_kernel(ScanArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(16))) float lds[ScanBlock<R, 2, 16>::FLOATS];
-  const int extra = (int)gridDim.z - n_entries;
+  const int extra = (int)gridDim.z - a.n_entries;
   const bool more = (int)blockIdx.z < extra;
-  int e = (int)gridDim.z - 1 - (int)blockIdx.z;      // (see delta_scan_kernel)
+  ScanEntry at{-1, 0, 0};
   if (more) {
     int nth = blockIdx.z;
-    e = -1;
-    for (int from = 0; from < n_entries; from += 64) {
-      const int i = min(from + (int)(threadIdx.x & 63), n_entries - 1);
-      unsigned long long wide = __ballot(from + (int)(threadIdx.x & 63) < n_entries && scan_wide(a.sh, a.q_start[i + 1] - a.q_start[i], a.n_tokens));
+    for (int from = 0; from < a.n_entries; from += 64) {
+      const int i = min(from + (int)(threadIdx.x & 63), a.n_entries - 1), first = a.q_start[i], count = a.q_start[i + 1] - first;
+      unsigned long long wide = __ballot(from + (int)(threadIdx.x & 63) < a.n_entries && scan_wide(a.sh, count, a.n_tokens));
       for (; wide != 0 && nth > 0; --nth) wide &= wide - 1;
       if (wide != 0) {
-        e = from + __builtin_ctzll(wide);
+        const int w = __builtin_ctzll(wide);
+        at = ScanEntry{from + w, __builtin_amdgcn_readlane(first, w), __builtin_amdgcn_readlane(count, w)};
         break;
       }
     }
-    if (e < 0) return;
-  }
-  const int first = a.q_start[e], count = a.q_start[e + 1] - first, group = blockIdx.x + (more ? gridDim.x : 0);
-  if (scan_wide(a.sh, count, a.n_tokens)) {
-    if (group * 8 < a.sh.vdim) scan_columns<R, 1, 32, W>(a, group, blockIdx.y, e, first, count, lds);
+    if (at.e < 0) return;
   } else {
-    scan_columns<R, 2, 16, W>(a, group, blockIdx.y, e, first, count, lds);
+    at = entry_at<ORDERED>(a, (int)blockIdx.z - extra);
+  }
+  const int group = blockIdx.x + (more ? gridDim.x : 0);
+  if (scan_wide(a.sh, at.count, a.n_tokens)) {
+    if (group * 8 < a.sh.vdim) scan_columns<R, 1, 32, W>(a, group, blockIdx.y, at.e, at.first, at.count, lds);
+  } else {
+    scan_columns<R, 2, 16, W>(a, group, blockIdx.y, at.e, at.first, at.count, lds);
   }
 #endif
 }
@@ -735,19 +794,22 @@ extern "C" int atoma_delta_scan(const float* qn, const float* kn, const float* v
   const dim3 grid((vdim + cols - 1) / cols, heads, n_entries + extra), block(256);
   const bool four = dim % 4 == 0 && s_offset % 4 == 0 && state_stride % 4 == 0 &&
                     ((uintptr_t)qn | (uintptr_t)kn | (uintptr_t)decay | (uintptr_t)state) % 16 == 0;
-  const ScanArgs args{qn, kn, vn, beta, decay, kq, sh, q_start, state_slots, state, state_stride, s_offset, o, n_tokens};
-#define ATOMA_SCAN(...)                                                                                                   \
+  const bool ordered = n_entries > 1 && n_tokens - n_entries + 1 >= kScanLong;
+  const int long_from = (int)std::min<int64_t>((int64_t)2 * n_tokens / n_entries + 1, n_tokens);      // (more than twice the mean)
+  const ScanArgs args{qn, kn, vn, beta, decay, kq, sh, q_start, state_slots, state, state_stride, s_offset, o, n_tokens, n_entries, long_from};
+#define ATOMA_SCAN(KERNEL, ...)                                                                                           \
   do {                                                                                                                    \
-    if (four) hipLaunchKernelGGL((delta_scan_kernel<__VA_ARGS__, 4>), grid, block, 0, stream, args);                      \
-    else hipLaunchKernelGGL((delta_scan_kernel<__VA_ARGS__, 1>), grid, block, 0, stream, args);                           \
+    if (four && ordered) hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 4, true>), grid, block, 0, stream, args);                \
+    else if (four) hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 4, false>), grid, block, 0, stream, args);                     \
+    else if (ordered) hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, true>), grid, block, 0, stream, args);                   \
+    else hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, false>), grid, block, 0, stream, args);                               \
   } while (0)
-  if (dim <= 16) ATOMA_SCAN(1, 1, 16);
-  else if (dim <= 32) ATOMA_SCAN(1, 2, 16);
-  else if (dim <= 64) ATOMA_SCAN(2, 2, 16);
-  else if (mixed && four) hipLaunchKernelGGL((delta_scan_long_kernel<4, 4>), grid, block, 0, stream, args, n_entries);
-  else if (mixed) hipLaunchKernelGGL((delta_scan_long_kernel<4, 1>), grid, block, 0, stream, args, n_entries);
-  else if (dim <= 128) ATOMA_SCAN(4, 2, 16);
-  else ATOMA_SCAN(8, 1, 32);
+  if (dim <= 16) ATOMA_SCAN(delta_scan_kernel, 1, 1, 16);
+  else if (dim <= 32) ATOMA_SCAN(delta_scan_kernel, 1, 2, 16);
+  else if (dim <= 64) ATOMA_SCAN(delta_scan_kernel, 2, 2, 16);
+  else if (mixed) ATOMA_SCAN(delta_scan_long_kernel, 4);
+  else if (dim <= 128) ATOMA_SCAN(delta_scan_kernel, 4, 2, 16);
+  else ATOMA_SCAN(delta_scan_kernel, 8, 1, 32);
 #undef ATOMA_SCAN
   ATOMA_LAUNCH_CHECK();
   return 0;

@@ -158,12 +158,13 @@ def test_the_recurrence_is_the_same_bits_however_it_is_cut(dim, vdim):
 @pytest.mark.parametrize("heads, kv, dim, vdim, taps", [(8, 4, 128, 128, 4), (6, 3, 70, 33, 3), (4, 2, 96, 24, 2), (2, 1, 66, 130, 1), (2, 2, 64, 20, 2),
                                                         (2, 1, 200, 9, 3), (3, 3, 30, 16, 4), (2, 2, 16, 40, 2)])
 def test_the_recurrence_is_the_same_bits_whatever_is_beside_it(heads, kv, dim, vdim, taps):
-    """Entries of 0 to 100 tokens, whole blocks of 16 and rests, alone (where long ones have 32 lanes a column) and all in one step, the long
-    ones first, last and in the middle; and against 64 bits."""
+    """Entries of 0 to 170 tokens, whole blocks of 16 and rests, alone (where long ones have 32 lanes a column) and all in one step, the long
+    ones first, last and in the middle of up to 64, 256 and more; and against 64 bits."""
     from atoma_infer_amd.kernels import ops
     g = torch.Generator().manual_seed(dim)
     r = lambda *n: torch.randn(*n, generator=g).to(DEV)
-    for counts in ([100, 1, 1, 0, 2], [1, 16, 17, 15, 1, 64, 33], [1] * 70 + [95, 80], [32, 31, 48, 7] * 6):
+    for counts in ([100, 1, 1, 0, 2], [1, 16, 17, 15, 1, 64, 33], [1] * 70 + [95, 80], [32, 31, 48, 7] * 6, [2, 0, 140, 1, 133, 1], [1] * 63 + [150],
+                   [170] + [1] * 64 + [0, 3], [1] * 40 + [0, 131, 2, 140] + [1] * 90, [1] * 150 + [141] + [1] * 120):
         t, n = sum(counts), len(counts)
         unit = lambda x: torch.nn.functional.normalize(x.view(t, kv, dim), dim=-1).reshape(t, -1)
         qn, kn, vn = unit(r(t, kv * dim)), unit(r(t, kv * dim)), r(t, heads * vdim)
