@@ -5,17 +5,15 @@
 // 64 rows 10 us a step in Python, their numbers another 5, and the GPU waits for both.
 #include <cstdint>
 
-extern "C" void sampling_uniforms(const uint64_t* seeds, const uint64_t* counters, int n, float* out) {
-  for (int i = 0; i < n; ++i) {
-    uint64_t z = seeds[i] * 0x9E3779B97F4A7C15ull + (counters[i] + 1) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    out[i] = (float)(z >> 40) * 0x1p-24f;
-  }
+namespace {
+float uniform(uint64_t seed, uint64_t counter) {
+  uint64_t z = seed * 0x9E3779B97F4A7C15ull + (counter + 1) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  return (float)(z >> 40) * 0x1p-24f;
 }
 
-namespace {
 struct PlanRow {               // as SamplingPlan.packed writes it
   float temperature, top_p, penalty;
   int32_t top_k;
@@ -38,7 +36,7 @@ extern "C" int sampling_pack(const void* plans, const uint64_t* counters, int n,
     meta[n + i] = r.top_p;
     meta[3 * (long)n + i] = r.penalty;
     top_k[i] = r.top_k;
-    sampling_uniforms(&r.seed, counters + i, 1, meta + 2 * (long)n + i);
+    meta[2 * (long)n + i] = uniform(r.seed, counters[i]);
     if (r.penalised) found |= kPenalised;
     if (r.greedy) continue;
     found &= ~kAllGreedy;

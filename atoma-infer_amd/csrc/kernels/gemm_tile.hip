@@ -63,7 +63,7 @@ struct Tile {
   static constexpr int XBUF = BM * 128, BUF = (BM + BN) * 128, LDS = S * BUF;  // bytes; X's rows, then W's
   // what a wave may still have on its way when the next step has to be there: the S - 2 steps behind it
   static constexpr int NEWER = (S - 2) * (XI + WI);
-  static_assert(S >= 2 && LDS <= 160 * 1024 && NEWER + XI + WI < 64, "");
+  static_assert(S >= 3 && LDS <= 160 * 1024 && NEWER + XI + WI < 64, "");
 };
 
 // silu(g) * u, as exact as g / (1 + expf(-g)) * u (measured over |g| <= 88: the same largest and mean error, 1.8e-7 and 3e-8
@@ -130,20 +130,15 @@ template <typename C>
 __device__ __forceinline__ void step(const char* __restrict__ rd, char* __restrict__ wr, bool more, rsrc_t xb, rsrc_t wb, int k,
                                      const uint32_t (&xo)[C::XI], const uint32_t (&wo)[C::WI], int wave, uint32_t xr, uint32_t wrow,
                                      int lane, Frag<C>& f0, Frag<C>& f1, f32x4 (&acc)[C::TN][C::TM]) {
-  auto loads = [&]() {
-    if (more) {
-      issue<C::QX, C::XI, C::NW>(wr, xb, k, xo, wave);
-      issue<C::QW, C::WI, C::NW>(wr + C::XBUF, wb, k, wo, wave);
-    }
-  };
-  // (with two buffers the loads have one step to arrive and go first; with more they wait until the first fragments' reads
-  // are out: 2,048 rows, N 3,072, K 8,192 by tiles of 256 x 128 111 -> 104 us; with two buffers 178 -> 198)
-  if constexpr (C::S == 2) loads();
   read<C>(rd, 0, xr, wrow, lane, f0);
   multiply<C>(f1, acc);
   interleave<C>();
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (C::S > 2) loads();
+  // (the loads wait until the first fragments' reads are out: 2,048 rows, N 3,072, K 8,192 by tiles of 256 x 128 111 -> 104 us)
+  if (more) {
+    issue<C::QX, C::XI, C::NW>(wr, xb, k, xo, wave);
+    issue<C::QW, C::WI, C::NW>(wr + C::XBUF, wb, k, wo, wave);
+  }
   read<C>(rd, 1, xr, wrow, lane, f1);
   multiply<C>(f0, acc);
   interleave<C>();

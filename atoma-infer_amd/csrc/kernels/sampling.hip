@@ -1146,13 +1146,12 @@ split_draw_kernel(const float* __restrict__ logits, int ld, int vocab, int parts
 constexpr int kFewMaxK = 128, kFewSpare = 16;
 constexpr int kFewCap = 384;                      // of a part's list
 constexpr int kFewNear = 1024;                    // weights in the k-th one's bin or above
-constexpr uint32_t kFewRefused = 0xffffffffu;
 struct FewRow {
   u64 part_mass[kMaxParts];          // of a part: the mass of its weights (rows with a top-p cut)
   float part_max_v[kMaxParts];       // its largest logit and that one's index
   int32_t part_max_i[kMaxParts];
   float part_floor[kMaxParts];       // what the list leaves out and might still be drawn is at most this
-  uint32_t part_count[kMaxParts];    // length of the list; kFewRefused: there is none
+  uint32_t part_count[kMaxParts];    // length of the list
   uint32_t part_nan[kMaxParts];      // values that are no numbers: they come first in the order of weights, and weigh nothing
   uint2 list[kMaxParts][kFewCap];    // (bits of the logit, index in the row), in no order
 };
@@ -1199,11 +1198,8 @@ few_list_kernel(const float* __restrict__ logits, int ld, int vocab, FewRow* __r
     r.part_max_v[part] = a.v;
     r.part_max_i[part] = a.i;
   }
-  if (!(temp > 0.f)) return;                       // (a greedy row needs no more)
-  if (k <= 0 || k > kFewMaxK) {
-    if (tid == 0) r.part_count[part] = kFewRefused;
-    return;
-  }
+  // (a greedy row needs no more, and one with another k is drawn without lists: what stands of them is not read as one then)
+  if (!(temp > 0.f) || k <= 0 || k > kFewMaxK) return;
   // From here on the values are numbers in their order, 0 where there is none: beyond the part's end, and what is no number, which is
   // counted
   // (indexes and floats are made anew where they are written, which the empty asm statements say to the compiler: sixteen more of

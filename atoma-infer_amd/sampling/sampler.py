@@ -39,7 +39,6 @@ def uniform(seed: int, counter: int) -> float:
 def _native() -> ctypes.CDLL:
     lib = load_host_library()
     ptr = ctypes.c_void_p
-    lib.sampling_uniforms.argtypes, lib.sampling_uniforms.restype = [ptr, ptr, ctypes.c_int, ptr], None
     lib.sampling_pack.argtypes = [ctypes.c_char_p, ptr, ctypes.c_int, ctypes.c_int, ptr]
     return lib
 
@@ -53,13 +52,6 @@ def _counters(steps: Sequence[int]) -> array:
         return array("q", steps)
     except OverflowError:
         return array("Q", [x & _MASK for x in steps])
-
-
-def write_uniforms(seeds: Sequence[int], counters: Sequence[int], address: int) -> None:
-    """``uniform`` of every (seed, counter) as float32 from ``address`` on, natively: a step of 64 rows spent 35 us on the
-    function above, more than the GPU on its draws."""
-    s, c = array("Q", [x & _MASK for x in seeds]), array("Q", [x & _MASK for x in counters])
-    _native().sampling_uniforms(s.buffer_info()[0], c.buffer_info()[0], len(s), address)
 
 
 def _found(plans: Sequence[SamplingPlan]) -> int:

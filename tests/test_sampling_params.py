@@ -57,12 +57,15 @@ def test_uniform_is_a_pure_function_in_the_unit_interval():
 def test_a_steps_uniform_numbers_written_natively_are_the_functions():
     import ctypes
 
-    from atoma_infer_amd.sampling.sampler import write_uniforms
+    from atoma_infer_amd.sampling import sampler
     seeds = [0, 1, 42, -1, 2 ** 63, 2 ** 64 - 1, 2 ** 64 + 5] * 40
-    counters = [i * i for i in range(len(seeds))]
-    got = (ctypes.c_float * len(seeds))()
-    write_uniforms(seeds, counters, ctypes.addressof(got))
-    assert list(got) == [uniform(s, c) for s, c in zip(seeds, counters)]
+    steps = [i * i for i in range(len(seeds))]
+    rows = len(seeds)
+    for counters in (steps, [s + 2 ** 63 for s in steps]):
+        got, c = (ctypes.c_float * (5 * rows))(), sampler._counters(counters)
+        sampler._native().sampling_pack(b"".join([plan(do_sample=True, temperature=0.7, random_seed=s).packed for s in seeds]), c.buffer_info()[0],
+                                        rows, 128, ctypes.addressof(got))
+        assert list(got)[2 * rows: 3 * rows] == [uniform(s, n) for s, n in zip(seeds, counters)]
 
 
 def test_a_steps_parameters_packed_natively_are_the_plans():
