@@ -89,10 +89,11 @@ def test_tile_plans_fit_the_kernel():
         for kind in (T_F32, T_RESID, T_SILU, T_ROPE):
             planes = kind in (T_F32, T_RESID)
             tile, slices, us = gemm_bf16.tile_plan(m, n, k, kind, planes)
-            assert 0 <= tile < len(gemm_bf16.TILES) and us > 0 and k % (64 * slices) == 0
+            assert us > 0 and k % (64 * slices) == 0
             assert 1 <= slices <= (gemm_bf16.TILE_MAX_SLICES if planes else 1)
-            assert kind != T_SILU or tile in gemm_bf16.TILES_SILU
-            assert kind != T_ROPE or tile in gemm_bf16.TILES_ROPE
+            # (what the kernel's `pick` takes for the result)
+            assert tile in {T_F32: (0, 1, 2, 3, 4, 5, 6, 7), T_RESID: (0, 1, 2, 3, 4, 5), T_SILU: (0, 1, 2, 3, 6), T_ROPE: (1, 2, 3, 4, 5, 8)}[kind]
+            assert tile in {T_F32: gemm_bf16.TILES_SUMS, T_RESID: gemm_bf16.TILES_SUMS, T_SILU: gemm_bf16.TILES_SILU, T_ROPE: gemm_bf16.TILES_ROPE}[kind]
 
 
 # measured on MI355X with the weights not in any cache, each with what follows it: (kind, rows, N, K, library us, tiles us)
