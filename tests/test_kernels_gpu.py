@@ -177,6 +177,22 @@ def test_gemm_float32_by_bfloat16_thirds(m, n, k):
     assert bool(ops.gemm_generic(a, w, torch.float32)[rows].isnan().all())
 
 
+@pytest.mark.parametrize("m,n,k", [(3, 4096, 8192), (16, 4096, 8192), (200, 4096, 8192), (17, 5000, 4096), (200, 4608, 4096), (900, 4608, 4096)])
+def test_gemm_float32_by_bfloat16_thirds_of_values_of_one_sign(m, n, k):
+    """The longest parts of K that go to the bfloat16 instruction, 1,024 values, with products of one sign, whose sums outgrow them the most.
+    A part is 96 additions, each at most 2^-24 of the part's sum off and a third of that squared in the mean square; the parts' errors meet by
+    their squares: 1.2e-7 and 1.7e-7 with eight and four parts.  Three times that is the bound; parts of 2,560 values, where what the
+    instruction drops of each product has added up, are 1.9e-6 off."""
+    from atoma_infer_amd.kernels import ops
+    parts = 8 if n <= 4096 else 4
+    g = torch.Generator(device=DEV).manual_seed(1)
+    for make in (lambda *s: torch.rand(*s, device=DEV, generator=g), lambda *s: 1 + 0.1 * torch.randn(*s, device=DEV, generator=g)):
+        a, w = make(m, k), make(n, k).bfloat16()
+        want = a.double() @ w.double().T
+        error = (ops.gemm_generic(a, w, torch.float32).double() - want).norm() / want.norm()
+        assert error <= 3 * (k / parts / 32) ** 0.5 * 2.0 ** -24 / parts ** 0.5
+
+
 @pytest.mark.parametrize("m", [1, 7, 16, 17, 48, 64])
 @pytest.mark.parametrize("n,k", [(16, 32), (100, 64), (3072, 2048), (2048, 8192), (1000, 96), (40000, 128),
                                  (70000, 64)])
