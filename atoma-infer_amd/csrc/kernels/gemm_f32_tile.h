@@ -148,14 +148,18 @@ __device__ __forceinline__ void f32_tile(float* __restrict__ lds, int K, int bit
 // ---- float32 rows against a bfloat16 weight -----------------------------------------------------------------------------
 // A float32 number is the sum of three bfloat16 numbers of its sign (24 bits of significand, eight at a time), so a product of
 // float32 rows and a bfloat16 weight is three bfloat16 ones, whose products float32 holds exactly and whose sums the matrix cores
-// keep in float32: nothing is rounded that the float32 instruction would not round, and 32 values of K take three instructions
-// where they took eight of twice the length.  A step of 32 values is added as the weight times the first, the second and the third
-// bfloat16 of each value, by v_mfma_f32_16x16x32_bf16 with lane group g holding values 8 g .. 8 g + 7; the parts of K are
-// those above.  Every kernel of the general product keeps to that.
-// Its error against 64-bit results is 0.6 of the float32 instruction's (200 rows, K of 2,048: 1.8e-7 and 2.9e-7 of the result, K of
-// 8,192 3.5e-7 and 5.7e-7, over normal, one-sided and heavy-tailed values).  What the matrix cores drop below a sum's last bit
-// counts against it only where all products have one sign and a part's sum outgrows them by far: in parts of 1,280 values the two are
-// even, in parts of 2,560 it is 1.9e-6 against 3.9e-7.  So parts longer than 1,024 values keep the float32 instruction.
+// keep in float32: 32 values of K take three instructions where they took eight of twice the length.  A step of 32 values is added as
+// the weight times the first, the second and the third bfloat16 of each value, by v_mfma_f32_16x16x32_bf16 with lane group g holding
+// values 8 g .. 8 g + 7; the parts of K are those above.  Every kernel of the general product keeps to that.
+// Its error against 64-bit results is smaller than the float32 instruction's, which rounds after each of a step's values.  By that one / by
+// this one, of the results' size, 200 rows, 4,096 columns, K of 2,048 and of 8,192: normal values 2.9e-7 / 1.9e-7 and 5.8e-7 / 3.5e-7,
+// those of either sign and size e^(2 normal) 2.0e-7 / 1.4e-7 and 5.3e-7 / 2.8e-7, uniform from 0 to 1 9.0e-8 / 6.9e-8 and 1.6e-7 / 1.1e-7,
+// 1 + 0.1 normal 8.8e-8 / 6.5e-8 and 1.6e-7 / 1.4e-7.
+// But it has a direction, where the float32 instruction's average is below 2e-9: normal values' results are too low by 1.5e-8 (K of 2,048)
+// to 5.7e-8 (8,192) of their size on average, whatever their own sign, and positive ones of parts of 1,024 values too high by up to 9e-8.
+// What sums over such results adds that up.  And it grows where all products have one sign and a part's sum outgrows them by far: in parts
+// of 1,280 values the two are even, in parts of 2,560 it is 1.9e-6 against 3.9e-7.  So parts longer than 1,024 values keep the float32
+// instruction.
 __host__ __device__ __forceinline__ constexpr bool split_product(int N, int K) { return K <= 1024 << f32_part_bits(N); }
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 
@@ -238,8 +242,8 @@ struct SplitTile {
 };
 
 // As f32_tile with SPLIT and no scale: total[i][j] of this wave's share (wave / WN of A's rows, wave % WN of W's).  A step's values
-// are asked for three steps ahead, wait in registers in two sets in turn, and are split and written to LDS beside the products of the
-// step before theirs: one barrier a step.
+// are asked for ST + 1 steps ahead, wait in registers in ST sets in turn (two, and four where a wave's share leaves room), and are split
+// and written to LDS beside the products of the step before theirs: one barrier a step.
 template <typename C, bool VEC, typename RowA, typename RowW>
 __device__ __forceinline__ void split_tile(char* __restrict__ lds, int K, int bits, RowA row_a, RowW row_w,
                                            f32x4_t (&total)[C::BN][C::BM]) {

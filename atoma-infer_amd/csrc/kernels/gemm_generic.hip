@@ -1,5 +1,6 @@
 // C[M, N] = A[M, K] * W[N, K]^T in true float32: products and sums are float32 fused multiply-adds (on the matrix
-// cores' float32 instruction), no reduced-precision mode.  A and W may be float32 or bfloat16 (widened exactly on
+// cores' float32 instruction), or, for float32 rows against a bfloat16 weight, exact products of all of a value's bits
+// with float32 sums; no reduced-precision mode.  A and W may be float32 or bfloat16 (widened exactly on
 // load); C float32 or bfloat16.  Any M, N, K.  It is the product of the 32-bit path and the fallback for shapes the
 // bfloat16 kernels refuse.
 //

@@ -401,9 +401,10 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 //   X0 W0 (W1 is read), X0 W1 (X1), X1 W1 (the next step's X0, into the registers of this one's), X1 W0 (its W0, into W1's)
 // So X0 and W0 of a step are read before the step begins, W1 and X1 by its middle, and with a barrier at either place the halves are
 // loaded anew a step and a half before they are read again, 32 KB at a time: the loads alone take 0.95 us a step.
-// us, before / now: gate-up with SiLU, 2,048 rows against 16,384 x 2,048 116 / 111, 16,384 x 3,072 164 / 156, 28,672 x 4,096 391 / 370;
-// float32 sums of 8,192^3 800 / 763.  What is left is power: the MFMAs alone would take 555 of the 763 and the loads alone 486, with all of them
-// served by the L2 the product still takes 735, and the clock is at 1.85 GHz; priorities for the MFMAs (s_setprio) cost 2 %.
+// us, before / now, on their own: gate-up with SiLU, 2,048 rows against 16,384 x 2,048 116 / 111, 16,384 x 3,072 164 / 156, 28,672 x 4,096
+// 391 / 370; in a program's steps 106 to 123, 149 and 355.  float32 sums of 8,192^3 800 / 763.  What is left is power: the MFMAs alone would
+// take 555 of the 763 and the loads alone 486, with all of them served by the L2 the product still takes 735, and the clock is at 1.85 GHz;
+// priorities for the MFMAs (s_setprio) cost 2 %.
 template <int BM_, int BN_, int WM_, int WN_>
 struct Phased {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM * WN;
@@ -572,7 +573,7 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   }
   if constexpr (EPI == kOutRope) {
     // (all sums at once do not fit LDS: a half of X's rows by a half of W's at a time.  2,048 rows against 6,144 x 4,096: 256 tiles of 256 x
-    // 192, 86 us; by 256 x 96 103, by the library with the rotation's kernel behind it 93)
+    // 192, 86 us on their own, 95 in the steps of a long prompt; by 256 x 96 103, by the library with the rotation's kernel behind it 93)
     constexpr int COLS = C::WH / C::WN;
     wait<0, true>();
     meet();                  // everybody's reads of the last step are done

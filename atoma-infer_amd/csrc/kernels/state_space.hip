@@ -711,7 +711,8 @@ extern "C" int atoma_ssd_scan(const float* xbc, const float* dt, const float* de
   return 0;
 }
 
-// The largest state size the chunk kernel takes (its tiles of B and C must fit the CU's LDS beside the rest).
+// The largest state size the chunk kernel is built for: a lane has a chunk's operands and its share of S in registers, 32 numbers of C, 32 of B
+// and 8 of S at 128.  LDS has room for more; nothing has been measured beyond.
 extern "C" int atoma_ssd_chunk_max_state() { return 128; }
 
 template <int NB, bool VEC>
