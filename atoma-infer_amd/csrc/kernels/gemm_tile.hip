@@ -393,11 +393,11 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 #endif
 }
 
-// ---- tiles of 256 x 256 ---------------------------------------------------------------------------------------------------
+// ---- tiles in phases ------------------------------------------------------------------------------------------------------
 // With one barrier a step a buffer is free, and the loads for the step after next can start, only when all of its fragments have been
-// read, and those loads must be there a step later: 64 KB of a burst and the latency behind it, 1.27 us a step on their own, about what
-// a step's MFMAs take.  Here a step is multiplied in four phases, half of X's rows by half of W's at a time, and a phase's fragments
-// are read under the MFMAs of the one before:
+// read, and those loads must be there a step later: 64 KB of a burst and the latency behind it for a tile of 256 x 256, 1.27 us a step on
+// their own, about what a step's MFMAs take.  Here a step is multiplied in four phases, half of X's rows by half of W's at a time, and a
+// phase's fragments are read under the MFMAs of the one before:
 //   X0 W0 (W1 is read), X0 W1 (X1), X1 W1 (the next step's X0, into the registers of this one's), X1 W0 (its W0, into W1's)
 // So X0 and W0 of a step are read before the step begins, W1 and X1 by its middle, and with a barrier at either place the halves are
 // loaded anew a step and a half before they are read again, 32 KB at a time: the loads alone take 0.95 us a step.
@@ -405,9 +405,17 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 // 391 / 370; in a program's steps 106 to 123, 149 and 355.  float32 sums of 8,192^3 800 / 763.  What is left is power: the MFMAs alone would
 // take 555 of the 763 and the loads alone 486, with all of them served by the L2 the product still takes 735, and the clock is at 1.85 GHz;
 // priorities for the MFMAs (s_setprio) cost 2 %.
-template <int BM_, int BN_, int WM_, int WN_>
+//
+// Two buffers instead of three or four also leave half of a CU's LDS to a second workgroup where a tile has 128 rows: one workgroup's first
+// loads and its results then pass under the other's products, and a barrier holds up half of a CU's waves.  Against tiles of the same 256 or
+// 128 rows with one barrier a step, four buffers and a workgroup a CU (some 18,000 products; geometric means of the time, by workgroups
+// a CU up to one / more): 128 x 128 0.95 to 0.98 / 0.84 to 0.89, 256 x 128 0.97 / 0.98, 128 x 192 against 256 x 96 0.92 to 0.97 / 0.85 to
+// 0.88, 128 x 64 1.01 / 0.83 to 0.88 (so only there).  us, before / now: q, k, v of 2,048 rows against 3,072 x 2,048 35.9 / 33.0, two slices of
+// 2,048 x 8,192 69.0 / 65.3.  (192 x 128, patches of eight rows of tiles and 128 x 160 gave nothing; 256 x 160 by halves of 80 lost 1 %.)
+// EU: waves a SIMD that the registers are to leave room for (four: two workgroups of eight waves).
+template <int BM_, int BN_, int WM_, int WN_, int EU_ = 2>
 struct Phased {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM * WN;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM * WN, EU = EU_;
   static constexpr int XH = BM / 2, WH = BN / 2;                              // rows of a half
   static constexpr int JX = XH / WM / 16, JW = WH / WN / 16;                  // blocks of 16 of a wave in a half
   static constexpr int QX = XH / 8, XI = (QX + NW - 1) / NW;                  // loads of eight rows: a half's, a wave's
@@ -450,7 +458,7 @@ __device__ __forceinline__ void phase(const bf16x8 (&w)[JW][2], const bf16x8 (&x
 
 // Two steps or more; ODD: their number is (a kernel that takes either spills registers).
 template <typename C, int EPI, bool GROUPED, bool ODD>
-__global__ void __launch_bounds__(64 * C::NW, 2)
+__global__ void __launch_bounds__(64 * C::NW, C::EU)
 gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int rows, int N, int ldx, int ldw, int k_len,
                    TileOut out, Groups groups) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -498,12 +506,13 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   const int wm = wave / C::WN, wn = wave % C::WN;
   const uint32_t xr = (wm * (C::XH / C::WM) + r16) * 128, wr = (wn * (C::WH / C::WN) + r16) * 128;
 
-  // lanes 0 .. 31: the wave's rows of X's first half, 32 .. 63: of the second
+  // lanes from 0 on: the wave's rows of X's first half, then those of the second
+  constexpr int ROWS = C::XH / C::WM;
   int pos_of = 0, page_of = -1, off_of = 0;
   if constexpr (EPI == kOutRope) {
-    static_assert(C::XH / C::WM == 32, "");
-    const int row = m0 + (lane >> 5) * C::XH + wm * 32 + (lane & 31);
-    if (row < M) {
+    static_assert(2 * ROWS <= 64 && (ROWS & (ROWS - 1)) == 0, "a lane a row");
+    const int row = m0 + lane / ROWS * C::XH + wm * ROWS + lane % ROWS;
+    if (lane < 2 * ROWS && row < M) {
       const int slot = out.rope.slot_mapping[row];
       pos_of = out.rope.positions[row];
       if (slot >= 0) page_of = slot / out.rope.page_size, off_of = slot - page_of * out.rope.page_size;
@@ -577,10 +586,10 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
     constexpr int COLS = C::WH / C::WN;
     wait<0, true>();
     meet();                  // everybody's reads of the last step are done
-    float* const sums = reinterpret_cast<float*>(lds) + wave * (32 * COLS);
+    float* const sums = reinterpret_cast<float*>(lds) + wave * (ROWS * COLS);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int from = h * 32 + (lane & 31), pos = __shfl(pos_of, from, 64), page = __shfl(page_of, from, 64), off = __shfl(off_of, from, 64);
+      const int from = h * ROWS + lane % ROWS, pos = __shfl(pos_of, from, 64), page = __shfl(page_of, from, 64), off = __shfl(off_of, from, 64);
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
 #pragma unroll
@@ -591,7 +600,7 @@ gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
         const int nw = n0 + g * C::WH + wn * COLS;
-        if (nw < N) rope_tile<32, COLS>(sums, m0 + h * C::XH + wm * 32, M, nw, N, pos, page, off, out.rope, (uint16_t*)out.c, out.ldc, lane);
+        if (nw < N) rope_tile<ROWS, COLS>(sums, m0 + h * C::XH + wm * ROWS, M, nw, N, pos, page, off, out.rope, (uint16_t*)out.c, out.ldc, lane);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
       }
@@ -643,42 +652,62 @@ static int launch(const void* x, const void* w, int M, int N, int K, int ldx, in
   return 0;
 }
 
-// (one step: by tiles of as many rows and half the columns)
+// (one step: by a tile of as many rows with one barrier a step)
 template <typename C, int EPI, bool GROUPED = false>
 static int launch_phased(const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
                          hipStream_t stream, const Groups& groups = Groups{}) {
   const int steps = K / slices / 64;
-  if (steps == 1) return launch<Tile<256, 128, 4, 2, 3>, EPI, GROUPED>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups);
+  if (steps == 1) return launch<Tile<C::BM, 128, C::BM / 64, 2, 3>, EPI, GROUPED>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups);
   return steps % 2 ? launch_phased<C, EPI, GROUPED, true>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups)
                    : launch_phased<C, EPI, GROUPED, false>(x, w, M, N, K, ldx, ldw, slices, out, stream, groups);
+}
+
+constexpr int kCUs = 256;
+
+// Tiles of which a CU can hold two where they go in phases, which is the quicker way once there is more than one for a CU.  One for each CU has
+// its LDS for four buffers: 128 x 64 takes 1.00 to 1.04 times as long in phases then, 128 x 192 with a long end 1.00 to 1.02, and 128 x 128 with
+// residual rows, 0.98 on its own, 1.02 within a prompt's steps.
+static bool two_a_cu(int M, int N, int bm, int bn, int slices) {
+  return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * slices > kCUs;
 }
 
 template <int EPI>
 static int pick(int tile, const void* x, const void* w, int M, int N, int K, int ldx, int ldw, int slices, const TileOut& out,
                 hipStream_t stream) {
-  constexpr bool GATED = EPI == kOutSilu;
+  constexpr bool GATED = EPI == kOutSilu, STORES = EPI == kOutResid || EPI == kOutRope;
   (void)GATED;
 #define ATOMA_TILE(...) return launch<Tile<__VA_ARGS__>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream)
+#define ATOMA_PHASED(...) return launch_phased<Phased<__VA_ARGS__>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream)
   switch (tile) {
-    case 0:
-      if constexpr (EPI != kOutRope)                  // (its sums do not fit LDS)
-        return launch_phased<Phased<256, 256, 2, 4>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream);
-      break;
-    case 1: ATOMA_TILE(256, 128, 4, 2, 3);
-    case 2: ATOMA_TILE(128, 128, 2, 4, 4);
-    case 3: ATOMA_TILE(128, 64, 2, 2, 4);
+    case 0: if constexpr (EPI != kOutRope) ATOMA_PHASED(256, 256, 2, 4); break;                  // (its sums do not fit LDS)
+    case 1: ATOMA_PHASED(256, 128, 4, 2);
+    // by four waves, whose larger shares read less LDS, or eight where the end is long, which gain by 2 to 13 percent there
+    case 2:
+      if constexpr (EPI == kOutResid)
+        if (!two_a_cu(M, N, 128, 128, slices)) ATOMA_TILE(128, 128, 2, 4, 4);
+      if constexpr (STORES) ATOMA_PHASED(128, 128, 2, 4, 4);
+      else ATOMA_PHASED(128, 128, 2, 2);
+    case 3:
+      if (two_a_cu(M, N, 128, 64, slices)) ATOMA_PHASED(128, 64, 4, 1, 4);
+      ATOMA_TILE(128, 64, 2, 2, 4);
     case 4: if constexpr (!GATED) ATOMA_TILE(256, 160, 4, 2, 3); break;     // (a wave's blocks are not in pairs)
-    case 5: if constexpr (!GATED) ATOMA_TILE(256, 96, 4, 2, 3); break;
+    case 5:
+      if constexpr (STORES) {
+        if (two_a_cu(M, N, 128, 192, slices)) ATOMA_PHASED(128, 192, 4, 2, 4);
+        ATOMA_TILE(128, 192, 2, 4, 4);
+      } else if constexpr (!GATED) {
+        ATOMA_PHASED(128, 192, 2, 2);
+      }
+      break;
     // 33 to 64 rows, and q, k, v and small weights with some hundred: bound by what a CU brings to LDS, so small tiles, two workgroups a CU, and K in slices.  64 rows, gate-up
     // of 16,384 x 2,048 in 64 x 64 17.7 us with four buffers, 18.8 with three, 18.2 with eight (one workgroup a CU); 64 x 128 with three
     // 21.6.  Planes of 3,072 x 8,192 13.7 by 64 x 128 in eight slices, 15.4 by 64 x 64.
     case 6: if constexpr (EPI == kOutF32 || GATED) ATOMA_TILE(64, 64, 2, 2, 4); break;
     case 7: if constexpr (EPI == kOutF32) ATOMA_TILE(64, 128, 2, 2, 3); break;
-    case 8:
-      if constexpr (EPI == kOutRope) return launch_phased<Phased<256, 192, 4, 2>, EPI>(x, w, M, N, K, ldx, ldw, slices, out, stream);
-      break;
+    case 8: if constexpr (EPI == kOutRope) ATOMA_PHASED(256, 192, 4, 2); break;
   }
 #undef ATOMA_TILE
+#undef ATOMA_PHASED
   return ATOMA_ERR_SHAPE;
 }
 
@@ -722,24 +751,22 @@ extern "C" int atoma_gemm_tile_groups(const void* x, const void* w, void* c, int
     return ATOMA_ERR_SHAPE;
   const TileOut out{c, kind == kOutSilu ? N / 2 : N, 0, RopeArgs{}};
   const Groups groups{tiles, offsets, perm, scale, top, plane_rows};
-#define ATOMA_TILE(BM, ...)                                                                                                \
+#define ATOMA_GROUPS(HOW, BM, ...)                                                                                        \
   do {                                                                                                                     \
     if (kind == kOutSilu)                                                                                                  \
-      return launch<Tile<BM, __VA_ARGS__>, kOutSilu, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);     \
+      return HOW<__VA_ARGS__, kOutSilu, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);                  \
     if (kind == kOutF32)                                                                                                   \
-      return launch<Tile<BM, __VA_ARGS__>, kOutF32, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);      \
+      return HOW<__VA_ARGS__, kOutF32, true>(x, w, max_tiles * BM, N, K, K, K, 1, out, stream, groups);                   \
   } while (0)
   switch (tile) {
-    case 0:
-      if (kind == kOutSilu)
-        return launch_phased<Phased<256, 256, 2, 4>, kOutSilu, true>(x, w, max_tiles * 256, N, K, K, K, 1, out, stream, groups);
-      if (kind == kOutF32)
-        return launch_phased<Phased<256, 256, 2, 4>, kOutF32, true>(x, w, max_tiles * 256, N, K, K, K, 1, out, stream, groups);
+    case 0: ATOMA_GROUPS(launch_phased, 256, Phased<256, 256, 2, 4>); break;
+    case 1: ATOMA_GROUPS(launch_phased, 256, Phased<256, 128, 4, 2>); break;
+    case 2: ATOMA_GROUPS(launch_phased, 128, Phased<128, 128, 2, 2>); break;
+    case 3:
+      if (two_a_cu(max_tiles * 128, N, 128, 64, 1)) ATOMA_GROUPS(launch_phased, 128, Phased<128, 64, 4, 1, 4>);
+      else ATOMA_GROUPS(launch, 128, Tile<128, 64, 2, 2, 4>);
       break;
-    case 1: ATOMA_TILE(256, 128, 4, 2, 3); break;
-    case 2: ATOMA_TILE(128, 128, 2, 4, 4); break;
-    case 3: ATOMA_TILE(128, 64, 2, 2, 4); break;
   }
-#undef ATOMA_TILE
+#undef ATOMA_GROUPS
   return ATOMA_ERR_SHAPE;
 }

@@ -1027,6 +1027,37 @@ def test_gemm_tile_in_phases_equals_the_one_by_steps(m, n, k):
         assert torch.equal(g[0], g[1])
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 320])
+def test_gemm_tiles_of_which_a_cu_holds_two_equal_the_others(k):
+    """Tiles of 128 rows with more workgroups than CUs go in phases: sums, residual rows, SiLU and (1,100 rows, 96 heads) q, k, v have the bits
+    of the tile of 256 x 128, with 1, 2, 3 and 5 steps of K and rows and columns that end inside a tile's first half."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    m, n, nh, nkv, hd, page = 1100, 6176, 80, 8, 64, 16
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    pos = (torch.arange(m) % 90).int().to(DEV)
+    slots = (torch.arange(m) + 3).int().to(DEV)
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    r0, want = rnd(m, n, seed=3), None
+    for tile in (1, 2, 3, 5):
+        bm, bn = gb.TILES[tile][:2]
+        assert tile == 1 or -(-m // bm) * -(-6144 // bn) > 256
+        c, r = torch.full((m, n), 7.0, device=DEV), r0.clone()
+        gb.tile_product(x, w, c, gb.TILE_F32, tile)
+        gb.tile_product(x, w, r, gb.TILE_RESID, tile)
+        q = torch.full((m, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+        kc = torch.full((m // page + 2, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
+        vc = kc.clone()
+        gb.tile_product(x, w[:6144], q, gb.TILE_ROPE, tile, rope=(pos, cos, sin, kc, vc, slots, page, nh, nkv, hd))
+        got = [c, r, q, kc, vc]
+        if tile in gb.TILES_SILU:
+            s = torch.full((m, n // 2), 7.0, dtype=torch.bfloat16, device=DEV)
+            gb.tile_product(x, w, s, gb.TILE_SILU, tile)
+            got.append(s)
+        want = want or got
+        assert all(torch.equal(a, b) for a, b in zip(want, got)), tile
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 32, 128), (41, 80, 192), (63, 544, 512), (64, 1056, 1024), (64, 2048, 8192), (1, 64, 128)])
 def test_gemm_tile_of_64_rows(m, n, k):
     """The tiles for 33 to 64 rows, as test_gemm_tile holds the others; then what parts call with as many rows: 41 and more leave the
