@@ -331,3 +331,38 @@ def test_waves_of_whole_ranges_at_the_lines(s, kv_heads, keys, head_size, want):
     starts, counts = np.arange(s, dtype=np.int32) % keys, np.ones(s, dtype=np.int32)
     # layers whose values are wider than their keys, or whose scores have a bias, keep eight
     assert A.plan_step(starts, counts, 4, 0, keys, kv_heads=kv_heads, max_waves=8, head_size=head_size, plain=False)[1][3] == 8
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_workgroups_of_mixed_steps_are_dealt_without_losing_a_task(seed):
+    """Decoded tokens of few and of many keys beside portions of prompts: the same tasks as the builder's, fours that share keys unbroken,
+    single ones together in fours where workgroups are more than the GPU takes, and every key seen once."""
+    rng = np.random.default_rng(700 + seed)
+    group, head_size = int(rng.choice([1, 3, 4, 40])), int(rng.choice([64, 128]))
+    window = int(rng.choice([0, 0, 700]))
+    s = int(rng.choice([3, 40, 150]))
+    counts = rng.choice([1, 1, 1, 1, 5, 40, 150], size=s).astype(np.int32)
+    starts = rng.choice([0, 5, 100, 300, 511, 800, 2400], size=s).astype(np.int32)
+    options = dict(kv_heads=8, max_waves=8, head_size=head_size)
+    arr, meta = A.build_tasks(starts, counts, group, window, **options)
+    got, mg = A.plan_step(starts, counts, group, window, **options)
+    coverage(got, mg, starts, counts, group, window)
+    live = lambda a, n: sorted(map(tuple, a[:n][a[:n, 0] >= 0].tolist()))
+    assert live(arr, meta[0]) == live(got, mg[0]) and np.array_equal(arr[meta[0]:], got[mg[0]:]) and mg[1:] == meta[1:]
+    fours = {tuple(map(tuple, f.tolist())) for f in got[: mg[0]].reshape(-1, 4, 12)}
+    kept = [tuple(map(tuple, f.tolist())) for f in arr[: meta[0]].reshape(-1, 4, 12) if (f[:, 0] >= 0).sum() > 1]
+    assert all(f in fours for f in kept)
+    full = meta[0] // 4 * 8 > 256 * (2 if head_size <= 64 else 1)
+    singles = sum((f[1:, 0] < 0).all() and f[0, 6] < 0 for f in arr[: meta[0]].reshape(-1, 4, 12))
+    assert mg[0] // 4 == meta[0] // 4 - (singles - -(-singles // 4) if full else 0)
+
+
+def test_chunks_run_among_prompt_tiles_only_where_they_take_a_share_of_the_time():
+    far = np.asarray([6000] + [2048] * 30), np.asarray([2018] + [1] * 30)
+    near = np.asarray([0] + [2048] * 32), np.asarray([2016] + [1] * 32)
+    for (starts, counts), mixed in ((far, False), (near, True)):
+        arr, meta = A.plan_step(starts, counts, 4, 0, kv_heads=8, max_waves=8)
+        chunked = arr[: meta[0]].reshape(-1, 4, 12)[:, 0, 6] >= 0
+        assert bool(chunked[: len(chunked) // 4].any()) == mixed
+        walks = (arr[: meta[0], 5] - arr[: meta[0], 4]).reshape(-1, 4).max(1)[~chunked]
+        assert not mixed or (np.diff(walks) <= 0).all()
