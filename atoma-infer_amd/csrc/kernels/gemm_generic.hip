@@ -30,6 +30,9 @@
 #include <cmath>
 #include <type_traits>
 
+#include "common.h"
+#include "cache_layout.h"
+#include "gate_act.h"
 #include "gemm_f32_tile.h"
 
 using namespace atoma;
@@ -298,10 +301,55 @@ split_stream_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, T
 // The same for up to 4 RW rows of A, 4 to 16, behind FULL blocks of 16 (none or one): sixteen lanes split a row's values of four steps and
 // hand them to the others through LDS, so that no lane splits what another splits too (every wave has its own corner of LDS, which it
 // fills and reads in order, with more than eight rows half a batch at a time).  A full block's rows are each lane's own.
-template <int FULL, int RW, int RT, int WK, typename TC>
+// END: what leaves.  kPlain: the sums; kGated: act(gate) * up [M][ldc] of a weight in blocks of 16 gate rows and their 16 up rows, a wave
+// having one of each (RT 2); kRotated: q rotated [M][ldc] and k, v in the float32 cache, the rows of q and k heads in pair order (columns 2 i and
+// 2 i + 1 are the members of pair i).  The sums are those of the other kernels, and the ends compute as the activation's and the rotation's own
+// kernels do, so the bits are theirs; what is saved is a launch.  Llama 1B sizes in float32, four layers, four requests: a pass of prompts and 16 decoded tokens 8.03 -> 7.76 ms.
+enum FewEnd : int { kPlain, kGated, kRotated };
+struct FewArgs {
+  GateAct act;
+  const int32_t* positions;      // [M]
+  const float* cos_t;            // [positions, hd / 2]
+  const float* sin_t;
+  float* kcache;                 // [pages, nkv, page_size * hd] tiles
+  float* vcache;
+  const int32_t* slot_mapping;   // [M]; negative: no cache write for the row
+  int page_size, nh, nkv, hd;
+};
+// outputs n .. n + 3 of a row of the fused q, k, v projection (n a multiple of 4, hd too: one head)
+__device__ __forceinline__ void rotate_store4(const FewArgs& f, float* __restrict__ q_row, int n, int pos, int slot, f32x4_t v) {
+  const int head = n / f.hd, d = n - head * f.hd, half = f.hd >> 1;
+  const int page = slot >= 0 ? slot / f.page_size : 0, off = slot >= 0 ? slot % f.page_size : 0;
+  if (head >= f.nh + f.nkv) {
+    if (slot < 0) return;
+    float* const tile = f.vcache + ((size_t)page * f.nkv + (head - f.nh - f.nkv)) * f.hd * f.page_size;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tile[value_offset(d + e, off, f.hd, f.page_size)] = v[e];
+    return;
+  }
+  const bool is_k = head >= f.nh;
+  if (is_k && slot < 0) return;
+  float* const ktile = is_k ? f.kcache + ((size_t)page * f.nkv + (head - f.nh)) * f.page_size * f.hd : nullptr;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int i = (d >> 1) + p;
+    const float c = f.cos_t[(size_t)pos * half + i], sv = f.sin_t[(size_t)pos * half + i];
+    const float x1 = v[2 * p], x2 = v[2 * p + 1];
+    const float o1 = fmaf(x1, c, -(x2 * sv)), o2 = fmaf(x1, sv, x2 * c);      // (as the compiler writes the rotation's own kernel)
+    if (is_k) {
+      ktile[key_offset(off, i, f.page_size)] = o1;
+      ktile[key_offset(off, i + half, f.page_size)] = o2;
+    } else {
+      q_row[head * f.hd + i] = o1;
+      q_row[head * f.hd + i + half] = o2;
+    }
+  }
+}
+
+template <int FULL, int RW, int RT, int WK, typename TC, int END = kPlain>
 __global__ void __launch_bounds__(64 * WK)
 split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* __restrict__ c, int M, int N, int K, int lda,
-                 int ldw, int ldc) {
+                 int ldw, int ldc, FewArgs few) {
   constexpr int BITS = WK == 8 ? 3 : 2, U = 4, H = RW > 2 ? U / 2 : U;      // steps of a batch, and at a time in LDS
   static_assert(WK == 1 << BITS, "a wave a part of K");
   __shared__ f32x4_t red[WK - 1][FULL + 1][RT][64];
@@ -319,6 +367,12 @@ split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* 
   const float* own[FULL + 1];                              // its own values of a step
 #pragma unroll
   for (int m = 0; m <= FULL; ++m) own[m] = a + (size_t)min(m * 16 + r16, M - 1) * lda + kg * 8;
+  int pos = 0, slot = -1;                                  // (asked for now: a trip to memory less behind the sums)
+  if constexpr (END == kRotated) {
+    static_assert(FULL == 0, "a lane a row");
+    pos = few.positions[min(r16, M - 1)];
+    slot = few.slot_mapping[min(r16, M - 1)];
+  }
   f32x4_t acc[FULL + 1][RT];
 #pragma unroll
   for (int m = 0; m <= FULL; ++m)
@@ -420,7 +474,16 @@ split_few_kernel(const float* __restrict__ a, const bf16_t* __restrict__ w, TC* 
     for (int i = 0; i < RT; ++i) {
 #pragma unroll
       for (int q = 0; q < WK - 1; ++q) acc[m][i] += red[q][m][i][lane];
-      put4(c + (size_t)(m * 16 + r16) * ldc, n0 + i * 16 + kg * 4, N, aligned, acc[m][i]);
+      if constexpr (END == kPlain) put4(c + (size_t)(m * 16 + r16) * ldc, n0 + i * 16 + kg * 4, N, aligned, acc[m][i]);
+      else if constexpr (END == kRotated)
+        if (n0 + i * 16 < N) rotate_store4(few, c + (size_t)r16 * ldc, n0 + i * 16 + kg * 4, pos, slot, acc[m][i]);
+    }
+    if constexpr (END == kGated) {
+      static_assert(RT == 2 && FULL == 0, "gate and up in a wave");
+      f32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = gated(acc[m][0][e], acc[m][1][e], few.act);
+      put4(c + (size_t)r16 * ldc, n0 / 2 + kg * 4, N / 2, aligned, o);
     }
   }
 }
@@ -448,13 +511,13 @@ static int launch_split_few(const float* a, const bf16_t* w, TC* c, int M, int N
   // (a wave a part of K)
   if constexpr (RT == 1) {
     if (FULL > 0 || RW > 2 || f32_part_bits(N) == 3) {      // (of many columns only up to eight rows come here)
-      hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+      hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 8, TC>), grid, dim3(512), 0, stream, a, w, c, M, N, K, lda, ldw, ldc, FewArgs{});
       ATOMA_LAUNCH_CHECK();
       return 0;
     }
   }
   if constexpr (FULL == 0 && RW <= 2) {
-    hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc);
+    hipLaunchKernelGGL((split_few_kernel<FULL, RW, RT, 4, TC>), grid, dim3(256), 0, stream, a, w, c, M, N, K, lda, ldw, ldc, FewArgs{});
     ATOMA_LAUNCH_CHECK();
   }
   return 0;
@@ -612,4 +675,57 @@ extern "C" int atoma_gemm_generic(const void* a, int a_dtype, const void* w, int
   if (a_dtype == kBF16)
     return launch_w<bf16_t>((const bf16_t*)a, w, w_dtype, c, c_dtype, M, N, K, lda, ldw, ldc, stream);
   return ATOMA_ERR_DTYPE;
+}
+
+// Whether products of up to eight float32 rows against a bfloat16 weight [N, K] have the two ends below.  gated: only weights of more than
+// 4,096 rows, whose workgroups have a block of gate rows and one of up rows each; a narrower one's have a block of sixteen, so that there
+// are enough of them.
+extern "C" int atoma_gemm_few_takes(int M, int N, int K, int gated) {
+  return M > 0 && M <= 8 && N > 0 && K > 0 && K % kF32Step == 0 && split_product(N, K) && N % (gated ? 32 : 16) == 0 &&
+         (!gated || f32_part_bits(N) == 2);
+}
+
+template <int END>
+static int launch_few_end(const float* a, const bf16_t* w, float* c, int M, int N, int K, int lda, int ldw, int ldc, const FewArgs& few, hipStream_t stream) {
+#define ATOMA_FEW(RW, RT, WK)                                                                                                          \
+  hipLaunchKernelGGL((split_few_kernel<0, RW, RT, WK, float, END>), dim3(ceil_div(N, 16 * RT)), dim3(64 * WK), 0, stream, a, w, c, M, N, K, \
+                     lda, ldw, ldc, few)
+  if (f32_part_bits(N) == 2) {
+    if (M <= 4) ATOMA_FEW(1, 2, 4);
+    else ATOMA_FEW(2, 2, 4);
+  } else if constexpr (END == kRotated) {
+    if (M <= 4) ATOMA_FEW(1, 1, 8);
+    else ATOMA_FEW(2, 1, 8);
+  } else {
+    return ATOMA_ERR_SHAPE;
+  }
+#undef ATOMA_FEW
+  ATOMA_LAUNCH_CHECK();
+  return 0;
+}
+
+static bool few_fits(const void* a, const void* w, const void* c, int K, int lda, int ldw) {
+  return lda >= K && ldw >= K && lda % 4 == 0 && ldw % 8 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)c) & 15) == 0;
+}
+
+// c [M, N / 2] = act(gate) * up of a [M <= 8, K] float32 times w [N, K] bfloat16 transposed, w in blocks of 16 gate rows and their 16 up rows.
+extern "C" int atoma_gemm_few_gated(const float* a, const void* w, float* c, int M, int N, int K, int lda, int ldw, int ldc, int kind, float limit,
+                                    float slope, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (!atoma_gemm_few_takes(M, N, K, 1) || !few_fits(a, w, c, K, lda, ldw) || ldc < N / 2 || !gate_act_ok(kind, limit)) return ATOMA_ERR_SHAPE;
+  FewArgs few{};
+  few.act = GateAct{kind, limit, slope};
+  return launch_few_end<kGated>(a, (const bf16_t*)w, c, M, N, K, lda, ldw, ldc, few, stream);
+}
+
+// q_out [M, nh hd] rotated, k (rotated) and v in the float32 cache, of a [M <= 8, K] float32 times the fused q, k, v weight in pair order.
+extern "C" int atoma_gemm_few_rotated(const float* a, const void* w, float* q_out, int M, int N, int K, int lda, int ldw, int ldq,
+                                      const int32_t* positions, const float* cos_t, const float* sin_t, float* kcache, float* vcache,
+                                      const int32_t* slot_mapping, int page_size, int nh, int nkv, int hd, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (!atoma_gemm_few_takes(M, N, K, 0) || !few_fits(a, w, q_out, K, lda, ldw) || nh <= 0 || nkv <= 0 || hd <= 0 || hd % 16 || N != (nh + 2 * nkv) * hd ||
+      ldq < nh * hd || page_size <= 0 || !positions || !cos_t || !sin_t || !kcache || !vcache || !slot_mapping)
+    return ATOMA_ERR_SHAPE;
+  const FewArgs few{GateAct{0, 0.f, 0.f}, positions, cos_t, sin_t, kcache, vcache, slot_mapping, page_size, nh, nkv, hd};
+  return launch_few_end<kRotated>(a, (const bf16_t*)w, q_out, M, N, K, lda, ldw, ldq, few, stream);
 }

@@ -322,6 +322,45 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, out: 
     return out
 
 
+def _few_rows(a: torch.Tensor, w: torch.Tensor, gated: bool) -> bool:
+    """Whether the product of up to eight float32 rows against a bfloat16 weight that ends in an activation or a rotation takes these."""
+    if not (a.dtype is torch.float32 and w.dtype is torch.bfloat16 and a.dim() == 2 and w.dim() == 2 and 0 < a.shape[0] <= 8
+            and a.shape[1] == w.shape[1] and a.stride(1) == 1 and w.stride(1) == 1 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (a.shape[0] == 1 or (a.stride(0) % 4 == 0 and a.stride(0) >= a.shape[1])) and w.stride(0) % 8 == 0 and w.stride(0) >= w.shape[1]):
+        return False
+    return bool(core().atoma_gemm_few_takes(a.shape[0], w.shape[0], w.shape[1], int(gated)))
+
+
+def gemm_few_gated(a: torch.Tensor, w: torch.Tensor, act="silu") -> Optional[torch.Tensor]:
+    """act(gate) * up of a [M <= 8, K] float32 times w [2 I, K] bfloat16 transposed, w in blocks of 16 gate rows and their 16 up rows: the bits
+    of ``swiglu(gemm_generic(a, w), block=16)`` by one launch; None where it does not take them."""
+    if not _few_rows(a, w, True):
+        return None
+    m, k = a.shape
+    n = w.shape[0]
+    out = torch.empty((m, n // 2), dtype=torch.float32, device=a.device)
+    _check(core().atoma_gemm_few_gated(_p(a), _p(w), _p(out), m, n, k, a.stride(0) if m > 1 else k, w.stride(0), n // 2, *_gate_args(act), _stream()),
+           "gemm_few_gated")
+    return out
+
+
+def gemm_few_rotated(a: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
+                     vcache: torch.Tensor, slot_mapping: torch.Tensor, page_size: int, nh: int, nkv: int, hd: int) -> Optional[torch.Tensor]:
+    """The fused q, k, v projection (rows of q and k heads in pair order) of a [M <= 8, K] float32: q rotated [M, nh hd] as the result, k and v in
+    the float32 cache, with the bits of ``gemm_generic`` and ``rope_cache_write`` behind it; None where it does not take them."""
+    if not (_few_rows(a, w, False) and hd % 16 == 0 and w.shape[0] == (nh + 2 * nkv) * hd and cos.dtype is torch.float32 and sin.dtype is torch.float32
+            and cos.is_contiguous() and sin.is_contiguous() and cos.shape == sin.shape and cos.shape[1] == hd // 2
+            and all(t.dtype is torch.float32 and t.is_contiguous() and tuple(t.shape[1:]) == (nkv, page_size * hd) for t in (kcache, vcache))
+            and all(t.dtype is torch.int32 and t.is_contiguous() and t.numel() >= a.shape[0] for t in (positions, slot_mapping))):
+        return None
+    m, k = a.shape
+    out = torch.empty((m, nh * hd), dtype=torch.float32, device=a.device)
+    _check(core().atoma_gemm_few_rotated(_p(a), _p(w), _p(out), m, w.shape[0], k, a.stride(0) if m > 1 else k, w.stride(0), nh * hd, _p(positions),
+                                         _p(cos), _p(sin), _p(kcache), _p(vcache), _p(slot_mapping), int(page_size), nh, nkv, hd, _stream()),
+           "gemm_few_rotated")
+    return out
+
+
 # ------------------------------------------------------------------------------------------------------------
 # mechanisms that only some architectures have: each module is compiled when a model first uses it
 

@@ -187,6 +187,9 @@ class PagedAttention(Mixer):
                                               cache.slot_mapping, cache.page_size, nh, nkv, hd)
         if qkv is None:
             x = as_tensor(x)
+            if self.paired and writes and x.dtype is torch.float32:
+                qkv = ops.gemm_few_rotated(x, w, ctx.positions, tables[0], tables[1], k_cache, v_cache, cache.slot_mapping,
+                                           cache.page_size, nh, nkv, hd)
         if qkv is not None:
             pass        # rotated and stored by the product's epilogue
         elif tables is not None or self.position is None:

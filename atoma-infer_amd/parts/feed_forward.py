@@ -73,6 +73,8 @@ class SwiGLU(FeedForward):
             h = gemm_bf16.try_linear_swiglu(x, self.w_gate_up, self.w_gate_up_tiled, self.activation)
             if h is None:
                 h = gemm_bf16.try_tile_swiglu(x, self.w_gate_up, self.activation)
+        if h is None and self.block and isinstance(x, torch.Tensor) and x.dtype is torch.float32:
+            h = ops.gemm_few_gated(x, self.w_gate_up, self.activation)
         if h is None:
             h = ops.swiglu(linear(x, self.w_gate_up), block=self.block, act=self.activation)
         return linear_delta(h, self.w_down, sink, self.w_down_tiled)

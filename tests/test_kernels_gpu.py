@@ -1058,6 +1058,41 @@ def test_gemm_tiles_of_which_a_cu_holds_two_equal_the_others(k):
         assert all(torch.equal(a, b) for a, b in zip(want, got)), tile
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu", ("clamped_sigmoid", 7.0, 1.702)])
+@pytest.mark.parametrize("m,inter,k", [(1, 2064, 32), (4, 2064, 160), (5, 4096, 2048), (8, 14336, 4096)])
+def test_few_float32_rows_end_in_the_activation(m, inter, k, act):
+    """The activation in the product's end has the bits of its own kernel behind the product: rows to eight, steps that fill no batch."""
+    from atoma_infer_amd.kernels import ops
+    wide = rnd(m, k + 4, seed=1)
+    a, w = wide[:, 4:], rnd(2 * inter, k, dtype=torch.bfloat16, seed=2)
+    got = ops.gemm_few_gated(a, w, act)
+    assert torch.equal(got, ops.swiglu(ops.gemm_generic(a, w, torch.float32), block=16, act=act))
+    assert ops.gemm_few_gated(rnd(9, k), w) is None and ops.gemm_few_gated(a, w[:4096]) is None       # (rows; a narrow weight)
+    assert ops.gemm_few_gated(a, w.float()) is None and ops.gemm_few_gated(wide[:, 2:-2] if m > 1 else wide[:, 2:-2].clone()[:, :k - 16], w) is None
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 8])
+@pytest.mark.parametrize("nh,nkv,hd,k,page", [(32, 8, 64, 2048, 16), (6, 2, 48, 96, 16), (40, 8, 128, 160, 32), (2, 2, 16, 64, 5)])
+def test_few_float32_rows_end_in_the_rotation(m, nh, nkv, hd, k, page):
+    """q, k and v by the product's end have the bits of the rotation's kernel behind the product; a row without a slot writes nothing."""
+    from atoma_infer_amd.kernels import ops
+    pages, n = -(-m // page) + 2, (nh + 2 * nkv) * hd
+    a, w = rnd(m, k, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    pos = (torch.arange(m) * 7 % 90).int().to(DEV)
+    slots = torch.randperm(pages * page, generator=torch.Generator().manual_seed(5))[:m].int()
+    if m > 2:
+        slots[2] = -1
+    slots = slots.to(DEV)
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    k1 = torch.full((pages, nkv, page * hd), 3.0, device=DEV)
+    v1, k2, v2, q2 = k1.clone(), k1.clone(), k1.clone(), torch.empty(m, nh * hd, device=DEV)
+    ops.rope_cache_write(ops.gemm_generic(a, w, torch.float32), pos, cos, sin, hd, k2, v2, slots, page, nh, nkv, hd, q2)
+    q1 = ops.gemm_few_rotated(a, w, pos, cos, sin, k1, v1, slots, page, nh, nkv, hd)
+    assert torch.equal(q1, q2) and torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert ops.gemm_few_rotated(rnd(9, k), w, pos, cos, sin, k1, v1, slots, page, nh, nkv, hd) is None
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 32, 128), (41, 80, 192), (63, 544, 512), (64, 1056, 1024), (64, 2048, 8192), (1, 64, 128)])
 def test_gemm_tile_of_64_rows(m, n, k):
     """The tiles for 33 to 64 rows, as test_gemm_tile holds the others; then what parts call with as many rows: 41 and more leave the
