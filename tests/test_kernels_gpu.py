@@ -1592,6 +1592,13 @@ def test_decode_chunks_that_grow_with_the_context(nh, nkv, hd, starts, chunk, wi
             assert err < 2e-2, f"request {e} at {s}: {err:.3e}"
 
 
+@pytest.mark.parametrize("nh,nkv,hd,starts,chunk", [(16, 1, 128, [2047, 600, 5], 256), (64, 2, 64, [2000, 1300, 9], 256), (24, 8, 128, [2040, 700], 256),
+                                                     (40, 1, 64, [2000, 300, 1], 256), (12, 1, 160, [2000, 31], 256)])
+def test_four_waves_merge_pieces_of_many_rows(nh, nkv, hd, starts, chunk):
+    """As above where a piece's live rows are more than one wave merges in one go, so that all waves of its last chunk share them."""
+    test_decode_chunks_that_grow_with_the_context(nh, nkv, hd, starts, chunk, 0)
+
+
 @pytest.mark.parametrize("plan", PLANS)
 @pytest.mark.parametrize("window", [64, 200, 1000])
 def test_decode_plans_behind_a_window(window, plan, monkeypatch):

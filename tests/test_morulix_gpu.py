@@ -142,6 +142,19 @@ def test_a_product_of_its_own_per_head(t, h, k, n, dtype):
     assert torch.equal(ops.head_linear(wide[:, : h * k], w.to(DEV, torch.bfloat16), dtype, gate.to(DEV)), got)
 
 
+@pytest.mark.parametrize("h, k, n", [(16, 128, 128), (3, 72, 20), (2, 8, 130)])
+def test_a_product_per_head_of_few_tokens_has_the_bits_of_many(h, k, n):
+    """Up to sixteen tokens, whose outputs the waves share, and the same tokens among forty."""
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(k)
+    x = torch.randn(40, h * k, generator=g).to(DEV, torch.bfloat16)
+    w, gate = torch.randn(h, n, k, generator=g).to(DEV, torch.bfloat16), torch.rand(40, h * n, generator=g).to(DEV)
+    for dtype in (torch.bfloat16, torch.float32):
+        many = ops.head_linear(x, w, dtype, gate)
+        for t in (1, 8, 16, 17):
+            assert torch.equal(ops.head_linear(x[:t], w, dtype, gate[:t].contiguous()), many[:t])
+
+
 # ---- the recurrence alone ---------------------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("inner, groups, rows", [(1030, 1, 1281), (2048, 1, 1300), (2048, 2, 700), (4096, 1, 1793), (6000, 2, 900), (4000, 1, 1792)])
