@@ -11,6 +11,7 @@
 //                 list of row tiles (expert, first place in perm) that the products below walk.  Which place a slot
 //                 gets inside its expert's range is not fixed; no result depends on it, since every row of a product
 //                 is computed by itself;
+//   route_few     both in one launch, for few tokens of up to 64 experts;
 //   expert_gemm   C[row(slot)] = (scale[slot] * A[src(slot)]) . W[expert]^T for all slots, tile by tile: true float32
 //                 multiply-adds (gemm_f32_tile.h) over float32 or bfloat16 operands, every row's sums in the same
 //                 order, so a row's result does not depend on the batch around it.  src is the slot's token (first product: the token's input, times its
@@ -27,16 +28,14 @@ constexpr int kTileM = 64, kTileN = 64;
 
 // Up to 64 experts: lane e holds expert e and counts the experts that go before it (a larger score, or the same and a
 // lower index), which is its place; the scores of the others come through scalar registers, one after the other, and no
-// step waits for the one before.
-__global__ void __launch_bounds__(256)
-route_rank_kernel(const float* __restrict__ logits, int ld, int experts, int top, int32_t* __restrict__ ids,
-                  float* __restrict__ weights, int n_tokens, int score, const float* __restrict__ correction,
-                  float scale, const float* __restrict__ bias, int groups, int groups_keep) {
+// step waits for the one before.  The place of lane e's expert among the choices of the wave's token (top or more: not
+// chosen), and its weight in `wt`.
+__device__ __forceinline__ int rank_expert(const float* __restrict__ row, int experts, int top, int score,
+                                           const float* __restrict__ correction, const float* __restrict__ bias,
+                                           int groups, int groups_keep, float& wt) {
   const int e = threadIdx.x & 63;
-  const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (t >= n_tokens) return;
   const bool real = e < experts;
-  float wt = real ? logits[(size_t)t * ld + e] + (bias != nullptr ? bias[e] : 0.f) : -INFINITY;
+  wt = real ? row[e] + (bias != nullptr ? bias[e] : 0.f) : -INFINITY;
   if (score == 1) {
     const float mx = wave_max(wt);
     wt = real ? expf(wt - mx) : 0.f;
@@ -67,15 +66,81 @@ route_rank_kernel(const float* __restrict__ logits, int ld, int experts, int top
     const float v = of(sc, i);
     place += v > sc || (v == sc && i < e);
   }
-  const bool chosen = real && place < top;
+  if (!real) place = top;
   if (score == 2) {
+    const bool chosen = place < top;
     const float mx = wave_max(chosen ? wt : -INFINITY);
     wt = chosen ? expf(wt - mx) : 0.f;
     wt /= wave_sum(wt);
   }
-  if (chosen) {
+  return place;
+}
+
+__global__ void __launch_bounds__(256)
+route_rank_kernel(const float* __restrict__ logits, int ld, int experts, int top, int32_t* __restrict__ ids,
+                  float* __restrict__ weights, int n_tokens, int score, const float* __restrict__ correction,
+                  float scale, const float* __restrict__ bias, int groups, int groups_keep) {
+  const int e = threadIdx.x & 63;
+  const int t = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (t >= n_tokens) return;
+  float wt;
+  const int place = rank_expert(logits + (size_t)t * ld, experts, top, score, correction, bias, groups, groups_keep, wt);
+  if (place < top) {
     ids[(size_t)t * top + place] = e;
     weights[(size_t)t * top + place] = wt * scale;
+  }
+}
+
+// route_topk and route_group of few tokens in one launch: each kernel is a few hundred instructions behind a launch and
+// a round trip to memory.  One workgroup; a wave ranks the experts of every sixteenth token and takes a number at the
+// counter of each chosen expert, which is the slot's place among that expert's.  Behind one barrier lane e of every wave
+// holds expert e's count, and a scan over the lanes gives where each expert's slots and tiles start.
+constexpr int kRouteFew = 64;        // tokens
+constexpr int kRouteWaves = 16;
+
+__global__ void __launch_bounds__(kRouteWaves * 64)
+route_few_kernel(const float* __restrict__ logits, int ld, int experts, int top, int32_t* __restrict__ ids,
+                 float* __restrict__ weights, int n_tokens, int score, const float* __restrict__ correction,
+                 float scale, const float* __restrict__ bias, int groups, int groups_keep, int32_t* __restrict__ perm,
+                 int32_t* __restrict__ offsets, int32_t* __restrict__ tiles, int max_tiles, int tile_m) {
+  __shared__ int32_t counts[64];
+  const int e = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (threadIdx.x < 64) counts[threadIdx.x] = 0;
+  __syncthreads();
+  constexpr int PER = kRouteFew / kRouteWaves;
+  int slot[PER], number[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int t = wave + j * kRouteWaves;
+    slot[j] = -1;
+    if (t >= n_tokens) continue;
+    float wt;
+    const int place = rank_expert(logits + (size_t)t * ld, experts, top, score, correction, bias, groups, groups_keep, wt);
+    if (place < top) {
+      slot[j] = t * top + place;
+      number[j] = atomicAdd(&counts[e], 1);
+      ids[slot[j]] = e;
+      weights[slot[j]] = wt * scale;
+    }
+  }
+  __syncthreads();
+  const int count = counts[e], mine = (count + tile_m - 1) / tile_m;
+  int at = count, tile = mine;         // inclusive sums over the lanes, then exclusive ones
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int a = __shfl_up(at, off, 64), b = __shfl_up(tile, off, 64);
+    if (e >= off) at += a, tile += b;
+  }
+  const int all = __shfl(tile, 63, 64);
+  at -= count, tile -= mine;
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (slot[j] >= 0) perm[at + number[j]] = slot[j];
+  if (wave == 0) {
+    if (e < experts) offsets[e] = at;
+    if (e == experts - 1) offsets[experts] = at + count;
+    for (int i = 0; i < mine; ++i) tiles[2 * (tile + i)] = e, tiles[2 * (tile + i) + 1] = at + i * tile_m;
+    for (int i = all + e; i < max_tiles; i += 64) tiles[2 * i] = -1, tiles[2 * i + 1] = 0;
   }
 }
 
@@ -661,6 +726,27 @@ extern "C" int atoma_route_topk(const float* logits, int ld, int experts, int to
 extern "C" int atoma_route_max_tiles(int n_slots, int experts, int tile_m) {
   const int full = n_slots / tile_m + experts;
   return full < n_slots ? full : (n_slots > 0 ? n_slots : 1);
+}
+
+// route_topk, then route_group with tiles of tile_m places, in one launch: up to 64 experts, up to 64 tokens
+extern "C" int atoma_route_few(const float* logits, int ld, int experts, int top, int32_t* ids, float* weights,
+                               int n_tokens, int score, const float* correction, float scale, const float* bias,
+                               int groups, int groups_keep, int32_t* perm, int32_t* offsets, int32_t* tiles,
+                               int max_tiles, int tile_m, hipStream_t stream) {
+  if (n_tokens <= 0) return 0;
+  if (n_tokens > kRouteFew || experts <= 0 || experts > 64 || top <= 0 || top > experts || ld < experts || score < 0 ||
+      score > 2 || (tile_m != 16 && tile_m != 64 && tile_m != 128 && tile_m != 256) ||
+      max_tiles < atoma_route_max_tiles(n_tokens * top, experts, tile_m))
+    return ATOMA_ERR_SHAPE;
+  if (groups < 0 || (groups > 0 && (experts % groups || groups_keep <= 0 || groups_keep > groups ||
+                                    groups_keep * (experts / groups) < top)))
+    return ATOMA_ERR_SHAPE;
+  if (groups <= groups_keep) groups = groups_keep = 0;      // (all groups are kept)
+  hipLaunchKernelGGL(route_few_kernel, dim3(1), dim3(kRouteWaves * 64), 0, stream, logits, ld, experts, top, ids, weights,
+                     n_tokens, score, correction, scale, bias, groups, groups_keep, perm, offsets, tiles, max_tiles,
+                     tile_m);
+  ATOMA_LAUNCH_CHECK();
+  return 0;
 }
 
 extern "C" int atoma_route_group(const int32_t* ids, int n_slots, int experts, int32_t* perm, int32_t* offsets,

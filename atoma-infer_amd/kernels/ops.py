@@ -873,15 +873,7 @@ def route_topk(logits: torch.Tensor, top: int, score: str = "sigmoid", correctio
     ones, times ``scale``.  ``bias`` [experts] joins the logits first.  ``groups`` = (count, keep): the experts form
     ``count`` equal runs of neighbours, a run's score is its best expert's, and only experts of the best ``keep`` runs
     can be chosen."""
-    _dev(logits, correction, bias)
-    _need(score in ROUTER_SCORES, f"route_topk: scores are one of {', '.join(ROUTER_SCORES)}")
-    _need(score != "softmax_chosen" or correction is None, "route_topk: a correction needs scores of its own")
-    if bias is not None:
-        _f32(bias, "bias", logits.shape[1])
-    if correction is not None:
-        _f32(correction, "correction", logits.shape[1])
-    _need(logits.dtype is torch.float32 and logits.dim() == 2 and logits.stride(1) == 1, "router logits: float32 [T, E]")
-    t, e = logits.shape
+    t, e = _router(logits, score, correction, bias)
     ids = torch.empty((t, top), dtype=torch.int32, device=logits.device)
     scores = torch.empty((t, top), dtype=torch.float32, device=logits.device)
     _check(_module("experts").atoma_route_topk(_p(logits), logits.stride(0), e, int(top), _p(ids), _p(scores), t,
@@ -889,6 +881,43 @@ def route_topk(logits: torch.Tensor, top: int, score: str = "sigmoid", correctio
                                                *((int(g) for g in groups) if groups else (0, 0)), _stream()),
            "route_topk")
     return ids, scores
+
+
+def _router(logits, score: str, correction, bias) -> Tuple[int, int]:
+    """What ``route_topk`` and ``route_few`` need of a router's outputs; (tokens, experts)."""
+    _dev(logits, correction, bias)
+    _need(score in ROUTER_SCORES, f"route_topk: scores are one of {', '.join(ROUTER_SCORES)}")
+    _need(score != "softmax_chosen" or correction is None, "route_topk: a correction needs scores of its own")
+    _need(logits.dtype is torch.float32 and logits.dim() == 2 and logits.stride(1) == 1, "router logits: float32 [T, E]")
+    if bias is not None:
+        _f32(bias, "bias", logits.shape[1])
+    if correction is not None:
+        _f32(correction, "correction", logits.shape[1])
+    return logits.shape
+
+
+# tokens and experts up to which one launch chooses and orders (csrc/kernels/experts.hip: kRouteFew, a lane an expert)
+ROUTE_FEW_TOKENS, ROUTE_FEW_EXPERTS = 64, 64
+
+
+def route_few(logits: torch.Tensor, top: int, score: str = "sigmoid", correction: Optional[torch.Tensor] = None,
+              scale: float = 1.0, bias: Optional[torch.Tensor] = None, groups: Optional[Tuple[int, int]] = None,
+              tile_m: int = 64):
+    """``route_topk`` and ``route_group`` in one launch, for up to ROUTE_FEW_TOKENS tokens and ROUTE_FEW_EXPERTS experts:
+    (ids, weights, perm, offsets, tiles)."""
+    t, e = _router(logits, score, correction, bias)
+    lib = _module("experts")
+    max_tiles = int(lib.atoma_route_max_tiles(t * top, e, int(tile_m)))
+    ids = torch.empty((t, top), dtype=torch.int32, device=logits.device)
+    scores = torch.empty((t, top), dtype=torch.float32, device=logits.device)
+    perm = torch.empty(t * top, dtype=torch.int32, device=logits.device)
+    offsets = torch.empty(e + 1, dtype=torch.int32, device=logits.device)
+    tiles = torch.empty((max_tiles, 2), dtype=torch.int32, device=logits.device)
+    _check(lib.atoma_route_few(_p(logits), logits.stride(0), e, int(top), _p(ids), _p(scores), t, ROUTER_SCORES[score],
+                               _p(correction), ctypes.c_float(scale), _p(bias),
+                               *((int(g) for g in groups) if groups else (0, 0)), _p(perm), _p(offsets), _p(tiles),
+                               max_tiles, int(tile_m), _stream()), "route_few")
+    return ids, scores, perm, offsets, tiles
 
 
 def route_group(ids: torch.Tensor, experts: int, tile_m: int = 64):

@@ -214,6 +214,37 @@ def test_experts_are_chosen_inside_the_groups_with_the_best_expert(experts, top,
     assert np.abs(wts.cpu().double().numpy() - 0.5 * want_w).max() < 1e-6
 
 
+@pytest.mark.parametrize("tokens, experts, top, groups, tile_m", [
+    (1, 1, 1, None, 16), (1, 8, 8, None, 64), (15, 64, 6, (8, 3), 16), (16, 33, 4, None, 16), (17, 64, 64, None, 16),
+    (64, 2, 1, None, 16), (64, 64, 8, None, 64), (63, 12, 5, (4, 3), 128), (64, 1, 1, None, 16)])
+@pytest.mark.parametrize("score", ["softmax", "sigmoid", "softmax_chosen"])
+def test_few_tokens_are_routed_in_one_launch_as_in_two(tokens, experts, top, groups, tile_m, score):
+    from atoma_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(tokens + experts)
+    z = torch.randn(tokens, experts + 3, generator=g).to(DEV)[:, :experts]      # (rows further apart than they are long)
+    z[tokens // 2] = 0.5
+    z[-1, ::2] = float("nan")
+    bias = torch.randn(experts, generator=g).to(DEV)
+    corr = None if score == "softmax_chosen" else torch.randn(experts, generator=g).to(DEV)
+    how = (z, top, score, corr, 0.7, bias, groups)
+    ids, weights, perm, offsets, tiles = ops.route_few(*how, tile_m)
+    want_ids, want_weights = ops.route_topk(*how)
+    want_perm, want_offsets, want_tiles = ops.route_group(want_ids.view(-1), experts, tile_m)
+    assert torch.equal(ids, want_ids) and torch.equal(weights.view(torch.int32), want_weights.view(torch.int32))
+    assert torch.equal(offsets, want_offsets) and torch.equal(tiles, want_tiles)
+    # (which place a slot has inside its expert's range is not fixed)
+    flat, perm = ids.view(-1).cpu(), perm.cpu().long()
+    assert torch.equal(perm.sort().values, torch.arange(tokens * top))
+    assert torch.equal(flat[perm], flat.sort().values)
+
+
+def test_one_launch_refuses_what_it_cannot_route():
+    from atoma_infer_amd.kernels import ops
+    for t, e, top in ((65, 8, 2), (4, 65, 2), (4, 8, 9)):
+        with pytest.raises(Exception):
+            ops.route_few(torch.zeros(t, e, device=DEV), top)
+
+
 @pytest.mark.parametrize("experts, groups", [(8, (2, 1)), (48, None), (128, (8, 2)), (300, None)])
 def test_logits_that_are_no_numbers_still_choose_experts_of_the_layer(experts, groups):
     from atoma_infer_amd.kernels import ops
