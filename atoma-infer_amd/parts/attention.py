@@ -23,7 +23,7 @@ import torch
 
 from ..kernels import ops
 from .base import CacheSpec, Mixer, PositionEncoding, WeightSpec, register_mixer
-from .linear import as_tensor, linear, linear_delta
+from .linear import LastProduct, as_tensor, linear, linear_delta
 from .position import rotation_frequencies
 
 
@@ -296,21 +296,24 @@ class TiedValueAttention(PagedAttention):
     accepts_begun = False
     takes_sink = False
 
-    def forward(self, x, ctx, cache, sink=None):
+    def first_weight(self):
+        return self.w_qk
+
+    def forward(self, x, ctx, cache, sink=None, first=None, to_last=False):
         nh, nkv, hd = self.nh, self.nkv, self.hd
         t = x.shape[0]
         writes = cache.writable
         if not writes:
             raise NotImplementedError("tied-value attention reads only a cache of its own")
-        w = self.w_qk
         # the projection leaves in float32: the norm over it and the rotation are float32 work
-        qk = linear(x, w, torch.float32)
+        qk = linear(x, self.w_qk, torch.float32) if first is None else first
         q = torch.empty((t, nh * hd), dtype=x.dtype, device=x.device)
         ops.qk_norm_rope(qk, ctx.positions, self.inv_freq, self.rotary_dim, self.q_norm, self.k_norm, self.norm_eps, q,
                          cache.k, cache.v, cache.slot_mapping, cache.page_size, nh, nkv, self.hd_in, hd)
         out = torch.empty((t, nh * hd), dtype=x.dtype, device=x.device)
         self.attend(q, cache.k, cache.v, out, ctx, cache)
-        return linear_delta(out, self.w_o, None, self.w_o_tiled)
+        last = LastProduct(out, self.w_o, self.w_o_tiled)
+        return last if to_last else last.delta()
 
 
 class HeadNormAttention(PagedAttention):

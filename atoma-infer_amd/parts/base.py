@@ -222,6 +222,12 @@ class Mixer(Part):
     def state_spec(self) -> Optional[StateSpec]:
         return None
 
+    def first_weight(self) -> Optional[torch.Tensor]:
+        """The weight of the product of x that starts the mixer, for parts whose ``forward`` has two keywords more:
+        ``first``, that product in float32 where the caller has it already, and ``to_last``: the result is then the
+        ``LastProduct`` that ends the mixer.  None for others."""
+        return None
+
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:
         """x [T, width] in the activation dtype -> [T, width].  ``cache`` is this layer call's ``LayerCache``."""
         raise NotImplementedError

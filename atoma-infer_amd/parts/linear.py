@@ -53,6 +53,37 @@ def linear(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
     return ops.gemm_generic(as_tensor(x), w, out_dtype, out)
 
 
+@dataclasses.dataclass
+class LastProduct:
+    """A mixer's output before its last product: ``linear_delta(x, w, None, tiled)`` is the output."""
+    x: torch.Tensor
+    w: torch.Tensor
+    tiled: object = None
+
+    def delta(self):
+        return linear_delta(self.x, self.w, None, self.tiled)
+
+
+def linear_pair(x, wa: torch.Tensor, wb: torch.Tensor):
+    """``linear(x, w, torch.float32)`` of two weights: one launch for few rows in bfloat16."""
+    if x.dtype is torch.bfloat16 and x.shape[0] <= 16:
+        from ..kernels import gemm_bf16
+        got = gemm_bf16.try_pair((x, wa), (x, wb), False)
+        if got is not None:
+            return got
+    return linear(x, wa, torch.float32), linear(x, wb, torch.float32)
+
+
+def delta_pair(a: LastProduct, b: LastProduct):
+    """The deltas of two last products: one launch for few rows in bfloat16."""
+    if a.x.dtype is torch.bfloat16 and a.x.shape[0] <= 16:
+        from ..kernels import gemm_bf16
+        got = gemm_bf16.try_pair((a.x, a.w), (b.x, b.w), True)
+        if got is not None:
+            return got
+    return a.delta(), b.delta()
+
+
 def linear_delta(x, w: torch.Tensor, sink: Optional[ResidualSink] = None, tiled=None):
     """A product whose result is only ever added to the residual stream.
 

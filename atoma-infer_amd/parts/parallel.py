@@ -15,6 +15,7 @@ from __future__ import annotations
 from typing import Dict, Optional, Sequence
 
 from .base import Mixer, WeightedSum, WeightSpec, register_mixer
+from .linear import delta_pair, linear_pair
 
 
 class ParallelMixer(Mixer):
@@ -70,8 +71,17 @@ class ParallelMixer(Mixer):
         found = self.step_planners(page_size, cache_dtype)
         return found[0] if found else None
 
+    def _outs(self, x, ctx, cache):
+        firsts = [b.first_weight() for b in self.branches]
+        if len(firsts) != 2 or firsts[0] is None or firsts[1] is None:
+            return [b.forward(x, ctx, cache) for b in self.branches]
+        # the branches' first products in one launch, then what is each one's own, then their last products in one
+        # launch (see linear_pair: few rows)
+        lasts = [b.forward(x, ctx, cache, first=f, to_last=True) for b, f in zip(self.branches, linear_pair(x, *firsts))]
+        return list(delta_pair(*lasts))
+
     def forward(self, x, ctx, cache):
-        outs = [b.forward(x, ctx, cache) for b in self.branches]
+        outs = self._outs(x, ctx, cache)
         if self.out_norms is None:
             return WeightedSum(list(zip(outs, self.scales)))
         from ..kernels import ops

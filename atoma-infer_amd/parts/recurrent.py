@@ -29,7 +29,7 @@ import torch
 
 from ..kernels import ops
 from .base import FREE, Mixer, StateSpec, WeightSpec, register_mixer
-from .linear import linear, linear_delta
+from .linear import LastProduct, linear, linear_delta
 from .position import rotation_frequencies
 
 
@@ -116,9 +116,17 @@ class GatedDeltaRule(Mixer):
     def device_bytes(self) -> int:
         return sum(w.numel() * w.element_size() for w in (self.w_in, self.w_ag, self.w_o))
 
-    def forward(self, x, ctx, cache):
-        state = cache.state
-        proj = linear(x, self.w_in, torch.float32)
+    def first_weight(self):
+        return self.w_in
+
+    def forward(self, x, ctx, cache, first=None, to_last=False):
+        last = LastProduct(self._mixed(x, ctx, cache.state, first), self.w_o, self.w_o_tiled)
+        return last if to_last else last.delta()
+
+    def _mixed(self, x, ctx, state, proj):
+        """What the output projection takes; ``proj``: the input projection, if it is there already."""
+        if proj is None:
+            proj = linear(x, self.w_in, torch.float32)
         # the second halves of the two low-rank maps read their columns of the float32 projection as they are
         low = proj[:, self.off_a1: self.off_g1 + self.gate_rank]
         pre = ops.lowrank_up(low, self.w_ag) if x.shape[0] <= ops.LOWRANK_UP_MAX_TOKENS else \
@@ -126,17 +134,15 @@ class GatedDeltaRule(Mixer):
         dt_pre, gate_pre = pre[:, : self.nd], pre[:, self.nd:]
         if (single_tokens(ctx) and ops.delta_step_pays(self.heads, self.kv_heads, self.dim, self.vdim, ctx.n_entries)
                 and ops.delta_step_fits(self.heads, self.kv_heads, self.dim, self.vdim, self.taps)):
-            y = ops.delta_step(proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim,
+            return ops.delta_step(proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim,
                                self.vdim, self.taps, ctx.q_start, ctx.state_slots, state, self.taps_w, dt_pre, self.dt_bias,
                                self.a_log, gate_pre, self.norm_w, self.norm_eps, x.dtype)
-            return linear_delta(y, self.w_o, None, self.w_o_tiled)
         qn, kn, vn, beta, decay, kq = ops.delta_prepare(
             proj, (self.off_q, self.off_k, self.off_v, self.off_b), self.heads, self.kv_heads, self.dim, self.vdim,
             self.taps, ctx.token_seq, ctx.q_start, ctx.state_slots, state, self.taps_w, dt_pre, self.dt_bias, self.a_log)
         o = ops.delta_scan(qn, kn, vn, beta, decay, kq, self.heads, self.kv_heads, self.dim, self.vdim, self.taps,
                            ctx.q_start, ctx.state_slots, state)
-        y = ops.delta_out(o, gate_pre, self.norm_w, self.norm_eps, self.heads, self.vdim, x.dtype)
-        return linear_delta(y, self.w_o, None, self.w_o_tiled)
+        return ops.delta_out(o, gate_pre, self.norm_w, self.norm_eps, self.heads, self.vdim, x.dtype)
 
 
 class StateSpaceDuality(Mixer):

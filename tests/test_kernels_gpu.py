@@ -1767,3 +1767,36 @@ def test_planes_of_a_split_product_over_a_tiled_weight_equal_the_row_major_ones(
         assert (got.double().sum(0).cpu() - ref).abs().max() <= 1e-2 * ref.abs().max()
     x = rnd(16, k, dtype=torch.bfloat16)
     assert torch.equal(gemm_bf16.linear_planes(x, w, tw), gemm_bf16.linear_planes(x, w))     # (few rows: row-major)
+
+
+# (8,172: 511 blocks of 16 columns, the most that waves of one block take)
+@pytest.mark.parametrize("planes", [False, True])
+@pytest.mark.parametrize("m, n0, k0, n1, k1", [(1, 4, 128, 20, 128), (3, 100, 640, 36, 1152), (8, 2560, 2048, 2240, 2048),
+                                               (8, 2048, 2048, 2048, 1024), (16, 8172, 1280, 4, 4096), (15, 16, 1152, 3072, 256)])
+def test_two_products_in_one_launch_have_the_bits_of_two(m, n0, k0, n1, k1, planes):
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    g = torch.Generator().manual_seed(m + n0 + k1)
+
+    def rows(r, c, extra):
+        return torch.randn(r, c + extra, generator=g).to(DEV, torch.bfloat16)[:, :c]
+    sides = [(rows(m, k, 8), rows(n, k, 16)) for n, k in ((n0, k0), (n1, k1))]
+    got = gb.try_pair(*sides, planes)
+    assert got is not None
+    for (x, w), y in zip(sides, got):
+        want = gb.linear_planes(x, w) if planes else gb.try_linear(x, w, torch.float32)
+        assert torch.equal(y, want)
+        ref = x.double() @ w.double().t()
+        # (K products of float32 sums, in any order)
+        bound = (x.double().abs() @ w.double().abs().t()) * (x.shape[1] * 2.0 ** -24)
+        assert bool(((y.sum(0) if planes else y).double() - ref).abs().le(bound).all())
+
+
+def test_two_products_of_other_plans_are_left_to_their_own_launches():
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+
+    def side(m, n, k, dtype=torch.bfloat16):
+        return torch.zeros(m, k, device=DEV, dtype=dtype), torch.zeros(n, k, device=DEV, dtype=dtype)
+    ok = side(8, 64, 256)
+    for other in (side(17, 64, 256), side(7, 64, 256), side(8, 8192, 256), side(8, 64, 96), side(8, 62, 256),
+                  side(8, 64, 256, torch.float32), side(0, 64, 256)):
+        assert gb.try_pair(ok, other, False) is None and gb.try_pair(other, ok, False) is None
