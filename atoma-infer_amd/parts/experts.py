@@ -166,25 +166,22 @@ class RoutedExperts(FeedForward):
             shared = self.shared_dense.device_bytes()
         return self.w_router.numel() * self.w_router.element_size() + self.top * per_expert + shared
 
-    def _route(self, logits, tile_m):
-        """(the slots' weights on the experts' inputs, on their outputs, perm, offsets, tiles)"""
-        how = (logits, self.top, self.score, self.correction, self.scale, self.router_b, self.groups)
-        if logits.shape[0] <= ops.ROUTE_FEW_TOKENS and self.experts <= ops.ROUTE_FEW_EXPERTS:
-            _, weights, *order = ops.route_few(*how, tile_m)
-        else:
-            ids, weights = ops.route_topk(*how)
-            order = ops.route_group(ids.view(-1), self.experts, tile_m)
-        flat = weights.view(-1)
-        return (flat, None, *order) if self.weighs_input else (None, flat, *order)
+    def _routed(self, x, ids, weights):
+        return self._products(x, lambda tile_m: (weights, *ops.route_group(ids.view(-1), self.experts, tile_m)))
 
-    def _routed(self, x, logits):
+    def _products(self, x, route):
+        """The experts' products; ``route(tile_m)`` gives (weights, perm, offsets, tiles) for tiles of ``tile_m`` places."""
+        def routed(tile_m):
+            weights, *order = route(tile_m)
+            flat = weights.view(-1)
+            return (flat, None, *order) if self.weighs_input else (None, flat, *order)
         t = x.shape[0]
         slots = t * self.top
         rows = self.w_gate_up.shape[1]
         if (self.mfma and x.dtype is torch.bfloat16 and slots <= stream_places(self.experts, self.w_gate_up.numel() + self.w_down.numel()) * self.experts
                 and ops.expert_stream_ok(x, rows, self.width) and self.width % 32 == 0 and self.inter % 128 == 0):
             # few places an expert: its weight is streamed, and the tokens' rows are read where they lie
-            w_in, w_out, perm, offsets, tiles = self._route(logits, ops.EXPERT_STREAM_PLACES)
+            w_in, w_out, perm, offsets, tiles = routed(ops.EXPERT_STREAM_PLACES)
             h = torch.empty((slots, self.inter), dtype=torch.bfloat16, device=x.device)
             ops.expert_stream(x, self.w_gate_up, h, perm, offsets, tiles, self.top, gather=True, scale=w_in,
                               swiglu=self.gated, relu2=not self.gated, act=self.activation)
@@ -198,7 +195,7 @@ class RoutedExperts(FeedForward):
             # many places an expert: the tile kernel of the dense products, a row of tiles an expert's run of places
             from ..kernels import gemm_bf16 as gb
             tile_m, up, down = gb.tile_groups_plan(slots, self.experts, rows, self.width, self.width, self.inter)
-            w_in, w_out, perm, offsets, tiles = self._route(logits, tile_m)
+            w_in, w_out, perm, offsets, tiles = routed(tile_m)
             xs = ops.gather_scale(x, w_in, perm, self.top)
             h = torch.empty((slots, self.inter), dtype=torch.bfloat16, device=x.device)
             gb.tile_groups(xs, self.w_gate_up, h, gb.TILE_SILU, up, tiles, offsets, perm, self.top)
@@ -209,7 +206,7 @@ class RoutedExperts(FeedForward):
             # tiles of 128 places where an expert has about a hundred or more (prompts): a weight fragment then
             # serves twice as many rows
             tile_m = 128 if slots >= 96 * self.experts else 64
-            w_in, w_out, perm, offsets, tiles = self._route(logits, tile_m)
+            w_in, w_out, perm, offsets, tiles = routed(tile_m)
             xs = ops.gather_scale(x, w_in, perm, self.top)
             h = torch.empty((slots, self.inter), dtype=torch.bfloat16, device=x.device)
             ops.expert_gemm_mfma(xs, self.w_gate_up, h, perm, offsets, tiles, self.top, swiglu=self.gated,
@@ -218,7 +215,7 @@ class RoutedExperts(FeedForward):
             ops.expert_gemm_mfma(h, self.w_down, out, perm, offsets, tiles, self.top, planes=True, tile_m=tile_m,
                                  out_scale=w_out)
             return out
-        w_in, w_out, perm, offsets, tiles = self._route(logits, 64)
+        w_in, w_out, perm, offsets, tiles = routed(64)
         if self.gated:
             gu = torch.empty((slots, 2 * self.inter), dtype=x.dtype, device=x.device)
             ops.expert_gemm(x, self.w_gate_up, gu, perm, offsets, tiles, self.top, gather=True, scale=w_in)
@@ -231,7 +228,12 @@ class RoutedExperts(FeedForward):
         return out
 
     def forward(self, x, ctx):
-        out = self._routed(x, linear(x, self.w_router, torch.float32))
+        logits = linear(x, self.w_router, torch.float32)
+        how = (logits, self.top, self.score, self.correction, self.scale, self.router_b, self.groups)
+        if logits.shape[0] <= ops.ROUTE_FEW_TOKENS and self.experts <= ops.ROUTE_FEW_EXPERTS:
+            out = self._products(x, lambda tile_m: ops.route_few(*how, tile_m)[1:])
+        else:
+            out = self._routed(x, *ops.route_topk(*how))
         if not self.shared:
             return out
         if self.shared_dense is not None:
