@@ -64,9 +64,13 @@ class LastProduct:
         return linear_delta(self.x, self.w, None, self.tiled)
 
 
+# rows up to which two products may share a launch; more fill the GPU by themselves
+PAIR_ROWS = 16
+
+
 def linear_pair(x, wa: torch.Tensor, wb: torch.Tensor):
-    """``linear(x, w, torch.float32)`` of two weights: one launch for few rows in bfloat16."""
-    if x.dtype is torch.bfloat16 and x.shape[0] <= 16:
+    """``linear(x, w, torch.float32)`` of two weights, for few rows: one launch where both are bfloat16 and of one plan."""
+    if x.dtype is torch.bfloat16:
         from ..kernels import gemm_bf16
         got = gemm_bf16.try_pair((x, wa), (x, wb), False)
         if got is not None:
@@ -75,8 +79,8 @@ def linear_pair(x, wa: torch.Tensor, wb: torch.Tensor):
 
 
 def delta_pair(a: LastProduct, b: LastProduct):
-    """The deltas of two last products: one launch for few rows in bfloat16."""
-    if a.x.dtype is torch.bfloat16 and a.x.shape[0] <= 16:
+    """The deltas of two last products, for few rows: one launch where both are bfloat16 and of one plan."""
+    if a.x.dtype is torch.bfloat16:
         from ..kernels import gemm_bf16
         got = gemm_bf16.try_pair((a.x, a.w), (b.x, b.w), True)
         if got is not None:

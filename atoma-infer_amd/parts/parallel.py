@@ -15,7 +15,7 @@ from __future__ import annotations
 from typing import Dict, Optional, Sequence
 
 from .base import Mixer, WeightedSum, WeightSpec, register_mixer
-from .linear import delta_pair, linear_pair
+from .linear import PAIR_ROWS, delta_pair, linear_pair
 
 
 class ParallelMixer(Mixer):
@@ -72,7 +72,7 @@ class ParallelMixer(Mixer):
         return found[0] if found else None
 
     def _outs(self, x, ctx, cache):
-        firsts = [b.first_weight() for b in self.branches]
+        firsts = [b.first_weight() for b in self.branches] if x.shape[0] <= PAIR_ROWS else []
         if len(firsts) != 2 or firsts[0] is None or firsts[1] is None:
             return [b.forward(x, ctx, cache) for b in self.branches]
         # the branches' first products in one launch, then what is each one's own, then their last products in one
