@@ -410,8 +410,8 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 // loads and its results then pass under the other's products, and a barrier holds up half of a CU's waves.  Against tiles of the same 256 or
 // 128 rows with one barrier a step, four buffers and a workgroup a CU (some 18,000 products; geometric means of the time, by workgroups
 // a CU up to one / more): 128 x 128 0.95 to 0.98 / 0.84 to 0.89, 256 x 128 0.97 / 0.98, 128 x 192 against 256 x 96 0.92 to 0.97 / 0.85 to
-// 0.88, 128 x 64 1.01 / 0.83 to 0.88 (so only there).  us, before / now: q, k, v of 2,048 rows against 3,072 x 2,048 35.9 / 33.0, two slices of
-// 2,048 x 8,192 69.0 / 65.3.  (192 x 128, patches of eight rows of tiles and 128 x 160 gave nothing; 256 x 160 by halves of 80 lost 1 %.)
+// 0.88, 128 x 64 1.01 / 0.83 to 0.88 (so only there).  us, before / now: q, k, v of 2,048 rows against 3,072 x 2,048 35.9 / 33.0 (one round
+// of 128 x 192, which keeps one barrier a step: 31.1), two slices of 2,048 x 8,192 69.0 / 65.3.  (192 x 128, patches of eight rows of tiles and 128 x 160 gave nothing; 256 x 160 by halves of 80 lost 1 %.)
 // EU: waves a SIMD that the registers are to leave room for (four: two workgroups of eight waves).
 template <int BM_, int BN_, int WM_, int WN_, int EU_ = 2>
 struct Phased {
