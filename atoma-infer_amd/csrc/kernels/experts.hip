@@ -92,13 +92,15 @@ route_rank_kernel(const float* __restrict__ logits, int ld, int experts, int top
 }
 
 // route_topk and route_group of few tokens in one launch: each kernel is a few hundred instructions behind a launch and
-// a round trip to memory.  One workgroup; a wave ranks the experts of every sixteenth token and takes a number at the
-// counter of each chosen expert, which is the slot's place among that expert's.  Behind one barrier lane e of every wave
-// holds expert e's count, and a scan over the lanes gives where each expert's slots and tiles start.
-constexpr int kRouteFew = 64;        // tokens
-constexpr int kRouteWaves = 16;
+// a round trip to memory.  One workgroup; a wave ranks the experts of its token and takes a number at the counter of each
+// chosen expert, which is the slot's place among that expert's.  Behind one barrier lane e of every wave holds expert e's
+// count, and a scan over the lanes gives where each expert's slots and tiles start.  Two launches / this one in a graph, us,
+// 1 / 8 / 16 tokens: 8 of 8 experts 3.7 / 4.4 / 4.7 -> 2.8 / 2.8 / 3.1, 4 of 32 5.6 / 6.8 / 7.2 -> 3.9 / 3.9 / 4.6, 6 of 64 in
+// eight groups 11.2 / 12.9 / 13.8 -> 7.9 / 8.3 / 10.7.  No more than a token a wave: with two in turn the last of these takes
+// 19.4 against 14.0, with four the second 11.2 against 7.6.
+constexpr int kRouteFew = 16;        // tokens, a wave each
 
-__global__ void __launch_bounds__(kRouteWaves * 64)
+__global__ void __launch_bounds__(kRouteFew * 64)
 route_few_kernel(const float* __restrict__ logits, int ld, int experts, int top, int32_t* __restrict__ ids,
                  float* __restrict__ weights, int n_tokens, int score, const float* __restrict__ correction,
                  float scale, const float* __restrict__ bias, int groups, int groups_keep, int32_t* __restrict__ perm,
@@ -107,20 +109,15 @@ route_few_kernel(const float* __restrict__ logits, int ld, int experts, int top,
   const int e = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (threadIdx.x < 64) counts[threadIdx.x] = 0;
   __syncthreads();
-  constexpr int PER = kRouteFew / kRouteWaves;
-  int slot[PER], number[PER];
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int t = wave + j * kRouteWaves;
-    slot[j] = -1;
-    if (t >= n_tokens) continue;
+  int slot = -1, number = 0;
+  if (wave < n_tokens) {
     float wt;
-    const int place = rank_expert(logits + (size_t)t * ld, experts, top, score, correction, bias, groups, groups_keep, wt);
+    const int place = rank_expert(logits + (size_t)wave * ld, experts, top, score, correction, bias, groups, groups_keep, wt);
     if (place < top) {
-      slot[j] = t * top + place;
-      number[j] = atomicAdd(&counts[e], 1);
-      ids[slot[j]] = e;
-      weights[slot[j]] = wt * scale;
+      slot = wave * top + place;
+      number = atomicAdd(&counts[e], 1);
+      ids[slot] = e;
+      weights[slot] = wt * scale;
     }
   }
   __syncthreads();
@@ -133,9 +130,7 @@ route_few_kernel(const float* __restrict__ logits, int ld, int experts, int top,
   }
   const int all = __shfl(tile, 63, 64);
   at -= count, tile -= mine;
-#pragma unroll
-  for (int j = 0; j < PER; ++j)
-    if (slot[j] >= 0) perm[at + number[j]] = slot[j];
+  if (slot >= 0) perm[at + number] = slot;
   if (wave == 0) {
     if (e < experts) offsets[e] = at;
     if (e == experts - 1) offsets[experts] = at + count;
@@ -728,7 +723,7 @@ extern "C" int atoma_route_max_tiles(int n_slots, int experts, int tile_m) {
   return full < n_slots ? full : (n_slots > 0 ? n_slots : 1);
 }
 
-// route_topk, then route_group with tiles of tile_m places, in one launch: up to 64 experts, up to 64 tokens
+// route_topk, then route_group with tiles of tile_m places, in one launch: up to 64 experts, up to 16 tokens
 extern "C" int atoma_route_few(const float* logits, int ld, int experts, int top, int32_t* ids, float* weights,
                                int n_tokens, int score, const float* correction, float scale, const float* bias,
                                int groups, int groups_keep, int32_t* perm, int32_t* offsets, int32_t* tiles,
@@ -742,7 +737,7 @@ extern "C" int atoma_route_few(const float* logits, int ld, int experts, int top
                                     groups_keep * (experts / groups) < top)))
     return ATOMA_ERR_SHAPE;
   if (groups <= groups_keep) groups = groups_keep = 0;      // (all groups are kept)
-  hipLaunchKernelGGL(route_few_kernel, dim3(1), dim3(kRouteWaves * 64), 0, stream, logits, ld, experts, top, ids, weights,
+  hipLaunchKernelGGL(route_few_kernel, dim3(1), dim3(kRouteFew * 64), 0, stream, logits, ld, experts, top, ids, weights,
                      n_tokens, score, correction, scale, bias, groups, groups_keep, perm, offsets, tiles, max_tiles,
                      tile_m);
   ATOMA_LAUNCH_CHECK();

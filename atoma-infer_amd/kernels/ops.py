@@ -896,8 +896,8 @@ def _router(logits, score: str, correction, bias) -> Tuple[int, int]:
     return logits.shape
 
 
-# tokens and experts up to which one launch chooses and orders (csrc/kernels/experts.hip: kRouteFew, a lane an expert)
-ROUTE_FEW_TOKENS, ROUTE_FEW_EXPERTS = 64, 64
+# tokens and experts up to which one launch chooses and orders (csrc/kernels/experts.hip: kRouteFew, a wave a token; a lane an expert)
+ROUTE_FEW_TOKENS, ROUTE_FEW_EXPERTS = 16, 64
 
 
 def route_few(logits: torch.Tensor, top: int, score: str = "sigmoid", correction: Optional[torch.Tensor] = None,

@@ -215,8 +215,8 @@ def test_experts_are_chosen_inside_the_groups_with_the_best_expert(experts, top,
 
 
 @pytest.mark.parametrize("tokens, experts, top, groups, tile_m", [
-    (1, 1, 1, None, 16), (1, 8, 8, None, 64), (15, 64, 6, (8, 3), 16), (16, 33, 4, None, 16), (17, 64, 64, None, 16),
-    (64, 2, 1, None, 16), (64, 64, 8, None, 64), (63, 12, 5, (4, 3), 128), (64, 1, 1, None, 16)])
+    (1, 1, 1, None, 16), (1, 8, 8, None, 64), (15, 64, 6, (8, 3), 16), (16, 33, 4, None, 16), (16, 64, 64, None, 16),
+    (16, 2, 2, None, 16), (16, 64, 8, None, 64), (13, 12, 5, (4, 3), 128), (16, 1, 1, None, 16)])
 @pytest.mark.parametrize("score", ["softmax", "sigmoid", "softmax_chosen"])
 def test_few_tokens_are_routed_in_one_launch_as_in_two(tokens, experts, top, groups, tile_m, score):
     from atoma_infer_amd.kernels import ops
@@ -240,7 +240,7 @@ def test_few_tokens_are_routed_in_one_launch_as_in_two(tokens, experts, top, gro
 
 def test_one_launch_refuses_what_it_cannot_route():
     from atoma_infer_amd.kernels import ops
-    for t, e, top in ((65, 8, 2), (4, 65, 2), (4, 8, 9)):
+    for t, e, top in ((17, 8, 2), (4, 65, 2), (4, 8, 9)):
         with pytest.raises(Exception):
             ops.route_few(torch.zeros(t, e, device=DEV), top)
 
