@@ -328,6 +328,7 @@ def _few_rows(a: torch.Tensor, w: torch.Tensor, gated: bool) -> bool:
             and a.shape[1] == w.shape[1] and a.stride(1) == 1 and w.stride(1) == 1 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (a.shape[0] == 1 or (a.stride(0) % 4 == 0 and a.stride(0) >= a.shape[1])) and w.stride(0) % 8 == 0 and w.stride(0) >= w.shape[1]):
         return False
+    _dev(a, w)
     return bool(core().atoma_gemm_few_takes(a.shape[0], w.shape[0], w.shape[1], int(gated)))
 
 
@@ -353,6 +354,7 @@ def gemm_few_rotated(a: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, 
             and all(t.dtype is torch.float32 and t.is_contiguous() and tuple(t.shape[1:]) == (nkv, page_size * hd) for t in (kcache, vcache))
             and all(t.dtype is torch.int32 and t.is_contiguous() and t.numel() >= a.shape[0] for t in (positions, slot_mapping))):
         return None
+    _dev(positions, cos, sin, kcache, vcache, slot_mapping)
     m, k = a.shape
     out = torch.empty((m, nh * hd), dtype=torch.float32, device=a.device)
     _check(core().atoma_gemm_few_rotated(_p(a), _p(w), _p(out), m, w.shape[0], k, a.stride(0) if m > 1 else k, w.stride(0), nh * hd, _p(positions),
