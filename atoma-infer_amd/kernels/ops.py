@@ -352,6 +352,7 @@ def gemm_few_rotated(a: torch.Tensor, w: torch.Tensor, positions: torch.Tensor, 
     if not (_few_rows(a, w, False) and hd % 16 == 0 and w.shape[0] == (nh + 2 * nkv) * hd and cos.dtype is torch.float32 and sin.dtype is torch.float32
             and cos.is_contiguous() and sin.is_contiguous() and cos.shape == sin.shape and cos.shape[1] == hd // 2
             and all(t.dtype is torch.float32 and t.is_contiguous() and tuple(t.shape[1:]) == (nkv, page_size * hd) for t in (kcache, vcache))
+            and kcache.shape == vcache.shape
             and all(t.dtype is torch.int32 and t.is_contiguous() and t.numel() >= a.shape[0] for t in (positions, slot_mapping))):
         return None
     _dev(positions, cos, sin, kcache, vcache, slot_mapping)

@@ -1,5 +1,5 @@
 """What the wrappers of products with fused ends refuse before anything is launched: a kernel takes addresses as they come, so an operand
-in host memory must not reach it.  The native module is replaced, so nothing here needs or touches a GPU."""
+in host memory or a cache that is too short must not reach it.  The native module is replaced, so nothing here needs or touches a GPU."""
 import pytest
 import torch
 
@@ -58,3 +58,15 @@ def test_few_rows_that_end_in_the_rotation_are_device_tensors(launched, host):
     with pytest.raises(ops.KernelError, match="device tensors only"):
         ops.gemm_few_rotated(**operands, page_size=PAGE, nh=NH, nkv=NKV, hd=HD)
     assert len(launched) == 1
+
+
+def test_few_rows_that_end_in_the_rotation_leave_caches_of_two_lengths(launched):
+    """To the rotation's own kernel, whose wrapper refuses them."""
+    operands = rotated_operands()
+    operands["vcache"] = there(4, NKV, PAGE * HD)
+    assert ops.gemm_few_rotated(**operands, page_size=PAGE, nh=NH, nkv=NKV, hd=HD) is None and not launched
+    qkv = there(3, (NH + 2 * NKV) * HD)
+    with pytest.raises(ops.KernelError, match="cache tensors"):
+        ops.rope_cache_write(qkv, operands["positions"], operands["cos"], operands["sin"], HD, operands["kcache"], operands["vcache"],
+                             operands["slot_mapping"], PAGE, NH, NKV, HD, there(3, NH * HD))
+    assert not launched
