@@ -297,7 +297,8 @@ class TiedValueAttention(PagedAttention):
     takes_sink = False
 
     def first_weight(self):
-        return self.w_qk
+        # (a forward put in this one's place need not know the keywords)
+        return self.w_qk if getattr(self.forward, "__func__", None) is TiedValueAttention.forward else None
 
     def forward(self, x, ctx, cache, sink=None, first=None, to_last=False):
         nh, nkv, hd = self.nh, self.nkv, self.hd

@@ -225,7 +225,7 @@ class Mixer(Part):
     def first_weight(self) -> Optional[torch.Tensor]:
         """The weight of the product of x that starts the mixer, for parts whose ``forward`` has two keywords more:
         ``first``, that product in float32 where the caller has it already, and ``to_last``: the result is then the
-        ``LastProduct`` that ends the mixer.  None for others."""
+        ``LastProduct`` that ends the mixer.  None for others, subclasses with a ``forward`` of their own among them."""
         return None
 
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:

@@ -72,7 +72,8 @@ class ParallelMixer(Mixer):
         return found[0] if found else None
 
     def _outs(self, x, ctx, cache):
-        firsts = [b.first_weight() for b in self.branches] if x.shape[0] <= PAIR_ROWS else []
+        offers = [getattr(b, "first_weight", None) for b in self.branches] if x.shape[0] <= PAIR_ROWS else []
+        firsts = [offer() if offer is not None else None for offer in offers]
         if len(firsts) != 2 or firsts[0] is None or firsts[1] is None:
             return [b.forward(x, ctx, cache) for b in self.branches]
         # the branches' first products in one launch, then what is each one's own, then their last products in one
