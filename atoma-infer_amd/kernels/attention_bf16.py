@@ -498,49 +498,82 @@ def whole_waves(pairs: int, keys: int, head_size: int) -> int:
     return 4 if pairs <= 512 or 768 < pairs <= 1024 else 8
 
 
-# A block of 32 keys of a chunk (bound by its bytes) against one of a prompt tile's task (bound by its arithmetic), in time; and the share of
-# the prompts' time from which on decoded tokens' chunks run among the prompt tiles
-DEAL_CHUNK_BLOCK, DEAL_MIN_SHARE = 3.4, 0.3
+# A block of 32 keys of a chunk (bound by its bytes) against one of a prompt tile's task (bound by its arithmetic), in time
+DEAL_CHUNK_BLOCK = 3.4
 
 
-def _deal(main: np.ndarray, kv_heads: int, head_size: int, compute_units: int) -> Optional[np.ndarray]:
+def _deal(main: np.ndarray, kv_heads: int, head_size: int, compute_units: int, waves: int) -> Optional[np.ndarray]:
     """The main tasks of a step of prompts and decoded tokens, a workgroup's four behind one another, in the order in which a mixed step is
-    quickest; None where they stay as they are.
+    quickest; None where they stay as they are: everywhere the GPU takes all workgroups at once.
 
-    * Entries of a single task (a decoded token of few keys) share workgroups, four of a length, where there are more workgroups than the
-      GPU takes at once: alone each keeps six of its eight waves idle (2,048 tokens, 32 heads of 64: 180 decoded tokens of 20 to 330 keys
-      beside 14 prompts of up to 300 31.2 -> 22.0 us, 100 tokens 22.8 -> 17.7; three short entries, which fill nothing, 5.8 -> 6.1, stay).
-    * The chunks of decoded tokens, which wait for memory, run among the prompt tiles, which compute, not behind them: 2,048 tokens, 16 / 32 /
-      63 of them decoded at 2,048 keys, 45.0 / 56.2 / 81.9 -> 41.5 / 48.6 / 72.2 us; 24 heads of 128, 20 decoded at up to 4,096 80.1 -> 72.5.
-      Not where the chunks are less than ``DEAL_MIN_SHARE`` of the tiles' time: tiles that walk long key ranges then only start later (30
-      chunked tokens beside 2,018 behind 6,000 others 154 -> 190 us)."""
+    * Entries of a single task (a decoded token of few keys) share workgroups (``_pays_to_share``): 2,048 tokens, 32 heads of 64, 180 decoded
+      tokens of 20 to 330 keys beside 14 prompts of up to 300 31.2 -> 22.0 us, 100 tokens 22.8 -> 17.7.
+    * The chunks of decoded tokens, which wait for memory, run among the prompt tiles, which compute, not behind them (``_pays_to_mix``): 2,048
+      tokens, 16 / 32 / 63 of them decoded at 2,048 keys, 45.0 / 56.2 / 81.9 -> 41.5 / 48.6 / 72.2 us; 24 heads of 128, 20 decoded at up
+      to 4,096 80.1 -> 72.5.  Not by launches of one wave a task, nor of heads beyond 192 columns, which have no other: a wave's chunk is
+      then the longest task there is and must not start late (40 heads of 48, 107 tokens at up to 6,900 keys beside portions of up to 19
+      63 -> 78 us).  Nor with KV heads that do not come in eights: workgroups go to the XCDs in turn, and tiles at a regular distance then
+      share a few (two KV heads, 63 tokens beside 961 behind 5,800 others 39 -> 54 us).
+
+    2,400 drawn steps (thirteen shapes of 1 to 32 KV heads of 32 to 256 columns, with windows and biases, 1 to 250 decoded tokens at 32 to
+    12,000 keys beside portions of 1 to 4,096 tokens, 512 to 4,096 in all), the attention kernel's time against tasks as they come: where they are
+    dealt 0.88 in the geometric mean, 1.8 percent of the steps more than 2 percent slower and two of 1,138 more than 5 (of the steps left
+    as they are, the same launch twice, 1.0 percent and three).  Dealt wherever there are more workgroups than the GPU takes, chunks
+    wherever they are 0.3 of the tiles' time: 7.9 percent of the steps and 73, up to 1.42 times as long."""
     groups = main.reshape(-1, 4, 12)
-    chunked = groups[:, 0, 6] >= 0
-    full = len(groups) * kv_heads > compute_units * (2 if head_size <= 64 else 1)
-    if not full and not chunked.any():
+    round_ = max(1, compute_units * (2 if head_size <= 64 else 1) // kv_heads)       # groups that the GPU takes at once
+    if len(groups) <= round_:
         return None
-    blocks = (groups[..., 5] - groups[..., 4]) * (groups[..., 0] >= 0)
-    single = ~chunked & (groups[:, 0, 0] >= 0) & (groups[:, 1:, 0] < 0).all(1) if full else np.zeros(len(groups), dtype=bool)
+    chunked = groups[:, 0, 6] >= 0
+    blocks = (groups[..., 5] - groups[..., 4]) / 32 * (groups[..., 0] >= 0)
+    single = ~chunked & (groups[:, 0, 0] >= 0) & (groups[:, 1:, 0] < 0).all(1)
+    if not _pays_to_share(blocks.max(1), chunked, single, round_):
+        single[:] = False
     tiles = groups[~chunked & ~single]
-    walks = blocks[~chunked & ~single]
+    walks = blocks[~chunked & ~single].max(1, initial=0)
+    order = np.argsort(-walks, kind="stable")
+    few = groups[single, 0]
+    few = few[np.argsort(few[:, 4] - few[:, 5], kind="stable")]
+    few = np.concatenate([few, np.tile(_NULL_TASK, (-len(few) % 4, 1))]).reshape(-1, 4, 12)
     chunks = groups[chunked]
-    order = np.argsort(-walks.max(1, initial=0), kind="stable")
-    few = groups[single]
-    if len(few):
-        few = few[:, 0]
-        few = few[np.argsort(few[:, 4] - few[:, 5], kind="stable")]
-        few = np.concatenate([few, np.tile(_NULL_TASK, (-len(few) % 4, 1))]).reshape(-1, 4, 12)
-    if len(chunks) and DEAL_CHUNK_BLOCK * blocks[chunked | single].sum() >= DEAL_MIN_SHARE * walks.sum():
+    if len(chunks) and waves >= 2 and head_size <= 192 and kv_heads % 8 == 0 and _pays_to_mix(
+            walks[order], blocks[~chunked & ~single].sum(), blocks[chunked | single].sum(), round_):
         tiles, others = tiles[order], np.concatenate([few, chunks])
         # (spread evenly: the i-th of n comes i / n of the way)
-        at = np.concatenate([np.arange(len(tiles)) / max(1, len(tiles)), (np.arange(len(others)) + 0.5) / len(others)])
+        at = np.concatenate([np.arange(len(tiles)) / len(tiles), (np.arange(len(others)) + 0.5) / len(others)])
         return np.concatenate([tiles, others])[np.argsort(at, kind="stable")].reshape(-1, 12)
     if not len(few):
         return None
     tiles = np.concatenate([tiles, few])
-    lengths = np.concatenate([walks.max(1, initial=0), (few[..., 5] - few[..., 4]).max(1)])
+    lengths = np.concatenate([walks, (few[..., 5] - few[..., 4]).max(1) / 32])
     order = np.argsort(-lengths, kind="stable")[_serpentine(len(tiles), kv_heads, compute_units, head_size)]
     return np.concatenate([tiles[order], chunks]).reshape(-1, 12)
+
+
+def _pays_to_share(walks: np.ndarray, chunked: np.ndarray, single: np.ndarray, round_: int) -> bool:
+    """Whether groups of a single task (a decoded token of few keys) share workgroups, four of a length: alone each keeps six of its eight
+    waves idle.  Where there are two rounds and more (0.83 of the time over 418 steps, 1.04 at most); and where one round is left and no such
+    task walks further than the tiles do (0.93 over 49, 1.02 at most).  Else there is little to gain, and a workgroup of four long walks may
+    be the last to end: 0.98 over 281, but 18 of them more than 2 percent slower (29 tokens of 511 keys beside tiles of 204, 16 heads over one
+    KV head, 16.6 -> 20.9 us; three short entries, which fill nothing, 5.8 -> 6.1)."""
+    n = len(walks)
+    if not single.any():
+        return False
+    shared = n - int(single.sum()) * 3 // 4
+    tiles = walks[~chunked & ~single].max(initial=0)
+    return n >= 2 * round_ or (shared <= round_ and walks[single].max() <= tiles)
+
+
+def _pays_to_mix(walks: np.ndarray, tile_blocks: float, other_blocks: float, round_: int) -> bool:
+    """Whether what decoded tokens run, which waits for memory, goes among the prompt tiles, which compute (``walks``: their blocks of 32
+    keys, longest first), and not behind them."""
+    n = len(walks)
+    if n < 0.9 * round_ or DEAL_CHUNK_BLOCK * other_blocks < 0.3 * tile_blocks:
+        return False
+    tiles = walks.sum() / round_
+    work = tiles + DEAL_CHUNK_BLOCK * other_blocks / 4 / round_
+    ends = np.arange(n) / n * work + 1.5 * walks
+    return walks[0] <= 2.2 * tiles and ends.max() <= 1.02 * max(work, 1.5 * walks[0])
 
 
 def plan_step(starts: np.ndarray, counts: np.ndarray, group: int, window: int, bucket_keys: Optional[int] = None, *, kv_heads: int,
@@ -552,7 +585,7 @@ def plan_step(starts: np.ndarray, counts: np.ndarray, group: int, window: int, b
     arr, meta = build_tasks(starts, counts, group, window, bucket_keys, kv_heads=kv_heads, head_size=head_size, keep=keep, **options)
     n_main, n_comb, n_part, waves, pieces, merge = meta
     if bucket_keys is None:
-        main = _deal(arr[:n_main], kv_heads, head_size, options.get("compute_units", 256))
+        main = _deal(arr[:n_main], kv_heads, head_size, options.get("compute_units", 256), waves)
         if main is not None:
             arr, meta = np.concatenate([main, arr[n_main:]]), (len(main), n_comb, n_part, waves, pieces, merge)
             n_main = len(main)

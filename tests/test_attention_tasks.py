@@ -336,7 +336,8 @@ def test_waves_of_whole_ranges_at_the_lines(s, kv_heads, keys, head_size, want):
 @pytest.mark.parametrize("seed", range(24))
 def test_workgroups_of_mixed_steps_are_dealt_without_losing_a_task(seed):
     """Decoded tokens of few and of many keys beside portions of prompts: the same tasks as the builder's, fours that share keys unbroken,
-    single ones together in fours where workgroups are more than the GPU takes, and every key seen once."""
+    single ones together in fours where workgroups are two rounds and more, or fit one round then and no tile ends before them, and every
+    key seen once."""
     rng = np.random.default_rng(700 + seed)
     group, head_size = int(rng.choice([1, 3, 4, 40])), int(rng.choice([64, 128]))
     window = int(rng.choice([0, 0, 700]))
@@ -352,9 +353,14 @@ def test_workgroups_of_mixed_steps_are_dealt_without_losing_a_task(seed):
     fours = {tuple(map(tuple, f.tolist())) for f in got[: mg[0]].reshape(-1, 4, 12)}
     kept = [tuple(map(tuple, f.tolist())) for f in arr[: meta[0]].reshape(-1, 4, 12) if (f[:, 0] >= 0).sum() > 1]
     assert all(f in fours for f in kept)
-    full = meta[0] // 4 * 8 > 256 * (2 if head_size <= 64 else 1)
-    singles = sum((f[1:, 0] < 0).all() and f[0, 6] < 0 for f in arr[: meta[0]].reshape(-1, 4, 12))
-    assert mg[0] // 4 == meta[0] // 4 - (singles - -(-singles // 4) if full else 0)
+    at_once = 256 * (2 if head_size <= 64 else 1) // 8
+    fours = arr[: meta[0]].reshape(-1, 4, 12)
+    alone, chunked = (fours[:, 1:, 0] < 0).all(1) & (fours[:, 0, 6] < 0), fours[:, 0, 6] >= 0
+    singles, walks = int(alone.sum()), (fours[..., 5] - fours[..., 4]).max(1)
+    left = len(fours) - singles + -(-singles // 4)
+    pays = len(fours) > at_once and singles and (len(fours) >= 2 * at_once or (
+        left <= at_once and walks[alone].max() <= walks[~alone & ~chunked].max(initial=0)))
+    assert mg[0] // 4 == (left if pays else len(fours))
 
 
 def test_chunks_run_among_prompt_tiles_only_where_they_take_a_share_of_the_time():
@@ -366,3 +372,18 @@ def test_chunks_run_among_prompt_tiles_only_where_they_take_a_share_of_the_time(
         assert bool(chunked[: len(chunked) // 4].any()) == mixed
         walks = (arr[: meta[0], 5] - arr[: meta[0], 4]).reshape(-1, 4).max(1)[~chunked]
         assert not mixed or (np.diff(walks) <= 0).all()
+
+
+@pytest.mark.parametrize("kv_heads,head_size,starts,counts,mixed", [
+    (8, 128, [6000] * 119 + [6406], [1] * 119 + [393], False),                  # (few tiles, of long walks: they start first, and all at once)
+    (2, 32, [5759] * 63 + [5800], [1] * 63 + [961], False),                     # (KV heads that are not in eights)
+    (8, 64, [4000] * 28 + [4294], [1] * 28 + [2020], False),                    # (behind a window: every tile walks as far)
+    (8, 64, [2048] * 63 + [0], [1] * 63 + [1985], True),
+    (24, 64, [2048] * 20 + [0], [1] * 20 + [2028], True),
+    (8, 128, [4096] * 20 + [0], [1] * 20 + [2028], True),
+    (8, 256, [4096] * 20 + [0], [1] * 20 + [2028], False)])                     # (one wave a task)
+def test_chunks_stay_behind_tiles_that_would_end_late(kv_heads, head_size, starts, counts, mixed):
+    window = 1024 if starts[-1] == 4294 else 0
+    arr, meta = A.plan_step(np.asarray(starts), np.asarray(counts), 4, window, kv_heads=kv_heads, max_waves=8 if head_size <= 192 else 1, head_size=head_size)
+    chunked = arr[: meta[0]].reshape(-1, 4, 12)[:, 0, 6] >= 0
+    assert chunked.any() and bool((np.diff(chunked.astype(int)) < 0).any()) == mixed
