@@ -510,8 +510,8 @@ def _deal(main: np.ndarray, kv_heads: int, head_size: int, compute_units: int, w
       tokens of 20 to 330 keys beside 14 prompts of up to 300 31.2 -> 22.0 us, 100 tokens 22.8 -> 17.7.
     * The chunks of decoded tokens, which wait for memory, run among the prompt tiles, which compute, not behind them (``_pays_to_mix``): 2,048
       tokens, 16 / 32 / 63 of them decoded at 2,048 keys, 45.0 / 56.2 / 81.9 -> 41.5 / 48.6 / 72.2 us; 24 heads of 128, 20 decoded at up
-      to 4,096 80.1 -> 72.5.  Not by launches of one wave a task, nor of heads beyond 192 columns, which have no other: a wave's chunk is
-      then the longest task there is and must not start late (40 heads of 48, 107 tokens at up to 6,900 keys beside portions of up to 19
+      to 4,096 80.1 -> 72.5.  Not by launches of one wave a task, the only ones of keys or values beyond 192 columns: a wave's
+      chunk is then the longest task there is and must not start late (40 heads of 48, 107 tokens at up to 6,900 keys beside portions of up to 19
       63 -> 78 us).  Nor with KV heads that do not come in eights: workgroups go to the XCDs in turn, and tiles at a regular distance then
       share a few (two KV heads, 63 tokens beside 961 behind 5,800 others 39 -> 54 us).
 
@@ -536,7 +536,7 @@ def _deal(main: np.ndarray, kv_heads: int, head_size: int, compute_units: int, w
     few = few[np.argsort(few[:, 4] - few[:, 5], kind="stable")]
     few = np.concatenate([few, np.tile(_NULL_TASK, (-len(few) % 4, 1))]).reshape(-1, 4, 12)
     chunks = groups[chunked]
-    if len(chunks) and waves >= 2 and head_size <= 192 and kv_heads % 8 == 0 and _pays_to_mix(
+    if len(chunks) and waves >= 2 and kv_heads % 8 == 0 and _pays_to_mix(
             walks[order], blocks[~chunked & ~single].sum(), blocks[chunked | single].sum(), round_):
         tiles, others = tiles[order], np.concatenate([few, chunks])
         # (spread evenly: the i-th of n comes i / n of the way)
@@ -554,7 +554,7 @@ def _pays_to_share(walks: np.ndarray, chunked: np.ndarray, single: np.ndarray, r
     """Whether groups of a single task (a decoded token of few keys) share workgroups, four of a length: alone each keeps six of its eight
     waves idle.  Where there are two rounds and more (0.83 of the time over 418 steps, 1.04 at most); and where one round is left and no such
     task walks further than the tiles do (0.93 over 49, 1.02 at most).  Else there is little to gain, and a workgroup of four long walks may
-    be the last to end: 0.98 over 281, but 18 of them more than 2 percent slower (29 tokens of 511 keys beside tiles of 204, 16 heads over one
+    be the last to end: 0.97 over 281, but 20 of them more than 2 percent slower (29 tokens of 511 keys beside tiles of 204, 16 heads over one
     KV head, 16.6 -> 20.9 us; three short entries, which fill nothing, 5.8 -> 6.1)."""
     n = len(walks)
     if not single.any():
@@ -566,7 +566,13 @@ def _pays_to_share(walks: np.ndarray, chunked: np.ndarray, single: np.ndarray, r
 
 def _pays_to_mix(walks: np.ndarray, tile_blocks: float, other_blocks: float, round_: int) -> bool:
     """Whether what decoded tokens run, which waits for memory, goes among the prompt tiles, which compute (``walks``: their blocks of 32
-    keys, longest first), and not behind them."""
+    keys, longest first), and not behind them.
+
+    Only where the tiles fill the GPU by themselves, about (0.9 of a round): fewer leave it to the chunks anyway (1.01 over 39 steps, up
+    to 1.21; where the GPU takes all workgroups at once 1.00 over 239, up to 1.41).  Not where the chunks are less than 0.3 of the tiles' time
+    (30 tokens beside 2,018 behind 6,000 others 154 -> 190 us), nor where a tile is a chain longer than the tiles' own rounds by more than a
+    lone prompt's longest is (twice; one of 2,767 keys among short ones 53 -> 60), nor where tiles of long walks, each half as long again
+    beside chunks, would begin too late to end with the others (all of a window's 1,024 keys, 47 -> 53)."""
     n = len(walks)
     if n < 0.9 * round_ or DEAL_CHUNK_BLOCK * other_blocks < 0.3 * tile_blocks:
         return False
@@ -585,7 +591,7 @@ def plan_step(starts: np.ndarray, counts: np.ndarray, group: int, window: int, b
     arr, meta = build_tasks(starts, counts, group, window, bucket_keys, kv_heads=kv_heads, head_size=head_size, keep=keep, **options)
     n_main, n_comb, n_part, waves, pieces, merge = meta
     if bucket_keys is None:
-        main = _deal(arr[:n_main], kv_heads, head_size, options.get("compute_units", 256), waves)
+        main = _deal(arr[:n_main], kv_heads, head_size, options.get("compute_units", 256), min(waves, options.get("max_waves", 2)))
         if main is not None:
             arr, meta = np.concatenate([main, arr[n_main:]]), (len(main), n_comb, n_part, waves, pieces, merge)
             n_main = len(main)

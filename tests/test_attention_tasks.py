@@ -381,9 +381,11 @@ def test_chunks_run_among_prompt_tiles_only_where_they_take_a_share_of_the_time(
     (8, 64, [2048] * 63 + [0], [1] * 63 + [1985], True),
     (24, 64, [2048] * 20 + [0], [1] * 20 + [2028], True),
     (8, 128, [4096] * 20 + [0], [1] * 20 + [2028], True),
-    (8, 256, [4096] * 20 + [0], [1] * 20 + [2028], False)])                     # (one wave a task)
+    (8, 256, [4096] * 20 + [0], [1] * 20 + [2028], False),                      # (one wave a task)
+    (8, 80, [4096] * 20 + [0], [1] * 20 + [2028], False)])                      # (so with values of 208 columns)
 def test_chunks_stay_behind_tiles_that_would_end_late(kv_heads, head_size, starts, counts, mixed):
     window = 1024 if starts[-1] == 4294 else 0
-    arr, meta = A.plan_step(np.asarray(starts), np.asarray(counts), 4, window, kv_heads=kv_heads, max_waves=8 if head_size <= 192 else 1, head_size=head_size)
+    arr, meta = A.plan_step(np.asarray(starts), np.asarray(counts), 4, window, kv_heads=kv_heads, max_waves=A.max_waves_for(head_size, 208 if head_size == 80 else None),
+                            head_size=head_size)
     chunked = arr[: meta[0]].reshape(-1, 4, 12)[:, 0, 6] >= 0
     assert chunked.any() and bool((np.diff(chunked.astype(int)) < 0).any()) == mixed
