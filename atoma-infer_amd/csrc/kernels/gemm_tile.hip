@@ -668,7 +668,9 @@ constexpr int kCUs = 256;
 
 // Tiles of which a CU can hold two where they go in phases, which is the quicker way once there is more than one for a CU.  One for each CU has
 // its LDS for four buffers: 128 x 64 takes 1.00 to 1.04 times as long in phases then, 128 x 192 with a long end 1.00 to 1.02, and 128 x 128 with
-// residual rows, 0.98 on its own, 1.02 within a prompt's steps.
+// residual rows, 0.98 on its own, 1.02 within a prompt's steps; with other ends 0.95 to 0.98, but beyond kLongSteps steps of K, where the loads set
+// the pace all the way, 1.00 to 1.02 and from 97 on 1.03 (sums, rotary) and 1.04 (SiLU), up to 1.15 (137 products).
+constexpr int kLongSteps = 64;
 static bool two_a_cu(int M, int N, int bm, int bn, int slices) {
   return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * slices > kCUs;
 }
@@ -685,8 +687,7 @@ static int pick(int tile, const void* x, const void* w, int M, int N, int K, int
     case 1: ATOMA_PHASED(256, 128, 4, 2);
     // by four waves, whose larger shares read less LDS, or eight where the end is long, which gain by 2 to 13 percent there
     case 2:
-      if constexpr (EPI == kOutResid)
-        if (!two_a_cu(M, N, 128, 128, slices)) ATOMA_TILE(128, 128, 2, 4, 4);
+      if ((EPI == kOutResid || K / slices / 64 > kLongSteps) && !two_a_cu(M, N, 128, 128, slices)) ATOMA_TILE(128, 128, 2, 4, 4);
       if constexpr (STORES) ATOMA_PHASED(128, 128, 2, 4, 4);
       else ATOMA_PHASED(128, 128, 2, 2);
     case 3:

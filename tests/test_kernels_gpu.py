@@ -1058,6 +1058,52 @@ def test_gemm_tiles_of_which_a_cu_holds_two_equal_the_others(k):
         assert all(torch.equal(a, b) for a, b in zip(want, got)), tile
 
 
+def _tile_results(tile, x, w, kinds, pos, cos, sin, slots, page, nh, nkv, hd, slices=1):
+    """What ``tile`` leaves of x w^T by kind: planes, residual rows, silu(gate) up, or (the rows of w that are its heads') q and both caches."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    m, n, out = x.shape[0], w.shape[0], []
+    if gb.TILE_F32 in kinds:
+        out.append(torch.full((slices, m, n), 7.0, device=DEV))
+        gb.tile_product(x, w, out[-1], gb.TILE_F32, tile, slices)
+    if gb.TILE_RESID in kinds:
+        out.append(rnd(m, n, seed=3))
+        gb.tile_product(x, w, out[-1], gb.TILE_RESID, tile)
+    if gb.TILE_SILU in kinds:
+        out.append(torch.full((m, n // 2), 7.0, dtype=torch.bfloat16, device=DEV))
+        gb.tile_product(x, w, out[-1], gb.TILE_SILU, tile)
+    if gb.TILE_ROPE in kinds:
+        q = torch.full((m, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+        kc = torch.full((-(-m // page) + 2, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
+        vc = kc.clone()
+        gb.tile_product(x, w[: (nh + 2 * nkv) * hd], q, gb.TILE_ROPE, tile, rope=(pos, cos, sin, kc, vc, slots, page, nh, nkv, hd))
+        out += [q, kc, vc]
+    return out
+
+
+def _rope_operands(m, hd, page, seed=5):
+    """Positions in any order, slots of which some are neighbours, some not and some none, and the tables."""
+    g = torch.Generator().manual_seed(seed)
+    pos = torch.randint(0, 90, (m,), generator=g).int().to(DEV)
+    slots = (torch.arange(m) + 5).int()
+    slots[: m // 3] = slots[: m // 3][torch.randperm(m // 3, generator=g)]
+    slots[2::7] = -1
+    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
+    return pos, torch.cos(ang).to(DEV), torch.sin(ang).to(DEV), slots.to(DEV), page
+
+
+@pytest.mark.parametrize("m,nh,nkv", [(300, 3, 1), (1100, 80, 8)])
+@pytest.mark.parametrize("k", [4096, 4160, 4224])
+def test_gemm_tile_at_the_steps_from_which_on_one_a_cu_goes_by_steps(k, m, nh, nkv):
+    """64 steps of K in phases, 65 and 66 by steps where there is a workgroup a CU at most: the bits of tiles that always go by steps."""
+    from atoma_infer_amd.kernels import gemm_bf16 as gb
+    hd = 64
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd((nh + 2 * nkv) * hd, k, dtype=torch.bfloat16, seed=2, scale=0.05)
+    rope = (*_rope_operands(m, hd, 16), nh, nkv, hd)
+    for other, kinds in ((4, (gb.TILE_F32, gb.TILE_RESID, gb.TILE_ROPE)), (6, (gb.TILE_SILU,))):
+        for got, want in zip(_tile_results(2, x, w, kinds, *rope), _tile_results(other, x, w, kinds, *rope)):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu", ("clamped_sigmoid", 7.0, 1.702)])
 @pytest.mark.parametrize("m,inter,k", [(1, 2064, 32), (4, 2064, 160), (5, 4096, 2048), (8, 14336, 4096)])
 def test_few_float32_rows_end_in_the_activation(m, inter, k, act):
