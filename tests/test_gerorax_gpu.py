@@ -241,7 +241,7 @@ def test_few_tokens_are_routed_in_one_launch_as_in_two(tokens, experts, top, gro
 def test_one_launch_refuses_what_it_cannot_route():
     from atoma_infer_amd.kernels import ops
     for t, e, top in ((17, 8, 2), (4, 65, 2), (4, 8, 9)):
-        with pytest.raises(Exception):
+        with pytest.raises(ops.KernelError, match="route_few: the kernel refuses these sizes"):
             ops.route_few(torch.zeros(t, e, device=DEV), top)
 
 
