@@ -387,6 +387,50 @@ def test_tied_value_attention_alone(hd, nh, nkv, chunk, rot, page, dtype):
         assert err < (2e-5 if dtype is torch.float32 else 2.5e-2), float(err)
 
 
+@pytest.mark.parametrize("tokens, counts", [(1, [1]), (16, [1] * 16), (16, [9, 7]), (17, [1] * 17)])
+@pytest.mark.parametrize("left, right, slices", [((4, 2, 64), (2, 1, 128, 128), 1), ((16, 8, 64), (8, 4, 64, 128), 2)])
+def test_mixers_side_by_side_in_shared_launches_are_the_branches_apart(left, right, slices, tokens, counts, monkeypatch):
+    """Inner widths and a model width that are multiples of 128, so that both ends of the branches share a launch up to 16 rows (planes of one
+    and of two K slices): outputs, caches and states have the bits of the branches run by themselves, and the scales join the right ones."""
+    from atoma_infer_amd.kernels import gemm_bf16, ops
+    from atoma_infer_amd.parts import GatedDeltaRule, TiedValueAttention
+    from atoma_infer_amd.parts.parallel import ParallelMixer
+    from atoma_infer_amd.weights.random_init import random_tensor
+    width, page, (nh, nkv, hd), bf16 = 256, 16, left, torch.bfloat16
+    part = ParallelMixer([TiedValueAttention(width, nh, nkv, hd, hd ** -0.5, 1e-5, 300.0, hd, chunk=64),
+                          GatedDeltaRule(width, *right, 4, 1e-5, decay_rank=32, gate_rank=32)], [0.7, -1.3], ["left", "right"])
+    _load(part, {n: random_tensor("p." + n, ws, 7, bf16).float() * (20 if n[-2:] in (".q", ".k", ".v", ".o") else 1)
+                 for n, ws in part.weight_specs().items()}, bf16)
+    g = torch.Generator().manual_seed(tokens + hd)
+    starts = [3 * i for i in range(len(counts))]
+    ctx = _ctx(starts, counts, list(range(len(counts))))
+    blocks = 6
+    slots = [(i * blocks + (s + j) // page) * page + (s + j) % page for i, (s, c) in enumerate(zip(starts, counts)) for j in range(c)]
+    bt = torch.arange(len(counts) * blocks, dtype=torch.int32, device=DEV).view(-1, blocks)
+    x = torch.randn(tokens, width, generator=g).to(DEV, bf16)
+    shape = (len(counts) * blocks, nkv, page * hd)
+    kv = [torch.randn(shape, generator=g).to(DEV, bf16) for _ in range(2)]
+    state = torch.randn((len(counts), part.state_spec().shape[0]), generator=g).to(DEV)
+    cache = lambda: types.SimpleNamespace(k=kv[0].clone(), v=kv[1].clone(), page_size=page, writable=True, block_tables=bt, state=state.clone(),
+                                          slot_mapping=torch.tensor(slots, dtype=torch.int32, device=DEV))
+    together, apart, paired, pair = cache(), cache(), [], gemm_bf16.try_pair
+    monkeypatch.setattr(gemm_bf16, "try_pair", lambda *a: paired.append(pair(*a)) or paired[-1])
+    terms = part.forward(x, ctx, together).terms
+    assert [p is not None for p in paired] == ([True, True] if tokens <= 16 else [])
+    want = [b.forward(x, ctx, apart) for b in part.branches]
+    for (got, scale), w, s in zip(terms, want, part.scales):
+        assert scale == s and torch.equal(got, w) and (tokens > 16 or tuple(got.shape) == (slices, tokens, width))
+    for name in ("k", "v", "state"):
+        assert torch.equal(getattr(together, name), getattr(apart, name)) and not torch.equal(getattr(together, name), getattr(cache(), name))
+    total = lambda y: (y.sum(0) if y.dim() == 3 else y).double()
+    ref = sum(total(w.double() if w.dim() == 3 else w) * s for w, s in zip(want, part.scales))
+    resid = torch.zeros(tokens, width, device=DEV)
+    ops.add_normed(resid, terms, None, 0.0)
+    # (a sum of at most four rounded terms)
+    bound = 8 * 2.0 ** -24 * sum((w.double().abs().sum(0) if w.dim() == 3 else w.double().abs()) * abs(s) for w, s in zip(want, part.scales))
+    assert bool(((resid.double() - ref).abs() <= bound).all()) and float(ref.abs().max()) > 0.1
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("edge", [-1, 0])
 def test_a_dominant_key_just_outside_and_just_inside_a_chunk(dtype, edge):
