@@ -590,10 +590,11 @@ def test_routed_experts_by_places(experts, top, width, ff, kw, monkeypatch):
 
 
 @pytest.mark.parametrize("tile", range(4))
-@pytest.mark.parametrize("counts,n,k", [((3, 0, 300), 64, 64), ((128, 257, 1), 288, 192), ((90, 90, 90, 90), 544, 640)])
+@pytest.mark.parametrize("counts,n,k", [((3, 0, 300), 64, 64), ((128, 257, 1), 288, 192), ((90, 90, 90, 90), 544, 640),
+                                        ((0, 1, 63, 65, 128, 129) * 5, 576, 256), ((129, 0, 64, 1, 127) * 5, 608, 320)])
 def test_gemm_tile_groups(tile, counts, n, k):
     """The tile kernel over experts' runs of places: whole, short and empty tiles, both results, against float64 (bounds as in
-    ``test_expert_stream``)."""
+    ``test_expert_stream``); more tiles of 128 x 64 than CUs, which go in phases, with an even and an odd number of steps."""
     from atoma_infer_amd.kernels import gemm_bf16 as gb, ops
     top = 2
     ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)]).int()
@@ -602,6 +603,7 @@ def test_gemm_tile_groups(tile, counts, n, k):
     t = ids.numel()
     x, w, score = rnd(t, k, dtype=torch.bfloat16, seed=2), rnd(len(counts), n, k, dtype=torch.bfloat16, seed=3), rnd(t, seed=4).abs()
     perm, offsets, tiles = ops.route_group(ids, len(counts), gb.TILES[tile][0])
+    assert tile != 3 or (tiles.shape[0] * -(-n // 64) > 256) == (len(counts) > 20)
     expert = ids.long()[perm.long()]            # (of a place)
     want = torch.stack([x[i].double() @ w[expert[i]].double().T for i in range(t)])
     size = torch.stack([x[i].double().abs() @ w[expert[i]].double().abs().T for i in range(t)])
@@ -1006,56 +1008,40 @@ def test_gemm_tile(tile, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (128, 128, 128), (129, 160, 192), (255, 96, 256), (385, 416, 320), (513, 800, 448), (300, 272, 640)])
 def test_gemm_tile_in_phases_equals_the_one_by_steps(m, n, k):
-    """The tiles of 256 x 256 sum in the order of the others, so the bits are theirs: 1 to 7 and 10 steps, in slices too (5 steps), with rows
-    that end in a tile's first or second half."""
+    """The tiles in phases sum in the order of those with one barrier a step (256 x 160, and 64 x 64 for SiLU), so the bits are theirs: 1 to 7
+    and 10 steps, in slices too (5 steps), with rows and columns that end in a tile's first or second half."""
     from atoma_infer_amd.kernels import gemm_bf16 as gb
     x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
+    none = (None,) * 5 + (1, 0, 1)
     for slices in (1, 2):
         if k % (64 * slices) == 0:
-            c = torch.full((2, slices, m, n), 7.0, device=DEV)
-            for i in range(2):
-                gb.tile_product(x, w, c[i], gb.TILE_F32, i, slices)
-            assert torch.equal(c[0], c[1])
-    r = rnd(m, n, seed=3)[None].repeat(2, 1, 1)
-    for i in range(2):
-        gb.tile_product(x, w, r[i], gb.TILE_RESID, i)
-    assert torch.equal(r[0], r[1])
+            kinds = (gb.TILE_F32, gb.TILE_RESID)
+            by_steps = _tile_results(4, x, w, kinds, *none, slices=slices)
+            for tile in (0, 1, 2, 5):
+                assert all(torch.equal(a, b) for a, b in zip(_tile_results(tile, x, w, kinds, *none, slices=slices), by_steps)), tile
     if n % 32 == 0:
-        g = torch.empty(2, m, n // 2, dtype=torch.bfloat16, device=DEV)
-        for i in range(2):
-            gb.tile_product(x, w, g[i], gb.TILE_SILU, i)
-        assert torch.equal(g[0], g[1])
+        by_steps, = _tile_results(6, x, w, (gb.TILE_SILU,), *none)
+        for tile in (0, 1, 2):
+            assert torch.equal(_tile_results(tile, x, w, (gb.TILE_SILU,), *none)[0], by_steps), tile
 
 
 @pytest.mark.parametrize("k", [64, 128, 192, 320])
 def test_gemm_tiles_of_which_a_cu_holds_two_equal_the_others(k):
-    """Tiles of 128 rows with more workgroups than CUs go in phases: sums, residual rows, SiLU and (1,100 rows, 96 heads) q, k, v have the bits
-    of the tile of 256 x 128, with 1, 2, 3 and 5 steps of K and rows and columns that end inside a tile's first half."""
+    """Tiles of 128 rows with more workgroups than CUs go in phases: sums, residual rows, SiLU and (1,100 rows, 96 heads, slots out of order and
+    missing) q, k, v have the bits of tiles with one barrier a step, with 1, 2, 3 and 5 steps of K and rows and columns that end inside a
+    tile's first half."""
     from atoma_infer_amd.kernels import gemm_bf16 as gb
     m, n, nh, nkv, hd, page = 1100, 6176, 80, 8, 64, 16
     x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2)
-    pos = (torch.arange(m) % 90).int().to(DEV)
-    slots = (torch.arange(m) + 3).int().to(DEV)
-    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
-    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
-    r0, want = rnd(m, n, seed=3), None
+    rope = (*_rope_operands(m, hd, page), nh, nkv, hd)
+    kinds = (gb.TILE_F32, gb.TILE_RESID, gb.TILE_ROPE)
+    by_steps, silu = _tile_results(4, x, w, kinds, *rope), _tile_results(6, x, w, (gb.TILE_SILU,), *rope)
     for tile in (1, 2, 3, 5):
         bm, bn = gb.TILES[tile][:2]
         assert tile == 1 or -(-m // bm) * -(-6144 // bn) > 256
-        c, r = torch.full((m, n), 7.0, device=DEV), r0.clone()
-        gb.tile_product(x, w, c, gb.TILE_F32, tile)
-        gb.tile_product(x, w, r, gb.TILE_RESID, tile)
-        q = torch.full((m, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
-        kc = torch.full((m // page + 2, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
-        vc = kc.clone()
-        gb.tile_product(x, w[:6144], q, gb.TILE_ROPE, tile, rope=(pos, cos, sin, kc, vc, slots, page, nh, nkv, hd))
-        got = [c, r, q, kc, vc]
+        assert all(torch.equal(a, b) for a, b in zip(_tile_results(tile, x, w, kinds, *rope), by_steps)), tile
         if tile in gb.TILES_SILU:
-            s = torch.full((m, n // 2), 7.0, dtype=torch.bfloat16, device=DEV)
-            gb.tile_product(x, w, s, gb.TILE_SILU, tile)
-            got.append(s)
-        want = want or got
-        assert all(torch.equal(a, b) for a, b in zip(want, got)), tile
+            assert torch.equal(_tile_results(tile, x, w, (gb.TILE_SILU,), *rope)[0], silu[0]), tile
 
 
 def _tile_results(tile, x, w, kinds, pos, cos, sin, slots, page, nh, nkv, hd, slices=1):
@@ -1323,29 +1309,15 @@ def test_gemm_tile_rope(m, nh, nkv, hd, k, page):
 @pytest.mark.parametrize("m,nh,nkv,hd,k", [(300, 6, 2, 64, 256), (385, 8, 2, 64, 320), (129, 4, 1, 128, 384), (641, 6, 2, 48, 448), (256, 5, 1, 64, 640),
                                            (513, 24, 8, 128, 704)])
 def test_gemm_tile_rope_in_phases_equals_the_one_by_steps(m, nh, nkv, hd, k):
-    """The tile of 256 x 192 sums as the others do, so q, k and v are theirs bit for bit: 4 to 7, 10 and 11 steps of K (none to four turns of
-    its loop behind an even and an odd number), rows that end in a tile's first and second half, columns that do and do not fill the
-    last tile, a padding row, and caches that keep what no token writes."""
+    """The tiles in phases sum as the one with a barrier a step does (256 x 160), so q, k and v are its bit for bit: 4 to 7, 10 and 11 steps of
+    K (none to four turns of their loop behind an even and an odd number), rows that end in a tile's first and second half, columns that do and
+    do not fill the last tile, padding rows, and caches that keep what no token writes."""
     from atoma_infer_amd.kernels import gemm_bf16 as gb
-    page, n = 16, (nh + 2 * nkv) * hd
-    pages = -(-m // page) + 2
-    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd(n, k, dtype=torch.bfloat16, seed=2, scale=0.2)
-    g = torch.Generator().manual_seed(5)
-    pos = torch.randint(0, 90, (m,), generator=g).int().to(DEV)
-    slots = (torch.arange(m) + 5).int()
-    slots[: m // 3] = slots[: m // 3][torch.randperm(m // 3, generator=g)]
-    slots[2] = -1
-    slots = slots.to(DEV)
-    ang = torch.arange(96).float()[:, None] / (10000.0 ** (torch.arange(0, hd, 2).float() / hd))[None]
-    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
-    out = []
-    for tile in (1, 8):
-        q = torch.full((m, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
-        kc = torch.full((pages, nkv, page * hd), 3.0, dtype=torch.bfloat16, device=DEV)
-        vc = kc.clone()
-        gb.tile_product(x, w, q, gb.TILE_ROPE, tile, rope=(pos, cos, sin, kc, vc, slots, page, nh, nkv, hd))
-        out.append((q, kc, vc))
-    assert all(torch.equal(a, b) for a, b in zip(*out))
+    x, w = rnd(m, k, dtype=torch.bfloat16, seed=1), rnd((nh + 2 * nkv) * hd, k, dtype=torch.bfloat16, seed=2, scale=0.2)
+    rope = (*_rope_operands(m, hd, 16), nh, nkv, hd)
+    by_steps = _tile_results(4, x, w, (gb.TILE_ROPE,), *rope)
+    for tile in (1, 2, 8):
+        assert all(torch.equal(a, b) for a, b in zip(_tile_results(tile, x, w, (gb.TILE_ROPE,), *rope), by_steps)), tile
 
 
 def _rms(x, g, eps):
