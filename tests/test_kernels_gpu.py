@@ -1613,8 +1613,64 @@ def test_decode_chunks_that_grow_with_the_context(nh, nkv, hd, starts, chunk, wi
 @pytest.mark.parametrize("nh,nkv,hd,starts,chunk", [(16, 1, 128, [2047, 600, 5], 256), (64, 2, 64, [2000, 1300, 9], 256), (24, 8, 128, [2040, 700], 256),
                                                      (40, 1, 64, [2000, 300, 1], 256), (12, 1, 160, [2000, 31], 256)])
 def test_four_waves_merge_pieces_of_many_rows(nh, nkv, hd, starts, chunk):
-    """As above where a piece's live rows are more than one wave merges in one go, so that all waves of its last chunk share them."""
+    """As above where a piece's live rows are more than one wave merges in one go, so that all waves of its last chunk share them; and the bits
+    of the same heads a few at a time, which one wave merges."""
+    import numpy as np
+    from atoma_infer_amd.kernels import attention_bf16
     test_decode_chunks_that_grow_with_the_context(nh, nkv, hd, starts, chunk, 0)
+    group, page, bucket = nh // nkv, 16, -(-(max(starts) + 1) // 256) * 256
+    _, _, kc, vc, bt = paged_setup([s + 1 for s in starts], nkv, hd, page, torch.bfloat16, seed=hd)
+    wide = torch.zeros((len(starts), bucket // page), dtype=torch.int32, device=DEV)
+    wide[:, : bt.shape[1]] = bt
+    q = (rnd(len(starts), nkv, group, hd, seed=3) * 1.5).bfloat16()
+
+    def attend(q):
+        g = q.shape[2]
+        ctx = FakeCtx(starts, [1] * len(starts))
+        arr, meta = attention_bf16.build_tasks(np.asarray(starts, dtype=np.int32), np.ones(len(starts), dtype=np.int32), g, 0, bucket, kv_heads=nkv,
+                                               max_waves=attention_bf16.max_waves_for(hd), head_size=hd)
+        assert meta[3] == 4 and meta[5] is True and (g * hd > 256) == (g == group)
+        ctx.plans = {attention_bf16.plan_key(g, 0, nkv, hd): (torch.from_numpy(arr).to(DEV), meta)}
+        out = torch.full((len(starts), nkv * g * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert attention_bf16.try_attention(q.reshape(len(starts), -1), kc, vc, out, ctx, FakeCache(wide, page), hd ** -0.5, 0, nkv * g, nkv, hd)
+        return set(map(tuple, arr[: meta[0]][:, [0, 4, 5]].tolist())), out.view(q.shape)
+    chunks, out = attend(q)
+    few = max(1, 256 // hd)
+    for lo in range(0, group, few):
+        part_chunks, part = attend(q[:, :, lo: lo + few].contiguous())
+        assert part_chunks == chunks and torch.equal(part, out[:, :, lo: lo + few])
+
+
+@pytest.mark.parametrize("nh,nkv,hd,decoded,portions", [
+    (32, 8, 64, [20 + 3 * i for i in range(100)] + [1500 + i for i in range(24)], [(0, 1924)]),        # shared workgroups and chunks among the tiles
+    (32, 8, 64, [20 + 2 * i for i in range(150)], [(0, 250)] * 4),                                     # shared workgroups alone
+    (24, 8, 128, [2000 + 7 * i for i in range(20)], [(0, 1500), (0, 500)])])                           # chunks alone
+def test_a_mixed_step_s_tasks_have_the_same_bits_in_any_order(nh, nkv, hd, decoded, portions):
+    """Decoded tokens of several requests in one workgroup, and their chunks among the prompt tiles, as a step's plan deals them, against the
+    builder's order, whose results other tests hold to a plain implementation."""
+    import numpy as np
+    from atoma_infer_amd.kernels import attention_bf16
+    starts = np.asarray(decoded + [s for s, _ in portions], dtype=np.int32)
+    counts = np.asarray([1] * len(decoded) + [c for _, c in portions], dtype=np.int32)
+    group, t = nh // nkv, int(counts.sum())
+    _, _, kc, vc, bt = paged_setup((starts + counts).tolist(), nkv, hd, 16, torch.bfloat16, seed=hd)
+    q = (rnd(t, nh * hd, seed=3) * 1.5).bfloat16()
+    options = dict(kv_heads=nkv, max_waves=attention_bf16.max_waves_for(hd), head_size=hd)
+    plans = [attention_bf16.build_tasks(starts, counts, group, 0, **options), attention_bf16.plan_step(starts, counts, group, 0, **options)]
+    fours = [a[: m[0]].reshape(-1, 4, 12) for a, m in plans]
+    shared = [f[(f[:, 0, 6] < 0) & (f[:, 1, 0] >= 0) & (f[:, 0, 0] != f[:, 1, 0])] for f in fours]
+    assert len(shared[0]) == 0 and (len(shared[1]) > 0) == (decoded[0] < 500)
+    among = [bool((np.diff((f[:, 0, 6] >= 0).astype(int)) < 0).any()) for f in fours]
+    assert among == [False, decoded[-1] > 500]
+    outs = []
+    for arr, meta in plans:
+        ctx = FakeCtx(starts.tolist(), counts.tolist())
+        ctx.plans = {attention_bf16.plan_key(group, 0, nkv, hd): (torch.from_numpy(np.ascontiguousarray(arr)).to(DEV), meta)}
+        for _ in range(2):                             # (the second launch finds the counters as the first left them)
+            out = torch.full((t, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+            assert attention_bf16.try_attention(q, kc, vc, out, ctx, FakeCache(bt, 16), hd ** -0.5, 0, nh, nkv, hd)
+            outs.append(out)
+    assert not bool(outs[0].isnan().any()) and all(torch.equal(o, outs[0]) for o in outs)
 
 
 @pytest.mark.parametrize("plan", PLANS)
