@@ -324,6 +324,30 @@ def _tile_tasks(e: int, start: int, count: int, tok_base: int, group: int, windo
     return lengths, t.reshape(tiles * fours, 4, 12)
 
 
+def _token_tasks(entries: np.ndarray, starts: np.ndarray, tok_bases: np.ndarray, group: int, window: int, row_tiles: int, keep: int):
+    """``_tile_tasks`` of the ``entries`` that bring one token each, all at once, as (entry, keys, tasks) a group of four tasks: a step of many
+    decoded tokens beside prompts spent most of its planning on them one by one (114 of them beside 9 portions 1.8 -> 0.4 ms of the host's)."""
+    piece = 32 * row_tiles
+    pieces = -(-group // piece)
+    fours = -(-pieces // 4)
+    pos = starts[entries].astype(np.int64)
+    kb, k_end = walk(pos, pos + 1, window, keep)
+    t = np.empty((len(entries), fours * 4, 12), dtype=np.int32)
+    t[:] = _NULL_TASK
+    body = t[:, :pieces]
+    body[..., 0] = entries[:, None]
+    body[..., 1] = 0
+    body[..., 2] = 1
+    body[..., 3] = piece * np.arange(pieces)
+    body[..., 4] = kb[:, None]
+    body[..., 5] = k_end[:, None]
+    body[..., 8] = tok_bases[entries][:, None]
+    body[..., 9] = 1
+    body[..., 10] = pos[:, None]
+    body[..., 11] = row_tiles
+    return np.repeat(entries, fours), np.repeat(k_end - kb, fours), t.reshape(-1, 4, 12)
+
+
 def _serpentine(n: int, kv_heads: int, compute_units: int, head_size: int = 64) -> np.ndarray:
     """The order of n groups of tasks, given longest first: the GPU takes a workgroup per (group, KV head) to its
     CUs in turn, and with head sizes up to 64 two workgroups share a CU.  So the groups of one round over all CUs
@@ -377,32 +401,37 @@ def build_tasks(starts: np.ndarray, counts: np.ndarray, group: int, window: int,
     direct_arrays = []
     n_part = 0
 
-    def splits(e):
-        first = int(first_key(int(starts[e]), window))
-        end = int(starts[e]) + int(counts[e])
-        if keep:
-            first, end = (int(v) for v in walk(int(starts[e]), end, window, keep))
-        return bucket is not None or (int(counts[e]) <= SPLIT_MAX_TOKENS and end - first >= SPLIT_MIN_KEYS)
-
-    split_entries = [e for e in range(len(starts)) if splits(e)]
+    ends = starts.astype(np.int64) + counts
+    firsts = first_key(starts.astype(np.int64), window)
+    if keep:
+        firsts, ends = walk(starts.astype(np.int64), ends, window, keep)
+    whole = (counts > SPLIT_MAX_TOKENS) | (ends - firsts < SPLIT_MIN_KEYS)
+    if bucket is not None:
+        whole[:] = False
+    split_entries = (~whole).nonzero()[0]
     chunk, waves, merge = CHUNK, 1, False
-    if split_entries:
+    if len(split_entries):
         most = bucket if bucket is not None else max(int(starts[e]) + int(counts[e]) for e in split_entries)
         if bucket is not None and window != 0:
             most = min(most, abs(window) + CHUNK + keep)
         chunk, waves = chunk_for(len(split_entries), most, kv_heads)
         waves = min(waves, max_waves)
         merge = merges_in_kernel(most)
-    for e in range(len(starts)):
+    if vectorized:
+        # (one token each, not split: built together)
+        tokens = (whole & (counts == 1)).nonzero()[0]
+        if len(tokens):
+            direct_arrays.append(_token_tasks(tokens, starts, tok_bases, group, window, row_tiles, keep))
+    for e in ((counts != 1) | ~whole).nonzero()[0].tolist() if vectorized else range(len(starts)):
         start, count = int(starts[e]), int(counts[e])
         qt = min(qt_max, count)
         rows = qt * group
-        do_split = splits(e)
+        do_split = not whole[e]
         tail = (int(tok_bases[e]), count, start, 0)
         if vectorized and not do_split:
             lengths, groups = _tile_tasks(e, start, count, int(tok_bases[e]), group, window, qt, row_tiles,
                                           keep)
-            direct_arrays.append((lengths, groups))
+            direct_arrays.append((np.full(len(lengths), e), lengths, groups))
             continue
         for tok0 in range(0, count, qt):
             last = min(tok0 + qt, count)
@@ -435,9 +464,8 @@ def build_tasks(starts: np.ndarray, counts: np.ndarray, group: int, window: int,
                     wave_tasks.append(null)
                 direct.append((k_end - kb, wave_tasks))
     if direct_arrays:
-        lengths = np.concatenate([l for l, _ in direct_arrays])
-        groups = np.concatenate([g for _, g in direct_arrays])                 # [n, 4, 12]
-        order = np.argsort(-lengths, kind="stable")
+        of, lengths, groups = (np.concatenate(x) for x in zip(*direct_arrays))        # (groups: [n, 4, 12])
+        order = np.lexsort((of, -lengths))                                            # (of one length in the entries' order)
         head = groups[order[_serpentine(len(order), kv_heads, compute_units, head_size)]].reshape(-1, 12)
     else:
         direct.sort(key=lambda x: -x[0])
@@ -520,48 +548,50 @@ def _deal(main: np.ndarray, kv_heads: int, head_size: int, compute_units: int, w
     dealt 0.88 in the geometric mean, 1.8 percent of the steps more than 2 percent slower and two of 1,138 more than 5 (of the steps left
     as they are, the same launch twice, 1.0 percent and three).  Dealt wherever there are more workgroups than the GPU takes, chunks
     wherever they are 0.3 of the tiles' time: 7.9 percent of the steps and 73, up to 1.42 times as long."""
-    groups = main.reshape(-1, 4, 12)
+    groups = main.reshape(-1, 48)                  # (a row: four tasks of twelve numbers; all of a tile's walk the same keys)
     round_ = max(1, compute_units * (2 if head_size <= 64 else 1) // kv_heads)       # groups that the GPU takes at once
     if len(groups) <= round_:
         return None
-    chunked = groups[:, 0, 6] >= 0
-    blocks = (groups[..., 5] - groups[..., 4]) / 32 * (groups[..., 0] >= 0)
-    single = ~chunked & (groups[:, 0, 0] >= 0) & (groups[:, 1:, 0] < 0).all(1)
-    if not _pays_to_share(blocks.max(1), chunked, single, round_):
-        single[:] = False
-    tiles = groups[~chunked & ~single]
-    walks = blocks[~chunked & ~single].max(1, initial=0)
-    order = np.argsort(-walks, kind="stable")
-    few = groups[single, 0]
-    few = few[np.argsort(few[:, 4] - few[:, 5], kind="stable")]
-    few = np.concatenate([few, np.tile(_NULL_TASK, (-len(few) % 4, 1))]).reshape(-1, 4, 12)
-    chunks = groups[chunked]
-    if len(chunks) and waves >= 2 and kv_heads % 8 == 0 and _pays_to_mix(
-            walks[order], blocks[~chunked & ~single].sum(), blocks[chunked | single].sum(), round_):
-        tiles, others = tiles[order], np.concatenate([few, chunks])
-        # (spread evenly: the i-th of n comes i / n of the way)
-        at = np.concatenate([np.arange(len(tiles)) / len(tiles), (np.arange(len(others)) + 0.5) / len(others)])
-        return np.concatenate([tiles, others])[np.argsort(at, kind="stable")].reshape(-1, 12)
-    if not len(few):
+    live = groups[:, ::12] >= 0
+    blocks = (groups[:, 5] - groups[:, 4]) / 32
+    whole = int((groups[:, 6] < 0).sum())          # (chunks stand behind the others)
+    single = live[:whole, 0] & ~live[:whole, 1:].any(1)
+    singles = single.nonzero()[0]
+    if not _pays_to_share(blocks[:whole], single, singles, len(groups), round_):
+        singles = singles[:0]
+    tiles = np.delete(np.arange(whole), singles) if len(singles) else np.arange(whole)
+    tiles = tiles[np.argsort(-blocks[tiles], kind="stable")]
+    fours = -(-len(singles) // 4)
+    few = np.empty((fours * 4, 12), dtype=np.int32)
+    few[: len(singles)] = groups[singles[np.argsort(-blocks[singles], kind="stable")], :12]
+    few[len(singles):] = _NULL_TASK
+    few = few.reshape(fours, 48)
+    if whole < len(groups) and waves >= 2 and kv_heads % 8 == 0:
+        work = (groups[:, 5::12] - groups[:, 4::12]).sum(1) / 32       # (an empty task walks nothing)
+        at_tiles = work[tiles].sum()
+        if _pays_to_mix(blocks[tiles], at_tiles, work.sum() - at_tiles, round_):
+            others = np.concatenate([few, groups[whole:]])
+            # (spread evenly: the i-th of n comes i / n of the way)
+            at = np.concatenate([np.arange(len(tiles)) / len(tiles), (np.arange(len(others)) + 0.5) / len(others)])
+            return np.concatenate([groups[tiles], others])[np.argsort(at, kind="stable")].reshape(-1, 12)
+    if not fours:
         return None
-    tiles = np.concatenate([tiles, few])
-    lengths = np.concatenate([walks, (few[..., 5] - few[..., 4]).max(1) / 32])
-    order = np.argsort(-lengths, kind="stable")[_serpentine(len(tiles), kv_heads, compute_units, head_size)]
-    return np.concatenate([tiles[order], chunks]).reshape(-1, 12)
+    lengths = np.concatenate([blocks[tiles], (few[:, 5] - few[:, 4]) / 32])
+    order = np.argsort(-lengths, kind="stable")[_serpentine(len(lengths), kv_heads, compute_units, head_size)]
+    return np.concatenate([np.concatenate([groups[tiles], few])[order], groups[whole:]]).reshape(-1, 12)
 
 
-def _pays_to_share(walks: np.ndarray, chunked: np.ndarray, single: np.ndarray, round_: int) -> bool:
+def _pays_to_share(walks: np.ndarray, single: np.ndarray, singles: np.ndarray, groups: int, round_: int) -> bool:
     """Whether groups of a single task (a decoded token of few keys) share workgroups, four of a length: alone each keeps six of its eight
     waves idle.  Where there are two rounds and more (0.83 of the time over 418 steps, 1.04 at most); and where one round is left and no such
     task walks further than the tiles do (0.93 over 49, 1.02 at most).  Else there is little to gain, and a workgroup of four long walks may
     be the last to end: 0.97 over 281, but 20 of them more than 2 percent slower (29 tokens of 511 keys beside tiles of 204, 16 heads over one
     KV head, 16.6 -> 20.9 us; three short entries, which fill nothing, 5.8 -> 6.1)."""
-    n = len(walks)
-    if not single.any():
+    if not len(singles):
         return False
-    shared = n - int(single.sum()) * 3 // 4
-    tiles = walks[~chunked & ~single].max(initial=0)
-    return n >= 2 * round_ or (shared <= round_ and walks[single].max() <= tiles)
+    if groups >= 2 * round_:
+        return True
+    return groups - len(singles) * 3 // 4 <= round_ and walks[singles].max() <= walks[~single].max(initial=0)
 
 
 def _pays_to_mix(walks: np.ndarray, tile_blocks: float, other_blocks: float, round_: int) -> bool:

@@ -389,3 +389,15 @@ def test_chunks_stay_behind_tiles_that_would_end_late(kv_heads, head_size, start
                             head_size=head_size)
     chunked = arr[: meta[0]].reshape(-1, 4, 12)[:, 0, 6] >= 0
     assert chunked.any() and bool((np.diff(chunked.astype(int)) < 0).any()) == mixed
+
+
+@pytest.mark.parametrize("group,window,keep,row_tiles", [(4, 0, 0, 1), (1, 700, 0, 1), (40, 0, 0, 2), (8, -512, 0, 1), (3, 600, 20, 1), (130, 0, 0, 1)])
+def test_entries_of_one_token_built_together_are_those_built_one_by_one(group, window, keep, row_tiles):
+    """Beside portions, splits and each other, in any order: the same records in the same order (longest first, then the entries')."""
+    rng = np.random.default_rng(group)
+    for s in (1, 2, 30, 150):
+        counts = rng.choice([1, 1, 1, 2, 16, 90], size=s).astype(np.int32)
+        starts = rng.choice([0, 5, 31, 32, 300, 510, 512, 20000], size=s).astype(np.int32)
+        options = dict(kv_heads=8, max_waves=8, head_size=64, keep=keep, row_tiles=row_tiles)
+        (a, ma), (b, mb) = (A.build_tasks(starts, counts, group, window, None, vectorized, **options) for vectorized in (True, False))
+        assert ma == mb and np.array_equal(a, b)
