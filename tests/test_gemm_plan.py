@@ -108,7 +108,7 @@ LIBRARY_QUICKER = [(T_RESID, 65, 5120, 5120, 35.2, 48.1), (T_RESID, 80, 8192, 81
 TILES_QUICKER = [(T_SILU, 2048, 16384, 2048, 127.5, 114.8), (T_SILU, 200, 16384, 2048, 33.9, 24.9), (T_ROPE, 2048, 3072, 2048, 38.1, 32.8),
                  (T_RESID, 128, 4096, 14336, 80.9, 37.8), (T_RESID, 200, 3072, 8192, 42.6, 29.5), (T_F32, 128, 4096, 4096, 30.3, 18.4),
                  (T_SILU, 2600, 16384, 4096, 410.4, 276.0), (T_RESID, 2048, 3584, 18944, 365.7, 222.8), (T_F32, 2048, 4096, 11008, 178.9, 158.1),
-                 (T_RESID, 2048, 4096, 14336, 217.5, 195.9)]
+                 (T_RESID, 2048, 4096, 14336, 217.5, 195.9), (T_SILU, 1368, 16384, 3072, 137.4, 128.9), (T_SILU, 2594, 8192, 2560, 146.6, 108.2)]
 
 
 def test_tile_rule_where_one_side_is_much_the_quicker():
