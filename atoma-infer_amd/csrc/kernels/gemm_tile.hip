@@ -409,7 +409,7 @@ gemm_tile_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
 // Two buffers instead of three or four also leave half of a CU's LDS to a second workgroup where a tile has 128 rows: one workgroup's first
 // loads and its results then pass under the other's products, and a barrier holds up half of a CU's waves.  Against tiles of the same 256 or
 // 128 rows with one barrier a step, four buffers and a workgroup a CU (some 18,000 products; geometric means of the time, by workgroups
-// a CU up to one / more): 128 x 128 0.95 to 0.98 / 0.84 to 0.89, 256 x 128 0.97 / 0.98, 128 x 192 against 256 x 96 0.92 to 0.97 / 0.85 to
+// a CU up to one / more): 128 x 128 0.95 to 0.98 (see kLongSteps) / 0.84 to 0.89, 256 x 128 0.97 / 0.98, 128 x 192 against 256 x 96 0.92 to 0.97 / 0.85 to
 // 0.88, 128 x 64 1.01 / 0.83 to 0.88 (so only there).  us, before / now: q, k, v of 2,048 rows against 3,072 x 2,048 35.9 / 33.0 (one round
 // of 128 x 192, which keeps one barrier a step: 31.1), two slices of 2,048 x 8,192 69.0 / 65.3.  (192 x 128, patches of eight rows of tiles and 128 x 160 gave nothing; 256 x 160 by halves of 80 lost 1 %.)
 // EU: waves a SIMD that the registers are to leave room for (four: two workgroups of eight waves).
@@ -456,7 +456,8 @@ __device__ __forceinline__ void phase(const bf16x8 (&w)[JW][2], const bf16x8 (&x
 }
 #endif
 
-// Two steps or more; ODD: their number is (a kernel that takes either spills registers).
+// Two steps or more; ODD: their number is (a kernel that takes either spills registers; of these only 128 x 192 with the rotary end, whose four waves
+// a SIMD leave 128, does: one a lane, outside the loop).
 template <typename C, int EPI, bool GROUPED, bool ODD>
 __global__ void __launch_bounds__(64 * C::NW, C::EU)
 gemm_phased_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int rows, int N, int ldx, int ldw, int k_len,
@@ -671,6 +672,7 @@ constexpr int kCUs = 256;
 // residual rows, 0.98 on its own, 1.02 within a prompt's steps; with other ends 0.95 to 0.98, but beyond kLongSteps steps of K, where the loads set
 // the pace all the way, 1.00 to 1.02 and from 97 on 1.03 (sums, rotary) and 1.04 (SiLU), up to 1.15 (137 products).
 constexpr int kLongSteps = 64;
+// (kernels/gemm_bf16.py: _rounds counts with the same line)
 static bool two_a_cu(int M, int N, int bm, int bn, int slices) {
   return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * slices > kCUs;
 }
