@@ -125,6 +125,15 @@ def test_tiles_of_256_by_256_where_they_are_the_quicker_ones(kind, m, n, k, wide
     assert gemm_bf16.tile_plan(m, n, k, kind, True)[:2] == ((0, slices) if wide_us < other_us else other)
 
 
+# us of both products of ``tokens`` rows for each of ``top`` of ``experts`` chosen at random, by the plan and by the one in its place
+@pytest.mark.parametrize("tokens, experts, top, width, inter, plan, us, other, other_us", [
+    (196, 8, 4, 6144, 3072, (128, 2, 2), 315.4, (128, 3, 3), 405.8), (767, 4, 1, 2560, 3072, (128, 2, 2), 68.0, (128, 3, 2), 81.4),
+    (976, 4, 1, 4096, 2560, (128, 2, 2), 136.1, (128, 3, 2), 160.4), (1296, 4, 1, 4096, 14336, (256, 0, 1), 732.0, (128, 2, 3), 905.6),
+    (382, 16, 4, 3072, 1536, (128, 2, 2), 173.2, (128, 3, 3), 206.6)])
+def test_experts_plans_count_tiles_of_128_by_64_by_whole_rounds(tokens, experts, top, width, inter, plan, us, other, other_us):
+    assert us < other_us and gemm_bf16.tile_groups_plan(tokens * top, experts, 2 * inter, width, width, inter) == plan != other
+
+
 def test_few_rows_plans_count_what_their_reader_pays_for_a_plane():
     """41 to 64 rows: sizes where more planes were measured slower than fewer, or than the streaming kernel's (None), and sizes where
     they are the quicker ones; beyond 64 rows no slice of more than 1,536 values of K."""
