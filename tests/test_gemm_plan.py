@@ -129,8 +129,8 @@ def test_tiles_of_256_by_256_where_they_are_the_quicker_ones(kind, m, n, k, wide
 @pytest.mark.parametrize("tokens, experts, top, width, inter, plan, us, other, other_us", [
     (196, 8, 4, 6144, 3072, (128, 2, 2), 315.4, (128, 3, 3), 405.8), (767, 4, 1, 2560, 3072, (128, 2, 2), 68.0, (128, 3, 2), 81.4),
     (976, 4, 1, 4096, 2560, (128, 2, 2), 136.1, (128, 3, 2), 160.4), (1296, 4, 1, 4096, 14336, (256, 0, 1), 732.0, (128, 2, 3), 905.6),
-    (382, 16, 4, 3072, 1536, (128, 2, 2), 173.2, (128, 3, 3), 206.6)])
-def test_experts_plans_count_tiles_of_128_by_64_by_whole_rounds(tokens, experts, top, width, inter, plan, us, other, other_us):
+    (382, 16, 4, 3072, 1536, (128, 2, 2), 173.2, (128, 3, 3), 206.6), (679, 16, 8, 5120, 8192, (256, 0, 1), 1904.4, (128, 2, 2), 2225.6)])
+def test_experts_plans_count_rounds_as_their_tiles_take_them(tokens, experts, top, width, inter, plan, us, other, other_us):
     assert us < other_us and gemm_bf16.tile_groups_plan(tokens * top, experts, 2 * inter, width, width, inter) == plan != other
 
 
